@@ -211,6 +211,11 @@ def prepare(case, seed):
                           page_size=PAGE, prefill_chunk_size=PORTION, num_pages=pages, cuda_graphs=False)
     runner = Runner.from_random(config_of(case), seed, options, std=0.02, norm_jitter=0.1)
     if case["new"]:
+        # as start-up does: the largest decode step once kernel by kernel, then its graph
+        seqs = [runner.open(r) for r in range(case["requests"])]
+        runner.step([StepEntry(seq, [0], [0]) for seq in seqs])
+        for seq in seqs:
+            runner.close(seq)
         runner.enable_graphs(case["requests"], max(len(t) for t in texts))
         runner.capture_graphs([case["requests"]])
     logits = torch.empty((sum(want for step in steps for *_, want in step), VOCAB), dtype=torch.float32, device="cuda:0")
