@@ -16,6 +16,7 @@
 #include "common.h"
 
 #define ATT_WAVES 4
+#define ATT_BATCH 8
 
 template <typename T>
 struct Vec8;  // eight consecutive elements, loaded as wide as the type allows
@@ -99,6 +100,9 @@ __global__ void paged_attention_kernel(T* __restrict__ out, const T* __restrict_
       if (head_dim & 7) {  // a head that is no whole number of 16-byte pieces: element by element
         for (int d = 0; d < head_dim; ++d) dot = fmaf(qbuf[d], to_float(kr[d]), dot);
       } else {
+        // (loads of 64 elements of the key go out together: with the loop rolled a lane waited for memory
+        // at every eight)
+#pragma unroll 8
         for (int d = 0; d < head_dim; d += 8) dot = Vec8<T>::dot(qbuf + d, kr + d, dot);
       }
       s = dot * scale;
@@ -118,20 +122,33 @@ __global__ void paged_attention_kernel(T* __restrict__ out, const T* __restrict_
 #pragma unroll
     for (int i = 0; i < DIMS_PER_LANE; ++i) acc[i] *= corr;
     const int count = (pos - base + 1 < PYLON_WAVE) ? pos - base + 1 : PYLON_WAVE;
-    for (int kk = 0; kk < count; ++kk) {
-      const float pk = __shfl(p, kk, PYLON_WAVE);
-      const int physk = __shfl(phys, kk, PYLON_WAVE);
-      // values transposed inside their page: [page, kv head, element, slot in page]
-      const T* vr = v_transposed
-                        ? v_cache + (static_cast<size_t>(physk / page_size) * n_kv_heads + kvh) * v_dim * page_size +
-                              physk % page_size
-                        : v_cache + (static_cast<size_t>(physk) * n_kv_heads + kvh) * v_row;
-      const size_t vstep = v_transposed ? page_size : 1;
+    // values transposed inside their page: [page, kv head, element, slot in page]
+    const size_t vstep = v_transposed ? page_size : 1;
+    // Eight keys' values are sent for before the first is used (a wave otherwise waits out a trip to
+    // memory per key: float32, 32 heads of 128, steps of 3 and 270 tokens of about 110 keys together 107 -> 36
+    // us a launch); the sums keep their order.
+    for (int k0 = 0; k0 < count; k0 += ATT_BATCH) {
+      float pk[ATT_BATCH], vv[ATT_BATCH][DIMS_PER_LANE];
 #pragma unroll
-      for (int i = 0; i < DIMS_PER_LANE; ++i) {
-        const int d = lane + PYLON_WAVE * i;
-        if (d < v_dim) acc[i] = fmaf(pk, to_float(vr[d * vstep]), acc[i]);
+      for (int u = 0; u < ATT_BATCH; ++u) {
+        const int kk = k0 + u < count ? k0 + u : count - 1;
+        pk[u] = __shfl(p, kk, PYLON_WAVE);
+        const int physk = __shfl(phys, kk, PYLON_WAVE);
+        const T* vr = v_transposed
+                          ? v_cache + (static_cast<size_t>(physk / page_size) * n_kv_heads + kvh) * v_dim * page_size +
+                                physk % page_size
+                          : v_cache + (static_cast<size_t>(physk) * n_kv_heads + kvh) * v_row;
+#pragma unroll
+        for (int i = 0; i < DIMS_PER_LANE; ++i) {
+          const int d = lane + PYLON_WAVE * i;
+          vv[u][i] = d < v_dim ? to_float(vr[d * vstep]) : 0.f;
+        }
       }
+#pragma unroll
+      for (int u = 0; u < ATT_BATCH; ++u)
+        if (k0 + u < count)
+#pragma unroll
+          for (int i = 0; i < DIMS_PER_LANE; ++i) acc[i] = fmaf(pk[u], vv[u][i], acc[i]);
     }
     m = m_new;
   }

@@ -1,9 +1,10 @@
-// out[M, N] = a[M, K] * w[N, K]^T with float accumulation on the vector ALUs (no matrix
-// cores, no reduced-precision mode): the matrix product of the true 32-bit path, and
-// the fallback for element type pairings the fast kernels do not take.  Each output
-// element is one chain of fused multiply-adds over k = 0..K-1 in ascending order, so its
-// value does not depend on M, on the tile it falls in, or on what else is in the batch.
+// out[M, N] = a[M, K] * w[N, K]^T with float accumulation and no reduced-precision mode.  float32
+// operands with 16-byte aligned rows go to gemm_f32.hip; the kernel here, on the vector ALUs, is for
+// the element type pairings and alignments that no fast kernel takes.  Each output element is one
+// chain of fused multiply-adds over k = 0..K-1 in ascending order, so its value does not depend on
+// M, on the tile it falls in, or on what else is in the batch.
 #include "common.h"
+#include "gemm_f32.h"
 
 #define GT_BM 64
 #define GT_BN 64
@@ -83,6 +84,9 @@ extern "C" int pylon_gemm_tiled(void* out, int out_dtype, const void* a, int a_d
   PYLON_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_tiled: a leading dimension is too short");
   if (M == 0) return 0;
   PYLON_REQUIRE((M + GT_BM - 1) / GT_BM <= 65535, "gemm_tiled: M=%d is too large for one launch", M);
+  if (out_dtype == PYLON_F32 && a_dtype == PYLON_F32 && w_dtype == PYLON_F32 && gemm_f32_takes(a, w, K, lda, ldw) &&
+      gemm_f32_launch((float*)out, (const float*)a, (const float*)w, M, N, K, lda, ldw, ldc, stream))
+    PYLON_LAUNCHED("gemm_f32");
   const int key = a_dtype * 100 + w_dtype * 10 + out_dtype;
   switch (key) {
     case 0:  // f32 f32 f32

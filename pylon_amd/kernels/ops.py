@@ -1276,7 +1276,8 @@ def attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
 
 def gemm_tiled(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.dtype] = None,
                out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """``x @ weight.T`` with float accumulation on the vector units (no matrix cores)."""
+    """``x @ weight.T`` with float accumulation and full-precision products: float32 operands with
+    16-byte aligned rows on the float32 matrix instruction, everything else on the vector units."""
     if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
         raise KernelError(f"gemm: cannot multiply {tuple(x.shape)} by the transpose of {tuple(weight.shape)}")
     m, k = x.shape
