@@ -1,0 +1,431 @@
+// out[M, N] = x[M, K] * w[N, K]^T in bfloat16 for the many rows of prompt portions, on the matrix
+// cores, with the activation of a feed-forward on the float sums before they are rounded: the products
+// of a prompt step, bound by the matrix cores where the rows are many and by moving w where they are few.
+//
+// Four wavefronts a workgroup, two by two, each a quarter of a tile of 64 to 256 rows by 64 to 256
+// columns in accumulators.  K is walked in chunks of 64 elements; both operands of a chunk go from
+// memory straight into LDS (buffer_load_dwordx4 ... lds: eight whole 128-byte row segments a load;
+// segments of 64 bytes, chunks of 32, were a quarter slower).  In LDS piece q of row R (16 bytes)
+// lies at place q ^ (R & 7) of its row, so that operand reads are free of bank conflicts.
+//
+// A chunk is two turns of matrix instructions.  While a turn multiplies, the operands of the next one
+// leave LDS and a part of a later chunk's loads is sent, one read or load every few matrix instructions
+// (the order is fixed with sched_barrier; with all loads of a chunk sent at once a wave stands for the
+// 700 clocks that the loads of four waves take to be accepted).  One barrier a chunk, between its turns,
+// behind a counted wait: the next chunk has landed, and nobody reads this one's place any more.
+//
+// Two ways to lay chunks out in LDS.  STAGES > 0: that many stages of x and w, as many as fit.
+// STAGES = 0 (square tiles): a ring of five places, each x or w of one chunk; two and a half chunks of a
+// 256 x 256 tile fill the 160 KB, where two stages keep too few bytes in flight for the latency of
+// memory (2048 rows, gate/up 2 x 12288 x 4096: 346 -> 307 us).
+//
+// Which tile: gw_choose, by a model of the launch's rounds over the compute units.  A layer of a prompt step,
+// library products and activation kernel before, gate/up here after (us, in whole steps): 4B sizes at 250,
+// 600, 1024, 1600, 2048 tokens 195, 262, 352, 482, 567 -> 176, 253, 347, 438, 519; 8B sizes 263, 401, 502, 828,
+// 794 -> 248, 390, 488, 810, 773; 32B sizes at 1024 and 2048 1218, 1829 -> 1138, 1775.  The products without an
+// activation: plan.wide_beats_library.  256 x 256 tiles multiply at 1.45 PFLOP/s (2048 x 2 x 12288 x 4096 in 285
+// us with its activation; with loads and LDS reads left out the loop reaches 1.7).
+//
+// A kernel's code has to stay small: two compute units share 64 KB of instruction cache.  Results stored with
+// an unrolled fallback for odd widths, software rounding and a peeled first chunk (55 to 87 KB of code instead
+// of 14 to 37) cost 15 % of a step's launches, though nothing of launches back to back.
+#include "common.h"
+
+#include <type_traits>
+#include <utility>
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+#define GW_LDS(T) __attribute__((address_space(3))) T
+#define GW_CHUNK 64
+#define GW_ROW_BYTES 128
+#define GW_PLACES 5  // of the ring of square tiles
+
+// What happens to the sums: nothing; act(gate) * up of a fused gate/up matrix; max(v, 0)^2.
+enum GwEpilogue { GW_PLAIN = 0, GW_SILU = 1, GW_RELU2 = 2, GW_GELU = 3, GW_CAPPED = 4 };
+
+template <int V>
+using Int = std::integral_constant<int, V>;
+template <typename F, int... I>
+__device__ __forceinline__ void gw_for_(F&& f, std::integer_sequence<int, I...>) {
+  (f(Int<I>{}), ...);
+}
+// f(0), f(1), ... f(N - 1) with the number a constant each time.
+template <int N, typename F>
+__device__ __forceinline__ void gw_for(F&& f) {
+  gw_for_(f, std::make_integer_sequence<int, N>{});
+}
+
+// All but the N loads sent last have landed, this wave's LDS reads have returned, and every wave is here.
+// (A fence would wait for every load, because the loads write LDS.)
+template <int N>
+__device__ __forceinline__ void gw_sync() {
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+struct GwShape {
+  int M, N, K;
+  long long ldx, ldw, ldo;
+  int m_tiles, n_tiles;
+  float alpha, offset, limit;  // of the capped gate
+  int epilogue;
+};
+
+// Gates of results that are about to be rounded to bfloat16: the hardware's exponential and reciprocal (about
+// one part in 2^22 each).
+__device__ __forceinline__ float gw_sigmoid_times(float z, float slope) {  // z / (1 + exp(-slope z))
+  return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * slope * z));
+}
+__device__ __forceinline__ float gw_gelu(float z) {  // pylon_gelu_tanh
+  const float u = 1.5957691216057308f * fmaf(0.044715f * z * z, z, z);
+  return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * u));
+}
+__device__ __forceinline__ float gw_capped(float g, float u, const GwShape& p) {
+  if (p.limit > 0.f) {
+    g = fminf(g, p.limit);
+    u = fminf(fmaxf(u, -p.limit), p.limit);
+  }
+  return gw_sigmoid_times(g, p.alpha) * (u + p.offset);
+}
+
+// MT, NT: tiles of 16 rows and of 16 columns per wave.  GATED: w is a fused matrix of 2 N rows, gate rows
+// first; a pair of a wave's column tiles is 16 gate rows and their 16 up rows, N rows further down.
+// (The body is a device function: the host pass does not know the descriptor type and would drop a kernel
+// that names it, launch stub and all.)
+template <int MT, int NT, int STAGES, bool GATED>
+__device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
+                                               const uint16_t* __restrict__ w, const GwShape p) {
+  constexpr bool RING = STAGES == 0;
+  static_assert(!RING || MT == NT, "the ring's places hold x or w");
+  static_assert(!GATED || NT % 2 == 0, "a gate tile and its up tile belong to one wave");
+  constexpr int TM = 32 * MT, TN = 32 * NT;
+  constexpr int XL = TM / 32, WL = TN / 32, LOADS = XL + WL;  // loads a wave sends per chunk
+  constexpr int STAGE_BYTES = (TM + TN) * GW_ROW_BYTES, PLACE_BYTES = TM * GW_ROW_BYTES;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[RING ? GW_PLACES * PLACE_BYTES : STAGES * STAGE_BYTES];
+
+  // Every eighth workgroup runs on one die: a die gets consecutive tiles, rows of tiles fastest, so that
+  // its cache serves most of what its workgroups read.
+  const int tiles = p.m_tiles * p.n_tiles, per_die = (tiles + 7) >> 3;
+  const int id = (blockIdx.x & 7) * per_die + (blockIdx.x >> 3);
+  if (static_cast<int>(blockIdx.x >> 3) >= per_die || id >= tiles) return;
+  constexpr int DEEP = TM >= 256 ? 8 : 16;  // tile rows walked together
+  const int deep_tiles = DEEP * p.n_tiles, stripe = id / deep_tiles, within = id - stripe * deep_tiles;
+  const int deep = p.m_tiles - stripe * DEEP < DEEP ? p.m_tiles - stripe * DEEP : DEEP;
+  const int m0 = (stripe * DEEP + within % deep) * TM, n0 = within / deep * (GATED ? TN / 2 : TN);
+
+  const int lane = threadIdx.x & (PYLON_WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PYLON_WAVE);
+  const int r = lane & 15, g = lane >> 4, wm = wave & 1, wn = wave >> 1;
+  const int chunks = p.K / GW_CHUNK;
+  const uint16_t* xt = x + static_cast<size_t>(m0) * p.ldx;
+  const uint16_t* wt = w + static_cast<size_t>(n0) * p.ldw;
+
+  // Load i of wave v brings rows 8 (v XL + i) .. + 7 of the tile.  Rows beyond M or N are read as the last
+  // one (their results go nowhere).
+  unsigned x_at[XL], w_at[WL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int row = 8 * (wave * XL + i) + (lane >> 3);
+    const int at = m0 + row < p.M ? row : p.M - 1 - m0;
+    x_at[i] = static_cast<unsigned>(at) * static_cast<unsigned>(p.ldx) * 2u + ((lane & 7) ^ (row & 7)) * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < WL; ++i) {
+    const int row = 8 * (wave * WL + i) + (lane >> 3);
+    int at = GATED ? (row >> 5) * 16 + (row & 15) : row;
+    at = n0 + at < p.N ? at : p.N - 1 - n0;
+    if (GATED && (row & 16)) at += p.N;
+    w_at[i] = static_cast<unsigned>(at) * static_cast<unsigned>(p.ldw) * 2u + ((lane & 7) ^ (row & 7)) * 16;
+  }
+  // Beyond K the descriptor spans nothing: the load fetches nothing, and every count of loads stays exact.
+  auto rows_of = [&](bool is_x, int chunk) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(is_x ? xt : wt), 0, chunk < chunks ? 0x7fffffff : 0,
+                                             0x00020000);
+  };
+  auto load = [&](__amdgpu_buffer_rsrc_t rows, bool is_x, int chunk, int base, int i) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rows, (GW_LDS(void)*)(lds + base + (wave * (is_x ? XL : WL) + i) * 1024), 16, is_x ? x_at[i] : w_at[i],
+        chunk * GW_ROW_BYTES, 0, 0);
+  };
+
+  // Operands: lane (r, g) takes piece 4 s + g of row r of a tile for turn s.
+  unsigned piece_at[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) piece_at[s] = r * GW_ROW_BYTES + ((4 * s + g) ^ (r & 7)) * 16;
+  bf16x8 xf[2][MT], wf[2][NT];
+  constexpr int READS = MT + NT;
+  auto read = [&](int s, int x_base, int w_base, int q) __attribute__((always_inline)) {
+    if (q < NT)
+      wf[s][q] = *reinterpret_cast<const GW_LDS(bf16x8)*>((const GW_LDS(unsigned char)*)lds + w_base +
+                                                          (wn * NT + q) * 2048 + piece_at[s]);
+    else
+      xf[s][q - NT] = *reinterpret_cast<const GW_LDS(bf16x8)*>((const GW_LDS(unsigned char)*)lds + x_base +
+                                                               (wm * MT + q - NT) * 2048 + piece_at[s]);
+  };
+
+  constexpr int PRODUCTS = MT * NT;  // of a turn
+  floatx4 acc[NT][MT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      acc[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      // zeros of its own: told that all accumulators start as one value, the compiler moves them about in the loop
+      if constexpr (PRODUCTS >= 64)
+        asm volatile("" : "+a"(acc[j][t]));
+      else
+        asm volatile("" : "+v"(acc[j][t]));
+    }
+
+  // Turn S: its products; between them the reads of the other turn's operands and `send(Int<i>)` for
+  // i = 0 .. SENDS - 1, spread over the first SPREAD products.
+  auto turn = [&](auto S, int x_base, int w_base, auto SENDS, auto SPREAD, auto send) __attribute__((always_inline)) {
+    constexpr int s = decltype(S)::value, sends = decltype(SENDS)::value, spread = decltype(SPREAD)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    gw_for<PRODUCTS>([&](auto I) __attribute__((always_inline)) {
+      constexpr int i = decltype(I)::value;
+      constexpr int q = (i * READS + PRODUCTS - 1) / PRODUCTS;  // the read that falls due here, if one does
+      if constexpr (q < READS && q * PRODUCTS / READS == i) read(s ^ 1, x_base, w_base, q);
+      if constexpr (sends > 0) {
+        constexpr int l = (i * sends + spread - 1) / spread;
+        if constexpr (l < sends && l * spread / sends == i) send(Int<l>{});
+        if constexpr (sends > spread && l + 1 < sends && (l + 1) * spread / sends == i) send(Int<l + 1>{});
+      }
+      acc[i / MT][i % MT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][i / MT], xf[s][i % MT], acc[i / MT][i % MT], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+
+  if constexpr (RING) {
+    // x of chunk c lies at place 2 c, w at 2 c + 1 (modulo five).  In flight besides the chunk in use: the
+    // next one and x of the one after it.
+    auto whole = [&](bool is_x, int chunk, int place) __attribute__((always_inline)) {
+      const __amdgpu_buffer_rsrc_t rows = rows_of(is_x, chunk);
+#pragma unroll
+      for (int i = 0; i < XL; ++i) load(rows, is_x, chunk, place * PLACE_BYTES, i);
+    };
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      whole(true, c, 2 * c);
+      whole(false, c, 2 * c + 1);
+    }
+    gw_sync<2 * XL>();
+#pragma unroll
+    for (int q = 0; q < READS; ++q) read(0, 0, PLACE_BYTES, q);
+    int place = 0;  // of the chunk's x
+    auto at = [&](int d) __attribute__((always_inline)) {
+      const int v = place + d;
+      return (v >= GW_PLACES ? v - GW_PLACES : v) * PLACE_BYTES;
+    };
+    for (int c = 0; c < chunks; ++c) {
+      const __amdgpu_buffer_rsrc_t xr = rows_of(true, c + 2), wr = rows_of(false, c + 2);
+      turn(Int<0>{}, at(0), at(1), Int<XL>{}, Int<PRODUCTS>{},
+           [&](auto I) __attribute__((always_inline)) { load(xr, true, c + 2, at(4), decltype(I)::value); });
+      gw_sync<XL>();  // all of the next chunk; x of the one after it is on its way
+      turn(Int<1>{}, at(2), at(3), Int<WL>{}, Int<PRODUCTS / 2>{},
+           [&](auto I) __attribute__((always_inline)) { load(wr, false, c + 2, at(0), decltype(I)::value); });
+      place = place + 2 >= GW_PLACES ? place + 2 - GW_PLACES : place + 2;
+    }
+  } else {
+    constexpr int HALF = (LOADS + 1) / 2;  // of a chunk's loads, sent per turn
+    auto load_one = [&](__amdgpu_buffer_rsrc_t xr, __amdgpu_buffer_rsrc_t wr, int chunk, int stage, int i)
+                        __attribute__((always_inline)) {
+      if (i < XL)
+        load(xr, true, chunk, stage * STAGE_BYTES, i);
+      else
+        load(wr, false, chunk, stage * STAGE_BYTES + TM * GW_ROW_BYTES, i - XL);
+    };
+#pragma unroll
+    for (int c = 0; c < STAGES; ++c) {
+      const __amdgpu_buffer_rsrc_t xr = rows_of(true, c), wr = rows_of(false, c);
+#pragma unroll
+      for (int i = 0; i < (c + 1 < STAGES ? LOADS : HALF); ++i) load_one(xr, wr, c, c, i);
+    }
+    gw_sync<(STAGES - 2) * LOADS + HALF>();
+#pragma unroll
+    for (int q = 0; q < READS; ++q) read(0, 0, TM * GW_ROW_BYTES, q);
+    int stage = 0;
+    // Chunk c + STAGES goes to the place of chunk c: half of its loads in c's second turn, the others in the
+    // first turn of c + 1.
+    for (int c = 0; c < chunks; ++c) {
+      const int next = stage + 1 == STAGES ? 0 : stage + 1, before = stage == 0 ? STAGES - 1 : stage - 1;
+      const int base = stage * STAGE_BYTES, next_base = next * STAGE_BYTES;
+      {
+        const __amdgpu_buffer_rsrc_t xr = rows_of(true, c - 1 + STAGES), wr = rows_of(false, c - 1 + STAGES);
+        turn(Int<0>{}, base, base + TM * GW_ROW_BYTES, Int<LOADS - HALF>{}, Int<PRODUCTS>{},
+             [&](auto I) __attribute__((always_inline)) { load_one(xr, wr, c - 1 + STAGES, before, HALF + decltype(I)::value); });
+      }
+      gw_sync<(STAGES - 2) * LOADS>();
+      const __amdgpu_buffer_rsrc_t xr = rows_of(true, c + STAGES), wr = rows_of(false, c + STAGES);
+      turn(Int<1>{}, next_base, next_base + TM * GW_ROW_BYTES, Int<HALF>{}, Int<PRODUCTS>{},
+           [&](auto I) __attribute__((always_inline)) { load_one(xr, wr, c + STAGES, stage, decltype(I)::value); });
+      stage = next;
+    }
+  }
+  // Loads beyond K fetch nothing but do write (zeros) into LDS: the wave sees them through before it leaves.
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+
+  // acc[j][t][i] is out[16 t + r][16 j + 4 g + i] of the wave's quarter (a pair of column tiles with GATED).
+  // N is a multiple of four: a lane's four values are all there or all beyond it.
+  auto store = [&](auto value) __attribute__((always_inline)) {
+    uint16_t* const base = out + static_cast<size_t>(m0 + wm * MT * 16 + r) * p.ldo + n0 + wn * NT * (GATED ? 8 : 16) + 4 * g;
+    const int rows = p.M - (m0 + wm * MT * 16 + r), cols = p.N - (n0 + wn * NT * (GATED ? 8 : 16) + 4 * g);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      if (16 * t >= rows) break;
+      uint16_t* const row = base + static_cast<size_t>(16 * t) * p.ldo;
+#pragma unroll
+      for (int j = 0; j < NT; j += GATED ? 2 : 1) {
+        const int at = j * (GATED ? 8 : 16);
+        bf16x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = static_cast<__bf16>(value(acc[j][t][i], acc[GATED ? j + 1 : j][t][i]));
+        if (at < cols) *reinterpret_cast<bf16x4*>(row + at) = v;
+      }
+    }
+  };
+  if constexpr (GATED) {
+    if (p.epilogue == GW_SILU)
+      store([&](float gate, float up) __attribute__((always_inline)) { return pylon_silu_for_bf16(gate) * up; });
+    else if (p.epilogue == GW_GELU)
+      store([&](float gate, float up) __attribute__((always_inline)) { return gw_gelu(gate) * up; });
+    else
+      store([&](float gate, float up) __attribute__((always_inline)) { return gw_capped(gate, up, p); });
+  } else if (p.epilogue == GW_RELU2) {
+    store([](float v, float) __attribute__((always_inline)) {
+      const float pos = fmaxf(v, 0.f);
+      return pos * pos;
+    });
+  } else {
+    store([](float v, float) __attribute__((always_inline)) { return v; });
+  }
+}
+
+// Two workgroups to a compute unit where their LDS fits.
+template <int MT, int NT, int STAGES>
+constexpr int gw_per_unit() {
+  const int bytes = (STAGES == 0 ? GW_PLACES * 32 * MT : STAGES * 32 * (MT + NT)) * GW_ROW_BYTES;
+  return 2 * bytes <= 160 * 1024 ? 2 : 1;
+}
+
+template <int MT, int NT, int STAGES, bool GATED>
+__global__ __launch_bounds__(256, (gw_per_unit<MT, NT, STAGES>())) void gemm_wide_kernel(
+    uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const GwShape p) {
+  gemm_wide_body<MT, NT, STAGES, GATED>(out, x, w, p);
+}
+
+// The tiles: rows, columns, workgroups per compute unit, and what a chunk of 64 of K costs a workgroup in
+// nanoseconds where the launch's last round leaves it alone on its unit (for one workgroup a unit: leaves
+// units idle) and in full rounds (measured over the layer sizes of 4B to 32B, each launch behind 256 MB of
+// other traffic, as in a step: launched back to back the small tiles look a third faster than they are).
+struct GwTile {
+  int rows, cols, per_unit, alone_ns, full_ns;
+};
+static const GwTile kTiles[] = {
+    {64, 64, 2, 230, 380},      // 2 x 2, five stages
+    {64, 128, 1, 400, 400},     // 2 x 4, six stages
+    {128, 64, 1, 400, 400},     // 4 x 2, six stages
+    {128, 128, 1, 580, 600},    // 4 x 4, four stages
+    {128, 128, 2, 700, 930},    // 4 x 4, the ring
+    {128, 192, 1, 690, 700},    // 4 x 6, three stages
+    {128, 192, 2, 850, 1330},   // 4 x 6, two stages
+    {96, 256, 1, 740, 750},     // 3 x 8, three stages
+    {256, 128, 1, 840, 840},    // 8 x 4, three stages
+    {128, 256, 1, 860, 870},    // 4 x 8, three stages
+    {160, 256, 1, 920, 970},    // 5 x 8, three stages
+    {256, 256, 1, 1300, 1380},  // 8 x 8, the ring
+};
+#define GW_ROUND_US 3.5  // of a round: the first chunks' way to LDS, and the results' way out
+static const int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
+
+static double gw_time_us(const GwTile& t, int M, int N, int K, bool gated, int units) {
+  const int cols = gated ? t.cols / 2 : t.cols;
+  const long long tiles = static_cast<long long>((M + t.rows - 1) / t.rows) * ((N + cols - 1) / cols);
+  const long long slots = static_cast<long long>(units) * t.per_unit;
+  const long long rounds = tiles / slots, left = tiles - rounds * slots;
+  const double chunks = 1e-3 * (K / GW_CHUNK);
+  const double last = left == 0 ? 0.0 : chunks * (left <= units ? t.alone_ns : t.full_ns) + GW_ROUND_US;
+  return rounds * (chunks * t.full_ns + GW_ROUND_US) + last;
+}
+
+static int gw_choose(int M, int N, int K, bool gated, int units) {
+  int best = 0;
+  double least = 1e30;
+  for (int i = 0; i < kTileCount; ++i) {
+    const double us = gw_time_us(kTiles[i], M, N, K, gated, units);
+    if (us < least) least = us, best = i;
+  }
+  return best;
+}
+
+// The tile that pylon_gemm_wide takes for a product of these sizes (units 0: the current device's), and in
+// *us the time that the model gives it.  Touches no device memory.
+extern "C" int pylon_gemm_wide_plan(int M, int N, int K, int gated, int units, int* tile, float* us) {
+  PYLON_REQUIRE(tile != nullptr && us != nullptr && M >= 1 && N >= 1 && K >= GW_CHUNK, "gemm_wide_plan: bad arguments");
+  if (units <= 0) units = pylon_compute_units();
+  PYLON_REQUIRE(units > 0, "gemm_wide_plan: no device to take the number of compute units from");
+  *tile = gw_choose(M, N, K, gated != 0, units);
+  *us = static_cast<float>(gw_time_us(kTiles[*tile], M, N, K, gated != 0, units));
+  return 0;
+}
+
+template <int MT, int NT, int STAGES>
+static void launch_wide(void* out, const void* x, const void* w, GwShape p, hipStream_t stream) {
+  const bool gated = p.epilogue != GW_PLAIN && p.epilogue != GW_RELU2;
+  const int cols = gated ? 16 * NT : 32 * NT;
+  p.m_tiles = (p.M + 32 * MT - 1) / (32 * MT), p.n_tiles = (p.N + cols - 1) / cols;
+  const dim3 grid((static_cast<unsigned>(p.m_tiles) * p.n_tiles + 7) / 8 * 8), block(256);
+  if (gated)
+    hipLaunchKernelGGL((gemm_wide_kernel<MT, NT, STAGES, true>), grid, block, 0, stream, (uint16_t*)out, (const uint16_t*)x,
+                       (const uint16_t*)w, p);
+  else
+    hipLaunchKernelGGL((gemm_wide_kernel<MT, NT, STAGES, false>), grid, block, 0, stream, (uint16_t*)out, (const uint16_t*)x,
+                       (const uint16_t*)w, p);
+}
+
+// x: [M, ldx] bf16; w: [N, ldw] bf16, or with a gate [2 N, ldw], gate rows first; out: [M, ldo] bf16, rounded
+// once.  epilogue: GwEpilogue; alpha, offset, limit: of the capped gate, min(g, limit) sigmoid(alpha g) times
+// clamp(u, -limit, limit) + offset (limit <= 0: no caps).  tile: an index of kTiles, or -1 for the rule; the
+// sums do not depend on it.
+extern "C" int pylon_gemm_wide(void* out, const void* x, const void* w, int M, int N, int K, long long ldx, long long ldw,
+                               long long ldo, int epilogue, float alpha, float offset, float limit, int tile,
+                               hipStream_t stream) {
+  PYLON_REQUIRE(epilogue >= GW_PLAIN && epilogue <= GW_CAPPED, "gemm_wide: unknown epilogue %d", epilogue);
+  PYLON_REQUIRE(M >= 0 && N > 0 && K > 0 && K % GW_CHUNK == 0, "gemm_wide: bad sizes M=%d N=%d K=%d (K a multiple of %d)",
+                M, N, K, GW_CHUNK);
+  PYLON_REQUIRE(ldx >= K && ldw >= K && ldo >= N && ldx % 8 == 0 && ldw % 8 == 0, "gemm_wide: bad row strides");
+  PYLON_REQUIRE((reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0,
+                "gemm_wide: operands must be 16-byte aligned");
+  const bool gated = epilogue != GW_PLAIN && epilogue != GW_RELU2;
+  PYLON_REQUIRE(ldx * 512 < (1ll << 31) && (static_cast<long long>(gated ? N : 0) + 256) * ldw * 2 < (1ll << 31),
+                "gemm_wide: the rows of a tile are beyond the 2 GB that one view of them may span");
+  PYLON_REQUIRE(N % 4 == 0 && ldo % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0,
+                "gemm_wide: rows of the result are multiples of 4 elements at 8-byte aligned addresses");
+  PYLON_REQUIRE(tile >= -1 && tile < kTileCount, "gemm_wide: there is no tile %d", tile);
+  PYLON_REQUIRE(static_cast<long long>((M + 63) / 64) * ((N + 31) / 32) < (1ll << 30), "gemm_wide: too many tiles for one launch");
+  if (M == 0) return 0;
+  if (tile < 0) {
+    const int units = pylon_compute_units();
+    PYLON_REQUIRE(units > 0, "gemm_wide: the device's number of compute units is unknown");
+    tile = gw_choose(M, N, K, gated, units);
+  }
+  const GwShape p{M, N, K, ldx, ldw, ldo, 0, 0, alpha, offset, limit, epilogue};
+  switch (tile) {
+    case 0: launch_wide<2, 2, 5>(out, x, w, p, stream); break;
+    case 1: launch_wide<2, 4, 6>(out, x, w, p, stream); break;
+    case 2: launch_wide<4, 2, 6>(out, x, w, p, stream); break;
+    case 3: launch_wide<4, 4, 4>(out, x, w, p, stream); break;
+    case 4: launch_wide<4, 4, 0>(out, x, w, p, stream); break;
+    case 5: launch_wide<4, 6, 3>(out, x, w, p, stream); break;
+    case 6: launch_wide<4, 6, 2>(out, x, w, p, stream); break;
+    case 7: launch_wide<3, 8, 3>(out, x, w, p, stream); break;
+    case 8: launch_wide<8, 4, 3>(out, x, w, p, stream); break;
+    case 9: launch_wide<4, 8, 3>(out, x, w, p, stream); break;
+    case 10: launch_wide<5, 8, 3>(out, x, w, p, stream); break;
+    default: launch_wide<8, 8, 0>(out, x, w, p, stream); break;
+  }
+  PYLON_LAUNCHED("gemm_wide");
+}

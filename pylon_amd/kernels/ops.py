@@ -1391,6 +1391,49 @@ def gemm_rows(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype =
     return out
 
 
+WIDE_CHUNK = 64  # elements of K that the tiled kernel walks at a time
+_WIDE_EPILOGUES = {"none": 0, "silu": 1, "relu2": 2, "gelu_tanh": 3, "capped": 4}
+
+
+def _wide_ok(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool:
+    """Operands that :func:`gemm_wide` takes and is meant for: bfloat16, more rows than the streaming
+    kernels hold, K in whole chunks, rows of multiples of 8 elements at 16-byte aligned addresses, results of
+    a multiple of 4 columns, and rows of w that one view of 2 GB spans."""
+    return (x.shape[0] > STREAM_ROWS and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda
+            and x.dim() == 2 and weight.shape[1] % WIDE_CHUNK == 0 and x.stride(1) == 1
+            and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and x.stride(0) < 2 ** 22
+            and weight.shape[0] % (8 if gated else 4) == 0
+            and ((weight.shape[0] // 2 if gated else 0) + 256) * weight.stride(0) < 2 ** 30)
+
+
+def gemm_wide(x: torch.Tensor, weight: torch.Tensor, *, epilogue: str = "none", alpha: float = 1.0, offset: float = 0.0,
+              limit: float = 0.0, tile: int = -1, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``x @ weight.T`` for many rows of bfloat16 ``x``, bfloat16 result, rounded once after ``epilogue``:
+    ``relu2`` is ``max(v, 0)^2``; with ``silu``, ``gelu_tanh`` and ``capped`` (:func:`gated_act`'s ``alpha``,
+    ``offset``, ``limit``) ``weight`` is a fused ``[2N, K]`` gate/up matrix and the result the activated gate
+    times up.  ``tile``: the kernel's own choice (-1) or one of its tiles; the result does not depend on it."""
+    if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
+        raise KernelError(f"gemm_wide: cannot multiply {tuple(x.shape)} by the transpose of {tuple(weight.shape)}")
+    if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+        raise KernelError("gemm_wide takes bfloat16 operands")
+    if not (x.is_cuda and weight.is_cuda) or x.stride(1) != 1 or weight.stride(1) != 1:
+        raise KernelError("gemm_wide: operands must be on the GPU with contiguous rows")
+    m, k = x.shape
+    n = weight.shape[0]
+    if epilogue not in ("none", "relu2"):
+        if n % 2:
+            raise KernelError("gemm_wide: a fused gate/up matrix has an even number of rows")
+        n //= 2
+    if out is None:
+        out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    elif out.shape != (m, n) or out.dtype != torch.bfloat16 or not out.is_cuda or not out.is_contiguous():
+        raise KernelError(f"gemm_wide: out must be contiguous bfloat16, on the GPU and of shape {(m, n)}")
+    _lib.call("pylon_gemm_wide", out.data_ptr(), x.data_ptr(), weight.data_ptr(), m, n, k, x.stride(0), weight.stride(0), n,
+              _WIDE_EPILOGUES[epilogue], float(alpha), float(offset), float(limit), int(tile), _stream())
+    return out
+
+
 def _library_float(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``x @ weight.T`` of bfloat16 operands as float32: the library's product with a float32
     result, that is its float32 sums before any rounding."""
@@ -1404,7 +1447,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
     """``x @ weight.T`` (into ``out`` if given: contiguous, of the result's shape and type).
 
     bfloat16 by bfloat16: up to 64 rows go to a weight-streaming kernel where one is faster
-    (:func:`plan.plan_projection`), more rows to the library matrix product (as the
+    (:func:`plan.plan_projection`), more rows to :func:`gemm_wide` where that is
+    (:func:`plan.wide_beats_library`) and else to the library matrix product (as the
     reference's ``nn.Linear`` does).  With a bfloat16 result the float32 sums are rounded once
     either way; with a float32 result (the logits) they come back unrounded either way (the
     library then writes its float32 sums): what a request's logits are rounded to does not
@@ -1423,6 +1467,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
                 return gemm_skinny(x, weight, out_dtype=out_dtype, out=out)
         if out_dtype == torch.float32:
             return _library_float(x, weight, out)
+        if _wide_ok(x, weight) and plan.wide_beats_library(x.shape[0], weight.shape[0]):
+            return gemm_wide(x, weight, out=out)
         y = torch.nn.functional.linear(x, weight)
         y = y if out_dtype == torch.bfloat16 else y.to(out_dtype)
         return y if out is None else out.copy_(y)
@@ -1446,8 +1492,8 @@ def linear_for_residual(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: tor
     to 128 bfloat16 rows it comes back as unrounded float32 sums, which the fused residual norm
     adds: partial sums ``[parts, M, N]`` of a streaming kernel (K cut over workgroups), or,
     from 17 rows on for a matrix at which the library is faster, the library's float32
-    result (:func:`plan.plan_residual`).  For more rows (prompt portions) it is the library's
-    product rounded once to bfloat16."""
+    result (:func:`plan.plan_residual`).  For more rows (prompt portions) it is the product rounded
+    once to bfloat16 (:func:`linear`)."""
     if _streaming_ok(x, weight, SPLIT_ROWS):
         choice = plan.plan_residual(x.shape[0], *weight.shape, units=_lib.compute_units())
         if choice.kernel == "rows":
@@ -1459,11 +1505,13 @@ def linear_for_residual(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: tor
 
 
 def linear_glu(x: torch.Tensor, gate_up: torch.Tensor, *, out_dtype: torch.dtype, act: str = "silu") -> torch.Tensor:
-    """``act(x @ gate.T) * (x @ up.T)`` for a fused ``[2I, K]`` gate/up matrix.  Up to 128
-    bfloat16 rows: the activation works on the float32 sums and its result is rounded once
-    (in a streaming kernel's epilogue; or, where the library is faster and beyond 64 rows,
-    from its float32 result: :func:`plan.plan_gated`).  More rows (prompt portions): the
-    library's product rounded to bfloat16 first."""
+    """``act(x @ gate.T) * (x @ up.T)`` for a fused ``[2I, K]`` gate/up matrix.  The activation works
+    on the float32 sums and its result is rounded once: in a streaming kernel's epilogue or, where
+    the library is faster, from its float32 result (up to 64 rows: :func:`plan.plan_gated`), beyond in
+    :func:`gemm_wide`'s epilogue.  Operands that kernel does not take: up to 128 rows the library's
+    float32 result, more rows its product rounded to bfloat16 first."""
+    if out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True):
+        return gemm_wide(x, gate_up, epilogue=act)
     if _streaming_ok(x, gate_up, SPLIT_ROWS) and x.is_cuda and gate_up.shape[0] % 2 == 0:
         choice = plan.plan_gated(x.shape[0], gate_up.shape[0] // 2, gate_up.shape[1], gate_up.stride(0))
         if choice.kernel == "rows":
@@ -1474,11 +1522,25 @@ def linear_glu(x: torch.Tensor, gate_up: torch.Tensor, *, out_dtype: torch.dtype
     return silu_gate(linear(x, gate_up, out_dtype=out_dtype), act=act)
 
 
+def linear_capped(x: torch.Tensor, gate_up: torch.Tensor, *, alpha: float, offset: float, limit: float,
+                  out_dtype: torch.dtype) -> torch.Tensor:
+    """:func:`gated_act` of ``x @ gate_up.T`` for a fused ``[2I, K]`` gate/up matrix: on the product's
+    float32 sums up to 128 rows and, beyond 64, in :func:`gemm_wide`'s epilogue; for operands that it does
+    not take the library's product, beyond 128 rows rounded first."""
+    if out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True):
+        return gemm_wide(x, gate_up, epilogue="capped", alpha=alpha, offset=offset, limit=limit)
+    sums = torch.float32 if x.shape[0] <= SPLIT_ROWS else out_dtype
+    return gated_act(linear(x, gate_up, out_dtype=sums), alpha=alpha, offset=offset, limit=limit, out_dtype=out_dtype)
+
+
 def linear_relu2(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype) -> torch.Tensor:
     """``max(x @ weight.T, 0)^2``.  Up to 128 bfloat16 rows the activation works on the product's float32
     sums and its result is rounded once: in a streaming kernel's epilogue where one is the faster
-    product (:func:`plan.plan_projection`), else from the library's float32 result.  More rows: the
-    library's product rounded first."""
+    product (:func:`plan.plan_projection`), else from the library's float32 result.  More than 64 rows:
+    in :func:`gemm_wide`'s epilogue, or for operands that it does not take from the library's product,
+    beyond 128 rows rounded first."""
+    if out_dtype == torch.bfloat16 and _wide_ok(x, weight):
+        return gemm_wide(x, weight, epilogue="relu2")
     if _streaming_ok(x, weight, STREAM_ROWS):
         choice = plan.plan_projection(x.shape[0], *weight.shape)
         if choice.kernel == "rows":

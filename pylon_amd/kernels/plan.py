@@ -165,6 +165,23 @@ def plan_summed_later(rows: int, n: int, k: int, units: int = UNITS) -> Product:
     return plan_projection(rows, n, k)
 
 
+def wide_beats_library(rows: int, n: int) -> bool:
+    """Whether a product of more than 64 rows without an activation behind it goes to the engine's own
+    tiled kernel (``gemm_wide``) or to the library's.  The own kernel's tile is chosen so that the launch fills
+    whole rounds of the compute units; for many rows the library's 256 x 256 tile is the faster main loop where
+    a matrix is wide enough for it.  A layer of a prompt step in us, library against own kernel (both with
+    gate/up in the own kernel's epilogue):
+
+    out and down: 4B sizes (2560 wide) at 160, 800, 1024, 1300, 2048 tokens 195, 328, 352, 404, 567 against
+    175, 315, 364, 386, 570; 8B (4096) at 160, 600, 1300, 1600, 2048 270, 401, 628, 828, 794 against 237, 410,
+    610, 692, 781; 32B (5120) at 160, 600, 1300, 1600, 1800, 2048 529, 868, 1456, 1927, 1707, 1829 against 422,
+    814, 1333, 1681, 1691, 2164.
+    q/k/v (6144 wide; 32B 10240): 4B at 100, 250, 1300, 1800, 2048 175, 195, 404, 516, 567 against 158, 187, 395,
+    530, 569; 8B at 160, 1024, 1800, 2048 270, 502, 746, 794 against 265, 502, 759, 809; 32B at 2048 1829 against
+    1902."""
+    return rows <= 1700 or n <= 4096
+
+
 def plan_gated(rows: int, n_half: int, k: int, row_stride: int) -> Product:
     """``silu(x gate^T) * (x up^T)`` over a fused matrix of ``2 * n_half`` rows; "library" means
     its product followed by the activation kernel (up to 64 rows its float32 result).

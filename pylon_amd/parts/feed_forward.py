@@ -53,9 +53,8 @@ class GatedFeedForward(Part):
 
 class CappedGatedFeedForward(Part):
     """``down(a(g) * (u + offset))``, ``g = min(gate(h), limit)``, ``u = clamp(up(h), -limit,
-    limit)``, ``a(g) = g * sigmoid(alpha * g)``.  As in the plain gated feed-forward, up to 128
-    rows the activation works on the float32 sums of the product and its result is rounded
-    once; beyond, the library's product is rounded first."""
+    limit)``, ``a(g) = g * sigmoid(alpha * g)``.  As in the plain gated feed-forward the activation
+    works on the float32 sums of the product and its result is rounded once (:func:`ops.linear_capped`)."""
 
     def __init__(self, spec: CappedGatedFeedForwardSpec, *, dtype: torch.dtype, device) -> None:
         super().__init__()
@@ -68,15 +67,14 @@ class CappedGatedFeedForward(Part):
 
     def forward(self, h: torch.Tensor, ctx) -> torch.Tensor:
         spec = self.spec
-        sums = torch.float32 if h.shape[0] <= ops.SPLIT_ROWS else self.dtype
-        gate_up = ops.linear(h, self.params["gate_up"], out_dtype=sums)
-        hidden = ops.gated_act(gate_up, alpha=spec.alpha, offset=spec.offset, limit=spec.limit, out_dtype=self.dtype)
+        hidden = ops.linear_capped(h, self.params["gate_up"], alpha=spec.alpha, offset=spec.offset, limit=spec.limit,
+                                   out_dtype=self.dtype)
         return ops.linear_for_residual(hidden, self.params["down"], out_dtype=self.dtype)
 
 
 class PlainFeedForward(Part):
-    """``down(max(up(h), 0)^2)``.  Up to 128 rows the activation works on the float32 sums of the
-    product and its result is rounded once; beyond, the library's product is rounded first."""
+    """``down(max(up(h), 0)^2)``.  The activation works on the float32 sums of the product and its result
+    is rounded once (:func:`ops.linear_relu2`)."""
 
     def __init__(self, spec: PlainFeedForwardSpec, *, dtype: torch.dtype, device) -> None:
         super().__init__()

@@ -1,0 +1,111 @@
+"""The tiled bfloat16 product of prompt portions (``ops.gemm_wide``): every tile at its edges and with
+every activation against float64, the rule that picks a tile, and the products that are led to it."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+TILES = [(64, 64), (64, 128), (128, 64), (128, 128), (128, 128), (128, 192), (128, 192), (96, 256), (256, 128), (128, 256),
+         (160, 256), (256, 256)]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from pylon_amd.kernels import ops
+
+    return ops
+
+
+def draw(seed, rows, k, pad=0):
+    gen = torch.Generator(DEV).manual_seed(seed)
+    return torch.randn(rows, k + pad, generator=gen, device=DEV).to(torch.bfloat16)[:, :k]
+
+
+def wanted(x, w, epilogue):
+    v = x.double() @ w.double().T
+    if epilogue == "none":
+        return v
+    if epilogue == "relu2":
+        return v.clamp(min=0) ** 2
+    g, u = v.chunk(2, 1)
+    if epilogue == "silu":
+        return g * torch.sigmoid(g) * u
+    if epilogue == "gelu_tanh":
+        return torch.nn.functional.gelu(g, approximate="tanh") * u
+    g, u = g.clamp(max=7.0), u.clamp(-7.0, 7.0)
+    return g * torch.sigmoid(1.702 * g) * (u + 1.0)
+
+
+def close(got, want):
+    """One rounding to bfloat16 (seven bits behind the leading one: at most 2^-8 of the value), and float32
+    sums and an activation ahead of it (2^-16 of the largest value)."""
+    room = want.abs() * 1.01 * 2.0 ** -8 + want.abs().max() * 2.0 ** -16
+    return bool(((got.double() - want).abs() <= room).all())
+
+
+# K: one chunk (fewer than any tile keeps in flight), a few, more than all that are in flight
+@pytest.mark.parametrize("k", [64, 128, 320, 704])
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_every_tile_at_its_edges(ops, tile, k):
+    rows, cols = TILES[tile]
+    for m, n in ((rows, cols), (rows + 1, cols - 4), (2 * rows - 3, cols + 4), (5, 3 * cols + 12)):
+        x, w = draw(m, m, k, 8), draw(n + k, n, k, 64)
+        got = ops.gemm_wide(x, w, tile=tile)
+        assert close(got, wanted(x, w, "none")), (m, n)
+        assert torch.equal(got, ops.gemm_wide(x, w, tile=(tile + 3) % len(TILES))), (m, n)  # one order of sums
+
+
+@pytest.mark.parametrize("epilogue", ["silu", "relu2", "gelu_tanh", "capped"])
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_every_activation(ops, tile, epilogue):
+    rows, cols = TILES[tile]
+    m, n, k = rows + 7, cols + 4, 192
+    x, w = draw(1, m, k), draw(2, 2 * n, k, 64) * 0.2
+    got = ops.gemm_wide(x, w, epilogue=epilogue, alpha=1.702, offset=1.0, limit=7.0, tile=tile)
+    assert close(got, wanted(x, w, epilogue))
+
+
+def test_the_rule_names_a_tile_that_fills_the_chip():
+    from pylon_amd.kernels import library
+
+    tile, us = ctypes.c_int(), ctypes.c_float()
+    for m, n, k, gated, expected in ((2048, 12288, 4096, 1, (256, 256)), (2048, 4096, 12288, 0, (256, 128)),
+                                     (2048, 9728, 2560, 1, (160, 256)), (100, 2560, 4096, 0, (64, 64)),
+                                     (656, 5120, 25600, 0, (128, 128))):
+        assert library.load().pylon_gemm_wide_plan(m, n, k, gated, 256, ctypes.byref(tile), ctypes.byref(us)) == 0
+        assert TILES[tile.value] == expected, (m, n, k, tile.value, us.value)
+
+
+@pytest.mark.parametrize("rows", [65, 128, 129, 300, 1537])
+def test_products_that_are_led_to_it(ops, rows):
+    """Each dispatcher beside its own answer for rows it leads elsewhere or takes apart: K of no whole
+    chunks, rows off a 16-byte boundary, odd strides of the result."""
+    x, w = draw(rows, rows, 256), draw(3, 600, 256) * 0.1
+    for k in (256, 248):  # 248: the library
+        a, b = x[:, :k], w[:, :k]
+        assert close(ops.linear(a, b), wanted(a, b, "none"))
+        twice = k == 248  # the library rounds before the activation
+        for got, want in ((ops.linear_glu(a, b, out_dtype=torch.bfloat16), wanted(a, b, "silu")),
+                          (ops.linear_glu(a, b, out_dtype=torch.bfloat16, act="gelu_tanh"), wanted(a, b, "gelu_tanh")),
+                          (ops.linear_relu2(a, b, out_dtype=torch.bfloat16), wanted(a, b, "relu2")),
+                          (ops.linear_capped(a, b, alpha=1.702, offset=1.0, limit=7.0, out_dtype=torch.bfloat16),
+                           wanted(a, b, "capped"))):
+            assert close(got, want) or (twice and (got.double() - want).abs().max() <= 2e-2 * want.abs().max())
+    into = torch.empty(rows, 600, dtype=torch.bfloat16, device=DEV)
+    assert ops.linear(x, w, out=into) is into and close(into, wanted(x, w, "none"))
+    assert close(ops.linear(x, w[:599]), wanted(x, w[:599], "none"))  # columns that are no multiple of 4: the library
+    shifted = torch.zeros(rows * 256 + 1, dtype=torch.bfloat16, device=DEV)[1:].view(rows, 256).copy_(x)
+    assert close(ops.linear(shifted, w), wanted(x, w, "none"))
+    assert ops.linear(x, w, out_dtype=torch.float32).dtype == torch.float32
+
+
+def test_infinities_stay_in_their_rows_and_columns(ops):
+    x, w = draw(5, 100, 128), draw(6, 72, 128)
+    x[3, 5], w[9, 0] = float("inf"), float("nan")
+    got = ops.gemm_wide(x, w)
+    keep = torch.ones(100, 72, dtype=torch.bool, device=DEV)
+    keep[3], keep[:, 9] = False, False
+    assert torch.isfinite(got[keep]).all() and torch.isnan(got[:, 9]).all() and not torch.isfinite(got[3]).any()
