@@ -153,8 +153,8 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
     }
   };
   floatx4 x_even[MT][4], x_odd[MT][4];
-  load_x(x_even, chunk, turns > 0);
-  issue(tile, chunk, 0, turns > 0);
+  load_x(x_even, chunk, true);
+  issue(tile, chunk, 0, true);
   advance();
   for (int turn = 0; turn < turns; turn += 2) {
     turn_of(turn, x_even, x_odd, 0);
@@ -169,9 +169,8 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
     floatx4 half[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int p = 0; p < GF_RANGES; ++p)
-      if (gf_range_begin(p, chunks) < gf_range_begin(p + 1, chunks))  // a short K leaves ranges empty
-        half[p / (GF_RANGES / 2)] +=
-            *reinterpret_cast<const floatx4*>(sums + (((tl * GF_RANGES + p) * MT + t) * PYLON_WAVE + lane) * 4);
+      half[p / (GF_RANGES / 2)] +=
+          *reinterpret_cast<const floatx4*>(sums + (((tl * GF_RANGES + p) * MT + t) * PYLON_WAVE + lane) * 4);
     const floatx4 v = half[0] + half[1];
     const int m = 16 * t + r, n = row0 + tl * 16 + 4 * g;
     if (m >= M) continue;
@@ -290,8 +289,8 @@ __device__ __forceinline__ void gemm_f32_tiles_body(float* __restrict__ out, con
           for (int t = 0; t < T; ++t)
             acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j][i], xf[t][i], acc[j][t], 0, 0, 0);
     }
-    while (range < GF_RANGES && gf_range_begin(range + 1, chunks) <= c) ++range;  // a short K leaves ranges empty
     if (gf_range_begin(range + 1, chunks) == c + 1) {  // the range ends with this chunk
+      ++range;
 #pragma unroll
       for (int j = 0; j < T; ++j)
 #pragma unroll
@@ -377,12 +376,15 @@ static int gf_group_tiles(int N, int units) {
   return per < 1 ? 1 : (per > GF_GROUP_TILES ? GF_GROUP_TILES : static_cast<int>(per));
 }
 
-// Whether the kernels of this file take the operands: whole 16-byte pieces of rows, and offsets
-// within a workgroup's rows that a buffer descriptor spans.  Nothing here depends on M except that
-// a launch's rows of x stay within a descriptor, which gemm_f32_launch cuts them to.
+// Whether the kernels of this file take the operands: whole 16-byte pieces of rows, offsets within a
+// workgroup's rows that a buffer descriptor spans, and a chunk of K for every range.  The last is not a
+// matter of time (one row, 512 outputs: 44.0 us at K = 508 in gemm_tiled, 3.1 us at K = 512 here; 300 rows
+// of 2048 outputs: 47.9 and 12.0): a shorter K would leave ranges empty, and models that small keep the
+// one ascending chain that recorded runs of theirs hold, choices between near ties included.  Nothing here
+// depends on M.
 bool gemm_f32_takes(const void* x, const void* w, int K, long long ldx, long long ldw) {
-  return K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && ldx <= (1ll << 21) && ldw <= (1ll << 21) &&
-         (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
+  return K >= GF_RANGES * GF_CHUNK && K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && ldx <= (1ll << 21) &&
+         ldw <= (1ll << 21) && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
 }
 
 // M >= 1; false if the device is unknown or the launch would be too large (nothing launched then).

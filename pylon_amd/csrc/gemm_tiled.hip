@@ -1,6 +1,6 @@
 // out[M, N] = a[M, K] * w[N, K]^T with float accumulation and no reduced-precision mode.  float32
-// operands with 16-byte aligned rows go to gemm_f32.hip; the kernel here, on the vector ALUs, is for
-// the element type pairings and alignments that no fast kernel takes.  Each output element is one
+// operands with 16-byte aligned rows of at least 512 elements go to gemm_f32.hip; the kernel here, on the
+// vector ALUs, is for the element type pairings, alignments and short rows that no fast kernel takes.  Each output element is one
 // chain of fused multiply-adds over k = 0..K-1 in ascending order, so its value does not depend on
 // M, on the tile it falls in, or on what else is in the batch.
 #include "common.h"
