@@ -119,6 +119,7 @@ class StepContext:
     logits_out: Optional[torch.Tensor] = None  # float32 [>= n_logits, vocab]: where the logits go, if given
     arena: Optional[MetadataArena] = None  # pinned staging for what parts put on the device themselves
     _tiles: Dict[Tuple[int, int, int], torch.Tensor] = field(default_factory=dict)
+    _singles: Optional[int] = None
     # what a part has derived from the step's metadata and layers of its kind can share (by a key of
     # the part's choosing): made once a step instead of once a layer
     memo: Dict[object, object] = field(default_factory=dict)
@@ -130,8 +131,10 @@ class StepContext:
     def leading_singles(self) -> int:
         """How many rows at the head of the step bring exactly one token (the decoding
         requests, which the engine puts first): token t of them is row t."""
-        more = np.nonzero(self.counts != 1)[0]
-        return int(more[0]) if more.size else self.rows
+        if self._singles is None:  # asked by every attention layer
+            more = np.nonzero(self.counts != 1)[0]
+            self._singles = int(more[0]) if more.size else self.rows
+        return self._singles
 
     def token_tiles(self, tokens_per_tile: int, skip_rows: int = 0, fold: int = 0) -> torch.Tensor:
         """int32 ``[n, 4]`` on the device: the step's tokens (without those of the first
@@ -270,12 +273,12 @@ def build_step(entries: Seq[StepEntry], manager: CacheManager, arena: MetadataAr
             off, n = layout[name]
             return block[off: off + n]
 
+        tables = [(dev(f"slot_map{g}"), dev(f"block_table{g}").view(rows, width)) for g in range(n_groups)]
         views: Dict[int, CacheView] = {}
         for cache_id in range(manager.n_caches):
             view = manager.view(cache_id)
             if view.group >= 0:
-                view.slot_map = dev(f"slot_map{view.group}")
-                view.block_table = dev(f"block_table{view.group}").view(rows, width)
+                view.slot_map, view.block_table = tables[view.group]
             views[cache_id] = view
         return StepContext(
             tokens=tokens, rows=rows,

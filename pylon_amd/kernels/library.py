@@ -9,7 +9,7 @@ import ctypes
 import threading
 from ctypes import c_char_p, c_float, c_int, c_longlong, c_void_p
 from pathlib import Path
-from typing import Optional
+from typing import Dict, Optional
 
 from ..csrc import build as _build
 
@@ -131,14 +131,21 @@ def load(*, quiet: bool = False) -> ctypes.CDLL:
     return _lib
 
 
-def call(name: str, *args) -> None:
-    lib = load()
-    fn = getattr(lib, name, None)
+_entry_points: Dict[str, object] = {}  # by name, looked up once: a step calls a few hundred times
+
+
+def _entry_point(name: str):
+    fn = getattr(load(), name, None)
     if fn is None:
         raise KernelError(f"the kernel library {_lib_path} has no entry point {name}")
-    status = fn(*args)
-    if status != 0:
-        raise KernelError(lib.pylon_last_error().decode(errors="replace"))
+    _entry_points[name] = fn
+    return fn
+
+
+def call(name: str, *args) -> None:
+    fn = _entry_points.get(name) or _entry_point(name)
+    if fn(*args) != 0:
+        raise KernelError(_lib.pylon_last_error().decode(errors="replace"))
 
 
 def check_device() -> None:

@@ -46,13 +46,15 @@ def _dev(t: Optional[torch.Tensor], name: str, dtype=None) -> int:
     """Device pointer of a checked tensor (0 for None)."""
     if t is None:
         return 0
+    if t.is_cuda and t.is_contiguous() and (dtype is None or t.dtype == dtype):
+        return t.data_ptr()
     if not t.is_cuda:
         raise KernelError(f"{name} must live on the GPU; there is no CPU path")
     if not t.is_contiguous():
         raise KernelError(f"{name} must be contiguous")
     if dtype is not None and t.dtype != dtype:
         raise KernelError(f"{name} must be {dtype}, got {t.dtype}")
-    return t.data_ptr()
+    raise KernelError(f"{name} is no tensor that a kernel takes")
 
 
 def embed(ids: torch.Tensor, table: torch.Tensor, *, scale: float = 1.0,
@@ -1306,7 +1308,7 @@ SPLIT_ROWS = plan.SPLIT_ROWS    # most rows the rows kernel takes, as two halves
 def _streaming_ok(x: torch.Tensor, weight: torch.Tensor, rows: int) -> bool:
     """Operands a weight-streaming kernel takes: bfloat16, at most ``rows`` rows of x, rows of
     multiples of 8 elements at 16-byte aligned addresses."""
-    return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and 0 < x.shape[0] <= rows
+    return (0 < x.shape[0] <= rows and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
             and weight.shape[1] % 8 == 0 and weight.stride(0) % 8 == 0 and x.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
@@ -1391,6 +1393,11 @@ def gemm_rows(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype =
     return out
 
 
+def _rows_apart(t: torch.Tensor) -> bool:
+    """Rows that hold something, do not overlap (an expanded row does) and are contiguous."""
+    return t.stride(1) == 1 and t.stride(0) >= t.shape[1] > 0
+
+
 WIDE_CHUNK = 64  # elements of K that the tiled kernel walks at a time
 _WIDE_EPILOGUES = {"none": 0, "silu": 1, "relu2": 2, "gelu_tanh": 3, "capped": 4}
 
@@ -1400,10 +1407,9 @@ def _wide_ok(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool
     kernels hold, K in whole chunks, rows of multiples of 8 elements at 16-byte aligned addresses, results of
     a multiple of 4 columns, and rows of w that one view of 2 GB spans."""
     return (x.shape[0] > STREAM_ROWS and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda
-            and x.dim() == 2 and weight.shape[1] % WIDE_CHUNK == 0 and x.stride(1) == 1
-            and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
+            and x.dim() == 2 and weight.shape[1] % WIDE_CHUNK == 0 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and x.stride(0) < 2 ** 22
-            and weight.shape[0] % (8 if gated else 4) == 0
+            and weight.shape[0] % (8 if gated else 4) == 0 and weight.shape[0] > 0 and _rows_apart(x) and _rows_apart(weight)
             and ((weight.shape[0] // 2 if gated else 0) + 256) * weight.stride(0) < 2 ** 30)
 
 
@@ -1465,10 +1471,14 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
                 return gemm_rows(x, weight, out_dtype=out_dtype, col_tiles=choice.col_tiles, out=out)
             if choice.kernel == "skinny":
                 return gemm_skinny(x, weight, out_dtype=out_dtype, out=out)
+            if (out is None and out_dtype == torch.bfloat16 and x.dim() == 2
+                    and plan.rows_match_library(x.shape[0], *weight.shape) and _rows_apart(x) and _rows_apart(weight)):
+                return gemm_rows(x, weight)
         if out_dtype == torch.float32:
             return _library_float(x, weight, out)
-        if _wide_ok(x, weight) and plan.wide_beats_library(x.shape[0], weight.shape[0]):
-            return gemm_wide(x, weight, out=out)
+        if out is None and _wide_ok(x, weight) and plan.wide_beats_library(x.shape[0], weight.shape[0]):
+            y = gemm_wide(x, weight)
+            return y if out_dtype == torch.bfloat16 else y.to(out_dtype)
         y = torch.nn.functional.linear(x, weight)
         y = y if out_dtype == torch.bfloat16 else y.to(out_dtype)
         return y if out is None else out.copy_(y)

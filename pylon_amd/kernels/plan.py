@@ -14,6 +14,7 @@ kernel wins almost everywhere; the exceptions are listed where they are decided.
 from __future__ import annotations
 
 from dataclasses import dataclass
+from functools import lru_cache
 
 FEW_ROWS = 16      # one tile of rows of x
 STREAM_ROWS = 64   # most rows of x a workgroup of a weight-streaming kernel takes
@@ -86,6 +87,7 @@ def deep_or_narrow(n: int, k: int) -> bool:
     return k >= 2 * n or n <= 4096
 
 
+@lru_cache(maxsize=4096)  # asked for every product of a step
 def plan_residual(rows: int, n: int, k: int, units: int = UNITS) -> Product:
     """A product about to be added to the float32 residual stream (out and down projections),
     ``rows`` <= 128: float32 sums, never rounded, from whichever kernel.
@@ -112,6 +114,7 @@ def plan_residual(rows: int, n: int, k: int, units: int = UNITS) -> Product:
     return Product("rows", *rows_split(n, k, rows, units))
 
 
+@lru_cache(maxsize=4096)  # asked for every product of a step
 def plan_projection(rows: int, n: int, k: int) -> Product:
     """Any other product (q/k/v; the vocabulary head); beyond 64 rows the library's.
 
@@ -137,6 +140,7 @@ def plan_projection(rows: int, n: int, k: int) -> Product:
     return Product("rows") if few else Product("library")
 
 
+@lru_cache(maxsize=4096)  # asked for every product of a step
 def plan_summed_later(rows: int, n: int, k: int, units: int = UNITS) -> Product:
     """A projection whose consumer can add float partial sums itself (q/k/v in front of the
     decode attention that prepares its own operands): K is cut over workgroups where the uncut
@@ -165,6 +169,16 @@ def plan_summed_later(rows: int, n: int, k: int, units: int = UNITS) -> Product:
     return plan_projection(rows, n, k)
 
 
+def rows_match_library(rows: int, n: int, k: int) -> bool:
+    """Whether a bfloat16 product of 17 to 48 rows that :func:`plan_projection` leaves to the library takes the
+    rows kernel after all: for matrices wide enough to fill the compute units uncut, whose rows are of no
+    power-of-two length, the device takes no longer (at 17, 32 and 48 rows 6144 x 2560 15.9, 15.6, 18.3 us
+    against 15.6, 15.8, 20.4; 7168 x 2560 16.2, 16.4, 18.7 against 16.5, 16.8, 20.9; 10240 x 5120 33.0, 33.5,
+    38.5 against 34.3, 35.2, 39.9; but 6144 x 4096 21.2, 21.1, 24.8 against 19.8, 20.1, 22.0) and the host 10
+    us instead of 26, which is what a step of few prompt tokens waits for."""
+    return rows <= 48 and 5120 <= n < TALL and not aliased_rows(k)
+
+
 def wide_beats_library(rows: int, n: int) -> bool:
     """Whether a product of more than 64 rows without an activation behind it goes to the engine's own
     tiled kernel (``gemm_wide``) or to the library's.  The own kernel's tile is chosen so that the launch fills
@@ -182,6 +196,7 @@ def wide_beats_library(rows: int, n: int) -> bool:
     return rows <= 1700 or n <= 4096
 
 
+@lru_cache(maxsize=4096)  # asked for every product of a step
 def plan_gated(rows: int, n_half: int, k: int, row_stride: int) -> Product:
     """``silu(x gate^T) * (x up^T)`` over a fused matrix of ``2 * n_half`` rows; "library" means
     its product followed by the activation kernel (up to 64 rows its float32 result).

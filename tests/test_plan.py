@@ -155,3 +155,11 @@ def test_decode_attention_cuts_the_keys_of_few_long_requests_over_workgroups():
                     cuts = ops.decode_cuts(tokens, heads, bound, units)
                     assert cuts & (cuts - 1) == 0 and 1 <= cuts <= 64
                     assert cuts == 1 or (tokens * heads * cuts <= units and cuts * 192 <= bound)
+
+
+@pytest.mark.parametrize("rows, n, k, own", [
+    (17, 6144, 2560, True), (48, 5120, 2560, True), (49, 6144, 2560, False), (32, 5119, 2560, False),
+    (32, plan.TALL - 1, 5120, True), (32, plan.TALL, 5120, False), (32, 6144, 4096, False)])
+def test_wide_projections_of_few_prompt_tokens_take_the_rows_kernel(rows, n, k, own):
+    assert plan.rows_match_library(rows, n, k) is own
+    assert not own or plan.plan_projection(rows, n, k).kernel == "library"  # what it stands in for
