@@ -341,6 +341,15 @@ __global__ __launch_bounds__(512) void attention_sink_kernel(
 // results (maximum, sum, unnormalised output, all float) meet in LDS and are merged in the order of
 // the waves: into the output if the keys are not cut, else into the cut's partial result for the
 // merge kernel.
+//
+// What bounds it is the chain of loads of a wave's few blocks, not the bytes: position, page, then the
+// block's keys, biases and values, which all go out before the first is used; the registers of each are
+// filled for the next block as soon as this block is done with them.  The biases are gathered by distance
+// straight from the table: a workgroup needs a few hundred entries of it, and copying all of a group's
+// tables to LDS first (32 KB at 2,048 distances and four heads) took longer than the walk itself.
+// 32 heads of 128 over 8 and 2,048 distances, 4 requests of 1,524 keys in 4 cuts with the merge: 29.9 us
+// with the tables in LDS and a block fetched when its turn came, 18.1 so (14.1 in 16 cuts); 16 requests 47.0
+// and 30.3; 64 of 1,000 keys, uncut, 88.1 and 63.2; without a bias, 2 of 2,524 in 8 cuts 25.1 and 16.5.
 template <int KS, int NV>
 __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, long long q_stride, const bf16_t* __restrict__ k_cache,
@@ -348,8 +357,8 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
     const int* __restrict__ positions, int n_heads, int n_kv_heads, int dim, int vdim, int page_size, float scale,
     const float* __restrict__ bias, int bucket_len, int sink, int cuts, float* __restrict__ partial, int window,
     float softcap, const float* __restrict__ sink_logit) {
-  extern __shared__ float bias_lds[];  // [group][bucket_len]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  extern __shared__ float mrg[];  // [4 waves][group][2 + vdim]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
   const int group = n_heads / n_kv_heads;
   int b = blockIdx.x;
@@ -360,16 +369,59 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
   const int pos = positions[tok];
   const int* table = block_table + static_cast<size_t>(tok) * table_width;
   const int my_head = kvh * group + (col < group ? col : group - 1);  // columns past the group repeat its last head
-  if (bias != nullptr) {
-    for (int i = threadIdx.x; i < group * bucket_len; i += 256) {
-      const int h = i / bucket_len;
-      bias_lds[i] = bias[static_cast<size_t>(kvh * group + h) * bucket_len + (i - h * bucket_len)];
-    }
-  }
-  __syncthreads();
-  const float* tbl = bias_lds + (col < group ? col : group - 1) * bucket_len;
-  const float far_bias = bias != nullptr ? tbl[bucket_len - 1] : 0.f;
+  const float* bias_row = bias + static_cast<size_t>(my_head) * bucket_len;  // read only if there is a bias
 
+  const int first_key = first_visible(pos, window);  // a window, a chunk: the walk starts at its block
+  const int kb_first = first_key / AS_BLOCK * AS_BLOCK;
+  const int n_blocks = (pos - kb_first) / AS_BLOCK + 1;
+  const int per_cut = (n_blocks + cuts - 1) / cuts;
+  const int kb_begin = kb_first + cut * per_cut * AS_BLOCK;
+  const int kb_end = kb_first + ((cut + 1) * per_cut < n_blocks ? (cut + 1) * per_cut : n_blocks) * AS_BLOCK;
+
+  u32x4 kraw[2][KS];
+  u32x2 vraw[NV][2];
+  float add[8];
+  auto load_keys = [&](int kb, int page) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const size_t slot = static_cast<size_t>(page) * page_size + kb % page_size + t * 16 + col;
+      const bf16_t* kr = k_cache + (slot * n_kv_heads + kvh) * dim;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int d = ks * 32 + grp * 8;
+        kraw[t][ks] = u32x4{0u, 0u, 0u, 0u};
+        if (d < dim) kraw[t][ks] = *reinterpret_cast<const u32x4*>(kr + d);
+      }
+    }
+  };
+  auto load_bias = [&](int kb) {
+    if (bias == nullptr) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) add[e] = 0.f;
+      return;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      int idx = pos - (kb + (e >> 2) * 16 + 4 * grp + (e & 3));
+      idx = idx < 0 ? 0 : (idx < bucket_len - 1 ? idx : bucket_len - 1);
+      add[e] = bias_row[idx];
+    }
+  };
+  auto load_values = [&](int kb, int page) {
+    const bf16_t* block = v_cache + (static_cast<size_t>(page) * n_kv_heads + kvh) * vdim * page_size + kb % page_size + 4 * grp;
+#pragma unroll
+    for (int dt = 0; dt < NV; ++dt) {
+      const int d = dt * 16 + col;
+      vraw[dt][0] = vraw[dt][1] = u32x2{0u, 0u};
+      if (d < vdim) {
+        const bf16_t* vr = block + static_cast<size_t>(d) * page_size;
+        vraw[dt][0] = *reinterpret_cast<const u32x2*>(vr);
+        vraw[dt][1] = *reinterpret_cast<const u32x2*>(vr + 16);
+      }
+    }
+  };
+
+  int kb = kb_begin + wave * AS_BLOCK;
   bf16x8 qf[KS];
   {
     const bf16_t* qr = q + static_cast<size_t>(tok) * q_stride + static_cast<size_t>(my_head) * dim;
@@ -381,6 +433,12 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
       qf[ks] = __builtin_bit_cast(bf16x8, raw);
     }
   }
+  if (kb < kb_end) {
+    const int page = table[kb / page_size];
+    load_keys(kb, page);
+    load_bias(kb);
+    load_values(kb, page);
+  }
   floatx4 o[NV];
 #pragma unroll
   for (int dt = 0; dt < NV; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -388,68 +446,29 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
   float m_run = first ? (sink_logit != nullptr ? sink_logit[my_head] : 0.f) : -INFINITY;
   float l_run = (first && grp == 0) ? 1.f : 0.f;
 
-  const int first_key = first_visible(pos, window);  // a window, a chunk: the walk starts at its block
-  const int kb_first = first_key / AS_BLOCK * AS_BLOCK;
-  const int n_blocks = (pos - kb_first) / AS_BLOCK + 1;
-  const int per_cut = (n_blocks + cuts - 1) / cuts;
-  const int kb_begin = kb_first + cut * per_cut * AS_BLOCK;
-  const int kb_end = kb_first + ((cut + 1) * per_cut < n_blocks ? (cut + 1) * per_cut : n_blocks) * AS_BLOCK;
-  for (int kb = kb_begin + wave * AS_BLOCK; kb < kb_end; kb += 4 * AS_BLOCK) {
-    const int page = table[kb / page_size];
-    const int in_page = kb % page_size;
+  for (; kb < kb_end; kb += 4 * AS_BLOCK) {
+    const int next = kb + 4 * AS_BLOCK;
+    const bool more = next < kb_end;
+    const int next_page = more ? table[next / page_size] : 0;
     floatx4 s[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const size_t slot = static_cast<size_t>(page) * page_size + in_page + t * 16 + col;
-      const bf16_t* kr = k_cache + (slot * n_kv_heads + kvh) * dim;
       s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int d = ks * 32 + grp * 8;
-        u32x4 raw = {0u, 0u, 0u, 0u};
-        if (d < dim) raw = *reinterpret_cast<const u32x4*>(kr + d);
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, raw), qf[ks], s[t], 0, 0, 0);
-      }
+      for (int ks = 0; ks < KS; ++ks)
+        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kraw[t][ks]), qf[ks], s[t], 0, 0, 0);
     }
-    bf16x8 vf[NV];
-    const bool ragged = kb + AS_BLOCK - 1 > pos;
-#pragma unroll
-    for (int dt = 0; dt < NV; ++dt) {
-      const int d = dt * 16 + col;
-      u32x4 raw = {0u, 0u, 0u, 0u};
-      if (d < vdim) {
-        const bf16_t* vr = v_cache + ((static_cast<size_t>(page) * n_kv_heads + kvh) * vdim + d) * page_size +
-                           in_page + 4 * grp;
-        const u32x2 a0 = *reinterpret_cast<const u32x2*>(vr);
-        const u32x2 a1 = *reinterpret_cast<const u32x2*>(vr + 16);
-        raw = u32x4{a0[0], a0[1], a1[0], a1[1]};
-        if (ragged) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int key = kb + (e >> 2) * 16 + 4 * grp + (e & 3);
-            if (key > pos) raw[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
-          }
-        }
-      }
-      vf[dt] = __builtin_bit_cast(bf16x8, raw);
-    }
+    if (more) load_keys(next, next_page);
     float sc[8];
-    const bool all_far = bias == nullptr || pos - (kb + AS_BLOCK - 1) >= bucket_len - 1;
     float top = m_run;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int key = kb + (e >> 2) * 16 + 4 * grp + (e & 3);
-      const int dist = pos - key;
-      float add = far_bias;
-      if (!all_far) {
-        int idx = dist < 0 ? 0 : dist;
-        idx = idx < bucket_len - 1 ? idx : bucket_len - 1;
-        add = tbl[idx];
-      }
-      const float v = capped_score(s[e >> 2][e & 3], scale, softcap) + add;
-      sc[e] = (dist >= 0 && key >= first_key) ? v : -INFINITY;
+      const float v = capped_score(s[e >> 2][e & 3], scale, softcap) + add[e];
+      sc[e] = (key <= pos && key >= first_key) ? v : -INFINITY;
       top = fmaxf(top, sc[e]);
     }
+    if (more) load_bias(next);
     top = fmaxf(top, __shfl_xor(top, 16, 64));
     top = fmaxf(top, __shfl_xor(top, 32, 64));
     const float corr = (top == -INFINITY || m_run == -INFINITY) ? (m_run == -INFINITY ? 0.f : 1.f) : __expf(m_run - top);
@@ -470,18 +489,28 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
       lo[e >> 1] = __builtin_amdgcn_perm(__float_as_uint(rc), __float_as_uint(ra), 0x07060302u);
     }
     const bf16x8 p_hi = __builtin_bit_cast(bf16x8, hi), p_lo = __builtin_bit_cast(bf16x8, lo);
+    const bool ragged = kb + AS_BLOCK - 1 > pos;
 #pragma unroll
     for (int dt = 0; dt < NV; ++dt) {
+      u32x4 raw = {vraw[dt][0][0], vraw[dt][0][1], vraw[dt][1][0], vraw[dt][1][1]};
+      if (ragged) {  // slots behind the token may hold anything
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int key = kb + (e >> 2) * 16 + 4 * grp + (e & 3);
+          if (key > pos) raw[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
+        }
+      }
+      const bf16x8 vf = __builtin_bit_cast(bf16x8, raw);
       floatx4 acc = o[dt];
       acc[0] *= corr; acc[1] *= corr; acc[2] *= corr; acc[3] *= corr;
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], p_hi, acc, 0, 0, 0);
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], p_lo, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p_hi, acc, 0, 0, 0);
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p_lo, acc, 0, 0, 0);
     }
+    if (more) load_values(next, next_page);
   }
   float l = l_run;
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
-  float* mrg = bias_lds + (bias != nullptr ? group * bucket_len : 4);  // [4 waves][group][2 + vdim]
   if (col < group) {
     float* mine = mrg + (wave * group + col) * (2 + vdim);
     if (grp == 0) {
@@ -524,28 +553,41 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
   }
 }
 
-// One wave per (token, head): out = sum_c o_c e^(m_c - m) / sum_c l_c e^(m_c - m), cuts in order.
+// One wave per 64 values of a (token, head): out = sum_c o_c e^(m_c - m) / sum_c l_c e^(m_c - m), cuts in
+// order.  All it does is wait for loads, so sixteen cuts' are sent for together with the maxima and sums.
 __global__ void attention_sink_merge_kernel(bf16_t* __restrict__ out, const float* __restrict__ partial, int items,
                                             int cuts, int vdim) {
-  const int item = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
+  const int chunks = (vdim + 63) / 64;
+  const int unit = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
+  const int item = unit / chunks, d = (unit - item * chunks) * 64 + (threadIdx.x & 63);
   const int lane = threadIdx.x & 63;
   if (item >= items) return;
   const float* src = partial + static_cast<size_t>(item) * cuts * (2 + vdim);
-  // lane c takes cut c's maximum and sum (at most 64 cuts); the values come in a loop whose loads
-  // do not wait for one another
+  // lane c takes cut c's maximum and sum (at most 64 cuts)
   const float mc = lane < cuts ? src[lane * (2 + vdim)] : -INFINITY;
   const float lc = lane < cuts ? src[lane * (2 + vdim) + 1] : 0.f;
+  const bool mine = d < vdim;  // every lane stays in the loop: its weight is read by the others
+  constexpr int BATCH = 16;
+  float part[BATCH];
+  auto load = [&](int c0) {
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {
+      part[j] = 0.f;
+      if (mine && c0 + j < cuts) part[j] = src[(c0 + j) * (2 + vdim) + 2 + d];
+    }
+  };
+  load(0);
   const float m = wave_max(mc);
   const float w = (mc == -INFINITY) ? 0.f : __expf(mc - m);
   const float inv = 1.0f / wave_sum(lc * w);
-  for (int d0 = 0; d0 < vdim; d0 += 64) {  // every lane stays in the loop: its weight is read by the others
-    const int d = d0 + lane;
-    const bool mine = d < vdim;
-    float acc = 0.f;
-#pragma unroll 8
-    for (int c = 0; c < cuts; ++c) acc = fmaf(mine ? src[c * (2 + vdim) + 2 + d] : 0.f, __shfl(w, c, 64), acc);
-    if (mine) out[static_cast<size_t>(item) * vdim + d].bits = float_to_bf16_bits(acc * inv);
+  float acc = 0.f;
+  for (int c0 = 0; c0 < cuts; c0 += BATCH) {
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j)  // beyond the last cut the weight and the value are zero
+      acc = fmaf(part[j], __shfl(w, c0 + j, 64), acc);
+    if (c0 + BATCH < cuts) load(c0 + BATCH);
   }
+  if (mine) out[static_cast<size_t>(item) * vdim + d].bits = float_to_bf16_bits(acc * inv);
 }
 
 // q: bf16 [tokens, n_heads, dim], rows q_stride elements apart; out: bf16 [tokens, n_heads, vdim].
@@ -578,10 +620,8 @@ extern "C" int pylon_attention_sink(void* out, const void* q, long long q_stride
                 "attention_sink: a bias by distance is a table of 1 to %d entries a head", AS_MAX_BIAS);
   PYLON_REQUIRE(cuts >= 1 && cuts <= 64, "attention_sink: 1 to 64 cuts, got %d", cuts);
   const int group = n_heads / n_kv_heads;
-  // single tokens whose group of heads fits a tile's columns and whose bias tables fit LDS: the
-  // kernel with the heads side by side, four partial results a cut
+  // single tokens whose group of heads fits a tile's columns: the kernel with the heads side by side
   const bool side_by_side = tiles == nullptr && group <= 16 &&
-                            (bias == nullptr || static_cast<long long>(group) * bucket_len * 4 <= 64 * 1024) &&
                             (cuts == 1 || (partial != nullptr &&
                                            partial_floats >= static_cast<long long>(tokens) * n_heads * cuts * (2 + vdim)));
   PYLON_REQUIRE(side_by_side || cuts == 1 ||
@@ -591,7 +631,7 @@ extern "C" int pylon_attention_sink(void* out, const void* q, long long q_stride
   if (side_by_side) {
     const long long wgs = static_cast<long long>(tokens) * n_kv_heads * cuts;
     PYLON_REQUIRE(wgs < (1ll << 31), "attention_sink: too many workgroups for one launch");
-    const size_t lds_d = sizeof(float) * ((bias != nullptr ? group * bucket_len : 4) + 4 * group * (2 + vdim));
+    const size_t lds_d = sizeof(float) * 4 * group * (2 + vdim);
     const int ks_d = (dim + 31) / 32, nv_d = (vdim + 15) / 16;
 #define GO_D(KS, NV)                                                                                                \
   do {                                                                                                              \
@@ -617,8 +657,8 @@ extern "C" int pylon_attention_sink(void* out, const void* q, long long q_stride
 #undef PICK_D
 #undef GO_D
     if (cuts > 1) {
-      const int items = tokens * n_heads;
-      hipLaunchKernelGGL(attention_sink_merge_kernel, dim3((items + 3) / 4), dim3(256), 0, stream, (bf16_t*)out,
+      const int items = tokens * n_heads, units = items * ((vdim + 63) / 64);
+      hipLaunchKernelGGL(attention_sink_merge_kernel, dim3((units + 3) / 4), dim3(256), 0, stream, (bf16_t*)out,
                          partial, items, cuts, vdim);
     }
     PYLON_LAUNCHED("attention_sink");
@@ -658,8 +698,8 @@ extern "C" int pylon_attention_sink(void* out, const void* q, long long q_stride
 #undef PICK_NV
 #undef GO
   if (cuts > 1) {
-    const int items = tokens * n_heads;
-    hipLaunchKernelGGL(attention_sink_merge_kernel, dim3((items + 3) / 4), dim3(256), 0, stream, (bf16_t*)out, partial,
+    const int items = tokens * n_heads, units = items * ((vdim + 63) / 64);
+    hipLaunchKernelGGL(attention_sink_merge_kernel, dim3((units + 3) / 4), dim3(256), 0, stream, (bf16_t*)out, partial,
                        items, cuts, vdim);
   }
   PYLON_LAUNCHED("attention_sink");

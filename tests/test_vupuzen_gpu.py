@@ -456,3 +456,33 @@ def test_greedy_generation_through_the_engine(tmp, name, dtype, graphs, page):
             assert produced == int(row.argmax()) or row.max() - row[produced] <= slack * np.abs(row).max(), \
                 (prompt[:3], result.output_ids)
             sequence.append(produced)
+
+
+# more cuts than blocks of keys, one block a wave, several; a group of heads whose bias tables exceed LDS
+@pytest.mark.parametrize("cuts", [1, 3, 16, 17, 64])
+@pytest.mark.parametrize("heads, groups, dim, vdim, buckets", [(8, 2, 128, 128, 0), (16, 1, 64, 200, 4096), (6, 2, 40, 68, 7)])
+@pytest.mark.parametrize("window", [None, 150])
+def test_single_tokens_whose_keys_are_cut(ops, cuts, heads, groups, dim, vdim, buckets, window):
+    page, lengths = 64, (1, 33, 129, 700, 1500)
+    gen = torch.Generator(DEV).manual_seed(heads + cuts)
+    width = -(-max(lengths) // page)
+    k = torch.randn(width, page, groups, dim, generator=gen, device=DEV).bfloat16()
+    v = torch.randn(width, groups, vdim, page, generator=gen, device=DEV).bfloat16()
+    q = torch.randn(len(lengths), heads, dim, generator=gen, device=DEV).bfloat16()
+    table = torch.randperm(width, generator=gen, device=DEV).int().expand(len(lengths), -1).contiguous()
+    bias = torch.randn(heads, buckets, generator=gen, device=DEV) if buckets else None
+    got = ops.attention_sink(q, k, v, table, None, i32([n - 1 for n in lengths]), page_size=page, scale=0.11, bias=bias,
+                             sink=True, cuts=cuts, window=window)
+    for r, n in enumerate(lengths):
+        keys = k[table[r].long()].reshape(-1, groups, dim)[:n].double()
+        values = v[table[r].long()].permute(0, 3, 1, 2).reshape(-1, groups, vdim)[:n].double()
+        first = max(0, n - window) if window else 0
+        for h in range(heads):
+            s = 0.11 * keys[first:, h * groups // heads] @ q[r, h].double()
+            if buckets:
+                s = s + bias[h].double()[(n - 1 - torch.arange(first, n, device=DEV)).clamp(max=buckets - 1)]
+            p = s.exp()
+            want = p @ values[first:, h * groups // heads] / (1.0 + p.sum())
+            # weights as two bfloat16 terms (2^-16 each), float32 sums, the result rounded once (2^-8)
+            room = 1.01 * 2.0 ** -8 * want.abs() + 2.0 ** -13 * (p @ values[first:, h * groups // heads].abs()) / (1.0 + p.sum())
+            assert ((got[r, h].double() - want).abs() <= room + 1e-30).all(), (n, h)
