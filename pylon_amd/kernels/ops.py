@@ -5,7 +5,7 @@ it launches, and launches on torch's current stream.  None has a CPU path.
 """
 from __future__ import annotations
 
-from typing import Optional
+from typing import Optional, Tuple
 
 import torch
 
@@ -1359,7 +1359,8 @@ def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype
 
 def gemm_rows(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype = torch.bfloat16,
               parts: int = 1, col_tiles: int = 1, glu: bool = False, relu2: bool = False, waves: int = 0, cols: int = 0,
-              out: Optional[torch.Tensor] = None, act: str = "silu") -> torch.Tensor:
+              out: Optional[torch.Tensor] = None, act: str = "silu",
+              capped: Optional[Tuple[float, float, float]] = None) -> torch.Tensor:
     """``x @ weight.T`` for at most 128 rows of bfloat16 ``x``: the rows of ``x`` pass through
     LDS once per workgroup of up to 64 (``col_tiles=1``) or 128 (``col_tiles=2``) columns and
     ``weight`` is streamed once (beyond 64 rows each half of the rows has workgroups of its
@@ -1369,7 +1370,10 @@ def gemm_rows(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype =
     (:data:`GATE_ACTS`), rounded once.  ``waves``: wavefronts per workgroup, 4 or 2 (0: the kernel's choice);
     ``cols``: columns per workgroup (0: the kernel's choice, an equal share for every
     workgroup of whole rounds over the compute units where that pays).  The sums depend on
-    neither.  ``relu2``: the result is ``max(x @ weight.T, 0)^2``, rounded once."""
+    neither.  ``relu2``: the result is ``max(x @ weight.T, 0)^2``, rounded once.  ``capped``, with ``glu``:
+    ``(alpha, offset, limit)`` of :func:`gated_act` instead of ``act``; the result is bfloat16."""
+    if capped is not None and not glu:
+        raise KernelError("gemm_rows: only a gate is capped")
     if relu2 and (glu or parts > 1):
         raise KernelError("gemm_rows: the squared relu takes the whole product, and no gate")
     if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
@@ -1391,8 +1395,8 @@ def gemm_rows(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype =
             or not out.is_cuda or not out.is_contiguous():
         raise KernelError(f"gemm_rows: out must be contiguous, on the GPU and of shape {shape}")
     _lib.call("pylon_gemm_rows", out.data_ptr(), dtype_code(out.dtype), x.data_ptr(), weight.data_ptr(),
-              m, n, k, x.stride(0), weight.stride(0), n, parts, m * n, int(col_tiles), _epilogue(glu, relu2, act), int(waves),
-              int(cols), _stream())
+              m, n, k, x.stride(0), weight.stride(0), n, parts, m * n, int(col_tiles),
+              5 if capped else _epilogue(glu, relu2, act), int(waves), int(cols), *(capped or (0.0, 0.0, 0.0)), _stream())
     return out
 
 
@@ -1537,11 +1541,15 @@ def linear_glu(x: torch.Tensor, gate_up: torch.Tensor, *, out_dtype: torch.dtype
 
 def linear_capped(x: torch.Tensor, gate_up: torch.Tensor, *, alpha: float, offset: float, limit: float,
                   out_dtype: torch.dtype) -> torch.Tensor:
-    """:func:`gated_act` of ``x @ gate_up.T`` for a fused ``[2I, K]`` gate/up matrix: on the product's
-    float32 sums up to 128 rows and, beyond 64, in :func:`gemm_wide`'s epilogue; for operands that it does
-    not take the library's product, beyond 128 rows rounded first."""
+    """:func:`gated_act` of ``x @ gate_up.T`` for a fused ``[2I, K]`` gate/up matrix: in the epilogue of the
+    rows kernel where :func:`plan.plan_gated` takes it and, beyond 64 rows, of :func:`gemm_wide`; else on the
+    product's float32 sums up to 128 rows, beyond them on the library's product, rounded first."""
     if out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True):
         return gemm_wide(x, gate_up, epilogue="capped", alpha=alpha, offset=offset, limit=limit)
+    if (out_dtype == torch.bfloat16 and x.is_cuda and x.dim() == 2 and _streaming_ok(x, gate_up, STREAM_ROWS)
+            and gate_up.shape[0] % 2 == 0 and plan.plan_gated(x.shape[0], gate_up.shape[0] // 2, gate_up.shape[1],
+                                                              gate_up.stride(0)).kernel == "rows"):
+        return gemm_rows(x, gate_up, glu=True, capped=(float(alpha), float(offset), float(limit)))
     sums = torch.float32 if x.shape[0] <= SPLIT_ROWS else out_dtype
     return gated_act(linear(x, gate_up, out_dtype=sums), alpha=alpha, offset=offset, limit=limit, out_dtype=out_dtype)
 

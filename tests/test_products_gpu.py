@@ -220,3 +220,23 @@ def test_operands_that_only_the_library_takes_stay_with_it(ops, rows):
     torch.testing.assert_close(ops.linear(one.repeat(rows, 1), w, out_dtype=torch.bfloat16, out=out), apart.float())
     assert ops.linear(one.repeat(rows, 1)[:, :0], w[:, :0]).eq(0).all()
     assert ops.linear(one.repeat(rows, 1), w[:0]).shape == (rows, 0)
+
+
+# the edges of the rows kernel's row tiles and a last workgroup with few columns; a matrix that the plan leaves to
+# the product with the activation kernel behind it (few rows of a small matrix)
+@pytest.mark.parametrize("rows", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("half, k, limit", [(4100, 200, 7.0), (4640, 2560, 2.0), (320, 264, 0.0)])
+def test_a_capped_gate_in_the_products_epilogue(ops, rows, half, k, limit):
+    gen = torch.Generator(DEV).manual_seed(rows + half)
+    x = torch.randn(rows, k, generator=gen, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(2 * half, k + 8, generator=gen, device=DEV) * 0.1).to(torch.bfloat16)[:, :k]
+    got = ops.linear_capped(x, w, alpha=1.702, offset=1.0, limit=limit, out_dtype=torch.bfloat16)
+    behind = ops.gated_act(ops.linear(x, w, out_dtype=torch.float32), alpha=1.702, offset=1.0, limit=limit,
+                           out_dtype=torch.bfloat16)
+    gate, up = (x.double() @ w.double().T).chunk(2, 1)
+    if limit:
+        gate, up = gate.clamp(max=limit), up.clamp(-limit, limit)
+    want = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
+    room = want.abs() * 1.01 * 2.0 ** -8 + want.abs().max() * 2.0 ** -16  # one rounding after float32 sums
+    assert ((got.double() - want).abs() <= room).all()
+    assert ((behind.double() - want).abs() <= room).all()
