@@ -486,3 +486,45 @@ def test_single_tokens_whose_keys_are_cut(ops, cuts, heads, groups, dim, vdim, b
             # weights as two bfloat16 terms (2^-16 each), float32 sums, the result rounded once (2^-8)
             room = 1.01 * 2.0 ** -8 * want.abs() + 2.0 ** -13 * (p @ values[first:, h * groups // heads].abs()) / (1.0 + p.sum())
             assert ((got[r, h].double() - want).abs() <= room + 1e-30).all(), (n, h)
+
+
+# the recurrent kernel of large states (16-byte pieces, 512 threads): rows of S that do not share out evenly, the
+# most rows a thread keeps, columns not in whole wavefronts, one below its least size, columns not in fours
+@pytest.mark.parametrize("form", ["retention", "lightning"])
+@pytest.mark.parametrize("dim, vdim", [(128, 128), (72, 60), (256, 256), (33, 252), (500, 20), (63, 64), (96, 66)])
+def test_recurrent_state_of_every_layout(ops, form, dim, vdim):
+    gen = torch.Generator(DEV).manual_seed(dim + vdim)
+    counts, heads, rot = (1, 3, 0, 2), 3, 0 if form == "lightning" else min(dim, 32) // 2 * 2
+    tokens = sum(counts)
+    proj = torch.randn(tokens, 2 * heads * (dim + vdim), generator=gen, device=DEV)
+    state = torch.randn(6, heads, dim, vdim, generator=gen, device=DEV)
+    decay = torch.tensor([0.5, 0.9, 0.99], device=DEV)
+    inv = torch.rand(rot // 2, generator=gen, device=DEV) if rot else None
+    positions, starts, slots = i32([7, 20, 21, 22, 3, 4]), i32([0, 1, 4, 4, 6]), i32([5, 0, 2, 3])
+    want_state, want = state.double(), torch.zeros(tokens, heads, vdim, dtype=torch.float64, device=DEV)
+    k_scale = 1.0 if form == "lightning" else 0.25
+    t = 0
+    for r, count in enumerate(counts):
+        for _ in range(count):
+            row = proj[t].double()
+            q, k = row[: heads * dim].view(heads, dim), row[heads * dim: 2 * heads * dim].view(heads, dim)
+            v, g = row[2 * heads * dim:].view(2, heads, vdim)
+            if form == "lightning":
+                q, k, v = (torch.nn.functional.silu(a) for a in (q, k, v))
+            else:
+                angle = (positions[t].float() * inv).double()  # the kernel's angle, a float
+                turn = lambda a: torch.cat([a[:, : rot // 2] * angle.cos() - a[:, rot // 2: rot] * angle.sin(),
+                                            a[:, rot // 2: rot] * angle.cos() + a[:, : rot // 2] * angle.sin(), a[:, rot:]], 1)
+                q, k = turn(q), turn(k) * k_scale
+            s = want_state[slots[r]]
+            s.mul_(decay.double().view(-1, 1, 1)).add_(k.unsqueeze(2) * v.unsqueeze(1))
+            o = (s * q.unsqueeze(2)).sum(1)
+            if form == "retention":
+                o = o / (o.square().mean(1, keepdim=True) + 1e-6).sqrt() * torch.nn.functional.silu(g)
+            want[t] = o
+            t += 1
+    got = ops.retention_recurrent(proj, state, decay, inv, positions, starts, slots, rows=len(counts), heads=heads, dim=dim,
+                                  vdim=vdim, rot_dims=rot, eps=1e-6, k_scale=k_scale, form=form)
+    # float32 throughout: chains of at most `dim` terms, a few roundings each
+    torch.testing.assert_close(state.double(), want_state, rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(got.double(), want.flatten(1), rtol=0, atol=float(dim * 2.0 ** -22 * max(1.0, want.abs().max())))
