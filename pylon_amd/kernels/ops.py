@@ -1483,7 +1483,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
                 return gemm_rows(x, weight)
         if out_dtype == torch.float32:
             return _library_float(x, weight, out)
-        if out is None and _wide_ok(x, weight) and plan.wide_beats_library(x.shape[0], weight.shape[0]):
+        if out is None and _wide_ok(x, weight) and plan.wide_beats_library(x.shape[0], *weight.shape):
             y = gemm_wide(x, weight)
             return y if out_dtype == torch.bfloat16 else y.to(out_dtype)
         y = torch.nn.functional.linear(x, weight)
@@ -1525,9 +1525,10 @@ def linear_glu(x: torch.Tensor, gate_up: torch.Tensor, *, out_dtype: torch.dtype
     """``act(x @ gate.T) * (x @ up.T)`` for a fused ``[2I, K]`` gate/up matrix.  The activation works
     on the float32 sums and its result is rounded once: in a streaming kernel's epilogue or, where
     the library is faster, from its float32 result (up to 64 rows: :func:`plan.plan_gated`), beyond in
-    :func:`gemm_wide`'s epilogue.  Operands that kernel does not take: up to 128 rows the library's
+    :func:`gemm_wide`'s epilogue (:func:`plan.wide_gated_beats_library`).  Otherwise: up to 128 rows the library's
     float32 result, more rows its product rounded to bfloat16 first."""
-    if out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True):
+    if (out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True)
+            and plan.wide_gated_beats_library(x.shape[0], gate_up.shape[0] // 2)):
         return gemm_wide(x, gate_up, epilogue=act)
     if _streaming_ok(x, gate_up, SPLIT_ROWS) and x.is_cuda and gate_up.shape[0] % 2 == 0:
         choice = plan.plan_gated(x.shape[0], gate_up.shape[0] // 2, gate_up.shape[1], gate_up.stride(0))

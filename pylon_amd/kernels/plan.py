@@ -179,7 +179,7 @@ def rows_match_library(rows: int, n: int, k: int) -> bool:
     return rows <= 48 and 5120 <= n < TALL and not aliased_rows(k)
 
 
-def wide_beats_library(rows: int, n: int) -> bool:
+def wide_beats_library(rows: int, n: int, k: int) -> bool:
     """Whether a product of more than 64 rows without an activation behind it goes to the engine's own
     tiled kernel (``gemm_wide``) or to the library's.  The own kernel's tile is chosen so that the launch fills
     whole rounds of the compute units; for many rows the library's 256 x 256 tile is the faster main loop where
@@ -192,8 +192,24 @@ def wide_beats_library(rows: int, n: int) -> bool:
     814, 1333, 1681, 1691, 2164.
     q/k/v (6144 wide; 32B 10240): 4B at 100, 250, 1300, 1800, 2048 175, 195, 404, 516, 567 against 158, 187, 395,
     530, 569; 8B at 160, 1024, 1800, 2048 270, 502, 746, 794 against 265, 502, 759, 809; 32B at 2048 1829 against
-    1902."""
+    1902.
+    A matrix at least as deep as wide has few tiles, and between one 64 x 64 tile a unit and a few of them the
+    own kernel, which does not cut K, leaves units waiting: out and down of 4B at 384, 450, 512, 700 tokens 211,
+    231, 234, 280 against 206, 245, 270, 297; of 8B at 260, 384, 512, 640, 700 287, 310, 345, 408, 432 against 310,
+    352, 365, 429, 438; of 32B at 260, 384, 450, 700 563, 609, 767, 927 against 584, 655, 693, 845."""
+    tiles = -(-rows // 64) * -(-n // 64)
+    if k >= n and UNITS < tiles <= (704 if n <= 4096 else 480):
+        return False
+    if n >= 32768 and not wide_gated_beats_library(rows, n // 2):  # a gate/up matrix on its way to the library
+        return False
     return rows <= 1700 or n <= 4096
+
+
+def wide_gated_beats_library(rows: int, n_half: int) -> bool:
+    """The same for gate/up, whose activation the own kernel has in its epilogue: everywhere but for very wide
+    matrices where a third tile of 128 rows (or a second of 256) is begun (layers of 32B at 260, 330, 384, 450
+    tokens 563, 588, 609, 767 us against 551, 604, 630, 754; 8B at 330, 384 299, 310 against 304, 310)."""
+    return not (n_half >= 16384 and 288 < rows <= 384)
 
 
 @lru_cache(maxsize=4096)  # asked for every product of a step

@@ -163,3 +163,19 @@ def test_decode_attention_cuts_the_keys_of_few_long_requests_over_workgroups():
 def test_wide_projections_of_few_prompt_tokens_take_the_rows_kernel(rows, n, k, own):
     assert plan.rows_match_library(rows, n, k) is own
     assert not own or plan.plan_projection(rows, n, k).kernel == "library"  # what it stands in for
+
+
+@pytest.mark.parametrize("rows, n, k, own", [
+    (384, 2560, 9728, True), (385, 2560, 9728, False), (1088, 2560, 4096, False), (1217, 2560, 4096, True),
+    (256, 4096, 4096, True), (257, 4096, 4096, False), (704, 4096, 12288, False), (705, 4096, 12288, True),
+    (384, 5120, 8192, False), (385, 5120, 8192, True), (384, 6144, 2560, True), (1701, 5120, 8192, False),
+    (2048, 4096, 4096, True)])
+def test_prompt_products_that_leave_units_waiting_stay_with_the_library(rows, n, k, own):
+    assert plan.wide_beats_library(rows, n, k) is own
+
+
+@pytest.mark.parametrize("rows, half, own", [(288, 25600, True), (289, 25600, False), (384, 16384, False), (385, 25600, True),
+                                             (330, 12288, True)])
+def test_gated_prompt_products_of_very_wide_matrices(rows, half, own):
+    assert plan.wide_gated_beats_library(rows, half) is own
+    assert own or not plan.wide_beats_library(rows, 2 * half, 5120)  # nor its product alone
