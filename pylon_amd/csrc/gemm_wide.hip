@@ -140,7 +140,8 @@ __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const
     if (GATED && (row & 16)) at += p.N;
     w_at[i] = static_cast<unsigned>(at) * static_cast<unsigned>(p.ldw) * 2u + ((lane & 7) ^ (row & 7)) * 16;
   }
-  // Beyond K the descriptor spans nothing: the load fetches nothing, and every count of loads stays exact.
+  // Beyond K the descriptor spans nothing and the chunk's offset is zero: the load fetches nothing, whether or
+  // not the range check counts the scalar offset, and every count of loads stays exact.
   auto rows_of = [&](bool is_x, int chunk) __attribute__((always_inline)) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(is_x ? xt : wt), 0, chunk < chunks ? 0x7fffffff : 0,
                                              0x00020000);
@@ -148,7 +149,7 @@ __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const
   auto load = [&](__amdgpu_buffer_rsrc_t rows, bool is_x, int chunk, int base, int i) __attribute__((always_inline)) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         rows, (GW_LDS(void)*)(lds + base + (wave * (is_x ? XL : WL) + i) * 1024), 16, is_x ? x_at[i] : w_at[i],
-        chunk * GW_ROW_BYTES, 0, 0);
+        chunk < chunks ? chunk * GW_ROW_BYTES : 0, 0, 0);
   };
 
   // Operands: lane (r, g) takes piece 4 s + g of row r of a tile for turn s.

@@ -109,3 +109,16 @@ def test_infinities_stay_in_their_rows_and_columns(ops):
     keep = torch.ones(100, 72, dtype=torch.bool, device=DEV)
     keep[3], keep[:, 9] = False, False
     assert torch.isfinite(got[keep]).all() and torch.isnan(got[:, 9]).all() and not torch.isfinite(got[3]).any()
+
+
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_operands_that_end_where_their_memory_ends(ops, tile):
+    """Loads ahead of the last chunks of K fetch nothing: the last rows of both operands are the last bytes of
+    allocations of their own (whole multiples of 2 MB, above what the allocator shares out)."""
+    torch.cuda.empty_cache()
+    x = draw(1, 5120, 1024).contiguous()
+    w = draw(2, 5120, 1024).contiguous()
+    got = ops.gemm_wide(x, w, tile=tile)
+    again = ops.gemm_wide(torch.cat([x, x[:8]]), torch.cat([w, w[:8]]), tile=tile)  # with memory behind them
+    assert torch.equal(got, again[:5120, :5120])
+    assert close(got[-300:], wanted(x[-300:], w, "none"))
