@@ -46,6 +46,15 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // What happens to the sums: nothing; act(gate) * up of a fused gate/up matrix; max(v, 0)^2.
 enum GwEpilogue { GW_PLAIN = 0, GW_SILU = 1, GW_RELU2 = 2, GW_GELU = 3, GW_CAPPED = 4 };
 
+// A gate of up to GW_EXACT_ROWS rows is expf and a true division, as in the kernels for fewer rows: up to there
+// the activation of a request's tokens has one precision whatever shares its step.  Beyond, where the other
+// route (the library's product rounded to bfloat16, then the activation) rounds gate and up by 2^-9 first, it is
+// the hardware's exponential and reciprocal, about 2^-22 off: the exact forms make the code of a 128 x 256 tile 46
+// KB instead of 19.  (Gate/up of 100 rows, silu, with them and with the hardware's: 4B 46.6 and 45.6 us, 8B 88.7 and
+// 87.3, 32B 153.0 and 149.9.)
+#define GW_EXACT_ROWS 128
+enum GwGate { GW_NO_GATE = 0, GW_FAST_GATE = 1, GW_EXACT_GATE = 2 };
+
 template <int V>
 using Int = std::integral_constant<int, V>;
 template <typename F, int... I>
@@ -74,31 +83,33 @@ struct GwShape {
   int epilogue;
 };
 
-// Gates of results that are about to be rounded to bfloat16: the hardware's exponential and reciprocal (about
-// one part in 2^22 each).
-__device__ __forceinline__ float gw_sigmoid_times(float z, float slope) {  // z / (1 + exp(-slope z))
-  return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * slope * z));
+// z / (1 + exp(-y)); the fast form about one part in 2^22 off.
+template <bool EXACT>
+__device__ __forceinline__ float gw_gate(float z, float y) {
+  if constexpr (EXACT) return z / (1.0f + expf(-y));
+  return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * y));
 }
+template <bool EXACT>
 __device__ __forceinline__ float gw_gelu(float z) {  // pylon_gelu_tanh
-  const float u = 1.5957691216057308f * fmaf(0.044715f * z * z, z, z);
-  return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * u));
+  return gw_gate<EXACT>(z, 1.5957691216057308f * fmaf(0.044715f * z * z, z, z));
 }
+template <bool EXACT>
 __device__ __forceinline__ float gw_capped(float g, float u, const GwShape& p) {
   if (p.limit > 0.f) {
     g = fminf(g, p.limit);
     u = fminf(fmaxf(u, -p.limit), p.limit);
   }
-  return gw_sigmoid_times(g, p.alpha) * (u + p.offset);
+  return gw_gate<EXACT>(g, p.alpha * g) * (u + p.offset);
 }
 
-// MT, NT: tiles of 16 rows and of 16 columns per wave.  GATED: w is a fused matrix of 2 N rows, gate rows
+// MT, NT: tiles of 16 rows and of 16 columns per wave.  With a gate w is a fused matrix of 2 N rows, gate rows
 // first; a pair of a wave's column tiles is 16 gate rows and their 16 up rows, N rows further down.
 // (The body is a device function: the host pass does not know the descriptor type and would drop a kernel
 // that names it, launch stub and all.)
-template <int MT, int NT, int STAGES, bool GATED>
+template <int MT, int NT, int STAGES, int GATE>
 __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
                                                const uint16_t* __restrict__ w, const GwShape p) {
-  constexpr bool RING = STAGES == 0;
+  constexpr bool RING = STAGES == 0, GATED = GATE != GW_NO_GATE, EXACT = GATE == GW_EXACT_GATE;
   static_assert(!RING || MT == NT, "the ring's places hold x or w");
   static_assert(!GATED || NT % 2 == 0, "a gate tile and its up tile belong to one wave");
   constexpr int TM = 32 * MT, TN = 32 * NT;
@@ -290,11 +301,11 @@ __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const
   };
   if constexpr (GATED) {
     if (p.epilogue == GW_SILU)
-      store([&](float gate, float up) __attribute__((always_inline)) { return pylon_silu_for_bf16(gate) * up; });
+      store([&](float gate, float up) __attribute__((always_inline)) { return gw_gate<EXACT>(gate, gate) * up; });
     else if (p.epilogue == GW_GELU)
-      store([&](float gate, float up) __attribute__((always_inline)) { return gw_gelu(gate) * up; });
+      store([&](float gate, float up) __attribute__((always_inline)) { return gw_gelu<EXACT>(gate) * up; });
     else
-      store([&](float gate, float up) __attribute__((always_inline)) { return gw_capped(gate, up, p); });
+      store([&](float gate, float up) __attribute__((always_inline)) { return gw_capped<EXACT>(gate, up, p); });
   } else if (p.epilogue == GW_RELU2) {
     store([](float v, float) __attribute__((always_inline)) {
       const float pos = fmaxf(v, 0.f);
@@ -312,10 +323,10 @@ constexpr int gw_per_unit() {
   return 2 * bytes <= 160 * 1024 ? 2 : 1;
 }
 
-template <int MT, int NT, int STAGES, bool GATED>
+template <int MT, int NT, int STAGES, int GATE>
 __global__ __launch_bounds__(256, (gw_per_unit<MT, NT, STAGES>())) void gemm_wide_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const GwShape p) {
-  gemm_wide_body<MT, NT, STAGES, GATED>(out, x, w, p);
+  gemm_wide_body<MT, NT, STAGES, GATE>(out, x, w, p);
 }
 
 // The tiles: rows, columns, workgroups per compute unit, and what a chunk of 64 of K costs a workgroup in
@@ -356,6 +367,7 @@ static int gw_choose(int M, int N, int K, bool gated, int units) {
   int best = 0;
   double least = 1e30;
   for (int i = 0; i < kTileCount; ++i) {
+    if (gated && M <= GW_EXACT_ROWS && kTiles[i].rows > GW_EXACT_ROWS) continue;  // these have no exact gate
     const double us = gw_time_us(kTiles[i], M, N, K, gated, units);
     if (us < least) least = us, best = i;
   }
@@ -379,12 +391,21 @@ static void launch_wide(void* out, const void* x, const void* w, GwShape p, hipS
   const int cols = gated ? 16 * NT : 32 * NT;
   p.m_tiles = (p.M + 32 * MT - 1) / (32 * MT), p.n_tiles = (p.N + cols - 1) / cols;
   const dim3 grid((static_cast<unsigned>(p.m_tiles) * p.n_tiles + 7) / 8 * 8), block(256);
-  if (gated)
-    hipLaunchKernelGGL((gemm_wide_kernel<MT, NT, STAGES, true>), grid, block, 0, stream, (uint16_t*)out, (const uint16_t*)x,
-                       (const uint16_t*)w, p);
-  else
-    hipLaunchKernelGGL((gemm_wide_kernel<MT, NT, STAGES, false>), grid, block, 0, stream, (uint16_t*)out, (const uint16_t*)x,
-                       (const uint16_t*)w, p);
+#define GO(GATE)                                                                                                     \
+  hipLaunchKernelGGL((gemm_wide_kernel<MT, NT, STAGES, GATE>), grid, block, 0, stream, (uint16_t*)out, (const uint16_t*)x, \
+                     (const uint16_t*)w, p)
+  if (!gated) {
+    GO(GW_NO_GATE);
+    return;
+  }
+  if constexpr (32 * MT <= GW_EXACT_ROWS) {
+    if (p.M <= GW_EXACT_ROWS) {
+      GO(GW_EXACT_GATE);
+      return;
+    }
+  }
+  GO(GW_FAST_GATE);
+#undef GO
 }
 
 // x: [M, ldx] bf16; w: [N, ldw] bf16, or with a gate [2 N, ldw], gate rows first; out: [M, ldo] bf16, rounded
@@ -406,6 +427,8 @@ extern "C" int pylon_gemm_wide(void* out, const void* x, const void* w, int M, i
   PYLON_REQUIRE(N % 4 == 0 && ldo % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0,
                 "gemm_wide: rows of the result are multiples of 4 elements at 8-byte aligned addresses");
   PYLON_REQUIRE(tile >= -1 && tile < kTileCount, "gemm_wide: there is no tile %d", tile);
+  PYLON_REQUIRE(tile < 0 || !gated || M > GW_EXACT_ROWS || kTiles[tile].rows <= GW_EXACT_ROWS,
+                "gemm_wide: a gate of up to %d rows takes a tile of up to as many rows", GW_EXACT_ROWS);
   PYLON_REQUIRE(static_cast<long long>((M + 63) / 64) * ((N + 31) / 32) < (1ll << 30), "gemm_wide: too many tiles for one launch");
   if (M == 0) return 0;
   if (tile < 0) {

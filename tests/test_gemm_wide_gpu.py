@@ -122,3 +122,28 @@ def test_operands_that_end_where_their_memory_ends(ops, tile):
     again = ops.gemm_wide(torch.cat([x, x[:8]]), torch.cat([w, w[:8]]), tile=tile)  # with memory behind them
     assert torch.equal(got, again[:5120, :5120])
     assert close(got[-300:], wanted(x[-300:], w, "none"))
+
+
+# one non-zero term a sum, so that the sums are exact and the gate alone is compared: up to 128 rows it is the
+# same expf and division as in the activation kernels, to the bit; beyond, the hardware's functions (2^-22, and
+# 2^-24 of the exponent's argument, ahead of the rounding)
+@pytest.mark.parametrize("rows", [65, 128, 129])
+@pytest.mark.parametrize("epilogue", ["silu", "gelu_tanh", "capped"])
+def test_a_gate_keeps_its_precision_up_to_128_rows(ops, rows, epilogue):
+    half, k, constants = 16384, 64, dict(alpha=1.702, offset=1.0, limit=7.0)
+    gen = torch.Generator(DEV).manual_seed(rows)
+    x = torch.zeros(rows, k, device=DEV)
+    x[torch.arange(rows), torch.arange(rows) % k] = 2.0 * torch.rand(rows, generator=gen, device=DEV) + 1.0
+    x, w = x.to(torch.bfloat16), draw(7, 2 * half, k) * 3
+    sums = torch.mm(x, w.t(), out_dtype=torch.float32)
+    if epilogue == "capped":
+        got = ops.linear_capped(x, w, out_dtype=torch.bfloat16, **constants)
+        behind = ops.gated_act(sums, out_dtype=torch.bfloat16, **constants)
+    else:
+        got = ops.linear_glu(x, w, out_dtype=torch.bfloat16, act=epilogue)
+        behind = ops.silu_gate(sums, out_dtype=torch.bfloat16, act=epilogue)
+    assert torch.equal(got, ops.gemm_wide(x, w, epilogue=epilogue, **constants))
+    if rows <= 128:
+        assert torch.equal(got, behind)
+    else:
+        torch.testing.assert_close(got, behind, rtol=2.0 ** -7, atol=1e-30)
