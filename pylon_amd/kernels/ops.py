@@ -1527,6 +1527,8 @@ def linear_glu(x: torch.Tensor, gate_up: torch.Tensor, *, out_dtype: torch.dtype
     the library is faster, from its float32 result (up to 64 rows: :func:`plan.plan_gated`), beyond in
     :func:`gemm_wide`'s epilogue (:func:`plan.wide_gated_beats_library`).  Otherwise: up to 128 rows the library's
     float32 result, more rows its product rounded to bfloat16 first."""
+    if act not in GATE_ACTS:  # also where the kernel has activations without a gate
+        raise KeyError(act)
     if (out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True)
             and plan.wide_gated_beats_library(x.shape[0], gate_up.shape[0] // 2)):
         return gemm_wide(x, gate_up, epilogue=act)
