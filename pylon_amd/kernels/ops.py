@@ -8,6 +8,7 @@ from __future__ import annotations
 from typing import Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from . import library as _lib
 from . import plan
@@ -1405,6 +1406,18 @@ def _rows_apart(t: torch.Tensor) -> bool:
     return t.stride(1) == 1 and t.stride(0) >= t.shape[1] > 0
 
 
+_PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def _watched(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether more is asked of a product than its values: a gradient, a tangent, a batch dimension of vmap, a
+    trace, a dispatch mode.  A kernel launch is seen by none of them."""
+    return (type(x) not in _PLAIN_TENSORS or type(weight) not in _PLAIN_TENSORS
+            or (x.requires_grad or weight.requires_grad) and torch.is_grad_enabled()
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None
+            or forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None)
+
+
 WIDE_CHUNK = 64  # elements of K that the tiled kernel walks at a time
 _WIDE_EPILOGUES = {"none": 0, "silu": 1, "relu2": 2, "gelu_tanh": 3, "capped": 4}
 
@@ -1462,7 +1475,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
     bfloat16 by bfloat16: up to 64 rows go to a weight-streaming kernel where one is faster
     (:func:`plan.plan_projection`), more rows to :func:`gemm_wide` where that is
     (:func:`plan.wide_beats_library`) and else to the library matrix product (as the
-    reference's ``nn.Linear`` does).  With a bfloat16 result the float32 sums are rounded once
+    reference's ``nn.Linear`` does), as does a product that is followed for its gradient, by vmap or by a trace.  With a bfloat16 result the float32 sums are rounded once
     either way; with a float32 result (the logits) they come back unrounded either way (the
     library then writes its float32 sums): what a request's logits are rounded to does not
     depend on how many rows share its step.  Every pairing that involves float32 operands runs
@@ -1479,11 +1492,13 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
             if choice.kernel == "skinny":
                 return gemm_skinny(x, weight, out_dtype=out_dtype, out=out)
             if (out is None and out_dtype == torch.bfloat16 and x.dim() == 2
-                    and plan.rows_match_library(x.shape[0], *weight.shape) and _rows_apart(x) and _rows_apart(weight)):
+                    and plan.rows_match_library(x.shape[0], *weight.shape) and _rows_apart(x) and _rows_apart(weight)
+                    and not _watched(x, weight)):
                 return gemm_rows(x, weight)
         if out_dtype == torch.float32:
             return _library_float(x, weight, out)
-        if out is None and _wide_ok(x, weight) and plan.wide_beats_library(x.shape[0], *weight.shape):
+        if (out is None and not _watched(x, weight) and _wide_ok(x, weight)
+                and plan.wide_beats_library(x.shape[0], *weight.shape)):
             y = gemm_wide(x, weight)
             return y if out_dtype == torch.bfloat16 else y.to(out_dtype)
         y = torch.nn.functional.linear(x, weight)

@@ -3,6 +3,8 @@ refused: on the CPU, with tensors that have a device and a shape but no data."""
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.autograd import forward_ad
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from pylon_amd.kernels import ops
 
@@ -16,3 +18,33 @@ def empty(*shape, dtype=torch.bfloat16):
 def test_what_is_no_gate_is_refused(rows, act):
     with FakeTensorMode(), pytest.raises(KeyError):
         ops.linear_glu(empty(rows, 256), empty(512, 256), out_dtype=torch.bfloat16, act=act)
+
+
+# rows and sizes that reach the tiled kernel, and the rows kernel in the library's stead
+@pytest.mark.parametrize("rows, n, k", [(300, 512, 256), (100, 2560, 4096), (32, 5120, 2560)])
+def test_a_traced_product_is_the_librarys(rows, n, k):
+    with FakeTensorMode():
+        assert ops.linear(empty(rows, k), empty(n, k)).shape == (rows, n)
+
+
+def test_a_product_that_is_followed_is_told_from_one_that_is_not():
+    x, w = torch.ones(3, 4), torch.nn.Parameter(torch.ones(2, 4), requires_grad=False)
+    seen = []
+
+    def ask(a):
+        seen.append(ops._watched(a, w))
+        return a * 2
+
+    ask(x)
+    ask(x.requires_grad_())
+    with torch.no_grad():
+        ask(x)
+    x = x.detach()
+    torch.vmap(ask)(x)
+    torch.func.jvp(ask, (x,), (x,))
+    with forward_ad.dual_level():
+        ask(forward_ad.make_dual(x, x))
+    make_fx(ask)(x)
+    torch.jit.trace(ask, (x,), check_trace=False)
+    ask(x)
+    assert seen == [False, True, False, True, True, True, True, True, False]

@@ -240,3 +240,15 @@ def test_a_capped_gate_in_the_products_epilogue(ops, rows, half, k, limit):
     room = want.abs() * 1.01 * 2.0 ** -8 + want.abs().max() * 2.0 ** -16  # one rounding after float32 sums
     assert ((got.double() - want).abs() <= room).all()
     assert ((behind.double() - want).abs() <= room).all()
+
+
+# one rounding to bfloat16 on either side: 2^-8 of the value each, and float32 sums (2^-16 of the largest)
+@pytest.mark.parametrize("rows, n, k", [(32, 5120, 192), (100, 512, 256)])
+def test_a_product_keeps_its_gradient(ops, rows, n, k):
+    x, w = (torch.randn(r, k, device=DEV).to(torch.bfloat16) for r in (rows, n))
+    x.requires_grad_()
+    y = ops.linear(x, w)
+    y.backward(torch.ones_like(y))
+    torch.testing.assert_close(x.grad.float(), w.float().sum(0).expand(rows, k), rtol=2.0 ** -8, atol=2.0 ** -16 * 300)
+    with torch.no_grad():
+        torch.testing.assert_close(ops.linear(x, w), y.detach(), rtol=2.0 ** -7, atol=2.0 ** -15 * 100)
