@@ -1427,7 +1427,7 @@ def _wide_ok(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool
     kernels hold, K in whole chunks, rows of multiples of 8 elements at 16-byte aligned addresses, results of
     a multiple of 4 columns, and rows of w that one view of 2 GB spans."""
     return (x.shape[0] > STREAM_ROWS and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda
-            and x.dim() == 2 and weight.shape[1] % WIDE_CHUNK == 0 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
+            and x.dim() == 2 and weight.dim() == 2 and weight.shape[1] % WIDE_CHUNK == 0 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and x.stride(0) < 2 ** 22
             and weight.shape[0] % (8 if gated else 4) == 0 and weight.shape[0] > 0 and _rows_apart(x) and _rows_apart(weight)
             and ((weight.shape[0] // 2 if gated else 0) + 256) * weight.stride(0) < 2 ** 30)

@@ -48,3 +48,14 @@ def test_a_product_that_is_followed_is_told_from_one_that_is_not():
     torch.jit.trace(ask, (x,), check_trace=False)
     ask(x)
     assert seen == [False, True, False, True, True, True, True, True, False]
+
+
+def test_a_vector_is_the_librarys():
+    x, w = torch.empty(300, 256, dtype=torch.bfloat16, device="meta"), torch.empty(256, dtype=torch.bfloat16, device="meta")
+
+    class OnTheDevice(torch.Tensor):  # what the checks ask for, and no more
+        is_cuda = True
+
+    assert ops._wide_ok(x.as_subclass(OnTheDevice), w) is False
+    with FakeTensorMode():
+        assert ops.linear(empty(300, 256), empty(256)).shape == (300,)
