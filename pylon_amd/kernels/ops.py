@@ -1418,17 +1418,24 @@ def _watched(x: torch.Tensor, weight: torch.Tensor) -> bool:
             or forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None)
 
 
+def _here(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Both operands on the current device, on whose stream a kernel is launched (the library goes to its operands'
+    device and refuses two)."""
+    here = _raw_device() if _raw_device is not None else torch.cuda.current_device()
+    return x.get_device() == here and weight.get_device() == here
+
+
 WIDE_CHUNK = 64  # elements of K that the tiled kernel walks at a time
 _WIDE_EPILOGUES = {"none": 0, "silu": 1, "relu2": 2, "gelu_tanh": 3, "capped": 4}
 
 
 def _wide_ok(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool:
-    """Operands that :func:`gemm_wide` takes and is meant for: bfloat16, more rows than the streaming
+    """Operands that :func:`gemm_wide` takes and is meant for: bfloat16 on this device, more rows than the streaming
     kernels hold, K in whole chunks, rows of multiples of 8 elements at 16-byte aligned addresses, results of
     a multiple of 4 columns, and rows of w that one view of 2 GB spans."""
     return (x.shape[0] > STREAM_ROWS and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda
-            and x.dim() == 2 and weight.dim() == 2 and weight.shape[1] % WIDE_CHUNK == 0 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and x.stride(0) < 2 ** 22
+            and x.dim() == 2 and weight.dim() == 2 and weight.shape[1] % WIDE_CHUNK == 0
+            and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 and _here(x, weight) and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and x.stride(0) < 2 ** 22
             and weight.shape[0] % (8 if gated else 4) == 0 and weight.shape[0] > 0 and _rows_apart(x) and _rows_apart(weight)
             and ((weight.shape[0] // 2 if gated else 0) + 256) * weight.stride(0) < 2 ** 30)
 
@@ -1445,6 +1452,8 @@ def gemm_wide(x: torch.Tensor, weight: torch.Tensor, *, epilogue: str = "none", 
         raise KernelError("gemm_wide takes bfloat16 operands")
     if not (x.is_cuda and weight.is_cuda) or x.stride(1) != 1 or weight.stride(1) != 1:
         raise KernelError("gemm_wide: operands must be on the GPU with contiguous rows")
+    if not _here(x, weight):
+        raise KernelError("gemm_wide: operands must be on the current device")
     m, k = x.shape
     n = weight.shape[0]
     if epilogue not in ("none", "relu2"):
@@ -1493,7 +1502,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
                 return gemm_skinny(x, weight, out_dtype=out_dtype, out=out)
             if (out is None and out_dtype == torch.bfloat16 and x.dim() == 2
                     and plan.rows_match_library(x.shape[0], *weight.shape) and _rows_apart(x) and _rows_apart(weight)
-                    and not _watched(x, weight)):
+                    and not _watched(x, weight) and _here(x, weight)):
                 return gemm_rows(x, weight)
         if out_dtype == torch.float32:
             return _library_float(x, weight, out)

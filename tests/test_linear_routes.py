@@ -59,3 +59,24 @@ def test_a_vector_is_the_librarys():
     assert ops._wide_ok(x.as_subclass(OnTheDevice), w) is False
     with FakeTensorMode():
         assert ops.linear(empty(300, 256), empty(256)).shape == (300,)
+
+
+@pytest.mark.parametrize("x_on, weight_on, current", [(1, 1, 0), (0, 1, 0), (1, 0, 0), (0, 0, 1)])
+def test_operands_of_other_devices_reach_no_kernel(monkeypatch, x_on, weight_on, current):
+    """The library goes to its operands' device, or refuses two; a launch would go to the current one."""
+    monkeypatch.setattr(ops, "_raw_device", lambda: current)
+    monkeypatch.setattr(ops, "_watched", lambda x, weight: False)
+    launched = []
+    monkeypatch.setattr(ops._lib, "call", lambda name, *args: launched.append(name))
+    with FakeTensorMode():
+        for rows, n, k in ((300, 512, 256), (32, 5120, 2560)):
+            x = torch.empty(rows, k, dtype=torch.bfloat16, device=f"cuda:{x_on}")
+            w = torch.empty(n, k, dtype=torch.bfloat16, device=f"cuda:{weight_on}")
+            if x_on == weight_on:
+                assert ops.linear(x, w).device == x.device
+            else:
+                with pytest.raises(RuntimeError):
+                    ops.linear(x, w)
+            with pytest.raises(ops.KernelError):
+                ops.gemm_wide(x, w)
+    assert not launched
