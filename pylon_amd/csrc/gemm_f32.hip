@@ -36,6 +36,7 @@ typedef int intx4 __attribute__((ext_vector_type(4)));
 #define GF_TILE_BYTES 4096    // 16 rows of one chunk
 #define GF_ROWS 32            // most rows of the streaming kernel
 #define GF_GROUP_TILES 4      // most column tiles of one of its workgroups
+#define GF_ROWS_LDS (GF_RANGES * 2 * GF_TILE_BYTES + GF_GROUP_TILES * GF_RANGES * 2 * 1024)  // most LDS of one
 #define GF_LDS(T) __attribute__((address_space(3))) T
 #define GF_OOB 0x80000000u
 
@@ -395,12 +396,13 @@ bool gemm_f32_launch(float* out, const float* x, const float* w, int M, int N, i
   if (M <= GF_ROWS) {
     const int per = gf_group_tiles(N, units);
     const int mt = M <= 16 ? 1 : 2;
-    const unsigned lds = GF_RANGES * 2 * GF_TILE_BYTES + per * GF_RANGES * mt * 1024;  // at most 128 KB
+    const unsigned lds = GF_RANGES * 2 * GF_TILE_BYTES + per * GF_RANGES * mt * 1024;  // at most GF_ROWS_LDS
     const dim3 grid((N + 16 * per - 1) / (16 * per)), block(GF_RANGES * PYLON_WAVE);
 #define GO(MT)                                                                                                          \
   do {                                                                                                                  \
+    /* one value for every launch: a thread must not lower what another has just set */                                 \
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<MT>),                                 \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);                                         \
+                              hipFuncAttributeMaxDynamicSharedMemorySize, GF_ROWS_LDS);                                 \
     hipLaunchKernelGGL((gemm_f32_rows_kernel<MT>), grid, block, lds, stream, out, x, w, M, N, K, ldx, ldw, ldo, per);    \
   } while (0)
     if (mt == 1) GO(1);

@@ -1,6 +1,8 @@
 """The float32 product (``ops.gemm_tiled`` with float32 operands): every kernel it is made of at the
 edges of their tiles, against a float64 product with the error bound of the order its sums are taken in,
 and one value per element whatever rows share the launch."""
+from concurrent.futures import ThreadPoolExecutor
+
 import pytest
 import torch
 
@@ -73,3 +75,22 @@ def test_numbers_at_the_ends_of_the_range(ops, rows):
     assert got[0, 0].item() == w[0, 0].item() and got[0, 1].item() == w[1, 0].item()
     assert torch.isinf(got[1, 2]) and got[0, 2].item() == 0.0
     assert torch.isnan(got[0, 3]) and torch.isnan(got[1, 0]) and got[0, 4].item() == 0.0
+
+
+def test_threads_with_launches_of_different_sizes(ops):
+    """Every host thread its own stream and shape: what one asks of the device for its kernel (LDS by the number of
+    columns and rows) must hold for the launches of all."""
+    shapes = [(3, 64, 512), (3, 26000, 512), (32, 26000, 512), (20, 300, 512)]
+    operands = [(draw(m, m, k), draw(n, n, k)) for m, n, k in shapes]
+    want = [ops.gemm_tiled(x, w) for x, w in operands]
+    torch.cuda.synchronize()
+
+    def work(i):
+        x, w = operands[i]
+        with torch.cuda.stream(torch.cuda.Stream()):
+            got = [ops.gemm_tiled(x, w) for _ in range(40)]
+            torch.cuda.current_stream().synchronize()
+            return all(torch.equal(g, want[i]) for g in got)
+
+    with ThreadPoolExecutor(len(shapes)) as pool:
+        assert all(pool.map(work, range(len(shapes))))

@@ -64,6 +64,8 @@ def test_a_vector_is_the_librarys():
 @pytest.mark.parametrize("x_on, weight_on, current", [(1, 1, 0), (0, 1, 0), (1, 0, 0), (0, 0, 1)])
 def test_operands_of_other_devices_reach_no_kernel(monkeypatch, x_on, weight_on, current):
     """The library goes to its operands' device, or refuses two; a launch would go to the current one."""
+    if torch.cuda.device_count() == 1:
+        pytest.skip("tensors without data can be put on any device of a machine that has none, or has two")
     monkeypatch.setattr(ops, "_raw_device", lambda: current)
     monkeypatch.setattr(ops, "_watched", lambda x, weight: False)
     launched = []
