@@ -368,6 +368,28 @@ static void launch_tiles(float* out, const float* x, const float* w, int M, int 
   hipLaunchKernelGGL((gemm_f32_tiles_kernel<T, TEAMS>), grid, block, 0, stream, out, x, w, M, N, K, ldx, ldw, ldo, m_tiles, n_tiles);
 }
 
+// Tiles of 64 x 64 for many rows that fill the chip three times over, else of 32 x 32 (us, 64 against
+// 32: 2048 rows 2560 x 9728 993, 1014 and 19456 x 2560 1861, 2057; 600 rows 19456 x 2560 591, 628; but
+// 400 rows 451, 440, 270 rows 2560 x 9728 245, 177 and 64 rows 230, 73; tiles of 128 x 128: 1487, 2024,
+// 606, 596, 743 and 727).  A launch holds less than 2^32 threads: 0 where neither does.
+static int gf_side(int M, int N, int units) {
+  auto fits = [&](int side, int threads) {
+    const long long groups = static_cast<long long>((M + side - 1) / side) * (((N + side - 1) / side + 7) / 8 * 8);
+    return groups * threads < (1ll << 32);
+  };
+  const bool many = M >= 512 && static_cast<long long>((M + 63) / 64) * ((N + 63) / 64) >= 3ll * units;
+  if (!many && fits(32, 512)) return 32;
+  return fits(64, 256) ? 64 : 0;
+}
+
+// The side of the tiles in which a product of these sizes is computed in float32 (units: compute units), 16 for the
+// streaming kernel; 0 where gemm_tiled takes it.  Touches no device.
+extern "C" int pylon_gemm_f32_plan(int M, int N, int units, int* side) {
+  PYLON_REQUIRE(M >= 1 && N >= 1 && units >= 1 && side != nullptr, "gemm_f32_plan: bad arguments");
+  *side = M <= GF_ROWS ? 16 : gf_side(M, N, units);
+  return 0;
+}
+
 // Column tiles per workgroup of the streaming kernel: two workgroups fit a compute unit, so as many
 // tiles as make the launch whole rounds of two per unit (at least one, at most four).
 static int gf_group_tiles(int N, int units) {
@@ -410,14 +432,10 @@ bool gemm_f32_launch(float* out, const float* x, const float* w, int M, int N, i
 #undef GO
     return true;
   }
-  if (static_cast<long long>((M + 31) / 32) * ((N + 31) / 32 + 7) >= (1ll << 31)) return false;
-  // Tiles of 64 x 64 for many rows that fill the chip three times over, else of 32 x 32 (us, 64 against
-  // 32: 2048 rows 2560 x 9728 993, 1014 and 19456 x 2560 1861, 2057; 600 rows 19456 x 2560 591, 628; but
-  // 400 rows 451, 440, 270 rows 2560 x 9728 245, 177 and 64 rows 230, 73; tiles of 128 x 128: 1487, 2024,
-  // 606, 596, 743 and 727).
-  if (M >= 512 && static_cast<long long>((M + 63) / 64) * ((N + 63) / 64) >= 3ll * units)
+  const int side = gf_side(M, N, units);
+  if (side == 64)
     launch_tiles<2, 1>(out, x, w, M, N, K, ldx, ldw, ldo, stream);
-  else
+  else if (side == 32)
     launch_tiles<1, 2>(out, x, w, M, N, K, ldx, ldw, ldo, stream);
-  return true;
+  return side != 0;
 }

@@ -1,9 +1,11 @@
 """The choice of product kernel by shape (pylon_amd/kernels/plan.py): pure functions, checked
 here without a GPU for the sizes of every Qwen3 dense model and for the properties the
 kernels rely on."""
+import ctypes
+
 import pytest
 
-from pylon_amd.kernels import plan
+from pylon_amd.kernels import library, plan
 
 # (hidden, q width, key/value width, feed-forward width) of the published Qwen3 dense sizes
 SIZES = {
@@ -179,3 +181,16 @@ def test_prompt_products_that_leave_units_waiting_stay_with_the_library(rows, n,
 def test_gated_prompt_products_of_very_wide_matrices(rows, half, own):
     assert plan.wide_gated_beats_library(rows, half) is own
     assert own or not plan.wide_beats_library(rows, 2 * half, 5120)  # nor its product alone
+
+
+# a launch holds less than 2^32 threads: the widest of 511 rows in tiles of 32 (512 threads) and one tile more, the
+# largest in tiles of 64 (256 threads) and what is left to the general kernel
+@pytest.mark.parametrize("m, n, side", [
+    (32, 2560, 16), (33, 2560, 32), (511, 2560, 32), (2048, 2560, 64), (511, 524279 * 32, 32),
+    (511, 524280 * 32 + 1, 64), (65536 * 64, 248 * 64, 64), (65535 * 64, 257 * 64, 0)])
+def test_float32_products_that_one_launch_holds(m, n, side):
+    got = ctypes.c_int()
+    assert library.load().pylon_gemm_f32_plan(m, n, 256, ctypes.byref(got)) == 0
+    assert got.value == side
+    if side in (32, 64):
+        assert -(-m // side) * (-(-n // side) + 7 & ~7) * {32: 512, 64: 256}[side] < 2 ** 32
