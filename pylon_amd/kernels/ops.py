@@ -1569,9 +1569,10 @@ def linear_glu(x: torch.Tensor, gate_up: torch.Tensor, *, out_dtype: torch.dtype
 def linear_capped(x: torch.Tensor, gate_up: torch.Tensor, *, alpha: float, offset: float, limit: float,
                   out_dtype: torch.dtype) -> torch.Tensor:
     """:func:`gated_act` of ``x @ gate_up.T`` for a fused ``[2I, K]`` gate/up matrix: in the epilogue of the
-    rows kernel where :func:`plan.plan_gated` takes it and, beyond 64 rows, of :func:`gemm_wide`; else on the
-    product's float32 sums up to 128 rows, beyond them on the library's product, rounded first."""
-    if out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True):
+    rows kernel where :func:`plan.plan_gated` takes it and, beyond 64 rows, of :func:`gemm_wide`
+    (:func:`plan.wide_gated_beats_library`); else on the product's float32 sums up to 128 rows, beyond them on the library's product, rounded first."""
+    if (out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True)
+            and plan.wide_gated_beats_library(x.shape[0], gate_up.shape[0] // 2)):
         return gemm_wide(x, gate_up, epilogue="capped", alpha=alpha, offset=offset, limit=limit)
     if (out_dtype == torch.bfloat16 and x.is_cuda and x.dim() == 2 and _streaming_ok(x, gate_up, STREAM_ROWS)
             and gate_up.shape[0] % 2 == 0 and plan.plan_gated(x.shape[0], gate_up.shape[0] // 2, gate_up.shape[1],

@@ -200,16 +200,18 @@ def wide_beats_library(rows: int, n: int, k: int) -> bool:
     tiles = -(-rows // 64) * -(-n // 64)
     if k >= n and UNITS < tiles <= (704 if n <= 4096 else 480):
         return False
-    if n >= 32768 and not wide_gated_beats_library(rows, n // 2):  # a gate/up matrix on its way to the library
+    if n >= 40960 and not wide_gated_beats_library(rows, n // 2):  # a gate/up matrix on its way to the library
         return False
     return rows <= 1700 or n <= 4096
 
 
 def wide_gated_beats_library(rows: int, n_half: int) -> bool:
-    """The same for gate/up, whose activation the own kernel has in its epilogue: everywhere but for very wide
-    matrices where a third tile of 128 rows (or a second of 256) is begun (layers of 32B at 260, 330, 384, 450
-    tokens 563, 588, 609, 767 us against 551, 604, 630, 754; 8B at 330, 384 299, 310 against 304, 310)."""
-    return not (n_half >= 16384 and 288 < rows <= 384)
+    """The same for gate/up, whose activation (a gate, capped or not) the own kernel has in its epilogue: everywhere
+    but for very wide matrices where a third tile of 160 rows is begun and the library's two of 192 hold them
+    (us that a layer of a prompt step takes longer with the library: 32B, 25600 wide, at 257, 289, 320, 321, 350,
+    384 tokens 14, 17, 16, -18, -17, -21, with a capped gate at 289, 320, 321, 384 11, 7, -18, -23; 17408 wide
+    at 289, 320, 321, 384 18, 17, 16, 15, capped 12, 10, 7, 10; 8B, 12288, at 330, 384 1, 3)."""
+    return not (n_half >= 20480 and 320 < rows <= 384)
 
 
 @lru_cache(maxsize=4096)  # asked for every product of a step

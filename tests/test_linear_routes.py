@@ -1,5 +1,7 @@
 """Which calls of the product entry points reach a kernel of the engine, which the library and which are
 refused: on the CPU, with tensors that have a device and a shape but no data."""
+import warnings
+
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -82,3 +84,32 @@ def test_operands_of_other_devices_reach_no_kernel(monkeypatch, x_on, weight_on,
             with pytest.raises(ops.KernelError):
                 ops.gemm_wide(x, w)
     assert not launched
+
+
+@pytest.fixture
+def routes(monkeypatch):
+    """What the entry points launch or hand to the library, in order; nothing is computed."""
+    seen = []
+    monkeypatch.setattr(ops, "_raw_device", lambda: 0)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_watched", lambda x, weight: False)
+    monkeypatch.setattr(ops, "_dev", lambda t, name, dtype=None: 0)
+    monkeypatch.setattr(ops._lib, "compute_units", lambda: 256)
+    monkeypatch.setattr(ops._lib, "call", lambda name, *args: seen.append(name.removeprefix("pylon_")))
+    real = torch.nn.functional.linear
+    monkeypatch.setattr(torch.nn.functional, "linear", lambda x, w: (seen.append("library"), real(x, w))[1])
+    with FakeTensorMode(), warnings.catch_warnings():
+        warnings.simplefilter("ignore")  # data pointers of tensors without data
+        yield seen
+
+
+# the widest gate/up matrices, where the library's tiles hold what begins a third one of the tiled kernel
+@pytest.mark.parametrize("rows, half, own", [(320, 25600, True), (321, 25600, False), (384, 25600, False), (385, 25600, True),
+                                             (350, 17408, True)])
+def test_gates_of_very_wide_matrices(routes, rows, half, own):
+    x, w = empty(rows, 256), empty(2 * half, 256)
+    ops.linear_capped(x, w, alpha=1.702, offset=1.0, limit=7.0, out_dtype=torch.bfloat16)
+    assert routes == (["gemm_wide"] if own else ["library", "gated_act"])
+    routes.clear()
+    ops.linear_glu(x, w, out_dtype=torch.bfloat16)
+    assert routes == (["gemm_wide"] if own else ["library", "silu_gate"])

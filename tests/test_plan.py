@@ -176,8 +176,8 @@ def test_prompt_products_that_leave_units_waiting_stay_with_the_library(rows, n,
     assert plan.wide_beats_library(rows, n, k) is own
 
 
-@pytest.mark.parametrize("rows, half, own", [(288, 25600, True), (289, 25600, False), (384, 16384, False), (385, 25600, True),
-                                             (330, 12288, True)])
+@pytest.mark.parametrize("rows, half, own", [(288, 25600, True), (320, 25600, True), (321, 25600, False), (384, 20480, False),
+                                             (385, 25600, True), (330, 12288, True), (330, 17408, True)])
 def test_gated_prompt_products_of_very_wide_matrices(rows, half, own):
     assert plan.wide_gated_beats_library(rows, half) is own
     assert own or not plan.wide_beats_library(rows, 2 * half, 5120)  # nor its product alone
