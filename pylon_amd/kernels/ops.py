@@ -5,6 +5,8 @@ it launches, and launches on torch's current stream.  None has a CPU path.
 """
 from __future__ import annotations
 
+import ctypes
+from functools import lru_cache
 from typing import Optional, Tuple
 
 import torch
@@ -1440,6 +1442,19 @@ def _wide_ok(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool
             and ((weight.shape[0] // 2 if gated else 0) + 256) * weight.stride(0) < 2 ** 30)
 
 
+@lru_cache(maxsize=4096)  # asked for every product of a step
+def _wide_us(rows: int, n: int, k: int, units: int) -> float:
+    """The time of :func:`gemm_wide` without a gate by the kernel's own model."""
+    tile, us = ctypes.c_int(), ctypes.c_float()
+    _lib.call("pylon_gemm_wide_plan", rows, n, k, 0, units, ctypes.byref(tile), ctypes.byref(us))
+    return us.value
+
+
+def _wide_relu2_beats_library(rows: int, n: int, k: int) -> bool:
+    units = _lib.compute_units()
+    return plan.wide_relu2_beats_library(rows, n, k, _wide_us(rows, n, k, units), units)
+
+
 def gemm_wide(x: torch.Tensor, weight: torch.Tensor, *, epilogue: str = "none", alpha: float = 1.0, offset: float = 0.0,
               limit: float = 0.0, tile: int = -1, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``x @ weight.T`` for many rows of bfloat16 ``x``, bfloat16 result, rounded once after ``epilogue``:
@@ -1586,10 +1601,13 @@ def linear_relu2(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtyp
     """``max(x @ weight.T, 0)^2``.  Up to 128 bfloat16 rows the activation works on the product's float32
     sums and its result is rounded once: in a streaming kernel's epilogue where one is the faster
     product (:func:`plan.plan_projection`), else from the library's float32 result.  More than 64 rows:
-    in :func:`gemm_wide`'s epilogue, or for operands that it does not take from the library's product,
-    beyond 128 rows rounded first."""
+    in :func:`gemm_wide`'s epilogue, or for operands that it does not take, and where it is the slower one
+    (:func:`plan.wide_relu2_beats_library`), from the library's product, beyond 128 rows rounded first."""
     if out_dtype == torch.bfloat16 and _wide_ok(x, weight):
-        return gemm_wide(x, weight, epilogue="relu2")
+        if _wide_relu2_beats_library(x.shape[0], *weight.shape):
+            return gemm_wide(x, weight, epilogue="relu2")
+        if x.shape[0] > SPLIT_ROWS:
+            return relu2(torch.nn.functional.linear(x, weight), out_dtype=out_dtype)
     if _streaming_ok(x, weight, STREAM_ROWS):
         choice = plan.plan_projection(x.shape[0], *weight.shape)
         if choice.kernel == "rows":
