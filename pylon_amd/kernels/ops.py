@@ -1409,6 +1409,10 @@ def _rows_apart(t: torch.Tensor) -> bool:
 
 
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
+# (a step without a graph asks for every projection and waits for the host: looked up once, 0.6 us a call)
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_transforms = torch._C._functorch.peek_interpreter_stack
+_traced = torch._C._get_tracing_state
 
 
 def _watched(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -1416,8 +1420,8 @@ def _watched(x: torch.Tensor, weight: torch.Tensor) -> bool:
     trace, a dispatch mode.  A kernel launch is seen by none of them."""
     return (type(x) not in _PLAIN_TENSORS or type(weight) not in _PLAIN_TENSORS
             or (x.requires_grad or weight.requires_grad) and torch.is_grad_enabled()
-            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None
-            or forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None)
+            or _dispatch_modes() > 0 or _transforms() is not None or forward_ad._current_level >= 0
+            or _traced() is not None)
 
 
 def _here(x: torch.Tensor, weight: torch.Tensor) -> bool:
