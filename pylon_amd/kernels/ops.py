@@ -1526,7 +1526,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
         if out_dtype == torch.float32:
             return _library_float(x, weight, out)
         if (out is None and not _watched(x, weight) and _wide_ok(x, weight)
-                and plan.wide_beats_library(x.shape[0], *weight.shape)):
+                and plan.wide_beats_library(x.shape[0], *weight.shape, units=_lib.compute_units())):
             y = gemm_wide(x, weight)
             return y if out_dtype == torch.bfloat16 else y.to(out_dtype)
         y = torch.nn.functional.linear(x, weight)

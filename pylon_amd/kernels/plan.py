@@ -179,7 +179,7 @@ def rows_match_library(rows: int, n: int, k: int) -> bool:
     return rows <= 48 and 5120 <= n < TALL and not aliased_rows(k)
 
 
-def wide_beats_library(rows: int, n: int, k: int) -> bool:
+def wide_beats_library(rows: int, n: int, k: int, units: int = UNITS) -> bool:
     """Whether a product of more than 64 rows without an activation behind it goes to the engine's own
     tiled kernel (``gemm_wide``) or to the library's.  The own kernel's tile is chosen so that the launch fills
     whole rounds of the compute units; for many rows the library's 256 x 256 tile is the faster main loop where
@@ -196,9 +196,21 @@ def wide_beats_library(rows: int, n: int, k: int) -> bool:
     A matrix at least as deep as wide has few tiles, and between one 64 x 64 tile a unit and a few of them the
     own kernel, which does not cut K, leaves units waiting: out and down of 4B at 384, 450, 512, 700 tokens 211,
     231, 234, 280 against 206, 245, 270, 297; of 8B at 260, 384, 512, 640, 700 287, 310, 345, 408, 432 against 310,
-    352, 365, 429, 438; of 32B at 260, 384, 450, 700 563, 609, 767, 927 against 584, 655, 693, 845."""
+    352, 365, 429, 438; of 32B at 260, 384, 450, 700 563, 609, 767, 927 against 584, 655, 693, 845.
+    Full portions of a narrow matrix: one round of 128 x 192 tiles that leaves units idle, where the library's 256
+    x 256 tiles come closer to their rate (us that a layer takes longer with the library, out and down of 4B at 1500,
+    1700, 1800, 1900, 2000, 2048 tokens 2, 6, 2, -8, -9, -15; of 8B, at 4096 columns, 15 to 22 from 1900 on).
+
+    The lines are read off whole steps of those widths and of 1024, 2048 and 1024 by 12288; near them either side is
+    the faster one by up to 2 % of a layer.  Whole steps, because up to about 350 tokens a step waits for the host,
+    to which the library's call costs 26 us and this one 10: on the device alone the own kernel, which does not cut
+    K, is the slower one for few rows of a deep matrix (160 rows of 2560 x 9728 58 us against 43, of 512 x 12288 62
+    against 26), in a step it is not (1024 wide models at 129 to 700 tokens 25 to 29 us a layer less, 4B at 200 to 330
+    10)."""
     tiles = -(-rows // 64) * -(-n // 64)
-    if k >= n and UNITS < tiles <= (704 if n <= 4096 else 480):
+    if k >= n and units < tiles <= (704 if n <= 4096 else 480):
+        return False
+    if rows > 1850 and n < 3072:
         return False
     if n >= 40960 and not wide_gated_beats_library(rows, n // 2):  # a gate/up matrix on its way to the library
         return False
