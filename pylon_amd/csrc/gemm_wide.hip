@@ -196,6 +196,7 @@ __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const
   // i = 0 .. SENDS - 1, spread over the first SPREAD products.
   auto turn = [&](auto S, int x_base, int w_base, auto SENDS, auto SPREAD, auto send) __attribute__((always_inline)) {
     constexpr int s = decltype(S)::value, sends = decltype(SENDS)::value, spread = decltype(SPREAD)::value;
+    static_assert(sends <= spread, "at most one load a product");
     __builtin_amdgcn_sched_barrier(0);
     gw_for<PRODUCTS>([&](auto I) __attribute__((always_inline)) {
       constexpr int i = decltype(I)::value;
@@ -204,7 +205,6 @@ __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const
       if constexpr (sends > 0) {
         constexpr int l = (i * sends + spread - 1) / spread;
         if constexpr (l < sends && l * spread / sends == i) send(Int<l>{});
-        if constexpr (sends > spread && l + 1 < sends && (l + 1) * spread / sends == i) send(Int<l + 1>{});
       }
       acc[i / MT][i % MT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][i / MT], xf[s][i % MT], acc[i / MT][i % MT], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
@@ -338,8 +338,6 @@ struct GwTile {
 };
 static const GwTile kTiles[] = {
     {64, 64, 2, 230, 380},      // 2 x 2, five stages
-    {64, 128, 1, 400, 400},     // 2 x 4, six stages
-    {128, 64, 1, 400, 400},     // 4 x 2, six stages
     {128, 128, 1, 580, 600},    // 4 x 4, four stages
     {128, 128, 2, 700, 930},    // 4 x 4, the ring
     {128, 192, 1, 690, 700},    // 4 x 6, three stages
@@ -439,16 +437,14 @@ extern "C" int pylon_gemm_wide(void* out, const void* x, const void* w, int M, i
   const GwShape p{M, N, K, ldx, ldw, ldo, 0, 0, alpha, offset, limit, epilogue};
   switch (tile) {
     case 0: launch_wide<2, 2, 5>(out, x, w, p, stream); break;
-    case 1: launch_wide<2, 4, 6>(out, x, w, p, stream); break;
-    case 2: launch_wide<4, 2, 6>(out, x, w, p, stream); break;
-    case 3: launch_wide<4, 4, 4>(out, x, w, p, stream); break;
-    case 4: launch_wide<4, 4, 0>(out, x, w, p, stream); break;
-    case 5: launch_wide<4, 6, 3>(out, x, w, p, stream); break;
-    case 6: launch_wide<4, 6, 2>(out, x, w, p, stream); break;
-    case 7: launch_wide<3, 8, 3>(out, x, w, p, stream); break;
-    case 8: launch_wide<8, 4, 3>(out, x, w, p, stream); break;
-    case 9: launch_wide<4, 8, 3>(out, x, w, p, stream); break;
-    case 10: launch_wide<5, 8, 3>(out, x, w, p, stream); break;
+    case 1: launch_wide<4, 4, 4>(out, x, w, p, stream); break;
+    case 2: launch_wide<4, 4, 0>(out, x, w, p, stream); break;
+    case 3: launch_wide<4, 6, 3>(out, x, w, p, stream); break;
+    case 4: launch_wide<4, 6, 2>(out, x, w, p, stream); break;
+    case 5: launch_wide<3, 8, 3>(out, x, w, p, stream); break;
+    case 6: launch_wide<8, 4, 3>(out, x, w, p, stream); break;
+    case 7: launch_wide<4, 8, 3>(out, x, w, p, stream); break;
+    case 8: launch_wide<5, 8, 3>(out, x, w, p, stream); break;
     default: launch_wide<8, 8, 0>(out, x, w, p, stream); break;
   }
   PYLON_LAUNCHED("gemm_wide");

@@ -8,7 +8,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
-TILES = [(64, 64), (64, 128), (128, 64), (128, 128), (128, 128), (128, 192), (128, 192), (96, 256), (256, 128), (128, 256),
+TILES = [(64, 64), (128, 128), (128, 128), (128, 192), (128, 192), (96, 256), (256, 128), (128, 256),
          (160, 256), (256, 256)]
 
 

@@ -2,6 +2,7 @@
 here without a GPU for the sizes of every Qwen3 dense model and for the properties the
 kernels rely on."""
 import ctypes
+import random
 
 import pytest
 
@@ -195,3 +196,16 @@ def test_float32_products_that_one_launch_holds(m, n, side):
     assert got.value == side
     if side in (32, 64):
         assert -(-m // side) * (-(-n // side) + 7 & ~7) * {32: 512, 64: 256}[side] < 2 ** 32
+
+
+def test_every_tile_of_the_wide_product_is_the_best_for_some_size():
+    lib, tile, us = library.load(), ctypes.c_int(), ctypes.c_float()
+    count = 0
+    while lib.pylon_gemm_wide(None, None, None, 0, 64, 64, 64, 64, 64, 0, 0.0, 0.0, 0.0, count, None) == 0:  # no rows: no launch
+        count += 1
+    rng, chosen = random.Random(1), set()
+    for _ in range(20000):
+        rows, n, k = rng.randint(65, 2200), 64 * rng.randint(1, 600), 64 * rng.randint(1, 400)
+        assert lib.pylon_gemm_wide_plan(rows, n, k, rng.randint(0, 1), 256, ctypes.byref(tile), ctypes.byref(us)) == 0
+        chosen.add(tile.value)
+    assert chosen == set(range(count)) and count > 1
