@@ -308,8 +308,10 @@ def attention_sink_ok(dtype: torch.dtype, *, head_dim: int, v_dim: int, page_siz
 
 def sink_cuts(tokens: int, n_heads: int, n_kv_heads: int, max_len: int, units: Optional[int] = None) -> int:
     """Workgroups that share the keys of one (token, key/value head) in a step of single tokens:
-    more than one while the launch would leave compute units idle and every cut keeps more than
-    64 keys of the longest request (``max_len`` may be an upper bound).  With the merge behind, at 32 heads of
+    more than one while the launch would leave compute units idle and the longest request (``max_len`` may be
+    an upper bound) has more than 64 keys a cut.  The kernel deals them in whole blocks of 32, as many to each cut:
+    at least three, but for the last cut that gets any, and up to a third of the cuts get none (131 blocks in 64
+    cuts: three each to 44) and leave partial results that weigh nothing.  With the merge behind, at 32 heads of
     128 over 8: 4 requests of 300 keys in 1, 2, 4, 8 cuts 14.0, 13.0, 10.4, 9.9 us; 4 of 1,524 in 4, 8, 16, 32
     18.1, 14.4, 14.1, 19.4; 1 of 8,000 in 8, 16, 32 30.0, 20.1, 16.2; 16 of 1,524 in 2, 4, 8 32.3, 30.3, 33.6; 64
     of 1,000 in 1, 2, 4 63.2, 67.8, 71.2."""

@@ -209,3 +209,21 @@ def test_every_tile_of_the_wide_product_is_the_best_for_some_size():
         assert lib.pylon_gemm_wide_plan(rows, n, k, rng.randint(0, 1), 256, ctypes.byref(tile), ctypes.byref(us)) == 0
         chosen.add(tile.value)
     assert chosen == set(range(count)) and count > 1
+
+
+def test_sink_attention_cuts_the_keys_in_whole_blocks():
+    """What a cut gets of the longest request: three blocks of 32 keys or more, the last one that gets any what is
+    left; at least two thirds of the cuts get some."""
+    ops = pytest.importorskip("pylon_amd.kernels.ops")
+    thresholds = [64 * 2 ** e + d for e in range(13) for d in (-33, -1, 0, 1, 2, 31, 33)]
+    for tokens, heads, kv_heads in ((1, 32, 8), (4, 32, 8), (16, 32, 8), (3, 6, 2), (64, 32, 8)):
+        for length in [300, 129, 4161, 2100] + thresholds:
+            cuts = ops.sink_cuts(tokens, heads, kv_heads, length, 256)
+            assert cuts & (cuts - 1) == 0 and 1 <= cuts <= 64
+            if cuts == 1:
+                continue
+            blocks = -(-length // 32)
+            per = -(-blocks // cuts)
+            with_keys = -(-blocks // per)
+            assert length > 64 * cuts and per >= 3 and 3 * with_keys >= 2 * cuts
+    assert ops.sink_cuts(1, 32, 8, 4161, 256) == 64
