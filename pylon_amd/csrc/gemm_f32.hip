@@ -44,11 +44,13 @@ __device__ __forceinline__ int gf_range_begin(int range, int chunks) {
   return static_cast<int>(static_cast<long long>(range) * chunks / GF_RANGES);
 }
 
-// vmcnt <= N; the other counters are left alone.
+// All but the N loads sent last have landed.  No load passes it: neither one that writes LDS nor one of a pointer
+// that may be written to (x of the streaming kernel, which is not __restrict__ for that reason: loads of one that is
+// are moved to where their values are used, past the wait that counts them).
 template <int N>
 __device__ __forceinline__ void gf_wait_loads() {
   static_assert(N >= 0 && N < 64, "vmcnt has six bits");
-  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 // Every wave's reads of LDS have returned and its loads into LDS have landed.
 __device__ __forceinline__ void gf_barrier() {
@@ -58,7 +60,7 @@ __device__ __forceinline__ void gf_barrier() {
 // The body is a device function: the host pass does not know the descriptor type and would drop a
 // kernel that names it, launch stub and all.
 template <int MT>
-__device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, const float* __restrict__ x,
+__device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, const float* x,
                                                    const float* __restrict__ w, int M, int N, int K, long long ldx,
                                                    long long ldw, long long ldo, int group_tiles) {
   // per wave two stages of one tile of w; then the ranges' sums, [tile][range][row tile][64 lanes][4]
@@ -130,7 +132,6 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
     issue(tile, chunk, stage ^ 1, turn + 1 < turns);
     advance();
     gf_wait_loads<4 * MT + 4>();  // all but the loads just sent
-    asm volatile("" ::: "memory");
     const GF_LDS(unsigned char)* base = (const GF_LDS(unsigned char)*)(stage_base + stage * GF_TILE_BYTES);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -188,7 +189,7 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
 
 template <int MT>
 __global__ __launch_bounds__(GF_RANGES* PYLON_WAVE) void gemm_f32_rows_kernel(
-    float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w, int M, int N, int K,
+    float* __restrict__ out, const float* x, const float* __restrict__ w, int M, int N, int K,
     long long ldx, long long ldw, long long ldo, int group_tiles) {
   gemm_f32_rows_body<MT>(out, x, w, M, N, K, ldx, ldw, ldo, group_tiles);
 }
