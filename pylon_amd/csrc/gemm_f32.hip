@@ -10,13 +10,15 @@
 // which gemm_tiled takes: logits of six layers are 2.6e-6 off 64 bits instead of 6.7e-6.)
 //
 // gemm_f32_rows_kernel, up to 32 rows: a step of a few tokens, bound by reading w once.  A
-// workgroup owns up to four tiles of 16 columns; its eight waves take one of the eight ranges
+// workgroup owns a tile of 16 columns; its eight waves take one of the eight ranges
 // each, so that even a matrix of 2560 rows has 1,280 waves that stream it, and the order of the
 // sums falls out of the order in which the waves' results are added through LDS.  A wave's share
 // of w goes from memory straight into LDS in whole 256-byte row segments (four rows a load;
 // gemm_rows measures what that is worth), one chunk of 16 rows ahead of the one it multiplies; the
 // few rows of x come in operand shape, a chunk ahead too.  No barrier until the end: a wave reads only
-// what it brought.
+// what it brought.  Two workgroups fit a compute unit, and more tiles a workgroup never paid (3 rows, us behind
+// 384 MB of other traffic, 1, 2, 3 and 4 tiles: 2560 x 9728 40, 51, 69, 83; 6144 x 2560 28, 28, 30, 32; 19456 x 2560
+// 66, 70, 70, 81; 151936 x 2560 289, 298, 311, 312).
 //
 // gemm_f32_tiles_kernel, more rows: LDS tiles, a chunk ahead, a wave a quarter of the tile.  One
 // 16-byte read from LDS feeds four matrix instructions of 32 clocks, so the matrix cores (157 TFLOP/s
@@ -35,8 +37,6 @@ typedef int intx4 __attribute__((ext_vector_type(4)));
 #define GF_RANGES 8
 #define GF_TILE_BYTES 4096    // 16 rows of one chunk
 #define GF_ROWS 32            // most rows of the streaming kernel
-#define GF_GROUP_TILES 4      // most column tiles of one of its workgroups
-#define GF_ROWS_LDS (GF_RANGES * 2 * GF_TILE_BYTES + GF_GROUP_TILES * GF_RANGES * 2 * 1024)  // most LDS of one
 #define GF_LDS(T) __attribute__((address_space(3))) T
 #define GF_OOB 0x80000000u
 
@@ -62,21 +62,18 @@ __device__ __forceinline__ void gf_barrier() {
 template <int MT>
 __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, const float* x,
                                                    const float* __restrict__ w, int M, int N, int K, long long ldx,
-                                                   long long ldw, long long ldo, int group_tiles) {
-  // per wave two stages of one tile of w; then the ranges' sums, [tile][range][row tile][64 lanes][4]
-  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+                                                   long long ldw, long long ldo) {
+  // per wave two stages of the tile of w; then the ranges' sums, [range][row tile][64 lanes][4]
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[GF_RANGES * 2 * GF_TILE_BYTES + GF_RANGES * MT * 1024];
   float* sums = reinterpret_cast<float*>(lds + GF_RANGES * 2 * GF_TILE_BYTES);
 
   const int lane = threadIdx.x & (PYLON_WAVE - 1);
   const int range = __builtin_amdgcn_readfirstlane(threadIdx.x / PYLON_WAVE);
   const int r = lane & 15, g = lane >> 4;
-  const int row0 = blockIdx.x * group_tiles * 16;  // first row of w of this workgroup
-  const int rows = (N - row0 < group_tiles * 16) ? N - row0 : group_tiles * 16;
-  const int tiles = (rows + 15) / 16;
+  const int row0 = blockIdx.x * 16;  // first row of w of this workgroup
+  const int rows = (N - row0 < 16) ? N - row0 : 16;
   const int chunks = (K + GF_CHUNK - 1) / GF_CHUNK;
   const int c_begin = gf_range_begin(range, chunks), c_end = gf_range_begin(range + 1, chunks);
-  const int per_tile = c_end - c_begin;
-  const int turns = tiles * per_tile;  // (tile, chunk) pairs, chunks within a tile
 
   const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(w + static_cast<size_t>(row0) * ldw), 0,
@@ -84,20 +81,19 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
   const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(x), 0, static_cast<int>((static_cast<long long>(M - 1) * ldx + K) * 4), 0x00020000);
 
-  // A load brings rows 4 q .. 4 q + 3 of a tile: lane l, for row R = 4 q + l / 16, the 16-byte piece
+  // A load brings rows 4 q .. 4 q + 3 of the tile: lane l, for row R = 4 q + l / 16, the 16-byte piece
   // (l % 16) ^ R, which lies at place l % 16 of that row in LDS: operand reads (lane r takes piece
   // 4 s + g of row r) then fall into different groups of banks.
   const int lrow = lane >> 4, lpos = lane & 15;
   unsigned char* stage_base = lds + range * 2 * GF_TILE_BYTES;
-  auto issue = [&](int tile, int chunk, int stage, bool live) {
+  auto issue = [&](int chunk, int stage) {
     const int k0 = chunk * GF_CHUNK;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int R = 4 * q + lrow;
       const int k = k0 + (lpos ^ R) * 4;
-      const int row = tile * 16 + R;
-      const bool ok = live && row < rows && k < K;
-      const unsigned at = static_cast<unsigned>(row) * static_cast<unsigned>(ldw) * 4u + static_cast<unsigned>(k) * 4u;
+      const bool ok = chunk < c_end && R < rows && k < K;
+      const unsigned at = static_cast<unsigned>(R) * static_cast<unsigned>(ldw) * 4u + static_cast<unsigned>(k) * 4u;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           wres, (GF_LDS(void)*)(stage_base + stage * GF_TILE_BYTES + q * 1024), 16, ok ? at : GF_OOB, 0, 0, 0);
     }
@@ -110,27 +106,21 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  auto load_x = [&](floatx4 (&xv)[MT][4], int chunk, bool live) {
+  auto load_x = [&](floatx4 (&xv)[MT][4], int chunk) {
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int k = chunk * GF_CHUNK + 16 * s + 4 * g;
         const int m = 16 * t + r;
-        const bool ok = live && m < M && k < K;
+        const bool ok = chunk < c_end && m < M && k < K;
         const unsigned at = static_cast<unsigned>(m) * static_cast<unsigned>(ldx) * 4u + static_cast<unsigned>(k) * 4u;
         xv[t][s] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xres, ok ? at : GF_OOB, 0, 0));
       }
   };
-  int tile = 0, chunk = c_begin;  // of the turn that is sent for
-  auto advance = [&]() {
-    if (++chunk == c_end) chunk = c_begin, ++tile;
-  };
-  int done_tile = 0, left = per_tile;  // of the turn that is multiplied: its tile, chunks left of it
-  auto turn_of = [&](int turn, floatx4 (&xv)[MT][4], floatx4 (&x_next)[MT][4], int stage) {
-    load_x(x_next, chunk, turn + 1 < turns);
-    issue(tile, chunk, stage ^ 1, turn + 1 < turns);
-    advance();
+  auto turn_of = [&](int chunk, floatx4 (&xv)[MT][4], floatx4 (&x_next)[MT][4], int stage) {
+    load_x(x_next, chunk + 1);
+    issue(chunk + 1, stage ^ 1);
     gf_wait_loads<4 * MT + 4>();  // all but the loads just sent
     const GF_LDS(unsigned char)* base = (const GF_LDS(unsigned char)*)(stage_base + stage * GF_TILE_BYTES);
 #pragma unroll
@@ -144,38 +134,31 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
     }
     // this wave's reads of the stage are over before the next turn's loads overwrite it
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (--left == 0) {  // the tile's range is done
-      left = per_tile;
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        *reinterpret_cast<floatx4*>(sums + (((done_tile * GF_RANGES + range) * MT + t) * PYLON_WAVE + lane) * 4) = acc[t];
-        acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-      }
-      ++done_tile;
-    }
   };
   floatx4 x_even[MT][4], x_odd[MT][4];
-  load_x(x_even, chunk, true);
-  issue(tile, chunk, 0, true);
-  advance();
-  for (int turn = 0; turn < turns; turn += 2) {
-    turn_of(turn, x_even, x_odd, 0);
-    if (turn + 1 < turns) turn_of(turn + 1, x_odd, x_even, 1);
+  load_x(x_even, c_begin);
+  issue(c_begin, 0);
+  for (int chunk = c_begin; chunk < c_end; chunk += 2) {
+    turn_of(chunk, x_even, x_odd, 0);
+    if (chunk + 1 < c_end) turn_of(chunk + 1, x_odd, x_even, 1);
   }
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+    *reinterpret_cast<floatx4*>(sums + ((range * MT + t) * PYLON_WAVE + lane) * 4) = acc[t];
   gf_barrier();
 
-  // Wave `range` now adds tiles in turn: element (row 16 t + r, column n0 + 4 g + i) of a tile.
+  // Wave t now adds row tile t: element (row 16 t + r, column row0 + 4 g + i).
   const bool wide = (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-  for (int item = range; item < tiles * MT; item += GF_RANGES) {
-    const int tl = item / MT, t = item - tl * MT;
+  if (range < MT) {
+    const int t = range;
     floatx4 half[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int p = 0; p < GF_RANGES; ++p)
       half[p / (GF_RANGES / 2)] +=
-          *reinterpret_cast<const floatx4*>(sums + (((tl * GF_RANGES + p) * MT + t) * PYLON_WAVE + lane) * 4);
+          *reinterpret_cast<const floatx4*>(sums + ((p * MT + t) * PYLON_WAVE + lane) * 4);
     const floatx4 v = half[0] + half[1];
-    const int m = 16 * t + r, n = row0 + tl * 16 + 4 * g;
-    if (m >= M) continue;
+    const int m = 16 * t + r, n = row0 + 4 * g;
+    if (m >= M) return;
     float* p = out + static_cast<size_t>(m) * ldo + n;
     if (wide && n + 3 < N) {
       *reinterpret_cast<floatx4*>(p) = v;
@@ -190,8 +173,8 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
 template <int MT>
 __global__ __launch_bounds__(GF_RANGES* PYLON_WAVE) void gemm_f32_rows_kernel(
     float* __restrict__ out, const float* x, const float* __restrict__ w, int M, int N, int K,
-    long long ldx, long long ldw, long long ldo, int group_tiles) {
-  gemm_f32_rows_body<MT>(out, x, w, M, N, K, ldx, ldw, ldo, group_tiles);
+    long long ldx, long long ldw, long long ldo) {
+  gemm_f32_rows_body<MT>(out, x, w, M, N, K, ldx, ldw, ldo);
 }
 
 // T: tiles of 16 rows and of 16 columns per wave; a workgroup's tile is 32 T by 32 T.  TEAMS: 1, or
@@ -391,15 +374,6 @@ extern "C" int pylon_gemm_f32_plan(int M, int N, int units, int* side) {
   return 0;
 }
 
-// Column tiles per workgroup of the streaming kernel: two workgroups fit a compute unit, so as many
-// tiles as make the launch whole rounds of two per unit (at least one, at most four).
-static int gf_group_tiles(int N, int units) {
-  const long long tiles = (N + 15) / 16;
-  const long long rounds = (tiles + 2ll * units * GF_GROUP_TILES - 1) / (2ll * units * GF_GROUP_TILES);
-  const long long per = (tiles + 2ll * units * rounds - 1) / (2ll * units * rounds);
-  return per < 1 ? 1 : (per > GF_GROUP_TILES ? GF_GROUP_TILES : static_cast<int>(per));
-}
-
 // Whether the kernels of this file take the operands: whole 16-byte pieces of rows, offsets within a
 // workgroup's rows that a buffer descriptor spans, and a chunk of K for every range.  The last is not a
 // matter of time (one row, 512 outputs: 44.0 us at K = 508 in gemm_tiled, 3.1 us at K = 512 here; 300 rows
@@ -417,20 +391,11 @@ bool gemm_f32_launch(float* out, const float* x, const float* w, int M, int N, i
   const int units = pylon_compute_units();
   if (units <= 0) return false;
   if (M <= GF_ROWS) {
-    const int per = gf_group_tiles(N, units);
-    const int mt = M <= 16 ? 1 : 2;
-    const unsigned lds = GF_RANGES * 2 * GF_TILE_BYTES + per * GF_RANGES * mt * 1024;  // at most GF_ROWS_LDS
-    const dim3 grid((N + 16 * per - 1) / (16 * per)), block(GF_RANGES * PYLON_WAVE);
-#define GO(MT)                                                                                                          \
-  do {                                                                                                                  \
-    /* one value for every launch: a thread must not lower what another has just set */                                 \
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_rows_kernel<MT>),                                 \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, GF_ROWS_LDS);                                 \
-    hipLaunchKernelGGL((gemm_f32_rows_kernel<MT>), grid, block, lds, stream, out, x, w, M, N, K, ldx, ldw, ldo, per);    \
-  } while (0)
-    if (mt == 1) GO(1);
-    else GO(2);
-#undef GO
+    const dim3 grid((N + 15) / 16), block(GF_RANGES * PYLON_WAVE);
+    if (M <= 16)
+      hipLaunchKernelGGL((gemm_f32_rows_kernel<1>), grid, block, 0, stream, out, x, w, M, N, K, ldx, ldw, ldo);
+    else
+      hipLaunchKernelGGL((gemm_f32_rows_kernel<2>), grid, block, 0, stream, out, x, w, M, N, K, ldx, ldw, ldo);
     return true;
   }
   const int side = gf_side(M, N, units);

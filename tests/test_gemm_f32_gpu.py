@@ -78,8 +78,7 @@ def test_numbers_at_the_ends_of_the_range(ops, rows):
 
 
 def test_threads_with_launches_of_different_sizes(ops):
-    """Every host thread its own stream and shape: what one asks of the device for its kernel (LDS by the number of
-    columns and rows) must hold for the launches of all."""
+    """Every host thread its own stream and shape, each with launches of other sizes beside it."""
     shapes = [(3, 64, 512), (3, 26000, 512), (32, 26000, 512), (20, 300, 512)]
     operands = [(draw(m, m, k), draw(n, n, k)) for m, n, k in shapes]
     want = [ops.gemm_tiled(x, w) for x, w in operands]
