@@ -94,6 +94,10 @@ def test_products_that_are_led_to_it(ops, rows):
                           (ops.linear_capped(a, b, alpha=1.702, offset=1.0, limit=7.0, out_dtype=torch.bfloat16),
                            wanted(a, b, "capped"))):
             assert close(got, want) or (twice and (got.double() - want).abs().max() <= 2e-2 * want.abs().max())
+    for got, epilogue in ((ops.linear(x, w), "none"), (ops.linear_relu2(x, w, out_dtype=torch.bfloat16), "relu2"),
+                          (ops.linear_glu(x, w, out_dtype=torch.bfloat16), "silu"),
+                          (ops.linear_capped(x, w, alpha=1.702, offset=1.0, limit=7.0, out_dtype=torch.bfloat16), "capped")):
+        assert torch.equal(got, ops.gemm_wide(x, w, epilogue=epilogue, alpha=1.702, offset=1.0, limit=7.0))
     into = torch.empty(rows, 600, dtype=torch.bfloat16, device=DEV)
     assert ops.linear(x, w, out=into) is into and close(into, wanted(x, w, "none"))
     assert close(ops.linear(x, w[:599]), wanted(x, w[:599], "none"))  # columns that are no multiple of 4: the library
@@ -147,3 +151,13 @@ def test_a_gate_keeps_its_precision_up_to_128_rows(ops, rows, epilogue):
         assert torch.equal(got, behind)
     else:
         torch.testing.assert_close(got, behind, rtol=2.0 ** -7, atol=1e-30)
+
+
+@pytest.mark.parametrize("rows", [100, 300])  # the exact gate and the hardware's
+@pytest.mark.parametrize("limit", [0.0, -1.0])
+def test_a_gate_without_caps(ops, rows, limit):
+    x, w = draw(1, rows, 192), draw(2, 160, 192) * 0.5
+    got = ops.gemm_wide(x, w, epilogue="capped", alpha=0.7, offset=0.25, limit=limit)
+    g, u = (x.double() @ w.double().T).chunk(2, 1)
+    assert g.abs().max() > 10  # more than the other tests' cap
+    assert close(got, g * torch.sigmoid(0.7 * g) * (u + 0.25))

@@ -126,3 +126,14 @@ def test_squared_relus_that_the_librarys_tiles_fit(routes, monkeypatch, rows, n,
     monkeypatch.setattr(ops._lib, "call", lambda name, *args: real(*args) if name == "pylon_gemm_wide_plan" else note(name, *args))
     ops.linear_relu2(empty(rows, k), empty(n, k), out_dtype=torch.bfloat16)
     assert routes == (["gemm_wide"] if own else ["library", "relu2"])
+
+
+# out and down of 4B, 8B and 32B sizes: few tiles, whole rounds, full portions; a q/k/v matrix; more than one rule
+@pytest.mark.parametrize("rows, n, k, own", [
+    (160, 2560, 9728, True), (512, 2560, 9728, False), (1300, 2560, 9728, True), (2048, 2560, 9728, False),
+    (2048, 4096, 12288, True), (700, 4096, 4096, False), (1024, 5120, 25600, True), (2048, 5120, 25600, False),
+    (1300, 6144, 4096, True), (2048, 6144, 4096, False)])
+def test_products_of_prompt_portions(routes, rows, n, k, own):
+    ops.linear(empty(rows, k), empty(n, k))
+    ops.linear_for_residual(empty(rows, k), empty(n, k), out_dtype=torch.bfloat16)
+    assert routes == ["gemm_wide" if own else "library"] * 2

@@ -490,13 +490,14 @@ def test_single_tokens_whose_keys_are_cut(ops, cuts, heads, groups, dim, vdim, b
 
 # the recurrent kernel of large states (16-byte pieces, 512 threads): rows of S that do not share out evenly, the
 # most rows a thread keeps, columns not in whole wavefronts, one below its least size, columns not in fours
-@pytest.mark.parametrize("form", ["retention", "lightning"])
+@pytest.mark.parametrize("form, dtype", [("retention", torch.float32), ("lightning", torch.float32),
+                                         ("retention", torch.bfloat16)])
 @pytest.mark.parametrize("dim, vdim", [(128, 128), (72, 60), (256, 256), (33, 252), (500, 20), (63, 64), (96, 66)])
-def test_recurrent_state_of_every_layout(ops, form, dim, vdim):
+def test_recurrent_state_of_every_layout(ops, form, dtype, dim, vdim):
     gen = torch.Generator(DEV).manual_seed(dim + vdim)
     counts, heads, rot = (1, 3, 0, 2), 3, 0 if form == "lightning" else min(dim, 32) // 2 * 2
     tokens = sum(counts)
-    proj = torch.randn(tokens, 2 * heads * (dim + vdim), generator=gen, device=DEV)
+    proj = torch.randn(tokens, 2 * heads * (dim + vdim), generator=gen, device=DEV).to(dtype)
     state = torch.randn(6, heads, dim, vdim, generator=gen, device=DEV)
     decay = torch.tensor([0.5, 0.9, 0.99], device=DEV)
     inv = torch.rand(rot // 2, generator=gen, device=DEV) if rot else None
@@ -525,6 +526,6 @@ def test_recurrent_state_of_every_layout(ops, form, dim, vdim):
             t += 1
     got = ops.retention_recurrent(proj, state, decay, inv, positions, starts, slots, rows=len(counts), heads=heads, dim=dim,
                                   vdim=vdim, rot_dims=rot, eps=1e-6, k_scale=k_scale, form=form)
-    # float32 throughout: chains of at most `dim` terms, a few roundings each
+    # float32 throughout: chains of at most `dim` terms, a few roundings each; the result rounded to its type once
     torch.testing.assert_close(state.double(), want_state, rtol=1e-5, atol=1e-5)
-    torch.testing.assert_close(got.double(), want.flatten(1), rtol=0, atol=float(dim * 2.0 ** -22 * max(1.0, want.abs().max())))
+    torch.testing.assert_close(got.double(), want.flatten(1), rtol=1.01 * 2.0 ** -8 if dtype == torch.bfloat16 else 0, atol=float(dim * 2.0 ** -22 * max(1.0, want.abs().max())))
