@@ -197,9 +197,10 @@ def wide_beats_library(rows: int, n: int, k: int, units: int = UNITS) -> bool:
     own kernel, which does not cut K, leaves units waiting: out and down of 4B at 384, 450, 512, 700 tokens 211,
     231, 234, 280 against 206, 245, 270, 297; of 8B at 260, 384, 512, 640, 700 287, 310, 345, 408, 432 against 310,
     352, 365, 429, 438; of 32B at 260, 384, 450, 700 563, 609, 767, 927 against 584, 655, 693, 845.
-    Full portions of a narrow matrix: one round of 128 x 192 tiles that leaves units idle, where the library's 256
-    x 256 tiles come closer to their rate (us that a layer takes longer with the library, out and down of 4B at 1500,
-    1700, 1800, 1900, 2000, 2048 tokens 2, 6, 2, -8, -9, -15; of 8B, at 4096 columns, 15 to 22 from 1900 on).
+    Full portions of a narrow matrix: one round of 128 x 192 tiles that leaves units idle, where the library has a
+    tile that suits 2048 rows, and none for the few that decode beside them (us that a layer takes longer with the
+    library, out and down of 4B at 1500, 1700, 1800, 1900, 2000, 2048, 2049, 2056, 2112 tokens 2, 6, 2, -8, -9, -15, 10,
+    9, 7; of 8B, at 4096 columns, 6 to 20 from 1900 on).
 
     The lines are read off whole steps of those widths and of 1024, 2048 and 1024 by 12288; near them either side is
     the faster one by up to 2 % of a layer.  Whole steps, because up to about 350 tokens a step waits for the host,
@@ -210,7 +211,7 @@ def wide_beats_library(rows: int, n: int, k: int, units: int = UNITS) -> bool:
     tiles = -(-rows // 64) * -(-n // 64)
     if k >= n and units < tiles <= (704 if n <= 4096 else 480):
         return False
-    if rows > 1850 and n < 3072:
+    if 1850 < rows <= 2048 and n < 3072:
         return False
     if n >= 40960 and not wide_gated_beats_library(rows, n // 2):  # a gate/up matrix on its way to the library
         return False

@@ -173,6 +173,7 @@ def test_wide_projections_of_few_prompt_tokens_take_the_rows_kernel(rows, n, k, 
     (256, 4096, 4096, True), (257, 4096, 4096, False), (704, 4096, 12288, False), (705, 4096, 12288, True),
     (384, 5120, 8192, False), (385, 5120, 8192, True), (384, 6144, 2560, True), (1701, 5120, 8192, False),
     (2048, 4096, 4096, True), (1850, 2560, 9728, True), (1851, 2560, 9728, False), (2048, 2560, 4096, False),
+    (2049, 2560, 9728, True),
     (2048, 3072, 4096, True)])
 def test_prompt_products_that_leave_units_waiting_stay_with_the_library(rows, n, k, own):
     assert plan.wide_beats_library(rows, n, k) is own
