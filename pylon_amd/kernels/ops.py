@@ -1407,7 +1407,7 @@ def gemm_rows(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype =
 
 def _rows_apart(t: torch.Tensor) -> bool:
     """Rows that hold something, do not overlap (an expanded row does) and are contiguous."""
-    return t.stride(1) == 1 and t.stride(0) >= t.shape[1] > 0
+    return t.is_contiguous() and t.size(1) > 1 or t.stride(1) == 1 and t.stride(0) >= t.size(1) > 0
 
 
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
@@ -1429,8 +1429,7 @@ def _watched(x: torch.Tensor, weight: torch.Tensor) -> bool:
 def _here(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Both operands on the current device, on whose stream a kernel is launched (the library goes to its operands'
     device and refuses two)."""
-    here = _raw_device() if _raw_device is not None else torch.cuda.current_device()
-    return x.get_device() == here and weight.get_device() == here
+    return x.get_device() == weight.get_device() == (_raw_device or torch.cuda.current_device)()
 
 
 WIDE_CHUNK = 64  # elements of K that the tiled kernel walks at a time
