@@ -1415,12 +1415,13 @@ _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 _dispatch_modes = torch._C._len_torch_dispatch_stack
 _transforms = torch._C._functorch.peek_interpreter_stack
 _traced = torch._C._get_tracing_state
+_compiled = torch.compiler.is_dynamo_compiling  # which the compiler knows: it looks into none of the others
 
 
 def _watched(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether more is asked of a product than its values: a gradient, a tangent, a batch dimension of vmap, a
-    trace, a dispatch mode.  A kernel launch is seen by none of them."""
-    return (type(x) not in _PLAIN_TENSORS or type(weight) not in _PLAIN_TENSORS
+    trace, a compiled graph, a dispatch mode.  A kernel launch is seen by none of them."""
+    return (_compiled() or type(x) not in _PLAIN_TENSORS or type(weight) not in _PLAIN_TENSORS
             or (x.requires_grad or weight.requires_grad) and torch.is_grad_enabled()
             or _dispatch_modes() > 0 or _transforms() is not None or forward_ad._current_level >= 0
             or _traced() is not None)

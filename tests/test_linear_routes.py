@@ -29,6 +29,17 @@ def test_a_traced_product_is_the_librarys(rows, n, k):
         assert ops.linear(empty(rows, k), empty(n, k)).shape == (rows, n)
 
 
+def test_a_compiled_product_is_the_librarys():
+    """All of it one graph: a check that the compiler cannot see through would refuse or break it."""
+    graphs = []
+    with FakeTensorMode():
+        x, w = empty(300, 256), empty(512, 256)
+    compiled = torch.compile(lambda a, b: ops.linear(a, b), fullgraph=True, dynamic=False,
+                             backend=lambda graph, example: graphs.append(graph) or graph.forward)
+    assert compiled(x, w).shape == (300, 512)
+    assert [node.target for node in graphs[0].graph.nodes if node.op == "call_function"] == [torch.nn.functional.linear]
+
+
 def test_a_product_that_is_followed_is_told_from_one_that_is_not():
     x, w = torch.ones(3, 4), torch.nn.Parameter(torch.ones(2, 4), requires_grad=False)
     seen = []
