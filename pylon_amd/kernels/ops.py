@@ -1443,7 +1443,8 @@ def _wide_ok(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool
     a multiple of 4 columns, and rows of w that one view of 2 GB spans."""
     return (x.shape[0] > STREAM_ROWS and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda
             and x.dim() == 2 and weight.dim() == 2 and weight.shape[1] % WIDE_CHUNK == 0
-            and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 and _here(x, weight) and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and x.stride(0) < 2 ** 22
+            and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 and x.stride(0) < 2 ** 22 and _here(x, weight)
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
             and weight.shape[0] % (8 if gated else 4) == 0 and weight.shape[0] > 0 and _rows_apart(x) and _rows_apart(weight)
             and ((weight.shape[0] // 2 if gated else 0) + 256) * weight.stride(0) < 2 ** 30)
 
@@ -1505,7 +1506,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
     bfloat16 by bfloat16: up to 64 rows go to a weight-streaming kernel where one is faster
     (:func:`plan.plan_projection`), more rows to :func:`gemm_wide` where that is
     (:func:`plan.wide_beats_library`) and else to the library matrix product (as the
-    reference's ``nn.Linear`` does), as does a product that is followed for its gradient, by vmap or by a trace.  With a bfloat16 result the float32 sums are rounded once
+    reference's ``nn.Linear`` does), as does a product that is followed for its gradient, by
+    vmap, a trace or the compiler.  With a bfloat16 result the float32 sums are rounded once
     either way; with a float32 result (the logits) they come back unrounded either way (the
     library then writes its float32 sums): what a request's logits are rounded to does not
     depend on how many rows share its step.  Every pairing that involves float32 operands runs
@@ -1591,7 +1593,8 @@ def linear_capped(x: torch.Tensor, gate_up: torch.Tensor, *, alpha: float, offse
                   out_dtype: torch.dtype) -> torch.Tensor:
     """:func:`gated_act` of ``x @ gate_up.T`` for a fused ``[2I, K]`` gate/up matrix: in the epilogue of the
     rows kernel where :func:`plan.plan_gated` takes it and, beyond 64 rows, of :func:`gemm_wide`
-    (:func:`plan.wide_gated_beats_library`); else on the product's float32 sums up to 128 rows, beyond them on the library's product, rounded first."""
+    (:func:`plan.wide_gated_beats_library`); else on the product's float32 sums up to 128 rows, beyond
+    them on the product (:func:`linear`) rounded first."""
     if (out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True)
             and plan.wide_gated_beats_library(x.shape[0], gate_up.shape[0] // 2)):
         return gemm_wide(x, gate_up, epilogue="capped", alpha=alpha, offset=offset, limit=limit)

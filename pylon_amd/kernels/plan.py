@@ -116,7 +116,8 @@ def plan_residual(rows: int, n: int, k: int, units: int = UNITS) -> Product:
 
 @lru_cache(maxsize=4096)  # asked for every product of a step
 def plan_projection(rows: int, n: int, k: int) -> Product:
-    """Any other product (q/k/v; the vocabulary head); beyond 64 rows the library's.
+    """Any other product (q/k/v; the vocabulary head) of up to 64 rows; what it leaves to the library and what has
+    more rows may still go to a kernel (:func:`rows_match_library`, :func:`wide_beats_library`).
 
     A head (tall matrix): the rows kernel with 128 columns per workgroup (151936 x 2560: 137 us
     against the skinny kernel's 154 at 8 rows; 173 against the library's 186 at 64 rows, 150

@@ -14,22 +14,22 @@ units, unless that would make it re-read more rows of x than it streams rows of 
 =========  ========================  =====================================  ===================
 product    1, 8, 16 rows             17, 48, 64 rows                        130 rows
 =========  ========================  =====================================  ===================
-4b qkv     rows CT1 2w 256x1 c24     rows CT1 up to 48 rows, then library   library, bfloat16
-4b out     rows CT1 4w 64x4 c40      rows CT1 4w 64x4 c40 at 17 rows,       library, bfloat16
+4b qkv     rows CT1 2w 256x1 c24     rows CT1 up to 48 rows, then library   gemm_wide
+4b out     rows CT1 4w 64x4 c40      rows CT1 4w 64x4 c40 at 17 rows,       gemm_wide
                                      40x4 c64 at 48 and 64
-4b gate/up rows GLU 4w 256x1 c38     rows GLU 4w 256x1 c38                  library + silu_gate
-4b down    rows CT1 4w 64x4 c40      rows CT2 4w 32x8 c80                   library, bfloat16
+4b gate/up rows GLU 4w 256x1 c38     rows GLU 4w 256x1 c38                  gemm_wide, silu
+4b down    rows CT1 4w 64x4 c40      rows CT2 4w 32x8 c80                   gemm_wide
 4b head    rows CT2 4w 1277x1 c119   rows CT2 4w 1187x1 c128                library, float32
-8b qkv     rows CT1 2w 256x1 c24     library                                library
-8b out     rows CT1 4w 64x4 c64      rows CT1 4w 64x4 c64                   library
-8b gate/up skinny GLU                rows GLU 4w 256x1 c48                  library + silu_gate
-8b down    rows CT1 4w 64x4 c64      rows CT2 4w 32x8 c128                  library
+8b qkv     rows CT1 2w 256x1 c24     library                                gemm_wide
+8b out     rows CT1 4w 64x4 c64      rows CT1 4w 64x4 c64                   gemm_wide
+8b gate/up skinny GLU                rows GLU 4w 256x1 c48                  gemm_wide, silu
+8b down    rows CT1 4w 64x4 c64      rows CT2 4w 32x8 c128                  gemm_wide
 8b head    rows CT1 4w 2533x1 c60    rows CT1 4w 2374x1 c64 at 17 rows,     library, float32
                                      library float32 at 48 and 64
-32b qkv    rows CT1 4w 256x1 c40     rows CT1 up to 48 rows, then library   library
-32b out    rows CT2 4w 64x4 c80      rows CT2 4w 64x4 c80                   library
-32b g/u    rows GLU 4w 512x1 c50     rows GLU 4w 512x1 c50                  library + silu_gate
-32b down   rows CT2 4w 64x4 c80      rows CT2 4w 64x4 c80                   library
+32b qkv    rows CT1 4w 256x1 c40     rows CT1 up to 48 rows, then library   gemm_wide
+32b out    rows CT2 4w 64x4 c80      rows CT2 4w 64x4 c80                   gemm_wide
+32b g/u    rows GLU 4w 512x1 c50     rows GLU 4w 512x1 c50                  gemm_wide, silu
+32b down   rows CT2 4w 64x4 c80      rows CT2 4w 64x4 c80                   gemm_wide
 32b head   rows CT2 4w 1277x1 c119   rows CT2 4w 1187x1 c128                library, float32
 =========  ========================  =====================================  ===================
 
@@ -40,7 +40,7 @@ as above.
 
 65 and 128 rows: the rows of x go as two halves, each to workgroups of its own, with the choices
 of 64 rows, for out, down and the q/k/v that a consumer adds; gate/up, the head and a plain q/k/v
-go to the library as at 130 rows.
+go where they go at 130 rows.
 """
 import ctypes
 import zlib
