@@ -5,8 +5,6 @@ it launches, and launches on torch's current stream.  None has a CPU path.
 """
 from __future__ import annotations
 
-import ctypes
-from functools import lru_cache
 from typing import Optional, Tuple
 
 import torch
@@ -1449,19 +1447,6 @@ def _wide_ok(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool
             and ((weight.shape[0] // 2 if gated else 0) + 256) * weight.stride(0) < 2 ** 30)
 
 
-@lru_cache(maxsize=4096)  # asked for every product of a step
-def _wide_us(rows: int, n: int, k: int, units: int) -> float:
-    """The time of :func:`gemm_wide` without a gate by the kernel's own model."""
-    tile, us = ctypes.c_int(), ctypes.c_float()
-    _lib.call("pylon_gemm_wide_plan", rows, n, k, 0, units, ctypes.byref(tile), ctypes.byref(us))
-    return us.value
-
-
-def _wide_relu2_beats_library(rows: int, n: int, k: int) -> bool:
-    units = _lib.compute_units()
-    return plan.wide_relu2_beats_library(rows, n, k, _wide_us(rows, n, k, units), units)
-
-
 def gemm_wide(x: torch.Tensor, weight: torch.Tensor, *, epilogue: str = "none", alpha: float = 1.0, offset: float = 0.0,
               limit: float = 0.0, tile: int = -1, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``x @ weight.T`` for many rows of bfloat16 ``x``, bfloat16 result, rounded once after ``epilogue``:
@@ -1592,11 +1577,12 @@ def linear_glu(x: torch.Tensor, gate_up: torch.Tensor, *, out_dtype: torch.dtype
 def linear_capped(x: torch.Tensor, gate_up: torch.Tensor, *, alpha: float, offset: float, limit: float,
                   out_dtype: torch.dtype) -> torch.Tensor:
     """:func:`gated_act` of ``x @ gate_up.T`` for a fused ``[2I, K]`` gate/up matrix: in the epilogue of the
-    rows kernel where :func:`plan.plan_gated` takes it and, beyond 64 rows, of :func:`gemm_wide`
-    (:func:`plan.wide_gated_beats_library`); else on the product's float32 sums up to 128 rows, beyond
-    them on the product (:func:`linear`) rounded first."""
-    if (out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True)
-            and plan.wide_gated_beats_library(x.shape[0], gate_up.shape[0] // 2)):
+    rows kernel where :func:`plan.plan_gated` takes it and, beyond 64 rows, of :func:`gemm_wide`; for operands
+    that it does not take on the product's float32 sums up to 128 rows, beyond them on the product
+    (:func:`linear`) rounded first.  (Where :func:`linear_glu` leaves a gate to the library this one stays: 350 rows
+    of 2 x 25600 x 5120 250 us against 225, but 1.7e-3 off 64 bits against 2.8e-3, and on the library's float32
+    result, as close, 246; at 384 rows 254, 235 and 260.)"""
+    if out_dtype == torch.bfloat16 and _wide_ok(x, gate_up, gated=True):
         return gemm_wide(x, gate_up, epilogue="capped", alpha=alpha, offset=offset, limit=limit)
     if (out_dtype == torch.bfloat16 and x.is_cuda and x.dim() == 2 and _streaming_ok(x, gate_up, STREAM_ROWS)
             and gate_up.shape[0] % 2 == 0 and plan.plan_gated(x.shape[0], gate_up.shape[0] // 2, gate_up.shape[1],
@@ -1610,13 +1596,13 @@ def linear_relu2(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtyp
     """``max(x @ weight.T, 0)^2``.  Up to 128 bfloat16 rows the activation works on the product's float32
     sums and its result is rounded once: in a streaming kernel's epilogue where one is the faster
     product (:func:`plan.plan_projection`), else from the library's float32 result.  More than 64 rows:
-    in :func:`gemm_wide`'s epilogue, or for operands that it does not take, and where it is the slower one
-    (:func:`plan.wide_relu2_beats_library`), from the library's product, beyond 128 rows rounded first."""
+    in :func:`gemm_wide`'s epilogue, or for operands that it does not take from the library's product,
+    beyond 128 rows rounded first.  (The library's tiles fill their rounds better at some counts, but a sum that
+    is rounded before it is squared is 3.7e-3 off 64 bits instead of 1.7e-3, and its float32 result costs what
+    it gains: 18432 x 4096 at 512, 576, 1344 rows 101, 103, 196 us here, 95, 95, 184 rounded first, 104, 108, 222 not;
+    38400 x 5120 at 512, 570, 960 250, 256, 375 here, 224, 228, 339 and 249, 264, 404.)"""
     if out_dtype == torch.bfloat16 and _wide_ok(x, weight):
-        if _wide_relu2_beats_library(x.shape[0], *weight.shape):
-            return gemm_wide(x, weight, epilogue="relu2")
-        if x.shape[0] > SPLIT_ROWS:
-            return relu2(torch.nn.functional.linear(x, weight), out_dtype=out_dtype)
+        return gemm_wide(x, weight, epilogue="relu2")
     if _streaming_ok(x, weight, STREAM_ROWS):
         choice = plan.plan_projection(x.shape[0], *weight.shape)
         if choice.kernel == "rows":

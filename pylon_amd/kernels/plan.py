@@ -220,24 +220,12 @@ def wide_beats_library(rows: int, n: int, k: int, units: int = UNITS) -> bool:
 
 
 def wide_gated_beats_library(rows: int, n_half: int) -> bool:
-    """The same for gate/up, whose activation (a gate, capped or not) the own kernel has in its epilogue: everywhere
+    """The same for gate/up, whose activation the own kernel has in its epilogue: everywhere
     but for very wide matrices where a third tile of 160 rows is begun and the library's two of 192 hold them
     (us that a layer of a prompt step takes longer with the library: 32B, 25600 wide, at 257, 289, 320, 321, 350,
-    384 tokens 14, 17, 16, -18, -17, -21, with a capped gate at 289, 320, 321, 384 11, 7, -18, -23; 17408 wide
-    at 289, 320, 321, 384 18, 17, 16, 15, capped 12, 10, 7, 10; 8B, 12288, at 330, 384 1, 3)."""
+    384 tokens 14, 17, 16, -18, -17, -21; 17408 wide at 289, 320, 321, 384 18, 17, 16, 15; 8B, 12288, at 330, 384 1, 3).
+    Not asked by :func:`ops.linear_capped` and :func:`ops.linear_relu2`, which keep their float32 sums."""
     return not (n_half >= 20480 and 320 < rows <= 384)
-
-
-def wide_relu2_beats_library(rows: int, n: int, k: int, own_us: float, units: int = UNITS) -> bool:
-    """The same for a product with the squared relu behind it, whose time in the own kernel its model puts at
-    ``own_us``: against the library's whole rounds of tiles of 192 x 256, 1.28 us for every 64 of K.  The own
-    kernel has no tile between 160 and 256 rows, and where the library's fill their rounds it is the slower one
-    though it saves the activation's launch (us that a layer of a prompt step takes longer with the library: 18432
-    x 4096 at 470, 530, 560, 580, 1024, 1344, 1856 tokens 6, -10, -12, 11, 22, -13, 4; 38400 x 5120 at 450, 500, 530,
-    570, 640, 832, 960, 1000, 2048 21, -22, -33, -20, 40, -23, -27, 48, 62).  For short K that launch weighs more
-    (14592 x 2560 at 704, 1024, 1300, 1500 tokens 4, 17, 35, 8)."""
-    rounds = -(-(-(-rows // 192) * -(-n // 256)) // units)
-    return k < 4096 or own_us < rounds * (k / 64 * 1.28 + 3.5)
 
 
 @lru_cache(maxsize=4096)  # asked for every product of a step
