@@ -26,8 +26,8 @@
 // rows still reaches every compute unit's matrix cores, by two teams of four waves with half of K each.
 //
 // Measured, 4B layer sizes, weights from memory, gemm_tiled (one chain per element on the vector ALUs)
-// before: the products of a step of 3 rows 16 + 12 + 42 + 23 us and the head 269 (5.8 TB/s) where a
-// launch took 615 on average; 270 rows 106 + 79 + 299 + 177 (80 to 90 TFLOP/s); 2048 rows 112 TFLOP/s.
+// before: of a step of 3 rows q/k/v 14 us, gate/up 35 (5.7 TB/s), out and down 34 together, the head 247 (6.3)
+// where a launch took 615 on average; 270 rows 106 + 79 + 299 + 177 (80 to 90 TFLOP/s); 2048 rows 112 TFLOP/s.
 #include "gemm_f32.h"
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
