@@ -6,13 +6,13 @@ static int decode_run_by_head_dim(int head_dim, AD_RUN_ARGS) {
   switch (head_dim / 64) {
     case 1:
       return pylon_decode_run_64(mode, out, q, k_cache, v_cache, block_table, table_width, tok_row, positions, tokens,
-                                 n_heads, n_kv_heads, page_size, window, scale, n_waves, prep, n_cuts, partial, stream);
+                                 n_heads, n_kv_heads, page_size, window, scale, n_waves, prep, n_cuts, partial, cache_slots, stream);
     case 2:
       return pylon_decode_run_128(mode, out, q, k_cache, v_cache, block_table, table_width, tok_row, positions, tokens,
-                                  n_heads, n_kv_heads, page_size, window, scale, n_waves, prep, n_cuts, partial, stream);
+                                  n_heads, n_kv_heads, page_size, window, scale, n_waves, prep, n_cuts, partial, cache_slots, stream);
     default:
       return pylon_decode_run_256(mode, out, q, k_cache, v_cache, block_table, table_width, tok_row, positions, tokens,
-                                  n_heads, n_kv_heads, page_size, window, scale, n_waves, prep, n_cuts, partial, stream);
+                                  n_heads, n_kv_heads, page_size, window, scale, n_waves, prep, n_cuts, partial, cache_slots, stream);
   }
 }
 
@@ -49,13 +49,14 @@ static int check_decode_geometry(const char* name, int tokens, int n_heads, int 
 
 // q, out: [tokens, n_heads, head_dim] bf16; n_waves (1, 2, 4 or 8) wavefronts share
 // the keys of one (token, key/value head), after n_cuts workgroups have shared them first
-// (n_cuts > 1 needs `partial`, scratch of pylon_attention_decode_scratch_floats floats).
+// (n_cuts > 1 needs `partial`, scratch of pylon_attention_decode_scratch_floats floats).  cache_slots: slots of
+// a cache, for which the addresses' arithmetic is chosen (0: any number).
 extern "C" int pylon_attention_decode(void* out, const void* q, const void* k_cache, const void* v_cache,
                                       const int* block_table, int table_width, const int* tok_row,
                                       const int* positions, int tokens, int n_heads, int n_kv_heads,
                                       int head_dim, int page_size, int window, float scale, int n_waves,
                                       int n_cuts, float* partial, long long partial_floats,
-                                      hipStream_t stream) {
+                                      long long cache_slots, hipStream_t stream) {
   if (check_decode_geometry("attention_decode", tokens, n_heads, n_kv_heads, head_dim, page_size, table_width,
                             window, n_waves) ||
       check_decode_cuts("attention_decode", tokens, n_heads, head_dim, n_cuts, partial, partial_floats))
@@ -64,7 +65,7 @@ extern "C" int pylon_attention_decode(void* out, const void* q, const void* k_ca
   const DecodePrep none = {};
   decode_run_by_head_dim(head_dim, AD_MODE_QUERIES, out, q, const_cast<void*>(k_cache), const_cast<void*>(v_cache),
                          block_table, table_width, tok_row, positions, tokens, n_heads, n_kv_heads, page_size, window,
-                         scale, n_waves, none, n_cuts, partial, stream);
+                         scale, n_waves, none, n_cuts, partial, cache_slots, stream);
   PYLON_LAUNCHED("attention_decode");
 }
 
@@ -81,7 +82,8 @@ extern "C" int pylon_attention_decode_fused(void* out, const void* qkv, long lon
                                             const int* tok_row, const int* positions, int tokens,
                                             int n_heads, int n_kv_heads, int head_dim, int page_size,
                                             int window, float scale, int n_waves, int n_cuts,
-                                            float* partial, long long partial_floats, hipStream_t stream) {
+                                            float* partial, long long partial_floats, long long cache_slots,
+                                            hipStream_t stream) {
   if (check_decode_geometry("attention_decode_fused", tokens, n_heads, n_kv_heads, head_dim, page_size,
                             table_width, window, n_waves) ||
       check_decode_cuts("attention_decode_fused", tokens, n_heads, head_dim, n_cuts, partial, partial_floats))
@@ -98,6 +100,6 @@ extern "C" int pylon_attention_decode_fused(void* out, const void* qkv, long lon
   const DecodePrep prep = {qkv, row_stride, qkv_parts, part_stride, q_weight, k_weight, eps, inv_freq, slot_map};
   decode_run_by_head_dim(head_dim, qkv_parts > 0 ? AD_MODE_PARTIAL_SUMS : AD_MODE_PROJECTION, out, nullptr, k_cache,
                          v_cache, block_table, table_width, tok_row, positions, tokens, n_heads, n_kv_heads, page_size,
-                         window, scale, n_waves, prep, n_cuts, partial, stream);
+                         window, scale, n_waves, prep, n_cuts, partial, cache_slots, stream);
   PYLON_LAUNCHED("attention_decode_fused");
 }

@@ -3,5 +3,5 @@
 
 int pylon_decode_run_64(AD_RUN_ARGS) {
   return decode_run<1>(mode, out, q, k_cache, v_cache, block_table, table_width, tok_row, positions, tokens, n_heads,
-                       n_kv_heads, page_size, window, scale, n_waves, prep, n_cuts, partial, stream);
+                       n_kv_heads, page_size, window, scale, n_waves, prep, n_cuts, partial, cache_slots, stream);
 }

@@ -86,75 +86,125 @@ __device__ __forceinline__ void load8_bf16(const uint16_t* __restrict__ src, flo
   }
 }
 
-// v = the sum of n_parts float vectors of 8 (32-byte aligned), stride elements apart, added in
-// order and rounded to bfloat16 once.  For the usual counts every load is issued before the
-// first addition.
-__device__ __forceinline__ void sum8_parts(const float* __restrict__ src, int n_parts, long long stride, float v[8]) {
-  auto take = [&](int p, float4& a, float4& b) {
-    const float4* at = reinterpret_cast<const float4*>(src + p * stride);
-    a = at[0], b = at[1];
-  };
-  float4 lo, hi;
-  if (n_parts == 2 || n_parts == 4) {
-    float4 a[4], b[4];
+// Eight elements of a projection's row, sent for (load) some time before they are needed (sum): bfloat16
+// ones, or with PARTS the sum of n_parts float vectors (32-byte aligned), stride elements apart, added in
+// order and rounded to bfloat16 once.  The first four parts are on their way together.
+template <bool PARTS>
+struct RawHead {
+  uint4 bits;
+  __device__ __forceinline__ void load(const void* src, size_t at, int, long long) {
+    bits = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(src) + at);
+  }
+  __device__ __forceinline__ void sum(const void*, size_t, int, long long, float v[8]) const {
+    const uint32_t w[4] = {bits.x, bits.y, bits.z, bits.w};
 #pragma unroll
-    for (int p = 0; p < 4; ++p) take(p < n_parts ? p : 0, a[p], b[p]);
-    lo = a[0], hi = b[0];
-#pragma unroll
-    for (int p = 1; p < 4; ++p) {
-      if (p < n_parts) {
-        lo.x += a[p].x, lo.y += a[p].y, lo.z += a[p].z, lo.w += a[p].w;
-        hi.x += b[p].x, hi.y += b[p].y, hi.z += b[p].z, hi.w += b[p].w;
-      }
-    }
-  } else {
-    take(0, lo, hi);
-    for (int p = 1; p < n_parts; ++p) {
-      float4 a, b;
-      take(p, a, b);
-      lo.x += a.x, lo.y += a.y, lo.z += a.z, lo.w += a.w;
-      hi.x += b.x, hi.y += b.y, hi.z += b.z, hi.w += b.w;
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(w[i] << 16);
+      v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
     }
   }
-  const float sums[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+};
+template <>
+struct RawHead<true> {
+  float4 lo[4], hi[4];
+  __device__ __forceinline__ void load(const void* src, size_t at, int n_parts, long long stride) {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(static_cast<uint32_t>(float_to_bf16_bits(sums[e])) << 16);
-}
+    for (int p = 0; p < 4; ++p) {
+      const float4* from = reinterpret_cast<const float4*>(static_cast<const float*>(src) + at + (p < n_parts ? p : 0) * stride);
+      lo[p] = from[0], hi[p] = from[1];
+    }
+  }
+  __device__ __forceinline__ void sum(const void* src, size_t at, int n_parts, long long stride, float v[8]) const {
+    float4 a = lo[0], b = hi[0];
+    auto add = [&](const float4& c, const float4& d) __attribute__((always_inline)) {
+      a.x += c.x, a.y += c.y, a.z += c.z, a.w += c.w;
+      b.x += d.x, b.y += d.y, b.z += d.z, b.w += d.w;
+    };
+    if (n_parts > 1) add(lo[1], hi[1]);
+    if (n_parts > 2) add(lo[2], hi[2]);
+    if (n_parts > 3) add(lo[3], hi[3]);
+    for (int p = 4; p < n_parts; ++p) {
+      const float4* from = reinterpret_cast<const float4*>(static_cast<const float*>(src) + at + p * stride);
+      add(from[0], from[1]);
+    }
+    const float sums[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(static_cast<__bf16>(sums[e]));
+  }
+};
 
 __device__ __forceinline__ void store8_bf16(uint16_t* __restrict__ dst, const float v[8]) {
-  uint32_t w[4];
+  typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+  bf16x8_t w;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    w[i] = static_cast<uint32_t>(float_to_bf16_bits(v[2 * i])) |
-           (static_cast<uint32_t>(float_to_bf16_bits(v[2 * i + 1])) << 16);
-  *reinterpret_cast<uint4*>(dst) = uint4{w[0], w[1], w[2], w[3]};
+  for (int e = 0; e < 8; ++e) w[e] = static_cast<__bf16>(v[e]);  // the hardware's: to nearest, ties to even
+  *reinterpret_cast<bf16x8_t*>(dst) = w;
 }
 
-// v: elements 8j .. 8j+7 of a head.  weight: the head's RMSNorm weight or null (per lane:
-// heads in one wave may differ).  cs: the token's rotation table or null.
+// v of another lane of the same row of 16, by a DPP control.
+template <int CTRL>
+__device__ __forceinline__ float lanes_turned(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+
+// Sum over the LPH (8, 16 or 32) lanes that share a head, in every lane: neighbours, pairs, quads, halves of a row
+// of 16, rows change places (the additions of a butterfly over lane ^ 1, 2, 4, 8, 16, without a trip through LDS).
+template <int LPH>
+__device__ __forceinline__ float head_sum(float v) {
+  static_assert(LPH == 8 || LPH == 16 || LPH == 32, "head sizes 64, 128, 256");
+  v += lanes_turned<0xB1>(v);
+  v += lanes_turned<0x4E>(v);
+  v += lanes_turned<0x141>(v);
+  if constexpr (LPH >= 16) v += lanes_turned<0x140>(v);
+  if constexpr (LPH >= 32) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  return v;
+}
+
+// v: elements 8j .. 8j+7 of a head.  weight: those of the head's RMSNorm weight, if it is `weighted`;
+// `rotated`: whether the head is (both per lane: heads in one wave may differ).  cs: the token's rotation
+// table, or null for the whole wave.
 template <int HD>
-__device__ __forceinline__ void norm_rotate8(float v[8], int j, const float* __restrict__ weight, float eps,
-                                             const float* __restrict__ cs) {
+__device__ __forceinline__ void norm_rotate8_with(float v[8], int j, bool weighted, const float weight[8], float eps,
+                                                  bool rotated, const float* __restrict__ cs) {
   constexpr int LPH = HD / 8;
   float ss = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
-#pragma unroll
-  for (int off = 1; off < LPH; off <<= 1) ss += __shfl_xor(ss, off, PYLON_WAVE);
-  if (weight != nullptr) {
+  ss = head_sum<LPH>(ss);
+  if (weighted) {
     const float inv = 1.0f / sqrtf(ss / static_cast<float>(HD) + eps);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = (v[e] * inv) * weight[8 * j + e];
+    for (int e = 0; e < 8; ++e) v[e] = (v[e] * inv) * weight[e];
   }
-  const bool rotate = cs != nullptr;
-  const bool low = j < LPH / 2;
-  const int pair0 = 8 * (j & (LPH / 2 - 1));
+  if (cs != nullptr) {
+    const bool low = j < LPH / 2;
+    const int pair0 = 8 * (j & (LPH / 2 - 1));
+    float other[8], c[8], sn[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float other = __shfl_xor(v[e], LPH / 2, PYLON_WAVE);
-    if (rotate) {
-      const float c = cs[pair0 + e], sn = cs[HD / 2 + pair0 + e];
-      v[e] = low ? v[e] * c - other * sn : v[e] * c + other * sn;
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (LPH == 16)
+        other[e] = lanes_turned<0x128>(v[e]);  // eight lanes further on in the row of 16
+      else
+        other[e] = __shfl_xor(v[e], LPH / 2, PYLON_WAVE);
+      c[e] = cs[pair0 + e], sn[e] = cs[HD / 2 + pair0 + e];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float turned = low ? v[e] * c[e] - other[e] * sn[e] : v[e] * c[e] + other[e] * sn[e];
+      v[e] = rotated ? turned : v[e];
     }
   }
+}
+
+// The same with the weights (or null) still in memory.
+template <int HD>
+__device__ __forceinline__ void norm_rotate8(float v[8], int j, const float* __restrict__ weight, float eps,
+                                             bool rotated, const float* __restrict__ cs) {
+  float own[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) own[e] = weight != nullptr ? weight[8 * j + e] : 0.f;
+  norm_rotate8_with<HD>(v, j, weight != nullptr, own, eps, rotated, cs);
 }

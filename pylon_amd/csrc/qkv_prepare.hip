@@ -194,7 +194,7 @@ __global__ __launch_bounds__(QKV_WAVES* PYLON_WAVE) void qkv_prepare_rows_kernel
     }
     float v[8];
     load8_bf16(src, v);
-    norm_rotate8<HD>(v, j, weight, eps, (rotate && inv_freq != nullptr) ? cs : nullptr);
+    norm_rotate8<HD>(v, j, weight, eps, rotate, inv_freq != nullptr ? cs : nullptr);
     if (valid && dst != nullptr) store8_bf16(dst, v);
   }
 }

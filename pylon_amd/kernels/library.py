@@ -52,8 +52,8 @@ _SIGNATURES = {
     "pylon_add_sinusoid": [P, P, P, I, I, P],
     "pylon_add_bias": [P, I, P, L, I, P],
     "pylon_scale": [P, L, F, P],
-    "pylon_attention_decode": [P, P, P, P, P, I, P, P, I, I, I, I, I, I, F, I, I, P, L, P],
-    "pylon_attention_decode_fused": [P, P, L, I, L, P, P, F, P, P, P, P, P, I, P, P, I, I, I, I, I, I, F, I, I, P, L, P],
+    "pylon_attention_decode": [P, P, P, P, P, I, P, P, I, I, I, I, I, I, F, I, I, P, L, L, P],
+    "pylon_attention_decode_fused": [P, P, L, I, L, P, P, F, P, P, P, P, P, I, P, P, I, I, I, I, I, I, F, I, I, P, L, L, P],
     "pylon_attention_prefill": [P, P, P, P, P, I, P, I, I, I, I, I, I, F, I, P],
     "pylon_gemm_tiled": [P, I, P, I, P, I, I, I, I, L, L, L, P],
     "pylon_gemm_skinny": [P, I, P, P, I, I, I, L, L, L, I, L, I, P],

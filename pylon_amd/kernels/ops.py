@@ -1155,7 +1155,7 @@ def attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
               _dev(tok_row, "tok_row", torch.int32), _dev(positions, "positions", torch.int32),
               tokens, n_heads, n_kv_heads, head_dim, page_size, mask_code(window, chunk), float(scale),
               int(n_splits), int(n_cuts), _dev(scratch, "scratch"), 0 if scratch is None else scratch.numel(),
-              _stream())
+              pages * page_size, _stream())
     return out
 
 
@@ -1221,7 +1221,7 @@ def attention_decode_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
               block_table.shape[1], _dev(tok_row, "tok_row", torch.int32),
               _dev(positions, "positions", torch.int32), tokens, n_heads, n_kv_heads, head_dim, page_size,
               int(window or 0), float(scale), int(n_splits), int(n_cuts), _dev(scratch, "scratch"),
-              0 if scratch is None else scratch.numel(), _stream())
+              0 if scratch is None else scratch.numel(), pages * page_size, _stream())
     return out
 
 

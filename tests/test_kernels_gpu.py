@@ -844,6 +844,45 @@ def test_sampling_where_most_of_the_row_has_no_mass(ops):
             assert first[r] == int(kept[0]) and last[r] == int(kept[-1]), (temp, top_p, r, first[r], last[r])
 
 
+# groups of every size at which the kernel takes its heads together, and of sizes between; keys around whole batches of
+# 32 and 64, around none, and beyond what the waves hold at once; pages of no power of two; cuts of no power of two
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+@pytest.mark.parametrize("heads, kv_heads", [(3, 3), (4, 2), (6, 2), (4, 1), (5, 1), (16, 2), (9, 1), (16, 1)])
+def test_decode_attention_at_its_edges(ops, head_dim, heads, kv_heads):
+    from pylon_amd.kernels import library
+
+    lengths = [1, 2, 32, 33, 34, 65, 66, 130, 257, 700]
+    for page, window, splits, cuts in ((16, None, 8, 1), (48, None, 2, 3), (24, 100, 4, 1), (64, None, 1, 2)):
+        per = -(-max(lengths) // page)
+        gen = torch.Generator(DEV).manual_seed(head_dim + heads + page)
+        tokens = len(lengths)
+        q = torch.randn(tokens, heads, head_dim, generator=gen, device=DEV).to(torch.bfloat16) * 2
+        kc = torch.randn(tokens * per, page, kv_heads, head_dim, generator=gen, device=DEV).to(torch.bfloat16)
+        vc = torch.randn(tokens * per, page, kv_heads, head_dim, generator=gen, device=DEV).to(torch.bfloat16)
+        table = torch.randperm(tokens * per, generator=gen, device=DEV).to(torch.int32).view(tokens, per)
+        positions = torch.tensor([n - 1 for n in lengths], dtype=torch.int32, device=DEV)
+        got = ops.attention_decode(q, kc, vc, table, None, positions, page_size=page, window=window,
+                                   scale=head_dim ** -0.5, n_splits=splits, n_cuts=cuts)
+        for t, n in enumerate(lengths):
+            rows = (table[t].long()[:, None] * page + torch.arange(page, device=DEV)).reshape(-1)[:n]
+            rows = rows if window is None else rows[-window:]
+            k = kc.view(-1, kv_heads, head_dim)[rows].double().repeat_interleave(heads // kv_heads, 1)
+            v = vc.view(-1, kv_heads, head_dim)[rows].double().repeat_interleave(heads // kv_heads, 1)
+            p = torch.softmax((k * q[t].double()[None]).sum(-1) * head_dim ** -0.5, 0)
+            want = (p[:, :, None] * v).sum(0)
+            # one rounding to bfloat16, and float scores of up to about 20 (2^-24 of them in the exponent) before it
+            room = want.abs() * 1.01 * 2.0 ** -8 + want.abs().max() * 2.0 ** -16
+            assert bool(((got[t].double() - want).abs() <= room).all()), (page, window, splits, cuts, n)
+        # the addresses' arithmetic for caches beyond 4 GB (the last number: slots of a cache, 0 for any)
+        far = torch.empty_like(got)
+        scratch = torch.empty(tokens * heads * cuts * (head_dim + 2), device=DEV)
+        assert library.load().pylon_attention_decode(
+            far.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), table.data_ptr(), per, None, positions.data_ptr(),
+            tokens, heads, kv_heads, head_dim, page, window or 0, head_dim ** -0.5, splits, cuts,
+            scratch.data_ptr() if cuts > 1 else None, scratch.numel(), 0, torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(far, got)
+
+
 @pytest.mark.parametrize("geom", [(8, 2, 128, True, True), (6, 6, 64, True, False), (5, 1, 256, False, True),
                                   (16, 1, 64, True, True), (3, 3, 128, False, False)])
 @pytest.mark.parametrize("store", [True, False])
