@@ -62,16 +62,31 @@ __device__ __forceinline__ float pylon_gate_act(float z, int act) {
   return act == PYLON_ACT_GELU ? pylon_gelu_tanh(z) : pylon_silu(z);
 }
 
-// Sum / max over the 64 lanes of a wavefront; every lane gets the result.
+// v of another lane of the same row of 16, by a DPP control.
+template <int CTRL>
+__device__ __forceinline__ float lanes_turned(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+
+// Over the 64 lanes of a wavefront; every lane gets the result, and the same bits: a butterfly over neighbours,
+// pairs, quads, halves of a row of 16, rows, halves of the wave, on the vector unit (six trips through LDS with
+// shuffles, about 130 clocks each).
+template <typename OP>
+__device__ __forceinline__ float wave_over(float v, OP op) {
+  v = op(v, lanes_turned<0xB1>(v));   // lane ^ 1
+  v = op(v, lanes_turned<0x4E>(v));   // lane ^ 2
+  v = op(v, lanes_turned<0x141>(v));  // lane ^ 7, whose quad holds the same
+  v = op(v, lanes_turned<0x140>(v));  // lane ^ 15, whose half of the row holds the same
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return op(__uint_as_float(h[0]), __uint_as_float(h[1]));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = PYLON_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, PYLON_WAVE);
-  return v;
+  return wave_over(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = PYLON_WAVE / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, PYLON_WAVE));
-  return v;
+  return wave_over(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // The first key that a token at position pos sees, for the one integer by which the attention

@@ -141,12 +141,6 @@ __device__ __forceinline__ void store8_bf16(uint16_t* __restrict__ dst, const fl
   *reinterpret_cast<bf16x8_t*>(dst) = w;
 }
 
-// v of another lane of the same row of 16, by a DPP control.
-template <int CTRL>
-__device__ __forceinline__ float lanes_turned(float v) {
-  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xf, 0xf, true));
-}
-
 // Sum over the LPH (8, 16 or 32) lanes that share a head, in every lane: neighbours, pairs, quads, halves of a row
 // of 16, rows change places (the additions of a butterfly over lane ^ 1, 2, 4, 8, 16, without a trip through LDS).
 template <int LPH>
