@@ -47,6 +47,7 @@ HIPCC_FLAGS = [
 EXTRA_FLAGS = {
     "attention_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "attention_latent.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "gemm_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],  # else its few sums change registers and back every chunk
 }
 
 

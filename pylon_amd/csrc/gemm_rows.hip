@@ -31,10 +31,20 @@
 // as others.)
 //
 // All loads go through buffer descriptors (of the workgroup's rows of w; of x): rows beyond
-// N or M and elements beyond K are read as zeros without a memory access and without a
-// branch, so every wave issues the same number of loads per chunk and the counted waits
-// are exact.
+// N or M are read as zeros without a memory access and without a branch, so every wave
+// issues the same number of loads per chunk and the counted waits are exact.
+//
+// A launch of a few microseconds is mostly its start and its end, and with one wavefront on a
+// SIMD every instruction takes four clocks or more: a load is two instructions (its offset
+// within the chunk is computed once, the chunk's is scalar), what is asked before the first
+// load comes with the launch, and nothing is sent beyond the range.  With a check a load and
+// loads beyond the range 6144 x 2560, 2560 x 4096, 2560 x 9728 and 2 x 9728 x 2560 took 8.3,
+// 6.3, 11.8 and 20.9 us at 8 rows, now 7.6, 5.6, 11.0 and 20.0; at 48 rows 10.5, 9.3, 14.3
+// and 25.2, now 9.3, 8.3, 12.9 and 23.4 (under a graph, matrices that no cache holds).
 #include "common.h"
+
+#include <type_traits>
+#include <utility>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -42,7 +52,6 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 #define GR_CHUNK 128
 #define GR_TILE_BYTES 4096  // 16 rows of one chunk
 #define GR_LDS(T) __attribute__((address_space(3))) T
-#define GR_OOB 0x80000000u
 
 // A barrier behind a wait for this wave's reads of LDS only.  The invariant it keeps: when a
 // wave passes it, every wave's operand reads of the chunk before have returned, so the loads
@@ -59,15 +68,24 @@ __device__ __forceinline__ void gr_wait_loads() {
   __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
 }
 
+template <typename F, int... I>
+__device__ __forceinline__ void gr_for_(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+// f(0), f(1), ... f(N - 1) with the number a constant each time.
+template <int N, typename F>
+__device__ __forceinline__ void gr_for(F&& f) {
+  gr_for_(f, std::make_integer_sequence<int, N>{});
+}
+
 // Stages of LDS for MT tiles of x and WAVES * CT tiles of w per chunk.
 template <int MT, int CT, int WAVES>
 struct GrShape {
   static constexpr int TILES = MT + WAVES * CT;
   static constexpr int STAGE_BYTES = TILES * GR_TILE_BYTES;
-  // Four stages where they fit and a wave brings one tile of w per chunk; with two tiles a wave
-  // (36 KB a stage and more) three do better by 1 to 2 % (gate/up 2 x 9728 x 2560 at 8 rows:
-  // 19.6 against 20.0 us; the head 139.1 against 140.2), and with one tile a wave three lose
-  // 4 to 7 %; six stages are slower everywhere.
+  // Four stages where they fit and a wave brings one tile of w per chunk, else three: 2560 x 9728 at
+  // 8 rows takes 11.9, 11.0, 11.2 and 11.6 us with three, four, six and eight, 2560 x 4096 6.2, 5.6, 5.8
+  // and 6.1; with two tiles a wave (36 KB a stage and more) three and four are within 1 %.
   static constexpr int STAGES = (4 * STAGE_BYTES <= 144 * 1024 && CT == 1) ? 4 : 3;
 };
 
@@ -90,8 +108,8 @@ enum GrGate { GR_NO_GATE = 0, GR_GATE = 1, GR_CAPPED_GATE = 2 };
 template <int MT, int CT, int GLU, int WAVES, typename TO>
 __device__ __forceinline__ void gemm_rows_body(
     TO* __restrict__ out, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int M, int N,
-    int K, long long ldx, long long ldw, long long ldo, long long part_stride, int chunks_per_part,
-    int wg_cols, int group, GrAct act) {
+    int K, int ldx, int ldw, long long ldo, long long part_stride, int chunks_per_part,
+    int wg_cols, int group, bool wide, GrAct act) {
   typedef GrShape<MT, CT, WAVES> Shape;
   constexpr int QW = 4 / WAVES;  // quarters of every tile of x that a wave fills
   constexpr int STAGES = Shape::STAGES;
@@ -102,55 +120,37 @@ __device__ __forceinline__ void gemm_rows_body(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PYLON_WAVE);
   const int r = lane & 15, g = lane >> 4;
   constexpr int WAVE_COLS = (GLU ? 1 : CT) * 16;  // columns of the output per wave
-  const int wg_row0 = group * wg_cols;  // first row of w the descriptor covers
-  const int wg_end = (N - wg_row0 < wg_cols) ? N : wg_row0 + wg_cols;
-  const int n0 = wg_row0 + wave * WAVE_COLS;
-  const int n_end = (wg_end - n0 < WAVE_COLS) ? wg_end : n0 + WAVE_COLS;  // <= n0: a wave without columns
+  const int wg_row0 = group * wg_cols;  // the workgroup's first row of w
+  const int wg_rows = N - wg_row0 < wg_cols ? N - wg_row0 : wg_cols;
+  const int first = wave * WAVE_COLS;  // the wave's first column, of the workgroup's
   const int part = blockIdx.y;
   const int chunks = (K + GR_CHUNK - 1) / GR_CHUNK;
   const int c_begin = part * chunks_per_part;
   const int c_end = (c_begin + chunks_per_part < chunks) ? c_begin + chunks_per_part : chunks;
 
-  // The descriptor of w starts at the workgroup's first row (with GLU it reaches N rows
-  // further, to its up rows).
-  const int wg_rows = wg_end - wg_row0;
-  const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(w + static_cast<size_t>(wg_row0) * ldw), 0,
-      static_cast<int>((static_cast<long long>((GLU ? N : 0) + wg_rows - 1) * ldw + K) * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(x), 0, static_cast<int>((static_cast<long long>(M - 1) * ldx + K) * 2), 0x00020000);
+  // Every view ends with its last row: a tile's rows beyond the workgroup's columns, or beyond M, lie outside it
+  // and fetch nothing.  With GLU the up rows have a view of their own, N rows further.
+  const uint16_t* const wg_w = w + static_cast<size_t>(wg_row0) * ldw;
+  const unsigned w_bytes = (static_cast<unsigned>(wg_rows - 1) * ldw + K) * 2u;
+  const unsigned x_bytes = (static_cast<unsigned>(M - 1) * ldx + K) * 2u;
 
   // A load fills rows 4 q .. 4 q + 3 of a tile (q: the quarter): lane l brings, for row
-  // R = 4 q + l / 16, the piece (l % 16) ^ R.
-  // x: this wave fills quarters QW * wave .. of every tile of x.
-  const int lrow = lane >> 4, lpos = lane & 15;
-  unsigned x_at[QW][MT];  // byte offset of this lane's piece in chunk 0, or out of range
-  int x_k[QW];            // its first element within a chunk
+  // R = 4 q + l / 16, the piece (l % 16) ^ R.  Byte offsets in chunk 0.
+  // x: this wave fills quarters QW * wave .. of every tile of x; w: all four of its own CT tiles.
+  const int lrow = lane >> 4, piece = (lane & 15) ^ lrow;
+  unsigned x_at[QW][MT], w_at[GLU ? 1 : CT][4];
 #pragma unroll
   for (int u = 0; u < QW; ++u) {
-    const int R = 4 * (QW * wave + u) + lrow;
-    x_k[u] = (lpos ^ R) * 8;
+    const int q = QW * wave + u;
 #pragma unroll
     for (int t = 0; t < MT; ++t)
-      x_at[u][t] = (16 * t + R < M)
-                       ? static_cast<unsigned>(16 * t + R) * static_cast<unsigned>(ldx) * 2u + 2u * x_k[u]
-                       : GR_OOB;
+      x_at[u][t] = static_cast<unsigned>(16 * t + 4 * q + lrow) * (2u * ldx) + ((piece ^ (4 * q)) * 16);
   }
-  // w: this wave fills all four quarters of its own CT tiles.
-  unsigned w_at[CT][4];
-  int w_k[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int R = 4 * q + lrow;
-    w_k[q] = (lpos ^ R) * 8;
+  for (int j = 0; j < (GLU ? 1 : CT); ++j)
 #pragma unroll
-    for (int j = 0; j < CT; ++j) {
-      // the row within the workgroup's columns, and where it lies from the descriptor's base
-      const int col = n0 - wg_row0 + (GLU ? R : 16 * j + R);
-      const unsigned row = static_cast<unsigned>(col) + ((GLU && j == 1) ? static_cast<unsigned>(N) : 0u);
-      w_at[j][q] = (wg_row0 + col < n_end) ? row * static_cast<unsigned>(ldw) * 2u + 2u * w_k[q] : GR_OOB;
-    }
-  }
+    for (int q = 0; q < 4; ++q)
+      w_at[j][q] = static_cast<unsigned>(first + 16 * j + 4 * q + lrow) * (2u * ldw) + ((piece ^ (4 * q)) * 16);
   // Operand reads: lane (r, g) takes piece 4 s + g of row r of a tile.
   unsigned piece_at[4];
 #pragma unroll
@@ -162,81 +162,97 @@ __device__ __forceinline__ void gemm_rows_body(
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // The loads of chunk c into a stage.  A chunk beyond the range issues the same loads with
-  // every offset out of range: nothing is fetched, and the count of loads per turn stays fixed.
-  auto issue = [&](int c, int stage) {
-    const bool live = c < c_end;
-    const unsigned k0 = static_cast<unsigned>(c) * GR_CHUNK;
-    unsigned char* base = lds + stage * Shape::STAGE_BYTES;
+  // The loads of chunk c into a stage, its offset their scalar one.  Pieces beyond K (of a chunk that K ends
+  // within) bring what follows in the view; their products are left out.
+  const __amdgpu_buffer_rsrc_t xres =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, x_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wres =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wg_w), 0, w_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t ures = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(wg_w + (GLU ? static_cast<size_t>(N) * ldw : 0)), 0, w_bytes, 0x00020000);
+  auto issue = [&](int c, int stage) __attribute__((always_inline)) {
+    const int at = c * (GR_CHUNK * 2);
+    unsigned char* const base = lds + stage * Shape::STAGE_BYTES;
 #pragma unroll
     for (int u = 0; u < QW; ++u)
 #pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        const bool ok = live && x_at[u][t] != GR_OOB && static_cast<int>(k0) + x_k[u] < K;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            xres, (GR_LDS(void)*)(base + t * GR_TILE_BYTES + (QW * wave + u) * 1024), 16,
-            ok ? x_at[u][t] + 2u * k0 : GR_OOB, 0, 0, 0);
-      }
+      for (int t = 0; t < MT; ++t)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (GR_LDS(void)*)(base + t * GR_TILE_BYTES + (QW * wave + u) * 1024), 16,
+                                                 x_at[u][t], at, 0, 0);
 #pragma unroll
     for (int j = 0; j < CT; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const bool ok = live && w_at[j][q] != GR_OOB && static_cast<int>(k0) + w_k[q] < K;
+      for (int q = 0; q < 4; ++q)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            wres, (GR_LDS(void)*)(base + (MT + wave * CT + j) * GR_TILE_BYTES + q * 1024), 16,
-            ok ? w_at[j][q] + 2u * k0 : GR_OOB, 0, 0, 0);
-      }
+            GLU && j == 1 ? ures : wres, (GR_LDS(void)*)(base + (MT + wave * CT + j) * GR_TILE_BYTES + q * 1024), 16,
+            w_at[GLU ? 0 : j][q], at, 0, 0);
   };
-  auto compute = [&](int stage) {
+  auto compute = [&](int stage, int left) __attribute__((always_inline)) {  // left: elements from the chunk's first to K
     const GR_LDS(unsigned char)* base = (const GR_LDS(unsigned char)*)(lds + stage * Shape::STAGE_BYTES);
+    auto product = [&](auto there) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      bf16x8 xf[MT], wf[CT];
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-        xf[t] = *reinterpret_cast<const GR_LDS(bf16x8)*>(base + t * GR_TILE_BYTES + piece_at[s]);
-#pragma unroll
-      for (int j = 0; j < CT; ++j)
-        wf[j] = *reinterpret_cast<const GR_LDS(bf16x8)*>(base + (MT + wave * CT + j) * GR_TILE_BYTES + piece_at[s]);
-#pragma unroll
-      for (int j = 0; j < CT; ++j)
+      for (int s = 0; s < 4; ++s) {
+        bf16x8 xf[MT], wf[CT];
 #pragma unroll
         for (int t = 0; t < MT; ++t)
-          acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[t], acc[j][t], 0, 0, 0);
-    }
+          xf[t] = there(*reinterpret_cast<const GR_LDS(bf16x8)*>(base + t * GR_TILE_BYTES + piece_at[s]), s);
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+          wf[j] = there(*reinterpret_cast<const GR_LDS(bf16x8)*>(base + (MT + wave * CT + j) * GR_TILE_BYTES + piece_at[s]), s);
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+#pragma unroll
+          for (int t = 0; t < MT; ++t)
+            acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[t], acc[j][t], 0, 0, 0);
+      }
+    };
+    if (left >= GR_CHUNK)
+      product([](bf16x8 v, int) __attribute__((always_inline)) { return v; });
+    else
+      product([&](bf16x8 v, int s) __attribute__((always_inline)) { return (4 * s + g) * 8 < left ? v : bf16x8{}; });
   };
 
   // Chunk c lives in stage (c - c_begin) % STAGES.  At the top of turn c the loads of chunks
   // c .. c + STAGES - 2 are outstanding; chunk c has landed once at most those of the later
   // ones are.  After the barrier every wave is past the products of chunk c - 1, whose stage
-  // chunk c + STAGES - 1 takes.
-#pragma unroll
-  for (int i = 0; i < STAGES - 1; ++i) issue(c_begin + i, i);
+  // chunk c + STAGES - 1 takes.  The last turns have nothing left to send and wait for fewer loads each (loads
+  // beyond the range, sent to keep one count, cost a launch 0.14 us a chunk).
   int stage = 0;
-  for (int c = c_begin; c < c_end; ++c) {
+  auto turn = [&](int c) __attribute__((always_inline)) {
+    if (first < wg_rows) compute(stage, K - c * GR_CHUNK);
+    stage = (stage + 1 == STAGES) ? 0 : stage + 1;
+  };
+#pragma unroll
+  for (int i = 0; i < STAGES - 1; ++i)
+    if (c_begin + i < c_end) issue(c_begin + i, i);
+  int c = c_begin;
+  for (; c + STAGES - 1 < c_end; ++c) {
     gr_wait_loads<LOADS*(STAGES - 2)>();
     gr_barrier();
     issue(c + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
-    if (n0 < n_end) compute(stage);
-    stage = (stage + 1 == STAGES) ? 0 : stage + 1;
+    turn(c);
   }
-  // The loads still outstanding are those past the range: they fetch nothing but do write
-  // (zeros) into LDS when they complete, so the wave sees them through before it leaves.
-  gr_wait_loads<0>();
+  gr_for<STAGES - 1>([&](auto I) __attribute__((always_inline)) {
+    constexpr int later = STAGES - 2 - decltype(I)::value;  // chunks behind this turn's
+    if (c + later < c_end) {
+      gr_wait_loads<LOADS * later>();
+      gr_barrier();
+      turn(c++);
+    }
+  });
 
-  // acc[j][t][i] is out[16 t + r][n0 + 16 j + 4 g + i] (with GLU: gate and up of column
-  // n0 + 4 g + i).  Four values of a lane go out as one store where every row of every part
-  // is aligned for it.
-  TO* dst = out + static_cast<size_t>(part) * part_stride;
-  const bool wide = (ldo & 3) == 0 && (part_stride & 3) == 0 &&
-                    (reinterpret_cast<uintptr_t>(out) & (4 * sizeof(TO) - 1)) == 0;
+  // acc[j][t][i] is out[16 t + r][first + 16 j + 4 g + i] of the workgroup's columns (with GLU: gate and up of
+  // column first + 4 g + i).  Four values of a lane go out as one store where every row of every part is
+  // aligned for it.
+  TO* dst = out + static_cast<size_t>(part) * part_stride + wg_row0;
+  wide = wide && (wg_row0 & 3) == 0;
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int m = t * 16 + r;
     if (m >= M) continue;
 #pragma unroll
     for (int j = 0; j < (GLU ? 1 : CT); ++j) {
-      const int n = n0 + 16 * j + 4 * g;
+      const int n = first + 16 * j + 4 * g;
       floatx4 v = acc[j][t];
       if constexpr (GLU == GR_GATE) {
 #pragma unroll
@@ -259,7 +275,7 @@ __device__ __forceinline__ void gemm_rows_body(
         }
       }
       TO* p = dst + static_cast<size_t>(m) * ldo + n;
-      if (wide && n + 3 < n_end && (n & 3) == 0) {
+      if (wide && n + 3 < wg_rows) {
         if constexpr (sizeof(TO) == 4) {
           *reinterpret_cast<floatx4*>(p) = v;
         } else {
@@ -271,17 +287,18 @@ __device__ __forceinline__ void gemm_rows_body(
       } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (n + i < n_end) p[i] = from_float<TO>(v[i]);
+          if (n + i < wg_rows) p[i] = from_float<TO>(v[i]);
       }
     }
   }
 }
 
+// The arguments that the first loads need are the first 16 words, which come with the launch.
 template <int MT, int CT, int GLU, int WAVES, typename TO>
 __global__ __launch_bounds__(WAVES* PYLON_WAVE) void gemm_rows_kernel(
-    TO* __restrict__ out, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int M, int N,
-    int K, long long ldx, long long ldw, long long ldo, long long part_stride, int chunks_per_part,
-    int wg_cols, int groups, int row_split, int variant) {
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int M, int N, int K, int ldx, int ldw,
+    int chunks_per_part, int wg_cols, int row_split, int groups, int flags, TO* __restrict__ out, long long ldo,
+    long long part_stride) {
   // More than 64 rows of x go as two halves of `row_split` rows, each to workgroups of its
   // own that take the same columns: blockIdx.x counts eight groups of columns for the first
   // half, the same eight for the second, then the next eight, so that the two workgroups that
@@ -297,16 +314,16 @@ __global__ __launch_bounds__(WAVES* PYLON_WAVE) void gemm_rows_kernel(
     M = (M - half * row_split < row_split) ? M - half * row_split : row_split;
   }
   gemm_rows_body<MT, CT, GLU, WAVES, TO>(out, x, w, M, N, K, ldx, ldw, ldo, part_stride, chunks_per_part, wg_cols,
-                                         group, GrAct{variant, 0.f, 0.f, 0.f});
+                                         group, (flags & 2) != 0, GrAct{flags & 1, 0.f, 0.f, 0.f});
 }
 
 // The same with a capped gate; up to 64 rows, whole K.
 template <int MT, int WAVES>
 __global__ __launch_bounds__(WAVES* PYLON_WAVE) void gemm_rows_capped_kernel(
-    bf16_t* __restrict__ out, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int M, int N, int K,
-    long long ldx, long long ldw, long long ldo, int wg_cols, GrAct act) {
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int M, int N, int K, int ldx, int ldw, int wg_cols,
+    int wide, bf16_t* __restrict__ out, long long ldo, GrAct act) {
   gemm_rows_body<MT, 2, GR_CAPPED_GATE, WAVES, bf16_t>(out, x, w, M, N, K, ldx, ldw, ldo, 0, (K + GR_CHUNK - 1) / GR_CHUNK,
-                                                       wg_cols, blockIdx.x, act);
+                                                       wg_cols, blockIdx.x, wide != 0, act);
 }
 
 // How a product is laid over the chip: wavefronts per workgroup, workgroups along the columns,
@@ -351,17 +368,21 @@ static void launch_rows_waves(void* out, int out_dtype, const void* x, const voi
   const int chunks = (K + GR_CHUNK - 1) / GR_CHUNK;
   const int per_part = (chunks + parts - 1) / parts;
   dim3 grid(row_split > 0 ? 2 * ((shape.groups + 7) / 8 * 8) : shape.groups, parts), block(WAVES * PYLON_WAVE);
+  // columns at multiples of four are aligned for a store of four in every row of every part
+  const int size = out_dtype == PYLON_F32 ? 4 : 2;
+  const int wide = (ldo & 3) == 0 && (part_stride & 3) == 0 &&
+                   (reinterpret_cast<uintptr_t>(out) & (4 * size - 1)) == 0;
   if constexpr (GLU == GR_CAPPED_GATE)
-    hipLaunchKernelGGL((gemm_rows_capped_kernel<MT, WAVES>), grid, block, 0, stream, (bf16_t*)out, (const uint16_t*)x,
-                       (const uint16_t*)w, M, N, K, ldx, ldw, ldo, shape.wg_cols, act);
+    hipLaunchKernelGGL((gemm_rows_capped_kernel<MT, WAVES>), grid, block, 0, stream, (const uint16_t*)x, (const uint16_t*)w,
+                       M, N, K, (int)ldx, (int)ldw, shape.wg_cols, wide, (bf16_t*)out, ldo, act);
   else if (out_dtype == PYLON_F32)
-    hipLaunchKernelGGL((gemm_rows_kernel<MT, CT, GLU, WAVES, float>), grid, block, 0, stream, (float*)out,
-                       (const uint16_t*)x, (const uint16_t*)w, M, N, K, ldx, ldw, ldo, part_stride, per_part,
-                       shape.wg_cols, shape.groups, row_split, act.variant);
+    hipLaunchKernelGGL((gemm_rows_kernel<MT, CT, GLU, WAVES, float>), grid, block, 0, stream, (const uint16_t*)x,
+                       (const uint16_t*)w, M, N, K, (int)ldx, (int)ldw, per_part, shape.wg_cols, row_split, shape.groups,
+                       act.variant | wide << 1, (float*)out, ldo, part_stride);
   else
-    hipLaunchKernelGGL((gemm_rows_kernel<MT, CT, GLU, WAVES, bf16_t>), grid, block, 0, stream, (bf16_t*)out,
-                       (const uint16_t*)x, (const uint16_t*)w, M, N, K, ldx, ldw, ldo, part_stride, per_part,
-                       shape.wg_cols, shape.groups, row_split, act.variant);
+    hipLaunchKernelGGL((gemm_rows_kernel<MT, CT, GLU, WAVES, bf16_t>), grid, block, 0, stream, (const uint16_t*)x,
+                       (const uint16_t*)w, M, N, K, (int)ldx, (int)ldw, per_part, shape.wg_cols, row_split, shape.groups,
+                       act.variant | wide << 1, (bf16_t*)out, ldo, part_stride);
 }
 
 // Workgroups of four waves, or of two where four would leave compute units without one.

@@ -322,6 +322,25 @@ def test_gemm_rows(ops, shape):
             ops.gemm_rows(a.to(DEV), w.to(DEV), parts=2, glu=True)
 
 
+# one chunk of 128 to two more than are in flight, whole and with 1, 8 and 15 pieces of 8 elements in the last
+@pytest.mark.parametrize("k", [c * 128 + e for c in range(7) for e in (8, 64, 120, 128)])
+def test_gemm_rows_leaves_out_what_lies_behind_k(ops, k):
+    """Operands in rows that go on with NaN: nothing of it is multiplied, in a product, in parts of K or with a gate."""
+    m, n = 1 + k % 64, 112
+    a, w = (torch.full((rows, k + 136), float("nan"), dtype=torch.bfloat16, device=DEV) for rows in (m, n))
+    a[:, :k], w[:, :k] = rnd((m, k), k, torch.bfloat16).to(DEV), rnd((n, k), k + 1, torch.bfloat16, 0.1).to(DEV)
+    a, w = a[:, :k], w[:, :k]
+    want = f64(a) @ f64(w).T
+    for parts, col_tiles, waves in ((1, 1, 2), (1, 2, 4), (2, 1, 4), (3, 2, 2)):
+        got = f64(ops.gemm_rows(a, w, out_dtype=torch.float32, parts=parts, col_tiles=col_tiles, waves=waves))
+        got = got.sum(0) if parts > 1 else got
+        assert np.abs(got - want).max() <= tol(torch.float32, np.abs(want).max()), (parts, col_tiles, waves)
+    g, u = want[:, : n // 2], want[:, n // 2:]
+    got = f64(ops.gemm_rows(a, w, out_dtype=torch.float32, glu=True))
+    want = g / (1 + np.exp(-g)) * u
+    assert np.abs(got - want).max() <= tol(torch.float32, np.abs(want).max())
+
+
 def plain_rope(x, pos, inv_freq, rot):
     # x: [..., d]; rotate the first `rot` elements, pairing i with i + rot/2
     ang = (np.float32(pos) * inv_freq.astype(np.float32)).astype(np.float64)
