@@ -35,7 +35,7 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 #define AS_MAX_BIAS 4096
 
 __device__ __forceinline__ uint32_t as_pack(float a, float b) {
-  return static_cast<uint32_t>(float_to_bf16_bits(a)) | (static_cast<uint32_t>(float_to_bf16_bits(b)) << 16);
+  return floats_to_bf16_pair(a, b);
 }
 
 // KS: steps of 32 key elements (dim <= 32 KS); NV: tiles of 16 value elements (vdim <= 16 NV).

@@ -23,7 +23,7 @@ from typing import List, Optional
 SOURCE_DIR = Path(__file__).resolve().parent
 LIB_NAME = "libpylon_hip.so"
 ARCH = "gfx950"
-# Packed-fp32 code generation is switched off for every kernel of this library.  The first 16 words of a kernel's
+# Packed-fp32 code generation is switched off for every kernel of this library.  The first 14 words of a kernel's
 # arguments come with the launch, in scalar registers, instead of being the first thing that it waits for (chats of
 # one user and of eight 55.5 -> 55.1 ms and 59.6 -> 59.3, ranudra's run 17.37 -> 17.28; same results).
 HIPCC_FLAGS = [

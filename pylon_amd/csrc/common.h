@@ -21,12 +21,16 @@ __device__ __forceinline__ float bf16_bits_to_float(uint16_t b) {
   return __uint_as_float(static_cast<uint32_t>(b) << 16);
 }
 
-// Round to nearest, ties to even; NaN stays NaN.
+// Round to nearest, ties to even; NaN stays NaN.  By the hardware's conversion: the same in integer arithmetic, with a
+// branch for NaN, was ten instructions a value, 0.4 us of a residual norm's 4.7.
 __device__ __forceinline__ uint16_t float_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
+}
+// Two of them in one word, `low` in its low half.
+__device__ __forceinline__ uint32_t floats_to_bf16_pair(float low, float high) {
+  typedef float pair_f __attribute__((ext_vector_type(2)));
+  typedef __bf16 pair_b __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((pair_f{low, high}), pair_b));
 }
 
 __device__ __forceinline__ float to_float(float v) { return v; }

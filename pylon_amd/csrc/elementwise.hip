@@ -2,6 +2,7 @@
 // residual sum that precedes it), and the gated activation of the feed-forward.
 // All reductions and all arithmetic are in float; only loads and stores see bf16.
 #include "common.h"
+#include "row_view.h"
 
 // ---- embedding ------------------------------------------------------------------
 // out[t, :] = table[ids[t], :] * scale, written as float (the residual stream).
@@ -59,8 +60,8 @@ __device__ __forceinline__ void store4(float* p, long long c, float a, float b, 
 }
 __device__ __forceinline__ void store4(bf16_t* p, long long c, float a, float b, float d, float e) {
   uint2 raw;
-  raw.x = static_cast<uint32_t>(float_to_bf16_bits(a)) | (static_cast<uint32_t>(float_to_bf16_bits(b)) << 16);
-  raw.y = static_cast<uint32_t>(float_to_bf16_bits(d)) | (static_cast<uint32_t>(float_to_bf16_bits(e)) << 16);
+  raw.x = floats_to_bf16_pair(a, b);
+  raw.y = floats_to_bf16_pair(d, e);
   reinterpret_cast<uint2*>(p)[c] = raw;
 }
 
@@ -69,8 +70,7 @@ __device__ __forceinline__ void store4(bf16_t* p, long long c, float a, float b,
 // One workgroup per output row. `row_idx` (optional) picks the input row of each
 // output row. With `delta`, the input is resid + factor * delta (float sum); `write_resid`
 // stores that sum back into resid (only meaningful without row_idx).
-// At most 512 threads per workgroup, so that a thread may hold the eight partial sums of its
-// sixteen elements in registers (a kernel that may be launched with 1,024 threads gets 128).
+// For rows of any length, type and alignment; float rows of whole fours go to the kernels below.
 template <typename TX, typename TD, typename TO>
 __global__ __launch_bounds__(512) void rmsnorm_kernel(TO* __restrict__ out, TX* x, const TD* __restrict__ delta,
                                int n_delta, long long delta_stride,
@@ -82,91 +82,6 @@ __global__ __launch_bounds__(512) void rmsnorm_kernel(TO* __restrict__ out, TX* 
   TX* xr = x + static_cast<size_t>(r_in) * dim;
   const TD* dr = delta ? delta + static_cast<size_t>(r_in) * dim : nullptr;
   TO* yr = out + static_cast<size_t>(r_out) * dim;
-
-  // Fast path (float rows whose length is a multiple of 4 and fits the registers): every
-  // load of the row is a 16-byte load issued before anything is stored, so the row costs
-  // one trip to memory.
-  constexpr int VEC = 4;  // float4 chunks per thread
-  if (sizeof(TX) == 4 && (dim & 3) == 0 && dim <= 4 * VEC * static_cast<int>(blockDim.x) &&
-      (delta_stride & 3) == 0) {
-    const int chunks = dim >> 2;
-    const float4* x4 = reinterpret_cast<const float4*>(xr);
-    const float4* w4 = reinterpret_cast<const float4*>(w);
-    float4 held[VEC], wt[VEC];
-#pragma unroll
-    for (int n = 0; n < VEC; ++n) {
-      const int c = threadIdx.x + n * blockDim.x;
-      held[n] = (c < chunks) ? x4[c] : float4{0.f, 0.f, 0.f, 0.f};
-      wt[n] = (c < chunks) ? w4[c] : float4{0.f, 0.f, 0.f, 0.f};
-    }
-    if (dr) {
-      // Partial sums of the previous matrix product are added in a fixed order.  For the
-      // usual counts every load is issued before the first addition: a loop over a count
-      // only known at run time would wait for memory once per partial sum.
-      const long long stride4 = delta_stride >> 2;
-      float4 d[VEC];
-#define PYLON_SUM_PARTS(ND)                                                                   \
-  do {                                                                                        \
-    float4 e[ND][VEC];                                                                        \
-    _Pragma("unroll") for (int p = 0; p < ND; ++p) _Pragma("unroll") for (int n = 0; n < VEC; ++n) { \
-      const int c = threadIdx.x + n * blockDim.x;                                             \
-      e[p][n] = (c < chunks) ? load4(dr, c + p * stride4) : float4{0.f, 0.f, 0.f, 0.f};       \
-    }                                                                                         \
-    _Pragma("unroll") for (int n = 0; n < VEC; ++n) {                                         \
-      d[n] = e[0][n];                                                                         \
-      _Pragma("unroll") for (int p = 1; p < ND; ++p) {                                        \
-        d[n].x += e[p][n].x; d[n].y += e[p][n].y; d[n].z += e[p][n].z; d[n].w += e[p][n].w;   \
-      }                                                                                       \
-    }                                                                                         \
-  } while (0)
-      if (n_delta == 1) {
-        PYLON_SUM_PARTS(1);
-      } else if (n_delta == 2) {
-        PYLON_SUM_PARTS(2);
-      } else if (n_delta == 4) {
-        PYLON_SUM_PARTS(4);
-      } else if (n_delta == 8) {
-        PYLON_SUM_PARTS(8);
-      } else {
-        PYLON_SUM_PARTS(1);
-        for (int p = 1; p < n_delta; ++p) {
-#pragma unroll
-          for (int n = 0; n < VEC; ++n) {
-            const int c = threadIdx.x + n * blockDim.x;
-            if (c < chunks) {
-              const float4 e = load4(dr, c + p * stride4);
-              d[n].x += e.x; d[n].y += e.y; d[n].z += e.z; d[n].w += e.w;
-            }
-          }
-        }
-      }
-#undef PYLON_SUM_PARTS
-#pragma unroll
-      for (int n = 0; n < VEC; ++n) {
-        held[n].x = fmaf(factor, d[n].x, held[n].x);
-        held[n].y = fmaf(factor, d[n].y, held[n].y);
-        held[n].z = fmaf(factor, d[n].z, held[n].z);
-        held[n].w = fmaf(factor, d[n].w, held[n].w);
-      }
-    }
-    float ss = 0.f;
-#pragma unroll
-    for (int n = 0; n < VEC; ++n)
-      ss += held[n].x * held[n].x + held[n].y * held[n].y + held[n].z * held[n].z + held[n].w * held[n].w;
-    const float total = block_sum(ss, scratch);
-    const float inv = 1.0f / sqrtf(total / static_cast<float>(dim) + eps);
-#pragma unroll
-    for (int n = 0; n < VEC; ++n) {
-      const int c = threadIdx.x + n * blockDim.x;
-      if (c < chunks) {
-        if (dr && write_resid) reinterpret_cast<float4*>(xr)[c] = held[n];
-        const float y0 = (held[n].x * inv) * wt[n].x, y1 = (held[n].y * inv) * wt[n].y;
-        const float y2 = (held[n].z * inv) * wt[n].z, y3 = (held[n].w * inv) * wt[n].w;
-        store4(yr, c, y0, y1, y2, y3);
-      }
-    }
-    return;
-  }
 
   float ss = 0.f;
   for (int i = threadIdx.x; i < dim; i += blockDim.x) {
@@ -190,6 +105,76 @@ __global__ __launch_bounds__(512) void rmsnorm_kernel(TO* __restrict__ out, TX* 
     }
     yr[i] = from_float<TO>((v * inv) * w[i]);
   }
+}
+
+// The same arithmetic for few rows: one trip to memory, and with one wavefront on a SIMD every instruction around
+// it counts.  All arguments come with the launch (14 words do), and nothing waits for a store.
+// Launches in a row, four parts, 8 rows of 2,560, 4,096 and 5,120: 3.8, 4.2 and 4.2 us -> 2.5, 2.7 and 3.2 (of an
+// empty kernel's 1.5); 48 rows 4.3, 4.9, 4.7 -> 2.8, 3.3, 3.5.
+// Float residual rows of a multiple of 4 elements, at most 4 NV a thread.  parts_apart: fours of elements from one
+// part to the next; sizes: dim, from bit 16 on the number of parts (0: no delta), from bit 24 on whether the sum is
+// stored.
+template <typename TD, typename TO, int NV, int THREADS>
+__device__ __forceinline__ void rmsnorm_few_body(float* x, const TD* delta, const float* w, TO* out, const int* row_idx,
+                                                 unsigned parts_apart, unsigned sizes, float eps, float factor) {
+  __shared__ float scratch[THREADS / PYLON_WAVE];
+  const int r_out = blockIdx.x, dim = sizes & 0xffff, parts = (sizes >> 16) & 0xff;
+  const int r_in = row_idx ? row_idx[r_out] : r_out;
+  const __amdgpu_buffer_rsrc_t x_row = row_view(x + static_cast<size_t>(r_in) * dim, dim), w_row = row_view(w, dim);
+  const int first = 4 * threadIdx.x;
+  constexpr int STEP = 4 * THREADS;
+  float4 held[NV], wt[NV];
+#pragma unroll
+  for (int n = 0; n < NV; ++n) held[n] = row_four<float>(x_row, first + n * STEP);
+#pragma unroll
+  for (int n = 0; n < NV; ++n) wt[n] = row_four<float>(w_row, first + n * STEP);
+  if (parts > 0) {
+    float4 d[NV];
+    row_sum_parts<TD, NV, THREADS>(d, delta + static_cast<size_t>(r_in) * dim, dim, parts, parts_apart);
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+      held[n] = float4{fmaf(factor, d[n].x, held[n].x), fmaf(factor, d[n].y, held[n].y), fmaf(factor, d[n].z, held[n].z),
+                       fmaf(factor, d[n].w, held[n].w)};
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int n = 0; n < NV; ++n) ss += row_squares(held[n]);
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // the weight is here: nothing below waits for the stores between
+  if (sizes >> 24) {
+#pragma unroll
+    for (int n = 0; n < NV; ++n) row_store<float>(x_row, first + n * STEP, held[n]);
+  }
+  const float total = row_block_sum<THREADS>(ss, scratch);
+  const float inv = 1.0f / sqrtf(total / static_cast<float>(dim) + eps);
+  const __amdgpu_buffer_rsrc_t y_row = row_view(out + static_cast<size_t>(r_out) * dim, dim);
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+    row_store<TO>(y_row, first + n * STEP, float4{(held[n].x * inv) * wt[n].x, (held[n].y * inv) * wt[n].y,
+                                                  (held[n].z * inv) * wt[n].z, (held[n].w * inv) * wt[n].w});
+}
+
+template <typename TD, typename TO, int NV, int THREADS>
+__global__ __launch_bounds__(THREADS) void rmsnorm_few_kernel(float* x, const TD* delta, const float* w, TO* out,
+                                                              const int* row_idx, unsigned parts_apart,
+                                                              unsigned sizes, float eps, float factor) {
+  rmsnorm_few_body<TD, TO, NV, THREADS>(x, delta, w, out, row_idx, parts_apart, sizes, eps, factor);
+}
+
+template <typename TD, typename TO, int THREADS>
+static void launch_rmsnorm_few(void* out, float* x, const TD* delta, int n_delta, long long delta_stride, const float* w,
+                               const int* row_idx, int rows, int dim, float eps, int write_resid, float factor,
+                               hipStream_t stream) {
+  const unsigned sizes = dim | (delta ? n_delta : 0) << 16 | write_resid << 24;
+#define GO(NV)                                                                                                         \
+  hipLaunchKernelGGL((rmsnorm_few_kernel<TD, TO, NV, THREADS>), dim3(rows), dim3(THREADS), 0, stream, x, delta, w, (TO*)out, \
+                     row_idx, static_cast<unsigned>(delta_stride >> 2), sizes, eps, factor)
+  switch ((dim + 4 * THREADS - 1) / (4 * THREADS)) {
+    case 1: GO(1); break;
+    case 2: GO(2); break;
+    case 3: GO(3); break;
+    default: GO(4); break;
+  }
+#undef GO
 }
 
 // The same arithmetic, in the same order, for steps of many rows (prompt portions): a
@@ -238,8 +223,7 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_many_kernel(TO* __restric
     float ss = 0.f;
 #pragma unroll
     for (int n = 0; n < VEC; ++n)
-      ss += held[i][n].x * held[i][n].x + held[i][n].y * held[i][n].y + held[i][n].z * held[i][n].z +
-            held[i][n].w * held[i][n].w;
+      ss += row_squares(held[i][n]);
     const float total = block_sum(ss, scratch);
     const float inv = 1.0f / sqrtf(total / static_cast<float>(dim) + eps);
     float* xr = resid + static_cast<size_t>(r0 + i) * dim;
@@ -270,6 +254,20 @@ static void launch_rmsnorm_out(void* out, int out_dtype, TX* x, const TD* delta,
 #define GO(TO, THREADS)                                                                                    \
   hipLaunchKernelGGL((add_rmsnorm_many_kernel<TD, TO, R, THREADS>), grid, dim3(THREADS), 0, stream, (TO*)out, x, \
                      delta, w, rows, dim, eps, factor)
+      if (dim > 4096) {
+        if (out_dtype == PYLON_F32) GO(float, 512); else GO(bf16_t, 512);
+      } else {
+        if (out_dtype == PYLON_F32) GO(float, 256); else GO(bf16_t, 256);
+      }
+#undef GO
+      return;
+    }
+  }
+  if constexpr (sizeof(TX) == 4) {
+    if ((dim & 3) == 0 && dim <= 8192 && (delta_stride & 3) == 0 && delta_stride < (1ll << 33) &&
+        row_aligned(x) && row_aligned(w) && row_aligned(delta) && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+#define GO(TO, THREADS) \
+  launch_rmsnorm_few<TD, TO, THREADS>(out, x, delta, n_delta, delta_stride, w, row_idx, rows, dim, eps, write_resid, factor, stream)
       if (dim > 4096) {
         if (out_dtype == PYLON_F32) GO(float, 512); else GO(bf16_t, 512);
       } else {
@@ -383,7 +381,7 @@ __global__ void silu_gate_bf16x8_kernel(uint4* __restrict__ out, const uint4* __
       const float u0 = __uint_as_float(uw[j] << 16), u1 = __uint_as_float(uw[j] & 0xffff0000u);
       const float a0 = pylon_gate_act(g0, act) * u0;
       const float a1 = pylon_gate_act(g1, act) * u1;
-      r[j] = static_cast<uint32_t>(float_to_bf16_bits(a0)) | (static_cast<uint32_t>(float_to_bf16_bits(a1)) << 16);
+      r[j] = floats_to_bf16_pair(a0, a1);
     }
     out[i] = uint4{r[0], r[1], r[2], r[3]};
   }
@@ -471,7 +469,7 @@ __global__ void gated_act_bf16x8_kernel(uint4* __restrict__ out, const uint4* __
         }
         a[k] = (gv[k] / (1.0f + expf(-alpha * gv[k]))) * (uv[k] + offset);
       }
-      r[j] = static_cast<uint32_t>(float_to_bf16_bits(a[0])) | (static_cast<uint32_t>(float_to_bf16_bits(a[1])) << 16);
+      r[j] = floats_to_bf16_pair(a[0], a[1]);
     }
     out[i] = uint4{r[0], r[1], r[2], r[3]};
   }
@@ -528,7 +526,7 @@ __global__ void relu2_bf16x8_kernel(uint4* __restrict__ out, const uint4* __rest
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float a = fmaxf(__uint_as_float(w[j] << 16), 0.f), b = fmaxf(__uint_as_float(w[j] & 0xffff0000u), 0.f);
-      r[j] = static_cast<uint32_t>(float_to_bf16_bits(a * a)) | (static_cast<uint32_t>(float_to_bf16_bits(b * b)) << 16);
+      r[j] = floats_to_bf16_pair(a * a, b * b);
     }
     out[i] = uint4{r[0], r[1], r[2], r[3]};
   }
@@ -685,7 +683,7 @@ __global__ void sigmoid_gate_bf16x8_kernel(uint4* __restrict__ x, const bf16_t* 
       const float ga = EACH ? 1.0f / (1.0f + __expf(-__uint_as_float(gw[j] << 16))) : one;
       const float gb = EACH ? 1.0f / (1.0f + __expf(-__uint_as_float(gw[j] & 0xffff0000u))) : one;
       const float a = __uint_as_float(w[j] << 16) * ga, b = __uint_as_float(w[j] & 0xffff0000u) * gb;
-      r[j] = static_cast<uint32_t>(float_to_bf16_bits(a)) | (static_cast<uint32_t>(float_to_bf16_bits(b)) << 16);
+      r[j] = floats_to_bf16_pair(a, b);
     }
     x[i] = uint4{r[0], r[1], r[2], r[3]};
   }

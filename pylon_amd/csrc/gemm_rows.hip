@@ -280,8 +280,8 @@ __device__ __forceinline__ void gemm_rows_body(
           *reinterpret_cast<floatx4*>(p) = v;
         } else {
           uint2 packed;
-          packed.x = float_to_bf16_bits(v[0]) | (static_cast<uint32_t>(float_to_bf16_bits(v[1])) << 16);
-          packed.y = float_to_bf16_bits(v[2]) | (static_cast<uint32_t>(float_to_bf16_bits(v[3])) << 16);
+          packed.x = floats_to_bf16_pair(v[0], v[1]);
+          packed.y = floats_to_bf16_pair(v[2], v[3]);
           *reinterpret_cast<uint2*>(p) = packed;
         }
       } else {
@@ -293,7 +293,7 @@ __device__ __forceinline__ void gemm_rows_body(
   }
 }
 
-// The arguments that the first loads need are the first 16 words, which come with the launch.
+// The arguments that the first loads need are the first 14 words, which come with the launch.
 template <int MT, int CT, int GLU, int WAVES, typename TO>
 __global__ __launch_bounds__(WAVES* PYLON_WAVE) void gemm_rows_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int M, int N, int K, int ldx, int ldw,

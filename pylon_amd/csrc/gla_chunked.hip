@@ -422,8 +422,8 @@ __global__ __launch_bounds__(256) void gla_chunked_kernel(
               y[i] = ((o[n][i] * inv) * wv[i]) * (g / (1.0f + __expf(-g)));
             }
             u32x2 packed;
-            packed[0] = static_cast<uint32_t>(float_to_bf16_bits(y[0])) | (static_cast<uint32_t>(float_to_bf16_bits(y[1])) << 16);
-            packed[1] = static_cast<uint32_t>(float_to_bf16_bits(y[2])) | (static_cast<uint32_t>(float_to_bf16_bits(y[3])) << 16);
+            packed[0] = floats_to_bf16_pair(y[0], y[1]);
+            packed[1] = floats_to_bf16_pair(y[2], y[3]);
             *reinterpret_cast<u32x2*>(o_row + e0) = packed;
           } else {
 #pragma unroll

@@ -17,8 +17,8 @@ __device__ __forceinline__ float4 ng_load4(const bf16_t* p, int c) {
 __device__ __forceinline__ void ng_store4(float* p, int c, float4 y) { reinterpret_cast<float4*>(p)[c] = y; }
 __device__ __forceinline__ void ng_store4(bf16_t* p, int c, float4 y) {
   uint2 raw;
-  raw.x = static_cast<uint32_t>(float_to_bf16_bits(y.x)) | (static_cast<uint32_t>(float_to_bf16_bits(y.y)) << 16);
-  raw.y = static_cast<uint32_t>(float_to_bf16_bits(y.z)) | (static_cast<uint32_t>(float_to_bf16_bits(y.w)) << 16);
+  raw.x = floats_to_bf16_pair(y.x, y.y);
+  raw.y = floats_to_bf16_pair(y.z, y.w);
   reinterpret_cast<uint2*>(p)[c] = raw;
 }
 __device__ __forceinline__ float ng_gate(float g, int silu) {

@@ -159,8 +159,7 @@ qkv_rotate_pieces_kernel(bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cach
         for (int j = 0; j < 4; ++j) {
           const float u = __uint_as_float(in[j] << 16), v = __uint_as_float(in[j] & 0xffff0000u);
           const float c = turn[(d >> 1) + j], s = turn[half + (d >> 1) + j];
-          o[j] = static_cast<uint32_t>(float_to_bf16_bits(u * c - v * s)) |
-                 (static_cast<uint32_t>(float_to_bf16_bits(v * c + u * s)) << 16);
+          o[j] = floats_to_bf16_pair(u * c - v * s, v * c + u * s);
         }
         y = uint4{o[0], o[1], o[2], o[3]};
       }

@@ -201,6 +201,49 @@ def test_residual_norm_adds_partial_sums(ops, dim, parts):
     assert np.abs(f64(got) - want[[4, 1]]).max() <= tol(torch.float32, np.abs(want).max())
 
 
+# one piece of 16 bytes, the last row that a number of pieces a thread holds and one piece more, the widest; and a
+# length of no whole pieces; parts that have code of their own and others
+@pytest.mark.parametrize("dim", [4, 1024, 1028, 2048, 2052, 3072, 3076, 4096, 4100, 6144, 6148, 8192, 4098])
+@pytest.mark.parametrize("parts", [0, 1, 2, 5, 8])
+def test_residual_norm_of_few_rows_at_its_edges(ops, dim, parts):
+    eps, rows, factor = 2e-6, 3, 0.25
+    frame = torch.full((rows + 2, dim), 7.0, device=DEV)  # rows before and behind: read and written by none
+    resid = frame[1: rows + 1]
+    resid.copy_(rnd((rows, dim), dim, torch.float32, 2.0))
+    before, stack = resid.clone(), rnd((max(parts, 1), rows, dim), dim + 1).to(DEV)
+    w = (1 + 0.3 * rnd((dim,), 14)).to(DEV)
+    summed = f64(before) + factor * f64(stack).sum(0) * (parts > 0)
+    want = summed / np.sqrt((summed * summed).mean(-1, keepdims=True) + eps) * f64(w)
+    out = torch.full((rows + 2, dim), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.add_rmsnorm(resid, stack if parts else None, w, eps, torch.bfloat16, out=out[1: rows + 1], factor=factor)
+    assert np.abs(f64(resid) - summed).max() <= 1e-6 * np.abs(summed).max()
+    assert np.abs(f64(out[1: rows + 1]) - want).max() <= tol(torch.bfloat16, np.abs(want).max())
+    for edge in (frame[0], frame[-1], out[0], out[-1]):
+        assert (edge == 7.0).all()
+    if parts < 2:  # a delta in bfloat16, rows picked, the residual left
+        delta = stack[0].to(torch.bfloat16) if parts else None
+        resid.copy_(before)
+        idx = torch.tensor([2, 0], dtype=torch.int32, device=DEV)
+        got = ops.add_rmsnorm(resid, delta, w, eps, torch.float32, row_idx=idx, factor=factor)
+        summed = (f64(before) + factor * (f64(delta) if parts else 0.0))[[2, 0]]
+        want = summed / np.sqrt((summed * summed).mean(-1, keepdims=True) + eps) * f64(w)
+        assert torch.equal(resid, before)
+        assert np.abs(f64(got) - want).max() <= tol(torch.float32, np.abs(want).max())
+
+
+def test_rounding_to_bfloat16_is_torchs(ops):
+    """Every high half of a float32 (zeros, subnormal numbers, infinities and NaN among them) with low halves around
+    the ties: the nearest, ties to even, NaN stays NaN."""
+    high = torch.arange(1 << 16, dtype=torch.int64)
+    bits = torch.stack([(high << 16) | low for low in (0, 1, 0x7fff, 0x8000, 0x8001, 0xffff)])
+    x = torch.where(bits >= 1 << 31, bits - (1 << 32), bits).to(torch.int32).view(torch.float32)
+    got = ops.qkv_bias_store(x.to(DEV), None, None, None, None, q_size=1 << 16, k_size=8, v_size=8, out_dtype=torch.bfloat16, store=False).cpu()
+    want = (x + 0.0).to(torch.bfloat16)  # on the CPU, in integers; a bias of zero makes -0 a 0
+    nan = torch.isnan(x)
+    assert torch.equal(torch.isnan(got), nan)
+    assert torch.equal(got.view(torch.int16)[~nan], want.view(torch.int16)[~nan])
+
+
 @pytest.mark.parametrize("shape", [(1, 96, 80), (8, 301, 176), (16, 130, 1000), (17, 64, 64),
                                    (64, 2560 + 8, 512 + 24), (33, 48, 4096), (8, 72, 9728)])
 def test_gemm_skinny(ops, shape):
