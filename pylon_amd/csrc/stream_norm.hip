@@ -12,6 +12,7 @@
 // elements of u between the passes, so that a row costs one trip to memory.  The order of every sum
 // depends on the row's length, the number of copies and of partial sums only.
 #include "common.h"
+#include "row_view.h"
 
 #define SN_BATCH 4  // partial sums whose loads are in flight together
 
@@ -55,8 +56,8 @@ template <int VEC>
 __device__ __forceinline__ void sn_store(bf16_t* p, int c, const SnVec<VEC>& a) {
   if constexpr (VEC == 4) {
     uint2 raw;
-    raw.x = static_cast<uint32_t>(float_to_bf16_bits(a.v[0])) | (static_cast<uint32_t>(float_to_bf16_bits(a.v[1])) << 16);
-    raw.y = static_cast<uint32_t>(float_to_bf16_bits(a.v[2])) | (static_cast<uint32_t>(float_to_bf16_bits(a.v[3])) << 16);
+    raw.x = floats_to_bf16_pair(a.v[0], a.v[1]);
+    raw.y = floats_to_bf16_pair(a.v[2], a.v[3]);
     reinterpret_cast<uint2*>(p)[c] = raw;
   } else {
     p[c] = from_float<bf16_t>(a.v[0]);
@@ -172,6 +173,104 @@ __global__ __launch_bounds__(1024) void stream_norm_kernel(
   }
 }
 
+// The same for up to four copies and rows of whole fours of elements (of a length up to 8192): every load is sent at
+// the start, through views of rows (row_view.h).  4 and 48 rows of 2,560, two copies, four parts: 3.8 and
+// 4.8 us -> 3.1 and 3.8; 2,048 rows, bfloat16 21.9 -> 18.9.
+template <typename TD, typename TO, int S, int NV, int THREADS>
+__device__ __forceinline__ void stream_norm_rows_body(TO* out, float* resid, const TD* delta, const float* w,
+                                                      const int* row_idx, unsigned parts_apart, unsigned sizes, float eps,
+                                                      unsigned copies_apart, const float* mix, const float* write,
+                                                      const float* read) {
+  __shared__ float scratch[2][THREADS / PYLON_WAVE];
+  const int r_out = blockIdx.x, dim = sizes & 0xffff, parts = (sizes >> 16) & 0xff;
+  const bool centre = (sizes >> 24 & 1) != 0, store = (sizes >> 25 & 1) != 0;
+  const int r_in = row_idx ? row_idx[r_out] : r_out;
+  const int first = 4 * threadIdx.x;
+  constexpr int STEP = 4 * THREADS;
+  float* const row = resid + static_cast<size_t>(r_in) * dim;
+  float4 x[S][NV], g[NV], u[NV];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const __amdgpu_buffer_rsrc_t view = row_view(row + static_cast<size_t>(s) * copies_apart * 4, dim);
+#pragma unroll
+    for (int n = 0; n < NV; ++n) x[s][n] = row_four<float>(view, first + n * STEP);
+  }
+  const __amdgpu_buffer_rsrc_t w_row = row_view(w, dim);
+#pragma unroll
+  for (int n = 0; n < NV; ++n) g[n] = row_four<float>(w_row, first + n * STEP);
+  float to[S], from[S], m[S][S];
+#pragma unroll
+  for (int t = 0; t < S; ++t) {
+    to[t] = write ? write[t] : 1.f;
+    from[t] = read ? read[t] : 1.f;
+#pragma unroll
+    for (int s = 0; s < S; ++s) m[s][t] = mix ? mix[s * S + t] : (s == t ? 1.f : 0.f);
+  }
+  auto fma4 = [](float f, const float4& v, const float4& c) __attribute__((always_inline)) {
+    return float4{fmaf(f, v.x, c.x), fmaf(f, v.y, c.y), fmaf(f, v.z, c.z), fmaf(f, v.w, c.w)};
+  };
+#pragma unroll
+  for (int n = 0; n < NV; ++n) u[n] = float4{0.f, 0.f, 0.f, 0.f};
+  if (parts > 0) {
+    float4 d[NV], y[S][NV];
+    row_sum_parts<TD, NV, THREADS>(d, delta + static_cast<size_t>(r_in) * dim, dim, parts, parts_apart);
+#pragma unroll
+    for (int t = 0; t < S; ++t)
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        float4 v = float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < S; ++s) v = fma4(m[s][t], x[s][n], v);
+        y[t][n] = fma4(to[t], d[n], v);
+        u[n] = fma4(from[t], y[t][n], u[n]);
+      }
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // the weight is here: nothing below waits for the stores between
+    if (store) {
+#pragma unroll
+      for (int t = 0; t < S; ++t) {
+        const __amdgpu_buffer_rsrc_t view = row_view(row + static_cast<size_t>(t) * copies_apart * 4, dim);
+#pragma unroll
+        for (int n = 0; n < NV; ++n) row_store<float>(view, first + n * STEP, y[t][n]);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < S; ++t)
+#pragma unroll
+      for (int n = 0; n < NV; ++n) u[n] = fma4(from[t], x[t][n], u[n]);
+  }
+  if (centre) {
+    float sum = 0.f;
+#pragma unroll
+    for (int n = 0; n < NV; ++n) sum += (u[n].x + u[n].y) + (u[n].z + u[n].w);
+    const float mean = row_block_sum<THREADS>(sum, scratch[0]) / static_cast<float>(dim);
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+      if (first + n * STEP < dim) {
+        u[n].x -= mean; u[n].y -= mean; u[n].z -= mean; u[n].w -= mean;
+      }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int n = 0; n < NV; ++n) ss += row_squares(u[n]);
+  const float inv = 1.0f / sqrtf(row_block_sum<THREADS>(ss, scratch[1]) / static_cast<float>(dim) + eps);
+  const __amdgpu_buffer_rsrc_t y_row = row_view(out + static_cast<size_t>(r_out) * dim, dim);
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+    row_store<TO>(y_row, first + n * STEP,
+                  float4{(u[n].x * inv) * g[n].x, (u[n].y * inv) * g[n].y, (u[n].z * inv) * g[n].z, (u[n].w * inv) * g[n].w});
+}
+
+template <typename TD, typename TO, int S, int NV, int THREADS>
+__global__ __launch_bounds__(THREADS) void stream_norm_rows_kernel(TO* out, float* resid, const TD* delta, const float* w,
+                                                                   const int* row_idx, unsigned parts_apart,
+                                                                   unsigned sizes, float eps, unsigned copies_apart,
+                                                                   const float* mix, const float* write,
+                                                                   const float* read) {
+  stream_norm_rows_body<TD, TO, S, NV, THREADS>(out, resid, delta, w, row_idx, parts_apart, sizes, eps, copies_apart, mix,
+                                                write, read);
+}
+
 // resid: float [streams, tokens, dim], the copies stream_stride elements apart, updated in place unless
 // row_idx picks rows (or delta is null).  delta: null (nothing is added, nothing mixed), [tokens, dim], or
 // n_delta such tensors delta_stride elements apart.  mix: float [streams, streams] (from, to) or null
@@ -191,6 +290,36 @@ extern "C" int pylon_stream_norm(void* out, int out_dtype, float* resid, long lo
   const uintptr_t bases = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(resid) |
                           reinterpret_cast<uintptr_t>(delta) | reinterpret_cast<uintptr_t>(w);
   const bool wide = dim % 4 == 0 && stream_stride % 4 == 0 && delta_stride % 4 == 0 && bases % 16 == 0;
+  if (wide && streams <= 4 && dim <= 8192 && n_delta < 256 && stream_stride < (1ll << 33) && delta_stride < (1ll << 33)) {
+    const unsigned sizes = dim | (delta != nullptr ? n_delta : 0) << 16 | (centre ? 1 : 0) << 24 | store << 25;
+#define GO(TD, TO, S, NV, THREADS)                                                                                   \
+  hipLaunchKernelGGL((stream_norm_rows_kernel<TD, TO, S, NV, THREADS>), dim3(rows), dim3(THREADS), 0, stream, (TO*)out, \
+                     resid, (const TD*)delta, w, row_idx, static_cast<unsigned>(delta_stride >> 2), sizes, eps,      \
+                     static_cast<unsigned>(stream_stride >> 2), mix, write, read)
+#define LENGTHS(TD, TO, S)                        \
+  do {                                            \
+    if (dim <= 1024) GO(TD, TO, S, 1, 256);       \
+    else if (dim <= 2048) GO(TD, TO, S, 2, 256);  \
+    else if (dim <= 3072) GO(TD, TO, S, 3, 256);  \
+    else if (dim <= 4096) GO(TD, TO, S, 2, 512);  \
+    else GO(TD, TO, S, 4, 512);                   \
+  } while (0)
+#define COPIES(TD, TO)                            \
+  do {                                            \
+    if (streams == 1) LENGTHS(TD, TO, 1);         \
+    else if (streams == 2) LENGTHS(TD, TO, 2);    \
+    else if (streams == 3) LENGTHS(TD, TO, 3);    \
+    else LENGTHS(TD, TO, 4);                      \
+  } while (0)
+    if (delta_dtype == PYLON_F32 && out_dtype == PYLON_F32) COPIES(float, float);
+    else if (delta_dtype == PYLON_F32) COPIES(float, bf16_t);
+    else if (out_dtype == PYLON_F32) COPIES(bf16_t, float);
+    else COPIES(bf16_t, bf16_t);
+#undef COPIES
+#undef LENGTHS
+#undef GO
+    PYLON_LAUNCHED("stream_norm");
+  }
   const int pieces = wide ? dim / 4 : dim;
   const int per = (pieces + 1023) / 1024 <= 1 ? 1 : (pieces + 1023) / 1024 <= 4 ? 4 : 16;
   const int threads = ((pieces + per - 1) / per + PYLON_WAVE - 1) / PYLON_WAVE * PYLON_WAVE;
@@ -200,8 +329,7 @@ extern "C" int pylon_stream_norm(void* out, int out_dtype, float* resid, long lo
                      streams, (const TD*)delta, n_delta, delta_stride, mix, write, read, w, row_idx, dim, eps, centre, store)
 #define PICK(TD, TO, S)                    \
   do {                                     \
-    if (wide && per == 1) GO(TD, TO, S, 1, 4);  \
-    else if (wide) GO(TD, TO, S, 4, 4);    \
+    if (wide) GO(TD, TO, S, 4, 4);         \
     else if (per <= 4) GO(TD, TO, S, 4, 1); \
     else GO(TD, TO, S, 16, 1);             \
   } while (0)

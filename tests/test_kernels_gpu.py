@@ -231,6 +231,50 @@ def test_residual_norm_of_few_rows_at_its_edges(ops, dim, parts):
         assert np.abs(f64(got) - want).max() <= tol(torch.float32, np.abs(want).max())
 
 
+@pytest.mark.parametrize("dim", [4, 1024, 1028, 2052, 3076, 4100, 8192, 8196, 16384, 2050])
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 8])
+def test_norms_of_pairs_and_streams_at_their_edges(ops, dim, parts):
+    """Rows that end inside and at the end of a workgroup's pieces, one piece longer, the widest of each size, and of no
+    whole pieces; a gain of one number and of one an element, with a bias and a scale; one to four copies, centred or not."""
+    eps, rows = 2e-6, 3
+    x, stack = rnd((rows, dim), 1, torch.float32, 2.0), rnd((parts, rows, dim), 2).to(DEV)
+    w, scale, bias = ((1 + 0.3 * rnd((dim,), seed)).to(DEV) for seed in (3, 4, 5))
+    one = torch.full((1,), 1.25, device=DEV)
+
+    def norm(v):
+        return v / np.sqrt((v * v).mean(-1, keepdims=True) + eps)
+
+    for gain, extra, out_dtype in ((w, dict(post_gain=one, post_eps=eps), torch.bfloat16),
+                                   (one, dict(delta_scale=scale, delta_bias=bias, factor=0.5), torch.float32),
+                                   (w, dict(factor=0.5), torch.bfloat16)):
+        d = f64(stack).sum(0) + (f64(bias) if "delta_bias" in extra else 0.0)
+        d = norm(d) * 1.25 if "post_gain" in extra else 0.5 * d * (f64(scale) if "delta_scale" in extra else 1.0)
+        want = norm(f64(x) + d) * f64(gain)
+        frame = torch.full((rows + 2, dim), 7.0, device=DEV)
+        frame[1:-1] = x.to(DEV)
+        got = ops.add_normed_rmsnorm(frame[1:-1], stack, gain, eps, out_dtype, **extra)
+        assert np.abs(f64(frame[1:-1]) - f64(x) - d).max() <= 2e-6 * np.abs(f64(x) + d).max()
+        assert np.abs(f64(got) - want).max() <= tol(out_dtype, np.abs(want).max())
+        assert (frame[[0, -1]] == 7.0).all()
+        idx = torch.tensor([2, 0], dtype=torch.int32, device=DEV)
+        frame[1:-1] = x.to(DEV)
+        got = ops.add_normed_rmsnorm(frame[1:-1], stack, gain, eps, out_dtype, row_idx=idx, **extra)
+        assert torch.equal(frame[1:-1].cpu(), x) and np.abs(f64(got) - want[[2, 0]]).max() <= tol(out_dtype, np.abs(want).max())
+    for copies in (1, 2, 3, 4, 5):
+        xs = rnd((copies, rows, dim), 6)
+        mix, write, read = (rnd(shape, seed) for shape, seed in (((copies, copies), 7), ((copies,), 8), ((copies,), 9)))
+        for centre, mixed in ((True, True), (False, False)):
+            new = (np.einsum("st,snd->tnd", f64(mix), f64(xs)) if mixed else f64(xs)) \
+                + (f64(write) if mixed else np.ones(copies))[:, None, None] * f64(stack).sum(0)
+            u = np.einsum("s,snd->nd", f64(read) if mixed else np.ones(copies), new)
+            want = norm(u - (u.mean(-1, keepdims=True) if centre else 0.0)) * f64(w)
+            resid = xs.to(DEV)
+            got = ops.stream_norm(resid, stack, w, eps, torch.bfloat16, centre=centre,
+                                  **(dict(mix=mix.to(DEV), write=write.to(DEV), read=read.to(DEV)) if mixed else {}))
+            assert np.abs(f64(resid) - new).max() <= 4e-6 * np.abs(new).max()
+            assert np.abs(f64(got) - want).max() <= tol(torch.bfloat16, np.abs(want).max())
+
+
 def test_rounding_to_bfloat16_is_torchs(ops):
     """Every high half of a float32 (zeros, subnormal numbers, infinities and NaN among them) with low halves around
     the ties: the nearest, ties to even, NaN stays NaN."""
