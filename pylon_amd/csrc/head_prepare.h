@@ -54,8 +54,7 @@ __device__ __forceinline__ void store_head_bf16(uint16_t* __restrict__ dst, int 
   } else {
 #pragma unroll
     for (int e = 0; e < EPL; e += 2) {
-      const uint32_t lo = float_to_bf16_bits(v[e]), hi = float_to_bf16_bits(v[e + 1 < EPL ? e + 1 : e]);
-      *reinterpret_cast<uint32_t*>(dst + lane * EPL + e) = lo | (hi << 16);
+      *reinterpret_cast<uint32_t*>(dst + lane * EPL + e) = floats_to_bf16_pair(v[e], v[e + 1 < EPL ? e + 1 : e]);
     }
   }
 }
@@ -64,17 +63,6 @@ __device__ __forceinline__ void store_head_bf16(uint16_t* __restrict__ dst, int 
 // head_dim/8 lanes share a head, 8 consecutive elements each, so a wavefront prepares
 // 512/head_dim heads at once.  j is the lane's index within its head (lane % (HD/8)).
 // Every lane of the wave must call these together (they exchange values inside a head).
-
-// cos(pos * f_i) and sin(pos * f_i) for the HD/2 rotation pairs of one token, by the whole
-// workgroup: cs[i] and cs[HD/2 + i].  A barrier must follow before cs is read.
-template <int HD>
-__device__ __forceinline__ void rotation_table(float* __restrict__ cs, const float* __restrict__ inv_freq, float pos) {
-  for (int i = threadIdx.x; i < HD / 2; i += blockDim.x) {
-    const float angle = pos * inv_freq[i];
-    cs[i] = cosf(angle);
-    cs[HD / 2 + i] = sinf(angle);
-  }
-}
 
 __device__ __forceinline__ void load8_bf16(const uint16_t* __restrict__ src, float v[8]) {
   const uint4 raw = *reinterpret_cast<const uint4*>(src);
@@ -191,14 +179,4 @@ __device__ __forceinline__ void norm_rotate8_with(float v[8], int j, bool weight
       v[e] = rotated ? turned : v[e];
     }
   }
-}
-
-// The same with the weights (or null) still in memory.
-template <int HD>
-__device__ __forceinline__ void norm_rotate8(float v[8], int j, const float* __restrict__ weight, float eps,
-                                             bool rotated, const float* __restrict__ cs) {
-  float own[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) own[e] = weight != nullptr ? weight[8 * j + e] : 0.f;
-  norm_rotate8_with<HD>(v, j, weight != nullptr, own, eps, rotated, cs);
 }

@@ -152,50 +152,85 @@ __global__ void qkv_prepare_wide_kernel(T* __restrict__ q_out, T* __restrict__ k
 // bfloat16 at head sizes 64/128/256 with the whole head rotated (or none of it): a
 // workgroup takes a share of one token's heads.  The token's rotation table is computed once
 // into LDS; then each wave prepares 512/head_dim heads at a time with 16-byte accesses.
-template <int HD>
+// With one wavefront's instructions behind another's on a SIMD this is bound by their number as much as by its bytes:
+// what does not depend on a lane is decided once a wave, and every load is sent before the angles are computed.
+// Of the arguments the first 14 words come with the launch.  (2,048 tokens of 32 + 16 heads of 128: 25.9 us with the
+// weights read an element at a time for every head and the loads behind the angles, 13.5 now, of 10 for the bytes; of
+// 64 + 16 heads 41.5 -> 18.6; 300 tokens 7.3 -> 4.8 and 10.3 -> 6.0.  Two rounds of heads on their way: four and three
+// are 1 to 5 % slower.)
+template <int HD, int ROUNDS>
 __global__ __launch_bounds__(QKV_WAVES* PYLON_WAVE) void qkv_prepare_rows_kernel(
-    uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
-    const uint16_t* __restrict__ qkv, long long row_stride, const float* __restrict__ q_weight,
-    const float* __restrict__ k_weight, float eps, const float* __restrict__ inv_freq,
-    const int* __restrict__ positions, const int* __restrict__ slot_map, int n_heads, int n_kv_heads,
-    int heads_per_token, int heads_per_block) {
-  constexpr int LPH = HD / 8, HPW = PYLON_WAVE / LPH;
-  __shared__ float cs[HD];
+    const uint16_t* __restrict__ qkv, const float* __restrict__ inv_freq, const int* __restrict__ positions,
+    const int* __restrict__ slot_map, const float* __restrict__ q_weight, const float* __restrict__ k_weight,
+    int row_stride, int heads_per_block, int heads_per_token, int n_heads, int n_kv_heads, float eps,
+    uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache) {
+  constexpr int LPH = HD / 8, HPW = PYLON_WAVE / LPH, STEP = QKV_WAVES * HPW;
+  typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));
+  __shared__ __attribute__((aligned(16))) float cs[HD];
   const int lane = threadIdx.x & (PYLON_WAVE - 1);
-  const int wave = threadIdx.x / PYLON_WAVE;
-  const int t = blockIdx.x;
-  if (inv_freq != nullptr) {
-    rotation_table<HD>(cs, inv_freq, static_cast<float>(positions[t]));
-    __syncthreads();
-  }
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PYLON_WAVE);
+  const int t = blockIdx.x, j = lane % LPH;
+  const bool rotated = inv_freq != nullptr;
+  const float freq = rotated && threadIdx.x < HD ? inv_freq[threadIdx.x & (HD / 2 - 1)] : 0.f;
+  const float pos = rotated ? static_cast<float>(positions[t]) : 0.f;
   const int h_begin = blockIdx.y * heads_per_block;
   const int h_end = h_begin + heads_per_block < heads_per_token ? h_begin + heads_per_block : heads_per_token;
   const int slot = heads_per_token > n_heads ? slot_map[t] : -1;
-  const uint16_t* row = qkv + static_cast<size_t>(t) * row_stride;
-  const int j = lane % LPH;
-  for (int h0 = h_begin + wave * HPW; h0 < h_end; h0 += QKV_WAVES * HPW) {
-    const int mine = h0 + lane / LPH;
-    const bool valid = mine < h_end;
-    const int s = valid ? mine : h_end - 1;
-    const uint16_t* src = row + static_cast<size_t>(s) * HD + 8 * j;  // heads lie in the order q, k, v
-    uint16_t* dst = nullptr;
-    const float* weight = nullptr;
-    bool rotate = false;
-    if (s < n_heads) {
-      dst = q_out + (static_cast<size_t>(t) * n_heads + s) * HD + 8 * j;
-      weight = q_weight;
-      rotate = true;
-    } else {
-      const bool is_key = s - n_heads < n_kv_heads;
-      const int kvh = is_key ? s - n_heads : s - n_heads - n_kv_heads;
-      if (slot >= 0) dst = (is_key ? k_cache : v_cache) + (static_cast<size_t>(slot) * n_kv_heads + kvh) * HD + 8 * j;
-      weight = is_key ? k_weight : nullptr;
-      rotate = is_key;
+  const uint16_t* const row = qkv + static_cast<size_t>(t) * static_cast<size_t>(row_stride) + 8 * lane;
+  uint4 raw[ROUNDS];
+  auto fetch = [&](int h) __attribute__((always_inline)) {  // heads h, h + STEP, ...: HPW of them a wave, one after the other
+#pragma unroll
+    for (int u = 0; u < ROUNDS; ++u)
+      if (h + u * STEP + lane / LPH < h_end) raw[u] = *reinterpret_cast<const uint4*>(row + static_cast<size_t>(h + u * STEP) * HD);
+  };
+  int h0 = h_begin + wave * HPW;
+  fetch(h0);
+  float4_any wq[2] = {}, wk[2] = {};
+  if (q_weight != nullptr) {
+    wq[0] = *reinterpret_cast<const float4_any*>(q_weight + 8 * j);
+    wq[1] = *reinterpret_cast<const float4_any*>(q_weight + 8 * j + 4);
+  }
+  if (k_weight != nullptr) {
+    wk[0] = *reinterpret_cast<const float4_any*>(k_weight + 8 * j);
+    wk[1] = *reinterpret_cast<const float4_any*>(k_weight + 8 * j + 4);
+  }
+  if (rotated) {  // cosines by some waves, sines by others
+    if (threadIdx.x < HD / 2)
+      cs[threadIdx.x] = cosf(pos * freq);
+    else if (threadIdx.x < HD)
+      cs[threadIdx.x] = sinf(pos * freq);
+    __syncthreads();
+  }
+  auto prepare = [&](const uint4& bits, int s, bool query, bool key) __attribute__((always_inline)) {
+    float v[8], weight[8];
+    const uint32_t w[4] = {bits.x, bits.y, bits.z, bits.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(w[i] << 16);
+      v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
     }
-    float v[8];
-    load8_bf16(src, v);
-    norm_rotate8<HD>(v, j, weight, eps, rotate, inv_freq != nullptr ? cs : nullptr);
-    if (valid && dst != nullptr) store8_bf16(dst, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) weight[e] = query ? wq[e / 4][e % 4] : wk[e / 4][e % 4];
+    norm_rotate8_with<HD>(v, j, query ? q_weight != nullptr : key && k_weight != nullptr, weight, eps, query || key,
+                          rotated ? cs : nullptr);
+    uint16_t* dst = nullptr;
+    if (query)
+      dst = q_out + (static_cast<size_t>(t) * n_heads + s) * HD + 8 * j;
+    else if (slot >= 0)
+      dst = (key ? k_cache : v_cache) + (static_cast<size_t>(slot) * n_kv_heads + (s - n_heads - (key ? 0 : n_kv_heads))) * HD + 8 * j;
+    if (s < h_end && dst != nullptr) store8_bf16(dst, v);
+  };
+  for (; h0 < h_end; h0 += ROUNDS * STEP) {
+#pragma unroll
+    for (int u = 0; u < ROUNDS; ++u) {
+      const int h = h0 + u * STEP, s = h + lane / LPH;  // heads lie in the order q, k, v
+      if (h >= h_end) break;
+      if (h + HPW <= n_heads)
+        prepare(raw[u], s, true, false);
+      else
+        prepare(raw[u], s, s < n_heads, s >= n_heads && s < n_heads + n_kv_heads);
+    }
+    if (h0 + ROUNDS * STEP < h_end) fetch(h0 + ROUNDS * STEP);
   }
 }
 
@@ -211,10 +246,15 @@ static bool launch_rows(uint16_t* q_out, uint16_t* k_cache, uint16_t* v_cache, c
   heads_per_block = (heads_per_block + per_round - 1) / per_round * per_round;
   shares = (heads_per_token + heads_per_block - 1) / heads_per_block;
   dim3 grid(tokens, shares), block(QKV_WAVES * PYLON_WAVE);
-#define GO(HD)                                                                                          \
-  hipLaunchKernelGGL((qkv_prepare_rows_kernel<HD>), grid, block, 0, stream, q_out, k_cache, v_cache, qkv, \
-                     row_stride, q_weight, k_weight, eps, inv_freq, positions, slot_map, n_heads,       \
-                     n_kv_heads, heads_per_token, heads_per_block)
+#define LAUNCH(HD, ROUNDS)                                                                                   \
+  hipLaunchKernelGGL((qkv_prepare_rows_kernel<HD, ROUNDS>), grid, block, 0, stream, qkv, inv_freq, positions, \
+                     slot_map, q_weight, k_weight, static_cast<int>(row_stride), heads_per_block, heads_per_token, \
+                     n_heads, n_kv_heads, eps, q_out, k_cache, v_cache)
+#define GO(HD)                                                  \
+  do {                                                          \
+    if (heads_per_block <= per_round) LAUNCH(HD, 1);            \
+    else LAUNCH(HD, 2);                                         \
+  } while (0)
   switch (head_dim) {
     case 64: GO(64); return true;
     case 128: GO(128); return true;
@@ -222,6 +262,7 @@ static bool launch_rows(uint16_t* q_out, uint16_t* k_cache, uint16_t* v_cache, c
     default: return false;
   }
 #undef GO
+#undef LAUNCH
 }
 
 template <typename T>
@@ -273,7 +314,7 @@ extern "C" int pylon_qkv_prepare(void* q_out, void* k_cache, void* v_cache, cons
   // whole-head rotation (or none) at head sizes 64/128/256 takes the vector form
   if ((inv_freq == nullptr || rot_dim == head_dim) && row_stride % 2 == 0) {
     bool done;
-    const bool vectors = dtype == PYLON_BF16 && row_stride % 8 == 0 &&
+    const bool vectors = dtype == PYLON_BF16 && row_stride % 8 == 0 && row_stride < (1ll << 31) &&
                          (reinterpret_cast<uintptr_t>(qkv) & 15) == 0 &&
                          (reinterpret_cast<uintptr_t>(q_out) & 15) == 0;
     if (vectors)

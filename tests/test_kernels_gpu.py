@@ -275,6 +275,34 @@ def test_norms_of_pairs_and_streams_at_their_edges(ops, dim, parts):
             assert np.abs(f64(got) - want).max() <= tol(torch.bfloat16, np.abs(want).max())
 
 
+@pytest.mark.parametrize("tokens", [1, 3, 1030])  # one round of heads a wave, and several
+@pytest.mark.parametrize("heads, kv_heads", [(6, 2), (7, 1), (32, 8), (64, 8)])  # waves of queries, keys and values together
+@pytest.mark.parametrize("dim", [64, 128, 256])
+def test_prepared_heads_are_those_of_the_general_path(ops, tokens, heads, kv_heads, dim):
+    """bfloat16 rows, with and without weights (which may lie anywhere), rotation and storing, beside the same numbers in
+    float32: at most one rounding apart."""
+    width = (heads + 2 * kv_heads) * dim
+    proj = rnd((tokens, width), dim, torch.bfloat16).to(DEV)
+    weights = (1 + 0.3 * rnd((2 * dim + 1,), 5)).to(DEV)
+    freq = (1e4 ** (-torch.arange(0, dim, 2) / dim)).float().to(DEV)
+    pos = ((torch.arange(tokens, dtype=torch.int32) * 77) % 5000).to(DEV)
+    slots = torch.randperm(tokens, generator=torch.Generator().manual_seed(1)).to(torch.int32).to(DEV)
+    slots[tokens // 2] = -1  # stores nothing
+    for weighted, rotated, store in ((True, True, True), (False, True, True), (True, False, True), (True, True, False)):
+        got = []
+        for dtype in (torch.bfloat16, torch.float32):
+            caches = [torch.full((1, tokens + 1, kv_heads, dim), 5.0, dtype=dtype, device=DEV) for _ in range(2)]
+            q = torch.empty((tokens, heads, dim), dtype=dtype, device=DEV)
+            rows = (proj if store else proj[:, : heads * dim].contiguous()).to(dtype)
+            ops.qkv_prepare(rows, q, *(caches if store else (None, None)), n_heads=heads, n_kv_heads=kv_heads, head_dim=dim,
+                            q_weight=weights[1: dim + 1] if weighted else None, k_weight=weights[dim + 1:] if weighted else None,
+                            eps=1e-6, inv_freq=freq if rotated else None, rot_dim=dim if rotated else 0,
+                            positions=pos if rotated else None, slot_map=slots if store else None, store_kv=store)
+            got.append([q, *caches])
+        for a, b in zip(*got):
+            assert ((a.float() - b).abs() <= b.abs() * 2.0 ** -8 + 1e-6).all()
+
+
 def test_rounding_to_bfloat16_is_torchs(ops):
     """Every high half of a float32 (zeros, subnormal numbers, infinities and NaN among them) with low halves around
     the ties: the nearest, ties to even, NaN stays NaN."""
