@@ -23,7 +23,7 @@ from typing import List, Optional
 import torch
 
 from ..config.specs import ModelSpec
-from ..kernels import ops
+from ..kernels import ops, plan
 from ..parts import build_part
 from ..parts.base import KVRequirement, Part, requirement_list
 from .batch import StepContext
@@ -52,7 +52,8 @@ class Model(Part):
         self.begins_pass = dict(begins)
         self.add_param("embed", (spec.vocab_size, spec.hidden_size), dtype, device)
         if not spec.tie_word_embeddings:
-            self.add_param("lm_head", (spec.vocab_size, spec.hidden_size), dtype, device)
+            self.add_param("lm_head", (spec.vocab_size, spec.hidden_size), dtype, device,
+                           row_padding=plan.head_row_padding(spec.hidden_size, dtype.itemsize))
         self.blocks: List[Part] = []
         for index, layer in enumerate(spec.layers):
             block = build_part("block", layer, dtype=dtype, device=device)

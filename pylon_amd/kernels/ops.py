@@ -1503,7 +1503,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
         if not x.is_cuda:
             raise KernelError("linear: operands must live on the GPU; there is no CPU path")
         if _streaming_ok(x, weight, STREAM_ROWS):
-            choice = plan.plan_projection(x.shape[0], *weight.shape)  # no rule of it counts compute units
+            choice = plan.plan_projection(x.shape[0], *weight.shape, weight.stride(0))  # no rule of it counts compute units
             if choice.kernel == "rows":
                 return gemm_rows(x, weight, out_dtype=out_dtype, col_tiles=choice.col_tiles, out=out)
             if choice.kernel == "skinny":

@@ -55,6 +55,15 @@ def gated_row_padding(k: int, element_size: int) -> int:
     return 64 if element_size == 2 and k >= 1024 else 0  # not worth doubling a toy's matrix
 
 
+def head_row_padding(k: int, element_size: int) -> int:
+    """The same behind the rows of a vocabulary head of its own (one that is the embedding too is read row by row
+    as it lies), where a row is a power-of-two length of 8 KB or more: 151936 x 4096 at 1, 8, 24, 48 and 64 rows
+    229, 236, 264, 271 and 274 us (the rows kernel, 64 columns a workgroup, beyond 32 rows the library) -> 211, 215,
+    223, 231 and 237 (the rows kernel, 128 columns; the library, padded, 243 and 259 at 48 and 64 rows).  Heads of
+    other widths are within 2 % either way and stay as they are."""
+    return 64 if element_size == 2 and aliased_rows(k) else 0
+
+
 def rows_split(n: int, k: int, rows: int = STREAM_ROWS, units: int = UNITS) -> tuple:
     """(parts, col_tiles) of the rows kernel for a product into the residual stream.
     Workgroups of 128 columns for deep matrices (beyond 16 rows, where the rows of x weigh
@@ -115,16 +124,18 @@ def plan_residual(rows: int, n: int, k: int, units: int = UNITS) -> Product:
 
 
 @lru_cache(maxsize=4096)  # asked for every product of a step
-def plan_projection(rows: int, n: int, k: int) -> Product:
+def plan_projection(rows: int, n: int, k: int, row_stride: int = 0) -> Product:
     """Any other product (q/k/v; the vocabulary head) of up to 64 rows; what it leaves to the library and what has
-    more rows may still go to a kernel (:func:`rows_match_library`, :func:`wide_beats_library`).
+    more rows may still go to a kernel (:func:`rows_match_library`, :func:`wide_beats_library`).  ``row_stride``: of the
+    matrix in memory, if its rows are further apart than they are long.
 
     A head (tall matrix): the rows kernel with 128 columns per workgroup (151936 x 2560: 137 us
     against the skinny kernel's 154 at 8 rows; 173 against the library's 186 at 64 rows, 150
     against 173 at 32; x 5120: 264 against 304 and 303 against 313).  With aliased rows (x 4096)
     64 columns per workgroup do better (220 against 227 us at 1 row, 230 against 235 at 8, 262
     against 272 at 32, the skinny kernel 237, 234 and, at 16 rows, 258 against 239), and beyond
-    32 rows the library (274 against 286 and 300 at 64 rows).
+    32 rows the library (274 against 286 and 300 at 64 rows); an engine's head of that width has
+    its rows apart (:func:`head_row_padding`) and goes as the others.
     A projection up to 16 rows: the rows kernel (6144 x 2560 at 8 rows 9.3 against the skinny
     kernel's 10.7 us, 10240 x 5120 21 against 31, 6144 x 4096 14.5 against 16).  Beyond 16
     rows the library: without K cut over workgroups the rows kernel is within 10 % of it either
@@ -135,7 +146,7 @@ def plan_projection(rows: int, n: int, k: int) -> Product:
     if rows > STREAM_ROWS:
         return Product("library")
     if n >= TALL:
-        if aliased_rows(k):
+        if aliased_rows(row_stride or k):
             return Product("rows", 1, 1) if rows <= 32 else Product("library")
         return Product("rows", 1, 2)
     return Product("rows") if few else Product("library")

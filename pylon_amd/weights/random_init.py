@@ -26,6 +26,25 @@ def _generator(seed: int, name: str, device="cpu") -> torch.Generator:
     return gen
 
 
+def _copy_flat(out: torch.Tensor, start: int, values: torch.Tensor) -> None:
+    """``values`` into the elements of ``out`` from number ``start`` on, counted row by row; the rows of a matrix may
+    be apart in memory."""
+    if out.is_contiguous():
+        out.view(-1)[start: start + values.numel()].copy_(values)
+        return
+    width, at = out.shape[1], 0
+    while at < values.numel():
+        row, col = divmod(start + at, width)
+        whole = (values.numel() - at) // width if col == 0 else 0
+        if whole:
+            out[row: row + whole].copy_(values[at: at + whole * width].view(whole, width))
+            at += whole * width
+        else:
+            n = min(width - col, values.numel() - at)
+            out[row, col: col + n].copy_(values[at: at + n])
+            at += n
+
+
 _SLAB = 1 << 26  # elements drawn at a time, so that no float32 copy of a large matrix is needed
 
 
@@ -57,13 +76,11 @@ def draw_tensor(seed: int, name: str, target, sigma: float, norm_jitter: float, 
     if target.init == "positive":
         out.copy_(torch.randn(tuple(out.shape), generator=gen, dtype=torch.float32, device=where).abs() * scale + shift)
         return
-    if out.is_contiguous():
-        flat = out.view(-1)
-        for start in range(0, flat.numel(), _SLAB):
-            part = flat[start: start + _SLAB]
-            part.copy_(torch.randn(part.numel(), generator=gen, dtype=torch.float32, device=where)
-                       * scale + shift)
-    else:
+    if out.is_contiguous() or target.param == "lm_head":
+        for start in range(0, out.numel(), _SLAB):
+            _copy_flat(out, start, torch.randn(min(_SLAB, out.numel() - start), generator=gen, dtype=torch.float32,
+                                               device=where) * scale + shift)
+    else:  # a gate/up matrix with its rows apart has always been drawn at once
         out.copy_(torch.randn(tuple(out.shape), generator=gen, dtype=torch.float32, device=where)
                   * scale + shift)
 

@@ -5,6 +5,7 @@ import ctypes
 import random
 
 import pytest
+import torch
 
 from pylon_amd.kernels import library, plan
 
@@ -78,6 +79,27 @@ def test_gate_up_rows_are_kept_apart_in_memory():
     assert plan.gated_row_padding(4096, 2) == 64 and plan.gated_row_padding(2560, 2) == 64
     assert plan.gated_row_padding(4096, 4) == 0  # the 32-bit path's matrices stay as they are
     assert plan.gated_row_padding(96, 2) == 0    # nor is a toy's matrix doubled
+
+
+def test_a_head_with_its_rows_apart_takes_the_rows_kernel():
+    """Only where its rows' length is a power of two of 8 KB or more; up to 64 rows, as the heads of other widths."""
+    assert [plan.head_row_padding(k, 2) for k in (2560, 4096, 5120, 8192)] == [0, 64, 0, 64]
+    assert plan.head_row_padding(4096, 4) == 0
+    for rows in (1, 16, 17, 48, 64):
+        assert plan.plan_projection(rows, VOCAB, 4096, 4160) == plan.Product("rows", 1, 2)
+        assert plan.plan_projection(rows, VOCAB, 4096, 4096) == plan.plan_projection(rows, VOCAB, 4096)
+    assert plan.plan_projection(65, VOCAB, 4096, 4160).kernel == "library"
+
+
+def test_drawing_into_rows_that_are_apart():
+    from pylon_amd.weights import random_init
+
+    values, apart = torch.randn(37 * 24), torch.zeros(37, 32)[:, :24]
+    for step in (7, 64, 100, 1000):
+        for start in range(0, values.numel(), step):
+            random_init._copy_flat(apart, start, values[start: start + step])
+        assert torch.equal(apart, values.view(37, 24))
+        apart.zero_()
     assert plan.plan_gated(8, 12288, 4096, 4096).kernel == "skinny"
     assert plan.plan_gated(8, 12288, 4096, 4096 + 64) == plan.Product("rows", 1, 2)
     assert plan.plan_gated(64, 12288, 4096, 4096 + 64) == plan.Product("rows", 1, 2)
