@@ -303,6 +303,48 @@ def test_prepared_heads_are_those_of_the_general_path(ops, tokens, heads, kv_hea
             assert ((a.float() - b).abs() <= b.abs() * 2.0 ** -8 + 1e-6).all()
 
 
+@pytest.mark.parametrize("tokens", [1, 3, 300])
+@pytest.mark.parametrize("heads, dim, vdim", [(1, 8, 8), (8, 128, 128), (3, 40, 72), (2, 12, 20)])  # the last: no whole pieces
+@pytest.mark.parametrize("transposed", [False, True])
+def test_keys_and_values_go_to_their_slots(ops, tokens, heads, dim, vdim, transposed):
+    k_row, v_row, size = heads * dim, heads * vdim, 32
+    proj = rnd((tokens, 8 + k_row + 16 + v_row), 1, torch.bfloat16).to(DEV)
+    slots = torch.randperm(11 * size, generator=torch.Generator().manual_seed(2))[:tokens].to(torch.int32)
+    k_cache = torch.full((11, size, heads, dim), 5.0, dtype=torch.bfloat16, device=DEV)
+    v_cache = torch.full((11, heads, vdim, size) if transposed else (11, size, heads, vdim), 5.0, dtype=torch.bfloat16, device=DEV)
+    want_k, want_v = k_cache.clone(), v_cache.clone()
+    for t, slot in enumerate(slots.tolist()):
+        want_k[slot // size, slot % size] = proj[t, 8: 8 + k_row].view(heads, dim)
+        v = proj[t, 24 + k_row:].view(heads, vdim)
+        if transposed:
+            want_v[slot // size, :, :, slot % size] = v
+        else:
+            want_v[slot // size, slot % size] = v
+    ops.kv_store(proj, k_cache, v_cache, slots.to(DEV), k_off=8, v_off=24 + k_row, v_transposed=transposed)
+    assert torch.equal(k_cache, want_k) and torch.equal(v_cache, want_v)
+
+
+@pytest.mark.parametrize("taps", [1, 2, 4, 8])
+@pytest.mark.parametrize("rows, width", [(1, 4), (5, 257), (48, 2560)])
+def test_a_convolution_of_single_tokens_is_that_of_a_tile(ops, taps, rows, width):
+    """The same sums and the same state, whether the bound on a row's tokens is one or more; a row without a token
+    keeps its state."""
+    w = rnd((width, taps), 1, torch.bfloat16).to(DEV)
+    state = rnd((rows + 1, max(taps - 1, 1), width), 2).to(DEV)
+    counts = [0 if rows > 1 and r == 1 else 1 for r in range(rows)]
+    start = torch.tensor(np.concatenate([[0], np.cumsum(counts)]), dtype=torch.int32, device=DEV)
+    slots = torch.arange(rows, 0, -1, dtype=torch.int32, device=DEV)
+    h, got = rnd((sum(counts), width), 3).to(DEV), []
+    for bound in (1, 2):
+        kept, outs = state.clone(), []
+        for step in range(3):
+            outs.append(ops.short_conv(h + step, w, kept if taps > 1 else None, start, slots, rows=rows, max_count=bound,
+                                       out_dtype=torch.float32))
+        got.append((kept, *outs))
+    for one, two in zip(*got):
+        assert torch.equal(one, two)
+
+
 def test_rounding_to_bfloat16_is_torchs(ops):
     """Every high half of a float32 (zeros, subnormal numbers, infinities and NaN among them) with low halves around
     the ties: the nearest, ties to even, NaN stays NaN."""
