@@ -163,7 +163,7 @@ __device__ __forceinline__ void gemm_rows_body(
     for (int t = 0; t < MT; ++t) acc[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   // The loads of chunk c into a stage, its offset their scalar one.  Pieces beyond K (of a chunk that K ends
-  // within) bring what follows in the view; their products are left out.
+  // within) bring what follows in the view, or zeros behind its last row; their products are left out.
   const __amdgpu_buffer_rsrc_t xres =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, x_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t wres =
@@ -171,7 +171,20 @@ __device__ __forceinline__ void gemm_rows_body(
   const __amdgpu_buffer_rsrc_t ures = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(wg_w + (GLU ? static_cast<size_t>(N) * ldw : 0)), 0, w_bytes, 0x00020000);
   auto issue = [&](int c, int stage) __attribute__((always_inline)) {
-    const int at = c * (GR_CHUNK * 2);
+    int at = c * (GR_CHUNK * 2);
+    if ((c + 1) * GR_CHUNK > K) {
+      // The range check does not count the scalar offset: in this chunk, which is the last that is sent, the lanes'
+      // offsets carry it, so that the last rows' pieces beyond K are beyond their views too.
+#pragma unroll
+      for (int u = 0; u < QW; ++u)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) x_at[u][t] += at;
+#pragma unroll
+      for (int j = 0; j < (GLU ? 1 : CT); ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w_at[j][q] += at;
+      at = 0;
+    }
     unsigned char* const base = lds + stage * Shape::STAGE_BYTES;
 #pragma unroll
     for (int u = 0; u < QW; ++u)
