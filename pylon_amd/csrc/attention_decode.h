@@ -558,7 +558,8 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
       }
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        const float fw = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), w0 + w));  // 0 past the last
+        if (w0 + w >= ranges) break;  // (the last range again: 0 times a sum beyond float32's range would be NaN)
+        const float fw = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), w0 + w));
 #pragma unroll
         for (int i = 0; i < EPL; ++i) o[i] = fmaf(a[w][i], fw, o[i]);
       }

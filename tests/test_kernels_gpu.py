@@ -1059,6 +1059,21 @@ def test_decode_attention_at_its_edges(ops, head_dim, heads, kv_heads):
         assert torch.equal(far, got)
 
 
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+@pytest.mark.parametrize("splits", [1, 2, 4, 8])
+def test_decode_attention_of_sums_beyond_the_range(ops, head_dim, splits):
+    """Values whose weighted sum is no float32 any more (each weighs as much as the largest: 1) give infinities, in
+    however many ranges the keys are taken."""
+    keys, page = 300, 64
+    q = torch.zeros(1, 2, head_dim, dtype=torch.bfloat16, device=DEV)
+    kc = rnd((5, page, 1, head_dim), 1, torch.bfloat16).to(DEV)
+    vc = torch.full((5, page, 1, head_dim), 3e38, dtype=torch.bfloat16, device=DEV)
+    table = torch.arange(5, dtype=torch.int32, device=DEV)[None]
+    positions = torch.tensor([keys - 1], dtype=torch.int32, device=DEV)
+    got = ops.attention_decode(q, kc, vc, table, None, positions, page_size=page, window=None, scale=1.0, n_splits=splits)
+    assert bool((got == math.inf).all())
+
+
 @pytest.mark.parametrize("geom", [(8, 2, 128, True, True), (6, 6, 64, True, False), (5, 1, 256, False, True),
                                   (16, 1, 64, True, True), (3, 3, 128, False, False)])
 @pytest.mark.parametrize("store", [True, False])
