@@ -17,7 +17,7 @@
 //
 // Scores come from the 16x16x32 bf16 matrix instruction with 16 keys as rows and the group's query heads, as often
 // as they fit, as columns; every copy then takes the softmax of other tiles.  The weighted sum of values takes
-// the probabilities as three bfloat16 parts each (exact, see there).  Softmax statistics are float throughout.
+// the probabilities as three bfloat16 parts each (exact for finite values; others are seen in the result).  Softmax statistics are float throughout.
 //
 // The kernel can also take over the step that precedes attention: given the raw q/k/v
 // projection instead of prepared queries, each workgroup first norms and rotates its
@@ -35,6 +35,8 @@
 #pragma once
 #include "common.h"
 #include "head_prepare.h"
+
+#include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -288,11 +290,14 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
   const int vkey = lane / LPK;
   uint32_t row_at[LOADS];  // the rows' numbers in the cache
   uint4 vv[LOADS];
-  auto find_rows = [&](int base) __attribute__((always_inline)) {
-    const int key = base + lane < k_end ? base + lane : k_end - 1, page = page_of(key);
+  auto own_row = [&](int base, int end) __attribute__((always_inline)) {  // of key base + lane (past the end: of the last)
+    const int key = base + lane < end ? base + lane : end - 1, page = page_of(key);
     int page_id = __shfl(table_entry, page & (PYLON_WAVE - 1), PYLON_WAVE);
-    if (page_of(k_end - 1) >= PYLON_WAVE && page >= PYLON_WAVE) page_id = table[page];
-    const uint32_t at = static_cast<uint32_t>(page_id * page_size + in_page(key, page)) * n_kv_heads + kvh;
+    if (page_of(end - 1) >= PYLON_WAVE && page >= PYLON_WAVE) page_id = table[page];
+    return static_cast<uint32_t>(page_id * page_size + in_page(key, page)) * n_kv_heads + kvh;
+  };
+  auto find_rows = [&](int base) __attribute__((always_inline)) {
+    const uint32_t at = own_row(base, k_end);
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) row_at[i] = __shfl(at, vkey * LOADS + i, PYLON_WAVE);
   };
@@ -363,7 +368,8 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
     const int share = (col / GP) % SHARES;
     float m_run = -INFINITY, l_run = 0.f;  // for head `head`, in every lane of it
     // The weighted values run on the matrix cores, too: a probability is the sum of three bfloat16 numbers to its
-    // last bit (24 = 3 x 8), the values are bfloat16, and the products of such numbers are exact in the float sums.
+    // last bit (24 = 3 x 8), the values are bfloat16, and the products of such numbers are exact in the float sums
+    // (of finite values: for others see below).
     // The three parts are rows of one operand: part 4 * (lane group) with up to four heads, which would be alone in
     // 16 rows otherwise; two and three instructions with 8 and 16.  Column n, element 8 g + i of the other operand
     // is a value that lane 16 g + n has loaded itself.  What the lanes of a group hold: with 128 elements one key
@@ -388,7 +394,7 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
       for (int e = 0; e < 8; ++e) acc[v][e] = floatx4{0.f, 0.f, 0.f, 0.f};
     const int k_row = (col % LOADS) * KPI + col / LOADS;  // of key 16 kt + col: (kt * 16 / LOADS) rows further
 
-    for (int base = k_begin; base < k_end; base += SUPER) {
+    auto batch = [&](int base, auto first_batch) __attribute__((always_inline)) {
       // all loads but the LOADS sent last (the values', or later ones) are through
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
       floatx4 sc[TILES];
@@ -450,7 +456,7 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
         }
       }
       tile_sum = over_columns<GP>(tile_sum, [](float a, float b) { return a + b; }) * (1.0f / COPIES);
-      if (base != k_begin) {  // rescale what has been accumulated: the factor of head h sits in lane h
+      if (!first_batch) {  // rescale what has been accumulated: the factor of head h sits in lane h
         const float corr = expf(m_run - m_new);
         l_run *= corr;
         // (row 4 grp + r is of head r, of head 4 (grp & 1) + r, of head 4 grp + r)
@@ -467,7 +473,7 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
       l_run += tile_sum;
       m_run = m_new;
       __builtin_amdgcn_wave_barrier();  // p_tile is private to the wave: program order suffices
-      // keys past the end weigh 0 and their value row is the (finite) last key's
+      // keys past the end weigh 0 and their value row is the last key's
 #pragma unroll
       for (int a = 0; a < LOADS; a += 8) {
         bf16x8 p[SETS][VARIANTS];
@@ -497,6 +503,14 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
         find_rows(base + SUPER);
         send_batch();
       }
+    };
+    // The first batch is code of its own where that is faster: with 128 elements (8 tokens of 170 keys 4.6 us, else
+    // 5.0) and where a batch takes few matrix instructions; with 256 elements two copies are up to 7 % slower than one.
+    if constexpr (HD == 128 || (HD == 64 ? GP < 16 : GP == 1)) {
+      batch(k_begin, std::true_type{});
+      for (int base = k_begin + SUPER; base < k_end; base += SUPER) batch(base, std::false_type{});
+    } else {
+      for (int base = k_begin; base < k_end; base += SUPER) batch(base, base == k_begin);
     }
 
     // The parts of a row are added over the lane groups that hold them, and what is left is spread over all lanes.
@@ -540,7 +554,8 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
   // the maximum and the sum of range w, so that all come at once.
   const int ranges = n_keys > 0 ? (n_keys + per_wave - 1) / per_wave : 0;
   const int mine = (lane & 15) < ranges ? lane & 15 : holds_last && (lane & 15) == AD_MAX_WAVES ? AD_MAX_WAVES : -1;
-  for (int h = wave; h < group; h += n_waves) {
+  float beyond = 0.f;  // NaN where a result is no finite number
+  auto merge = [&](int h, auto whole) __attribute__((always_inline)) {
     const float2 ml = *reinterpret_cast<const float2*>(part_ml + 2 * ((mine >= 0 ? mine : 0) * GP + h));
     const float m = over_row(mine >= 0 ? ml.x : -INFINITY, [](float a, float b) { return fmaxf(a, b); });
     const float f = mine >= 0 ? expf(ml.x - m) : 0.f;
@@ -548,20 +563,55 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
     float o[EPL];
 #pragma unroll
     for (int i = 0; i < EPL; ++i) o[i] = 0.f;
-    for (int w0 = 0; w0 < ranges; w0 += 4) {
-      float a[4][EPL];
+    if constexpr (decltype(whole)::value) {  // a key a lane for the probabilities, then EPL elements a lane
+      const uint16_t* const qrow = PREP ? q_lds + h * HD : q + (static_cast<size_t>(t) * n_heads + kvh * group + h) * HD;
+#pragma unroll 1
+      for (int base = c_begin; base < c_end; base += PYLON_WAVE) {
+        const uint32_t at = own_row(base, c_end);
+        float dot = 0.f;
+#pragma unroll 1
+        for (int c = 0; c < HD; c += 8) {
+          float a[8], b[8];
+          load8_bf16(qrow + c, a);
+          load8_bf16(k_cache + static_cast<size_t>(at) * HD + c, b);
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const float* arow = reinterpret_cast<const float*>(lds + (w0 + w < ranges ? w0 + w : ranges - 1) * WAVE_BYTES) + h * HD;
+          for (int e = 0; e < 8; ++e) dot = fmaf(a[e], b[e], dot);
+        }
+        const float p = expf(dot * scale - m);
+        const int keys = c_end - base < PYLON_WAVE ? c_end - base : PYLON_WAVE;
+#pragma unroll 1
+        for (int i0 = 0; i0 < keys; i0 += 4) {
+          float v[4][EPL];
 #pragma unroll
-        for (int i = 0; i < EPL; ++i) a[w][i] = arow[lane * EPL + i];
+          for (int u = 0; u < 4; ++u) {  // past the last: the last again, unused
+            const uint32_t row = __builtin_amdgcn_readlane(at, i0 + u < keys ? i0 + u : keys - 1);
+#pragma unroll
+            for (int i = 0; i < EPL; ++i) v[u][i] = bf16_bits_to_float(v_cache[static_cast<size_t>(row) * HD + lane * EPL + i]);
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if (i0 + u >= keys) break;
+            const float pu = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), i0 + u));
+#pragma unroll
+            for (int i = 0; i < EPL; ++i) o[i] = fmaf(v[u][i], pu, o[i]);
+          }
+        }
       }
+    } else {
+      for (int w0 = 0; w0 < ranges; w0 += 4) {
+        float a[4][EPL];
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        if (w0 + w >= ranges) break;  // (the last range again: 0 times a sum beyond float32's range would be NaN)
-        const float fw = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), w0 + w));
+        for (int w = 0; w < 4; ++w) {
+          const float* arow = reinterpret_cast<const float*>(lds + (w0 + w < ranges ? w0 + w : ranges - 1) * WAVE_BYTES) + h * HD;
 #pragma unroll
-        for (int i = 0; i < EPL; ++i) o[i] = fmaf(a[w][i], fw, o[i]);
+          for (int i = 0; i < EPL; ++i) a[w][i] = arow[lane * EPL + i];
+        }
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const float fw = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), w0 + w));  // 0 past the last
+#pragma unroll
+          for (int i = 0; i < EPL; ++i) o[i] = fmaf(a[w][i], fw, o[i]);
+        }
       }
     }
     if (holds_last) {
@@ -569,6 +619,8 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
 #pragma unroll
       for (int i = 0; i < EPL; ++i) o[i] = fmaf(bf16_bits_to_float(kv_new[HD + lane * EPL + i]), fw, o[i]);
     }
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) beyond = fmaf(o[i], 0.f, beyond);
     if (shape.n_cuts > 1) {
       // [token][head][cut][HD values, maximum, sum]
       float* prow = partial + ((static_cast<size_t>(t) * n_heads + kvh * group + h) * shape.n_cuts + cut) * (HD + 2);
@@ -584,6 +636,15 @@ __global__ __launch_bounds__(AD_MAX_WAVES* PYLON_WAVE) void attention_decode_ker
 #pragma unroll
       for (int i = 0; i < EPL; ++i) reinterpret_cast<__bf16*>(orow)[i] = static_cast<__bf16>(o[i] * inv);
     }
+  };
+  for (int h = wave; h < group; h += n_waves) merge(h, std::false_type{});
+  // An infinite or NaN value, or a sum beyond float32's range, leaves no finite number above, in other elements, too: a
+  // part of its probability may be 0 or negative, and rows of zeros and ranges past the last meet it.  The wave's
+  // heads are then merged once more from the keys themselves, with whole probabilities.  (Asked once, behind the
+  // stores, it costs nothing: 419 launches of one to 1,024 tokens within 0.1 % on average; asked a head 1.2 %.)
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(beyond != 0.f) != 0, 0)) {
+#pragma unroll 1
+    for (int h = wave; h < group; h += n_waves) merge(h, std::true_type{});
   }
 }
 

@@ -1074,6 +1074,42 @@ def test_decode_attention_of_sums_beyond_the_range(ops, head_dim, splits):
     assert bool((got == math.inf).all())
 
 
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+@pytest.mark.parametrize("heads, kv_heads", [(2, 2), (4, 2), (6, 2), (8, 1), (16, 1)])
+def test_decode_attention_of_infinite_and_nan_values(ops, head_dim, heads, kv_heads):
+    """Infinities and NaN in the cache reach the elements of the result that they are part of, as the products and sums of
+    numbers give them, and no others: in the first key, beside one of the other sign, in the last of a range, in the
+    token's own, and in the half of a row that lies beside others in an operand."""
+    lengths, page = [1, 40, 97, 130, 700], 64
+    per = -(-max(lengths) // page)
+    tokens, inf, nan = len(lengths), math.inf, math.nan
+    q = rnd((tokens, heads, head_dim), head_dim, torch.bfloat16)
+    kc, vc = (rnd((tokens * per, page, kv_heads, head_dim), seed, torch.bfloat16) for seed in (1, 2))
+    flat = vc.view(tokens, per * page, kv_heads, head_dim)
+    for t, n in enumerate(lengths):
+        flat[t, 0, :, 1] = inf
+        flat[t, n - 1, :, 5] = -inf  # the token's own key
+        flat[t, (n - 1) // 2, :, head_dim // 2 + 1] = nan
+        flat[t, max(n - 2, 0), 0, 7] = inf
+        flat[t, 0, :, 9], flat[t, (n - 1) // 3, :, 9] = inf, -inf
+        flat[t, n:, :, 11] = nan  # behind the last key: part of nothing
+    table = torch.arange(tokens * per, dtype=torch.int32).view(tokens, per)
+    positions = torch.tensor([n - 1 for n in lengths], dtype=torch.int32)
+    for splits, cuts in ((1, 1), (2, 1), (8, 1), (4, 3)):
+        got = ops.attention_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), table.to(DEV), None, positions.to(DEV), page_size=page,
+                                   window=None, scale=head_dim ** -0.5, n_splits=splits, n_cuts=cuts).cpu().double()
+        for t, n in enumerate(lengths):
+            k, v = (c.view(tokens, -1, kv_heads, head_dim)[t, :n].double().repeat_interleave(heads // kv_heads, 1) for c in (kc, vc))
+            p = torch.softmax((k * q[t].double()[None]).sum(-1) * head_dim ** -0.5, 0)
+            want = (p[:, :, None] * v).sum(0)
+            plain = torch.isfinite(want)
+            assert torch.equal(torch.isnan(got[t]), torch.isnan(want)), (splits, cuts, n)
+            assert torch.equal(got[t][torch.isinf(want)], want[torch.isinf(want)]), (splits, cuts, n)
+            # as where every value is finite: one rounding to bfloat16, and float scores before it
+            room = want[plain].abs() * 1.01 * 2.0 ** -8 + want[plain].abs().max() * 2.0 ** -16
+            assert bool(((got[t][plain] - want[plain]).abs() <= room).all()), (splits, cuts, n)
+
+
 @pytest.mark.parametrize("geom", [(8, 2, 128, True, True), (6, 6, 64, True, False), (5, 1, 256, False, True),
                                   (16, 1, 64, True, True), (3, 3, 128, False, False)])
 @pytest.mark.parametrize("store", [True, False])
