@@ -1503,7 +1503,13 @@ def linear(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: Optional[torch.d
         if not x.is_cuda:
             raise KernelError("linear: operands must live on the GPU; there is no CPU path")
         if _streaming_ok(x, weight, STREAM_ROWS):
-            choice = plan.plan_projection(x.shape[0], *weight.shape, weight.stride(0))  # no rule of it counts compute units
+            n, k = weight.shape
+            apart = weight.stride(0)
+            # rows that are apart make a head of this width the rows kernel's where it is the library's else, which
+            # a gradient or a trace sees and which goes to its operands' device
+            if n >= plan.TALL and plan.aliased_rows(k) and (_watched(x, weight) or not _here(x, weight)):
+                apart = 0
+            choice = plan.plan_projection(x.shape[0], n, k, apart)  # no rule of it counts compute units
             if choice.kernel == "rows":
                 return gemm_rows(x, weight, out_dtype=out_dtype, col_tiles=choice.col_tiles, out=out)
             if choice.kernel == "skinny":

@@ -137,3 +137,19 @@ def test_products_of_prompt_portions(routes, rows, n, k, own):
     ops.linear(empty(rows, k), empty(n, k))
     ops.linear_for_residual(empty(rows, k), empty(n, k), out_dtype=torch.bfloat16)
     assert routes == ["gemm_wide" if own else "library"] * 2
+
+
+@pytest.mark.parametrize("rows", [33, 64])
+def test_a_head_with_its_rows_apart_is_the_librarys_when_followed(routes, monkeypatch, rows):
+    """As one without, which is the library's at so many rows: followed for a gradient, or on another device."""
+    x, apart, close = empty(rows, 4096), empty(32768, 4160)[:, :4096], empty(32768, 4096)
+    ops.linear(x, apart)
+    ops.linear(x, close)
+    assert routes == ["gemm_rows", "library"]
+    routes.clear()
+    monkeypatch.setattr(ops, "_watched", lambda x, weight: True)
+    ops.linear(x, apart)
+    monkeypatch.setattr(ops, "_watched", lambda x, weight: False)
+    monkeypatch.setattr(ops, "_raw_device", lambda: 1)
+    ops.linear(x, apart)
+    assert routes == ["library"] * 2
