@@ -57,11 +57,18 @@ def gated_row_padding(k: int, element_size: int) -> int:
 
 def head_row_padding(k: int, element_size: int) -> int:
     """The same behind the rows of a vocabulary head of its own (one that is the embedding too is read row by row
-    as it lies), where a row is a power-of-two length of 8 KB or more: 151936 x 4096 at 1, 8, 24, 48 and 64 rows
-    229, 236, 264, 271 and 274 us (the rows kernel, 64 columns a workgroup, beyond 32 rows the library) -> 211, 215,
-    223, 231 and 237 (the rows kernel, 128 columns; the library, padded, 243 and 259 at 48 and 64 rows).  Heads of
-    other widths are within 2 % either way and stay as they are."""
-    return 64 if element_size == 2 and aliased_rows(k) else 0
+    as it lies), where a row is a multiple of 8 KB, but no power of two beyond it.  ``linear``, us, close -> apart, the
+    rows kernel with 64 and 128 columns a workgroup or, close and beyond 32 rows, the library:
+
+    151936 x 4096 at 1, 8, 24, 33, 48 and 64 rows 226, 229, 252, 258, 261, 270 -> 206, 205, 212, 215, 221, 228;
+    32000 x 4096 at 1, 32, 48, 64 rows 53, 57, 65, 60 -> 47, 49, 67, 50;
+    128256 x 12288 at 1, 8, 32, 48, 64 rows 546, 555, 574, 586, 613 -> 533, 536, 543, 544, 562;
+    65536 x 20480 at 1, 32, 64 rows 455, 477, 484 -> 451, 454, 472.
+    But 65536 x 8192 at 1, 32, 33, 48, 64 rows 233, 237, 214, 205, 216 -> 229, 235, 240, 242, 245; 151936 x 8192 at
+    33, 48 rows 494, 479 -> 512, 516; 128256 x 16384 at 33, 48 rows 755, 757 -> 787, 805: the library does well with
+    those as they lie.  From 65 rows on (the library) at most 1.5 % slower and up to 30 % faster; heads of other
+    widths are within 2 %."""
+    return 64 if element_size == 2 and aliased_rows(k) and (k == 4096 or k & (k - 1)) else 0
 
 
 def rows_split(n: int, k: int, rows: int = STREAM_ROWS, units: int = UNITS) -> tuple:
@@ -127,7 +134,7 @@ def plan_residual(rows: int, n: int, k: int, units: int = UNITS) -> Product:
 def plan_projection(rows: int, n: int, k: int, row_stride: int = 0) -> Product:
     """Any other product (q/k/v; the vocabulary head) of up to 64 rows; what it leaves to the library and what has
     more rows may still go to a kernel (:func:`rows_match_library`, :func:`wide_beats_library`).  ``row_stride``: of the
-    matrix in memory, if its rows are further apart than they are long.
+    matrix in memory; it counts at the widths of :func:`head_row_padding`.
 
     A head (tall matrix): the rows kernel with 128 columns per workgroup (151936 x 2560: 137 us
     against the skinny kernel's 154 at 8 rows; 173 against the library's 186 at 64 rows, 150
@@ -146,7 +153,7 @@ def plan_projection(rows: int, n: int, k: int, row_stride: int = 0) -> Product:
     if rows > STREAM_ROWS:
         return Product("library")
     if n >= TALL:
-        if aliased_rows(row_stride or k):
+        if aliased_rows(k) and not (head_row_padding(k, 2) and row_stride > k and not aliased_rows(row_stride)):
             return Product("rows", 1, 1) if rows <= 32 else Product("library")
         return Product("rows", 1, 2)
     return Product("rows") if few else Product("library")

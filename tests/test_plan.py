@@ -82,12 +82,17 @@ def test_gate_up_rows_are_kept_apart_in_memory():
 
 
 def test_a_head_with_its_rows_apart_takes_the_rows_kernel():
-    """Only where its rows' length is a power of two of 8 KB or more; up to 64 rows, as the heads of other widths."""
-    assert [plan.head_row_padding(k, 2) for k in (2560, 4096, 5120, 8192)] == [0, 64, 0, 64]
+    """Rows of a multiple of 8 KB, but no power of two beyond it; up to 64 rows, as the heads of other widths.  A
+    matrix of another width goes as it did, however far apart its rows are."""
+    assert [plan.head_row_padding(k, 2) for k in (2560, 4096, 5120, 8192, 12288, 16384, 20480)] == [0, 64, 0, 0, 64, 0, 64]
     assert plan.head_row_padding(4096, 4) == 0
-    for rows in (1, 16, 17, 48, 64):
+    for rows in (1, 16, 17, 32, 33, 48, 64):
+        close = plan.Product("rows", 1, 1) if rows <= 32 else plan.Product("library")
         assert plan.plan_projection(rows, VOCAB, 4096, 4160) == plan.Product("rows", 1, 2)
-        assert plan.plan_projection(rows, VOCAB, 4096, 4096) == plan.plan_projection(rows, VOCAB, 4096)
+        assert plan.plan_projection(rows, VOCAB, 12288, 12352) == plan.Product("rows", 1, 2)
+        for k, stride in ((4096, 0), (4096, 4096), (4096, 8192), (8192, 8192), (8192, 8256), (16384, 16448)):
+            assert plan.plan_projection(rows, VOCAB, k, stride) == close
+        assert plan.plan_projection(rows, VOCAB, 2560, 4096) == plan.Product("rows", 1, 2)
     assert plan.plan_projection(65, VOCAB, 4096, 4160).kernel == "library"
 
 
