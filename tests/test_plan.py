@@ -79,6 +79,9 @@ def test_gate_up_rows_are_kept_apart_in_memory():
     assert plan.gated_row_padding(4096, 2) == 64 and plan.gated_row_padding(2560, 2) == 64
     assert plan.gated_row_padding(4096, 4) == 0  # the 32-bit path's matrices stay as they are
     assert plan.gated_row_padding(96, 2) == 0    # nor is a toy's matrix doubled
+    assert plan.plan_gated(8, 12288, 4096, 4096).kernel == "skinny"
+    assert plan.plan_gated(8, 12288, 4096, 4096 + 64) == plan.Product("rows", 1, 2)
+    assert plan.plan_gated(64, 12288, 4096, 4096 + 64) == plan.Product("rows", 1, 2)
 
 
 def test_a_head_with_its_rows_apart_takes_the_rows_kernel():
@@ -105,9 +108,6 @@ def test_drawing_into_rows_that_are_apart():
             random_init._copy_flat(apart, start, values[start: start + step])
         assert torch.equal(apart, values.view(37, 24))
         apart.zero_()
-    assert plan.plan_gated(8, 12288, 4096, 4096).kernel == "skinny"
-    assert plan.plan_gated(8, 12288, 4096, 4096 + 64) == plan.Product("rows", 1, 2)
-    assert plan.plan_gated(64, 12288, 4096, 4096 + 64) == plan.Product("rows", 1, 2)
 
 
 def test_a_gate_up_matrix_beyond_a_descriptor_is_not_given_to_the_rows_kernel():
