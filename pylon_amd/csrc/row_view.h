@@ -36,6 +36,45 @@ __device__ __forceinline__ void row_store(__amdgpu_buffer_rsrc_t row, int i, con
                                           0, 0);
 }
 
+// The same of a row that begins anywhere, by a check a four instead of a descriptor.
+template <typename T>
+struct LooseRow {
+  T* p;
+  int elements;
+};
+typedef float loose_f4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned short loose_h4 __attribute__((ext_vector_type(4), aligned(2)));
+
+template <typename T>
+__device__ __forceinline__ float4 row_four(const LooseRow<T>& row, int i) {
+  if (i >= row.elements) return float4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (sizeof(T) == 4) {
+    const loose_f4 v = *reinterpret_cast<const loose_f4*>(row.p + i);
+    return float4{v.x, v.y, v.z, v.w};
+  } else {
+    const loose_h4 v = *reinterpret_cast<const loose_h4*>(row.p + i);
+    return float4{bf16_bits_to_float(v.x), bf16_bits_to_float(v.y), bf16_bits_to_float(v.z), bf16_bits_to_float(v.w)};
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void row_store(const LooseRow<T>& row, int i, const float4 v) {
+  if (i >= row.elements) return;
+  if constexpr (sizeof(T) == 4)
+    *reinterpret_cast<loose_f4*>(row.p + i) = loose_f4{v.x, v.y, v.z, v.w};
+  else
+    *reinterpret_cast<loose_h4*>(row.p + i) =
+        loose_h4{float_to_bf16_bits(v.x), float_to_bf16_bits(v.y), float_to_bf16_bits(v.z), float_to_bf16_bits(v.w)};
+}
+
+template <bool LOOSE, typename T>
+__device__ __forceinline__ auto row_of(const T* row, int elements) {
+  if constexpr (LOOSE)
+    return LooseRow<T>{const_cast<T*>(row), elements};
+  else
+    return row_view(row, elements);
+}
+
 // Whether rows `apart` elements apart from here on are such rows.
 template <typename T>
 static inline bool row_aligned(const T* p, long long apart = 0) {
@@ -62,10 +101,10 @@ __device__ __forceinline__ float row_block_sum(float v, float* scratch) {
 
 // d[n] = the sum over `parts` rows, `fours` fours of elements apart, of elements 4 (threadIdx.x + n THREADS) .. + 3, in
 // order; of 1, 2, 4 and 8 rows all loads are sent before the first sum.
-template <typename TD, int NV, int THREADS>
+template <typename TD, int NV, int THREADS, bool LOOSE = false>
 __device__ __forceinline__ void row_sum_parts(float4 (&d)[NV], const TD* row, int dim, int parts, unsigned fours) {
   auto part = [&](int p, float4* e) __attribute__((always_inline)) {
-    const __amdgpu_buffer_rsrc_t view = row_view(row + static_cast<size_t>(p) * fours * 4, dim);
+    const auto view = row_of<LOOSE>(row + static_cast<size_t>(p) * fours * 4, dim);
 #pragma unroll
     for (int n = 0; n < NV; ++n) e[n] = row_four<TD>(view, 4 * (threadIdx.x + n * THREADS));
   };

@@ -231,6 +231,35 @@ def test_residual_norm_of_few_rows_at_its_edges(ops, dim, parts):
         assert np.abs(f64(got) - want).max() <= tol(torch.float32, np.abs(want).max())
 
 
+@pytest.mark.parametrize("dim", [4, 1024, 2560, 4096, 6148, 8192])
+@pytest.mark.parametrize("parts", [0, 1, 2, 3, 4, 8])
+def test_residual_norm_of_rows_that_begin_anywhere(ops, dim, parts):
+    """The bits of the same rows at multiples of 16 bytes, wherever which operand begins; nothing beside them written."""
+    rows, eps, factor = 3, 2e-6, 0.25
+    x, stack = rnd((rows, dim), 1, torch.float32, 2.0), rnd((max(parts, 1), rows, dim), 2)
+    w = 1 + 0.3 * rnd((dim,), 3)
+
+    def at(t, off):
+        frame = torch.full((t.numel() + 32,), 7.0, dtype=t.dtype, device=DEV)
+        view = frame[16 + off: 16 + off + t.numel()].view(t.shape)
+        view.copy_(t)
+        return frame, view
+
+    for delta in (stack, stack[0].to(torch.bfloat16)) if parts < 2 else (stack,):
+        for out_dtype in DTYPES:
+            want = None
+            for offs in ((0, 0, 0, 0), (1, 0, 0, 0), (0, 1, 0, 0), (0, 0, 3, 0), (0, 0, 0, 1), (1, 2, 3, 5)):
+                (xf, xv), (df, dv), (_, wv), (of, ov) = (at(t, off) for t, off in zip(
+                    (x, delta, w, torch.empty((rows, dim), dtype=out_dtype)), offs))
+                ops.add_rmsnorm(xv, dv if parts else None, wv, eps, out_dtype, out=ov, factor=factor)
+                got = (xv.clone(), ov.clone(), ops.rmsnorm(xv, wv, eps))
+                want = want or got
+                assert all(torch.equal(a, b) for a, b in zip(got, want)), (offs, out_dtype)
+                for frame, view in ((xf, xv), (of, ov)):
+                    view.fill_(7.0)
+                    assert (frame == 7.0).all()
+
+
 @pytest.mark.parametrize("dim", [4, 1024, 1028, 2052, 3076, 4100, 8192, 8196, 16384, 2050])
 @pytest.mark.parametrize("parts", [1, 2, 3, 4, 8])
 def test_norms_of_pairs_and_streams_at_their_edges(ops, dim, parts):
