@@ -260,6 +260,25 @@ def test_residual_norm_of_rows_that_begin_anywhere(ops, dim, parts):
                     assert (frame == 7.0).all()
 
 
+@pytest.mark.parametrize("dim", [2, 250, 260, 1026, 2050, 4098, 8190, 9002, 2560, 8192])
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 8])
+def test_norms_of_pairs_an_element_at_a_time(ops, dim, parts):
+    """Rows of no whole fours of elements and, one element further on, rows that begin at no multiple of 16 bytes."""
+    rows, eps = 3, 2e-6
+    frame = torch.full((rows * dim + 8,), 7.0, device=DEV)
+    resid = frame[1: 1 + rows * dim].view(rows, dim)
+    x, stack = rnd((rows, dim), 1, torch.float32, 2.0), rnd((parts, rows, dim), 2).to(DEV)
+    resid.copy_(x)
+    w, one = (1 + 0.3 * rnd((dim,), 3)).to(DEV), torch.full((1,), 1.25, device=DEV)
+    d = f64(stack).sum(0)
+    summed = f64(x) + 1.25 * d / np.sqrt((d * d).mean(-1, keepdims=True) + eps)
+    want = summed / np.sqrt((summed * summed).mean(-1, keepdims=True) + eps) * f64(w)
+    got = ops.add_normed_rmsnorm(resid, stack, w, eps, torch.float32, post_gain=one, post_eps=eps)
+    assert np.abs(f64(resid) - summed).max() <= 2e-6 * np.abs(summed).max()
+    assert np.abs(f64(got) - want).max() <= tol(torch.float32, np.abs(want).max())
+    assert (frame[:1] == 7.0).all() and (frame[1 + rows * dim:] == 7.0).all()
+
+
 @pytest.mark.parametrize("dim", [4, 1024, 1028, 2052, 3076, 4100, 8192, 8196, 16384, 2050])
 @pytest.mark.parametrize("parts", [1, 2, 3, 4, 8])
 def test_norms_of_pairs_and_streams_at_their_edges(ops, dim, parts):
