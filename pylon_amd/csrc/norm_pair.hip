@@ -234,10 +234,12 @@ extern "C" int pylon_add_normed_rmsnorm(void* out, int out_dtype, float* resid, 
                      static_cast<unsigned>(delta_stride >> 2), delta_scale, delta_bias)
 #define PICK(TD, TO)                              \
   do {                                            \
-    if (dim <= 1024) GO(TD, TO, 1, 256);          \
+    if (dim <= 256) GO(TD, TO, 1, 64);            \
+    else if (dim <= 1024) GO(TD, TO, 1, 256);     \
     else if (dim <= 2048) GO(TD, TO, 2, 256);     \
     else if (dim <= 3072) GO(TD, TO, 3, 256);     \
     else if (dim <= 4096) GO(TD, TO, 4, 256);     \
+    else if (dim <= 6144) GO(TD, TO, 3, 512);     \
     else if (dim <= 8192) GO(TD, TO, 4, 512);     \
     else GO(TD, TO, 4, 1024);                     \
   } while (0)

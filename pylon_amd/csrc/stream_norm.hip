@@ -176,7 +176,10 @@ __global__ __launch_bounds__(1024) void stream_norm_kernel(
 // The same for up to four copies and rows of whole fours of elements (of a length up to 8192): every load is sent at
 // the start, through views of rows (row_view.h).  4 and 48 rows of 2,560, two copies, four parts: 3.8 and
 // 4.8 us -> 3.1 and 3.8; 2,048 rows, bfloat16 21.9 -> 18.9.
-template <typename TD, typename TO, int S, int NV, int THREADS>
+// ONE: an instance for no delta or one, whose registers hold no further parts, so that more rows are on their way where
+// a step has many: 2,048 rows of 8,192, one copy and two, no delta 21.8 -> 15.9 us and 28.7 -> 24.4, a bfloat16 one
+// 37.6 -> 34.3 and 60.6 -> 52.7.
+template <typename TD, typename TO, int S, int NV, int THREADS, bool ONE>
 __device__ __forceinline__ void stream_norm_rows_body(TO* out, float* resid, const TD* delta, const float* w,
                                                       const int* row_idx, unsigned parts_apart, unsigned sizes, float eps,
                                                       unsigned copies_apart, const float* mix, const float* write,
@@ -213,7 +216,13 @@ __device__ __forceinline__ void stream_norm_rows_body(TO* out, float* resid, con
   for (int n = 0; n < NV; ++n) u[n] = float4{0.f, 0.f, 0.f, 0.f};
   if (parts > 0) {
     float4 d[NV], y[S][NV];
-    row_sum_parts<TD, NV, THREADS>(d, delta + static_cast<size_t>(r_in) * dim, dim, parts, parts_apart);
+    if constexpr (ONE) {
+      const __amdgpu_buffer_rsrc_t d_row = row_view(delta + static_cast<size_t>(r_in) * dim, dim);
+#pragma unroll
+      for (int n = 0; n < NV; ++n) d[n] = row_four<TD>(d_row, first + n * STEP);
+    } else {
+      row_sum_parts<TD, NV, THREADS>(d, delta + static_cast<size_t>(r_in) * dim, dim, parts, parts_apart);
+    }
 #pragma unroll
     for (int t = 0; t < S; ++t)
 #pragma unroll
@@ -261,13 +270,13 @@ __device__ __forceinline__ void stream_norm_rows_body(TO* out, float* resid, con
                   float4{(u[n].x * inv) * g[n].x, (u[n].y * inv) * g[n].y, (u[n].z * inv) * g[n].z, (u[n].w * inv) * g[n].w});
 }
 
-template <typename TD, typename TO, int S, int NV, int THREADS>
+template <typename TD, typename TO, int S, int NV, int THREADS, bool ONE = false>
 __global__ __launch_bounds__(THREADS) void stream_norm_rows_kernel(TO* out, float* resid, const TD* delta, const float* w,
                                                                    const int* row_idx, unsigned parts_apart,
                                                                    unsigned sizes, float eps, unsigned copies_apart,
                                                                    const float* mix, const float* write,
                                                                    const float* read) {
-  stream_norm_rows_body<TD, TO, S, NV, THREADS>(out, resid, delta, w, row_idx, parts_apart, sizes, eps, copies_apart, mix,
+  stream_norm_rows_body<TD, TO, S, NV, THREADS, ONE>(out, resid, delta, w, row_idx, parts_apart, sizes, eps, copies_apart, mix,
                                                 write, read);
 }
 
@@ -290,19 +299,28 @@ extern "C" int pylon_stream_norm(void* out, int out_dtype, float* resid, long lo
   const uintptr_t bases = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(resid) |
                           reinterpret_cast<uintptr_t>(delta) | reinterpret_cast<uintptr_t>(w);
   const bool wide = dim % 4 == 0 && stream_stride % 4 == 0 && delta_stride % 4 == 0 && bases % 16 == 0;
-  if (wide && streams <= 4 && dim <= 8192 && n_delta < 256 && stream_stride < (1ll << 33) && delta_stride < (1ll << 33)) {
+  // Four copies of the longest rows are more than the registers hold of many rows at once: 2,048 rows of 8,192 without a
+  // delta 53 us with every load at the start, 46 copy by copy; 1,024 rows 25.2 and 24.3, 512 rows 13.8 and 15.0.
+  const bool copy_by_copy = streams == 4 && delta == nullptr && dim > 6144 && rows > 512;
+  if (wide && !copy_by_copy && streams <= 4 && dim <= 8192 && n_delta < 256 && stream_stride < (1ll << 33) && delta_stride < (1ll << 33)) {
+    const bool one = delta == nullptr || n_delta == 1;
     const unsigned sizes = dim | (delta != nullptr ? n_delta : 0) << 16 | (centre ? 1 : 0) << 24 | store << 25;
-#define GO(TD, TO, S, NV, THREADS)                                                                                   \
-  hipLaunchKernelGGL((stream_norm_rows_kernel<TD, TO, S, NV, THREADS>), dim3(rows), dim3(THREADS), 0, stream, (TO*)out, \
+#define GO(TD, TO, S, NV, THREADS, ONE)                                                                                       \
+  hipLaunchKernelGGL((stream_norm_rows_kernel<TD, TO, S, NV, THREADS, ONE>), dim3(rows), dim3(THREADS), 0, stream, (TO*)out, \
                      resid, (const TD*)delta, w, row_idx, static_cast<unsigned>(delta_stride >> 2), sizes, eps,      \
                      static_cast<unsigned>(stream_stride >> 2), mix, write, read)
-#define LENGTHS(TD, TO, S)                        \
-  do {                                            \
-    if (dim <= 1024) GO(TD, TO, S, 1, 256);       \
-    else if (dim <= 2048) GO(TD, TO, S, 2, 256);  \
-    else if (dim <= 3072) GO(TD, TO, S, 3, 256);  \
-    else if (dim <= 4096) GO(TD, TO, S, 2, 512);  \
-    else GO(TD, TO, S, 4, 512);                   \
+#define LENGTHS(TD, TO, S)                               \
+  do {                                                   \
+    if (dim <= 256) GO(TD, TO, S, 1, 64, false);         \
+    else if (dim <= 512) GO(TD, TO, S, 1, 128, false);   \
+    else if (dim <= 1024) GO(TD, TO, S, 1, 256, false);  \
+    else if (dim <= 2048) GO(TD, TO, S, 2, 256, false);  \
+    else if (dim <= 3072) GO(TD, TO, S, 3, 256, false);  \
+    else if (dim <= 4096) GO(TD, TO, S, 2, 512, false);  \
+    else if (dim <= 6144 && one) GO(TD, TO, S, 3, 512, true);  \
+    else if (dim <= 6144) GO(TD, TO, S, 3, 512, false);  \
+    else if (one) GO(TD, TO, S, 4, 512, true);           \
+    else GO(TD, TO, S, 4, 512, false);                   \
   } while (0)
 #define COPIES(TD, TO)                            \
   do {                                            \

@@ -279,7 +279,7 @@ def test_norms_of_pairs_an_element_at_a_time(ops, dim, parts):
     assert (frame[:1] == 7.0).all() and (frame[1 + rows * dim:] == 7.0).all()
 
 
-@pytest.mark.parametrize("dim", [4, 1024, 1028, 2052, 3076, 4100, 8192, 8196, 16384, 2050])
+@pytest.mark.parametrize("dim", [4, 256, 260, 512, 516, 1024, 1028, 2052, 3076, 4100, 6144, 6148, 8192, 8196, 16384, 2050])
 @pytest.mark.parametrize("parts", [1, 2, 3, 4, 8])
 def test_norms_of_pairs_and_streams_at_their_edges(ops, dim, parts):
     """Rows that end inside and at the end of a workgroup's pieces, one piece longer, the widest of each size, and of no
@@ -321,6 +321,20 @@ def test_norms_of_pairs_and_streams_at_their_edges(ops, dim, parts):
                                   **(dict(mix=mix.to(DEV), write=write.to(DEV), read=read.to(DEV)) if mixed else {}))
             assert np.abs(f64(resid) - new).max() <= 4e-6 * np.abs(new).max()
             assert np.abs(f64(got) - want).max() <= tol(torch.bfloat16, np.abs(want).max())
+
+
+@pytest.mark.parametrize("rows, dim", [(3, 256), (3, 512), (3, 4100), (3, 6144), (3, 6148), (513, 6148), (513, 8192)])
+@pytest.mark.parametrize("copies", [1, 3, 4])
+def test_norms_of_streams_that_nothing_is_added_to(ops, rows, dim, copies):
+    x, read, w = rnd((copies, rows, dim), 1), rnd((copies,), 2), 1 + 0.3 * rnd((dim,), 3)
+    u = np.einsum("s,snd->nd", f64(read), f64(x))
+    u -= u.mean(-1, keepdims=True)
+    want = u / np.sqrt((u * u).mean(-1, keepdims=True) + 1e-6) * f64(w)
+    resid = x.to(DEV)
+    got = ops.stream_norm(resid, None, w.to(DEV), 1e-6, torch.float32, centre=True, read=read.to(DEV))
+    # sums of up to four copies that cancel: their rounding, 2^-24 of the largest term, is as large beside the row's deviation
+    assert np.abs(f64(got) - want).max() <= 4 * tol(torch.float32, np.abs(want).max())
+    assert torch.equal(resid.cpu(), x)
 
 
 @pytest.mark.parametrize("tokens", [1, 3, 1030])  # one round of heads a wave, and several
