@@ -230,6 +230,7 @@ __global__ __launch_bounds__(QKV_WAVES* PYLON_WAVE) void qkv_prepare_rows_kernel
       else
         prepare(raw[u], s, s < n_heads, s >= n_heads && s < n_heads + n_kv_heads);
     }
+    if constexpr (ROUNDS == 1) break;  // all that a workgroup of one round has
     if (h0 + ROUNDS * STEP < h_end) fetch(h0 + ROUNDS * STEP);
   }
 }
