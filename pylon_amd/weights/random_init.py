@@ -46,6 +46,9 @@ def _copy_flat(out: torch.Tensor, start: int, values: torch.Tensor) -> None:
 
 
 _SLAB = 1 << 26  # elements drawn at a time, so that no float32 copy of a large matrix is needed
+# Parameters that are drawn at once, not slab by slab, where their rows are apart in memory (a numbers' matter: the two
+# give other numbers to matrices of more than a slab).  All others have the same numbers however they lie.
+_AT_ONCE = ("gate_up", "shared_gate_up")
 
 
 def draw_tensor(seed: int, name: str, target, sigma: float, norm_jitter: float, *, out: torch.Tensor,
@@ -76,11 +79,12 @@ def draw_tensor(seed: int, name: str, target, sigma: float, norm_jitter: float, 
     if target.init == "positive":
         out.copy_(torch.randn(tuple(out.shape), generator=gen, dtype=torch.float32, device=where).abs() * scale + shift)
         return
-    if out.is_contiguous() or target.param == "lm_head":
+    rows_apart = out.dim() == 2 and out.stride(1) == 1 and out.stride(0) > out.shape[1]
+    if out.is_contiguous() or rows_apart and target.param.rpartition(".")[2] not in _AT_ONCE:
         for start in range(0, out.numel(), _SLAB):
             _copy_flat(out, start, torch.randn(min(_SLAB, out.numel() - start), generator=gen, dtype=torch.float32,
                                                device=where) * scale + shift)
-    else:  # a gate/up matrix with its rows apart has always been drawn at once
+    else:
         out.copy_(torch.randn(tuple(out.shape), generator=gen, dtype=torch.float32, device=where)
                   * scale + shift)
 

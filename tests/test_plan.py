@@ -99,7 +99,10 @@ def test_a_head_with_its_rows_apart_takes_the_rows_kernel():
     assert plan.plan_projection(65, VOCAB, 4096, 4160).kernel == "library"
 
 
-def test_drawing_into_rows_that_are_apart():
+def test_drawing_into_rows_that_are_apart(monkeypatch):
+    """The numbers of rows that are close, whatever the parameter, across slabs that end in the middle of a row; a
+    gate/up matrix has those of one draw."""
+    from pylon_amd.config.registry import WeightTarget
     from pylon_amd.weights import random_init
 
     values, apart = torch.randn(37 * 24), torch.zeros(37, 32)[:, :24]
@@ -108,6 +111,17 @@ def test_drawing_into_rows_that_are_apart():
             random_init._copy_flat(apart, start, values[start: start + step])
         assert torch.equal(apart, values.view(37, 24))
         apart.zero_()
+
+    def drawn(param, out):
+        random_init.draw_tensor(3, "name", WeightTarget(param, (37, 24)), 0.5, 0.0, out=out)
+        return out.clone()
+
+    monkeypatch.setattr(random_init, "_SLAB", 100)
+    close = drawn("lm_head", torch.zeros(37, 24))
+    for param in ("lm_head", "blocks.0.another"):
+        assert torch.equal(drawn(param, apart), close)
+    together = torch.randn(37, 24, generator=random_init._generator(3, "name")) * 0.5
+    assert torch.equal(drawn("blocks.0.feed_forward.gate_up", apart), together) and not torch.equal(together, close)
 
 
 def test_a_gate_up_matrix_beyond_a_descriptor_is_not_given_to_the_rows_kernel():
