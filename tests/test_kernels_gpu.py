@@ -1229,6 +1229,45 @@ def test_decode_attention_that_prepares_q_k_v_itself(ops, geom, store):
         assert torch.equal(kc4, kc3) and torch.equal(vc4, vc3), parts
 
 
+@pytest.mark.parametrize("nh, nkv, hd, tokens", [(32, 8, 128, 48), (16, 16, 64, 48), (128, 8, 64, 40), (16, 8, 256, 40), (16, 1, 128, 300)])
+@pytest.mark.parametrize("splits, cuts", [(1, 1), (2, 1), (4, 1), (8, 1), (1, 2)])
+def test_decode_attention_of_more_workgroups_than_units_prepares_q_k_v(ops, nh, nkv, hd, tokens, splits, cuts):
+    """The waves that hold keys prepare q, k and v too (a workgroup has no others then), in several rounds where the group
+    is large: the bits of the two launches, also with the addresses of caches beyond 4 GB (slots given as 0)."""
+    from pylon_amd.kernels import library
+
+    assert tokens * nkv * cuts > library.compute_units()
+    page, per = 16, 20
+    qkv = rnd((tokens, (nh + 2 * nkv) * hd), 1, torch.bfloat16).to(DEV)
+    qw, kw = ((1 + 0.2 * rnd((hd,), seed)).to(DEV) for seed in (2, 3))
+    inv_freq = (1.0 / (10000.0 ** (torch.arange(0, hd, 2, dtype=torch.float32) / hd))).to(DEV)
+    positions = (torch.arange(tokens, dtype=torch.int32) * 37) % (per * page)
+    positions[:3] = torch.tensor([0, per * page - 1, 64])
+    table = torch.randperm(tokens * per, generator=torch.Generator().manual_seed(4)).to(torch.int32).view(tokens, per)
+    slots = table[torch.arange(tokens), (positions // page).long()] * page + positions % page
+    positions, table, slots = positions.to(DEV), table.to(DEV), slots.to(DEV)
+    caches = [(rnd((tokens * per, page, nkv, hd), seed, torch.bfloat16) * 0.5).to(DEV) for seed in (5, 6)]
+    once, far = [c.clone() for c in caches], [c.clone() for c in caches]
+    q = torch.empty((tokens, nh, hd), dtype=torch.bfloat16, device=DEV)
+    ops.qkv_prepare(qkv, q, *caches, n_heads=nh, n_kv_heads=nkv, head_dim=hd, q_weight=qw, k_weight=kw, eps=1e-6,
+                    inv_freq=inv_freq, rot_dim=hd, positions=positions, slot_map=slots, store_kv=True)
+    want = ops.attention_decode(q, *caches, table, None, positions, page_size=page, window=None, scale=hd ** -0.5,
+                                n_splits=splits, n_cuts=cuts)
+    got = ops.attention_decode_fused(qkv, *once, table, None, positions, n_heads=nh, q_weight=qw, k_weight=kw, eps=1e-6,
+                                     inv_freq=inv_freq, slot_map=slots, page_size=page, window=None, scale=hd ** -0.5,
+                                     n_splits=splits, n_cuts=cuts)
+    out = torch.empty_like(got)
+    scratch = torch.empty(tokens * nh * cuts * (hd + 2), device=DEV)
+    assert library.load().pylon_attention_decode_fused(
+        out.data_ptr(), qkv.data_ptr(), qkv.stride(0), 0, 0, qw.data_ptr(), kw.data_ptr(), 1e-6, inv_freq.data_ptr(),
+        far[0].data_ptr(), far[1].data_ptr(), slots.data_ptr(), table.data_ptr(), per, None, positions.data_ptr(), tokens, nh,
+        nkv, hd, page, 0, hd ** -0.5, splits, cuts, scratch.data_ptr() if cuts > 1 else None, scratch.numel(), 0,
+        torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(got, want) and torch.equal(out, want)
+    for k, v in (once, far):
+        assert torch.equal(k, caches[0]) and torch.equal(v, caches[1])
+
+
 def test_kernels_refuse_what_they_cannot_do(ops):
     from pylon_amd.kernels import KernelError
 

@@ -252,3 +252,17 @@ def test_a_product_keeps_its_gradient(ops, rows, n, k):
     torch.testing.assert_close(x.grad.float(), w.float().sum(0).expand(rows, k), rtol=2.0 ** -8, atol=2.0 ** -16 * 300)
     with torch.no_grad():
         torch.testing.assert_close(ops.linear(x, w), y.detach(), rtol=2.0 ** -7, atol=2.0 ** -15 * 100)
+
+
+# either side of 32 rows, where the close head goes to the library, and of 64, where the one apart does
+@pytest.mark.parametrize("rows", [1, 32, 33, 64, 65])
+def test_a_head_with_its_rows_apart(ops, rows):
+    """float32 logits of a tall head whose rows lie apart, and of one whose rows are close, as torch gives them in 64 bits."""
+    n, k = 32768 + 40, 4096
+    x = torch.randn(rows, k, device=DEV).to(torch.bfloat16)
+    apart = torch.full((n, k + 64), float("nan"), dtype=torch.bfloat16, device=DEV)[:, :k]
+    apart.copy_(torch.randn(n, k, device=DEV) * 0.02)
+    want = x.double() @ apart.double().T
+    for w in (apart, apart.contiguous()):
+        got = ops.linear(x, w, out_dtype=torch.float32)
+        assert ((got.double() - want).abs().max() <= 2.0 ** -18 * want.abs().max())  # float32 sums of 4,096 products
