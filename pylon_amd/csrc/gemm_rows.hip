@@ -135,7 +135,8 @@ __device__ __forceinline__ void gemm_rows_body(
   const unsigned x_bytes = (static_cast<unsigned>(M - 1) * ldx + K) * 2u;
 
   // A load fills rows 4 q .. 4 q + 3 of a tile (q: the quarter): lane l brings, for row
-  // R = 4 q + l / 16, the piece (l % 16) ^ R.  Byte offsets in chunk 0.
+  // R = 4 q + l / 16, the piece (l % 16) ^ R.  Byte offsets in chunk 0: of at most 128 rows of 8 MB, which the host sees
+  // to, so that none of them, nor with a chunk's added, passes 2^31.
   // x: this wave fills quarters QW * wave .. of every tile of x; w: all four of its own CT tiles.
   const int lrow = lane >> 4, piece = (lane & 15) ^ lrow;
   unsigned x_at[QW][MT], w_at[GLU ? 1 : CT][4];
@@ -350,11 +351,11 @@ struct GrLaunch {
 // share for every workgroup of as many whole rounds over the units as workgroups of full
 // width would need (at least 16 columns), unless that makes the workgroups re-read more rows
 // of x than they stream rows of w; then, and beyond 16 rows of x in launches of several rounds
-// whose last is not mostly empty, the full width.  Measured at 2560 x 9728, K cut in eight, 32 rows: 13.2 us with 80 columns
-// (256 workgroups) against 14.9 with 128 (160); 2560 x 4096 cut in four, 48 rows: 9.15 with
-// 40 columns against 9.08 with 64; the head of 151936 rows at 8 rows of x: 136.5 with 119
-// columns against 141; at 64 rows of x (4.6 rounds): 181 against 170.5; a gate/up matrix of
-// 2 x 17408 rows at 17 rows of x (1.06 rounds of 64 columns): 34 columns in 512 workgroups.
+// whose last is not mostly empty, the full width.  Measured at 2560 x 9728, K cut in eight, 32 rows: 11.2 us with 80
+// columns (256 workgroups) against 12.9 with 128 (160); 2560 x 4096 cut in four, 48 rows: 8.1 with
+// 40 columns against 8.4 with 64; the head of 151936 rows at 8 rows of x: 137.6 with 119
+// columns against 138.4; at 64 rows of x (4.6 rounds): 179.6 against 169.1; a gate/up matrix of
+// 2 x 17408 rows at 17 rows of x (1.06 rounds of 64 columns): 65 with 34 columns in 512 workgroups against 86.
 static GrLaunch gr_launch_shape(int M, int N, int parts, int col_tiles, int glu, int waves, int units, int cols) {
   const int wave_cols = (glu ? 1 : col_tiles) * 16;
   if (waves == 0)
@@ -466,6 +467,7 @@ extern "C" int pylon_gemm_rows(void* out, int out_dtype, const void* x, const vo
   PYLON_REQUIRE(parts == 1 || !glu, "gemm_rows: the gated epilogue needs the whole of K");
   PYLON_REQUIRE(parts == 1 || part_stride >= static_cast<long long>(M) * ldo,
                 "gemm_rows: partial results overlap");
+  // (one view once spanned gate and up rows; each has its own now, and larger matrices stay refused)
   PYLON_REQUIRE(!glu || (static_cast<long long>(N) + 64) * ldw * 2 < (1ll << 31),
                 "gemm_rows: a fused gate/up matrix of %d rows of %lld elements is beyond the 2 GB a "
                 "workgroup's view of it may span", 2 * N, ldw);

@@ -1070,7 +1070,7 @@ def decode_splits(tokens: int, n_kv_heads: int, max_len: Optional[int], units: i
     waves = 8
     if tokens * n_kv_heads > units:
         # more workgroups than compute units: smaller ones run side by side (64 tokens of 140
-        # keys: 13.8 us with four waves, 21.6 with eight; of 1,000 keys: 47 against 52)
+        # keys: 11.6 us with four waves, 13.7 with eight; of 1,000 keys: 48.0 against 48.5)
         waves = 4
     while waves > 1 and tokens * n_kv_heads * waves > 16 * units:
         waves //= 2
@@ -1094,11 +1094,11 @@ def decode_cuts(tokens: int, n_kv_heads: int, max_len: Optional[int], units: int
     the chip.  From 768 keys of ``max_len`` on (which may be an upper bound above the true
     lengths), each cut at least 192 keys, up to one workgroup per compute unit.  Measured on 256
     units with 8 key/value heads of 128, the launch with its merge against one workgroup per
-    (token, head): 1 token of 1,000 keys 14.1 us (4 cuts) against 20.6, of 2,000 keys 14.1 (8)
-    against 31, of 8,000 keys 19.1 (32) against 125; 8 tokens of 700 keys 15.2 (4) against 19.7,
-    of 2,000 keys 23.6 (4) against 42; 16 tokens of 2,000 keys 35 (2) against 49.  At 500 keys one
-    workgroup is within a microsecond (13.2 to 14.3 us); and once the workgroups fill the units
-    (32 tokens) a cut only adds the second kernel."""
+    (token, head): 1 token of 1,000 keys 7.9 us (4 cuts) against 10.7, of 2,000 keys 7.8 (8)
+    against 17.4, of 8,000 keys 12.6 (32) against 90; 8 tokens of 700 keys 10.0 (4, where the bound is 768) against
+    12.1, of 2,000 keys 18.0 (4) against 30; 16 tokens of 2,000 keys 29.1 (2) against 34.6.  At 500 keys one
+    workgroup is the fastest or within 0.1 us of it (6.3 to 7.9 us); and once the workgroups fill the units
+    (32 tokens of 2,000 keys: 49 us, 52 with two cuts) a cut only adds the second kernel."""
     if max_len is None or max_len < 768:
         return 1
     cuts = 1

@@ -36,7 +36,7 @@ class Product:
 def aliased_rows(k: int) -> bool:
     """Rows of a power-of-two length of 8 KB or more: the 256-byte segments that a chunk is of
     many rows then meet in few memory channels, and the rows kernel streams 10 to 20 % slower
-    (gate/up 2x12288 x 4096 at 8 rows: 44 us against the skinny kernel's 40)."""
+    (gate/up 2x12288 x 4096 at 8 rows: 42 us against the skinny kernel's 39)."""
     return k % 4096 == 0
 
 
@@ -45,8 +45,8 @@ def gated_row_padding(k: int, element_size: int) -> int:
     (of rows of at least 1,024 of them).
     A workgroup's gate rows and its up rows, half the matrix further, otherwise tend to meet in
     the same memory channels, most of all where a row is a power-of-two length of 8 KB or more:
-    2x12288 x 4096: the rows kernel at 8 rows 43.0 -> 34.7 us (which then beats the skinny
-    kernel's 37.4), at 64 rows 47.3 -> 39.3.  At other widths the streaming kernels gain little
+    2x12288 x 4096: the rows kernel at 8 rows 42.4 -> 35.4 us (which then beats the skinny
+    kernel's 38.7), at 64 rows 45.1 -> 37.9.  At other widths the streaming kernels gain little
     (2x9728 x 2560 at 8 rows 20.1 -> 19.5 us) and the library's product for prompt portions some
     (2,048 rows of 2x9728 x 2560: 212 -> 187 us alone, 0.2 ms of a 19.8 ms step): a whole step
     at the Qwen3-4B shape 2.526 -> 2.516 ms decoding and 19.81 -> 19.60 ms for 2,048 prompt tokens,
@@ -109,17 +109,19 @@ def plan_residual(rows: int, n: int, k: int, units: int = UNITS) -> Product:
     ``rows`` <= 128: float32 sums, never rounded, from whichever kernel.
 
     Up to 16 rows the rows kernel beats the skinny one for deep, narrow and moderately wide
-    matrices (2560x4096 at 8 rows: 6.2 against 8.3 us, 2560x9728 11.5 against 13.8, 5120x8192
-    20 against 23, 5120x25600 52 against 65).  From 17 to 64 rows the rows kernel with K cut
-    into parts beats the library, which does not cut K (at 64 rows: 2560x4096 10.0 against
-    14.3 us, 2560x9728 16.0 against 28.0, 4096x4096 11.0 against 15.1, 4096x12288 26.5 against
-    37.5, 5120x5120 16.3 against 21.8, 5120x8192 22.9 against 28.9, 5120x17408 42 against 86,
-    6144x6144 21.5 against 26.8, 10240x10240 48 against 60), except for wide matrices whose rows
-    are of a power-of-two length (8192x8192 36.4 against 33.7, 16384x4096 37.4 against 34.5).
+    matrices (2560x4096 at 8 rows: 5.8 against 8.5 us, 2560x9728 10.9 against 14.0, 5120x8192
+    20.1 against 23.2, 5120x25600 48 against 65).  Of wider ones those whose rows are of a power-of-two
+    length are the skinny kernel's (16384x4096 30 against 35); the others stay with it, too, since an earlier form of
+    the rows kernel (10240x10240 59, where the rows kernel now takes 36).  From 17 to 64 rows the rows
+    kernel with K cut into parts beats the library, which does not cut K (at 64 rows: 2560x4096 8.5 against
+    14.3 us, 2560x9728 13.4 against 28.0, 4096x4096 9.5 against 15.1, 4096x12288 22.4 against
+    36.6, 5120x5120 13.5 against 21.5, 5120x8192 21.4 against 28.8, 5120x17408 37 against 86,
+    6144x6144 17.7 against 25.4, 10240x10240 42 against 57), except for wide matrices whose rows
+    are of a power-of-two length (8192x8192 33.9 against 32.2, 16384x4096 36.0 against 32.6).
     From 65 to 128 rows the rows kernel takes the rows as two halves, each to workgroups of its
     own, two that stream the same rows of w side by side on one die: 2560x9728 at 65, 96 and 128
-    rows 22.6, 23.0 and 26.2 us against the library's 26.2, 26.9 and 52.9 (bfloat16 result),
-    2560x4096 14.1, 14.3 and 16.8 against 20.9, 20.9 and 22.9; the same choices as for 64 rows."""
+    rows 19.0, 19.9 and 22.4 us against the library's 25.3, 26.0 and 52.2 (bfloat16 result),
+    2560x4096 12.1, 13.2 and 15.0 against 13.1, 13.0 and 23.8; the same choices as for 64 rows."""
     few = rows <= FEW_ROWS
     if few:
         if deep_or_narrow(n, k) or n <= 8192:
@@ -137,18 +139,17 @@ def plan_projection(rows: int, n: int, k: int, row_stride: int = 0) -> Product:
     matrix in memory; it counts at the widths of :func:`head_row_padding`.
 
     A head (tall matrix): the rows kernel with 128 columns per workgroup (151936 x 2560: 137 us
-    against the skinny kernel's 154 at 8 rows; 173 against the library's 186 at 64 rows, 150
-    against 173 at 32; x 5120: 264 against 304 and 303 against 313).  With aliased rows (x 4096)
-    64 columns per workgroup do better (220 against 227 us at 1 row, 230 against 235 at 8, 262
-    against 272 at 32, the skinny kernel 237, 234 and, at 16 rows, 258 against 239), and beyond
-    32 rows the library (274 against 286 and 300 at 64 rows); an engine's head of that width has
-    its rows apart (:func:`head_row_padding`) and goes as the others.
-    A projection up to 16 rows: the rows kernel (6144 x 2560 at 8 rows 9.3 against the skinny
-    kernel's 10.7 us, 10240 x 5120 21 against 31, 6144 x 4096 14.5 against 16).  Beyond 16
-    rows the library: without K cut over workgroups the rows kernel is within 10 % of it either
-    way (6144 x 2560: 12.2 against 11.8 us at 32 rows, 17.8 against 15.5 at 64), and the rows of
-    x of a workgroup that covers 64 of many columns weigh most here; a consumer that adds
-    partial sums gets them (:func:`plan_summed_later`)."""
+    against the skinny kernel's 157 at 8 rows; 167 against the library's 184 at 64 rows, 147
+    against 171 at 32; x 5120: 267 against 302 and 294 against 310).  With aliased rows (x 4096)
+    64 columns per workgroup do better (221 against 224 us at 1 row, 229 against 231 at 8, 258
+    against 276 at 32), and beyond 32 rows the library (270 against 291 and 287 at 64 rows); an
+    engine's head of that width has its rows apart (:func:`head_row_padding`) and goes as the others.
+    A projection up to 16 rows: the rows kernel (6144 x 2560 at 8 rows 9.4 against the skinny
+    kernel's 12.1 us, 10240 x 5120 20 against 31, 6144 x 4096 11.7 against 16.2).  Beyond 16
+    rows the library, beside which the rows kernel without K cut over workgroups was within 10 % either way when
+    this line was drawn, with the rows of x of a workgroup that covers 64 of many columns weighing most (now 6144 x
+    2560 11.7 against 13.1 us at 32 rows, 13.2 against 15.5 at 64; 6144 x 4096 14.3 against 15.1 and 19.0
+    against 17.8); a consumer that adds partial sums gets them (:func:`plan_summed_later`)."""
     few = rows <= FEW_ROWS
     if rows > STREAM_ROWS:
         return Product("library")
@@ -166,15 +167,15 @@ def plan_summed_later(rows: int, n: int, k: int, units: int = UNITS) -> Product:
     launch would leave compute units without one.
 
     Up to 16 rows: workgroups of 64 columns and 2 or 4 parts, as many as keep the workgroups
-    within the units.  At 8 rows 6144 x 2560 takes 7.8 us (2 parts) against 10.3 uncut, 4096 x
-    2048 5.5 (4) against 8.5, 6144 x 4096 12.3 (2) against 14.5, 7168 x 5120 15.0 (2) against
-    17.6; 10240 x 5120 stays uncut (19.8 against 20.1).  With what the attention kernel then
-    pays for adding them, a whole step at the Qwen3-4B shape, batch 8: 2.603 -> 2.531 ms.
+    within the units.  At 8 rows 6144 x 2560 takes 7.6 us (2 parts) against 9.4 uncut, 4096 x
+    2048 5.0 (4) against 7.1, 7168 x 2560 8.6 against 9.3; 6144 x 4096 (12.1 against 11.7) and 7168 x 5120 (14.1
+    either way) gain nothing since an uncut launch starts sooner; 10240 x 5120 stays uncut.  With what the
+    attention kernel then pays for adding them, a whole step at the Qwen3-4B shape, batch 8, was 2.603 -> 2.531 ms.
     From 17 to 64 rows the rows kernel so cut beats the library, which does not cut K: 6144 x
-    2560 at 17, 32, 48 and 64 rows 9.0, 9.5, 10.8 and 11.7 us (four parts of 128 columns) against
-    11.0, 11.8, 15.3 and 15.5; 6144 x 4096 11.8 to 14.9 against 14.5 to 17.9; 10240 x 5120 (two
-    parts) 21.5 to 28.1 against 24.4 to 32.8.  From 65 to 128 rows, as two halves: 6144 x 2560 15.4 to
-    18.2 us against the library's 20.9 to 21.3.  Without a cut as :func:`plan_projection`."""
+    2560 at 17, 32, 48 and 64 rows 8.0, 8.3, 9.3 and 9.8 us (four parts of 128 columns) against
+    12.6, 13.1, 15.5 and 15.5; 6144 x 4096 10.4 to 12.3 against 14.6 to 17.8; 10240 x 5120 (two
+    parts) 19.7 to 23.1 against 23.8 to 31.8.  From 65 to 128 rows, as two halves: 6144 x 2560 13.1 to
+    15.8 us against the library's 16.3 to 19.0.  Without a cut as :func:`plan_projection`."""
     if n < TALL and rows <= FEW_ROWS:
         groups, parts = -(-n // 64), 1
         while parts < 4 and 2 * parts * groups <= units and k // (2 * parts) >= 256:
@@ -191,10 +192,11 @@ def plan_summed_later(rows: int, n: int, k: int, units: int = UNITS) -> Product:
 def rows_match_library(rows: int, n: int, k: int) -> bool:
     """Whether a bfloat16 product of 17 to 48 rows that :func:`plan_projection` leaves to the library takes the
     rows kernel after all: for matrices wide enough to fill the compute units uncut, whose rows are of no
-    power-of-two length, the device takes no longer (at 17, 32 and 48 rows 6144 x 2560 15.9, 15.6, 18.3 us
-    against 15.6, 15.8, 20.4; 7168 x 2560 16.2, 16.4, 18.7 against 16.5, 16.8, 20.9; 10240 x 5120 33.0, 33.5,
-    38.5 against 34.3, 35.2, 39.9; but 6144 x 4096 21.2, 21.1, 24.8 against 19.8, 20.1, 22.0) and the host 10
-    us instead of 26, which is what a step of few prompt tokens waits for."""
+    power-of-two length, the device takes no longer (at 17, 32 and 48 rows 6144 x 2560 10.8, 11.7, 11.6 us
+    against 12.6, 13.1, 15.5; 7168 x 2560 9.4, 9.9, 11.9 against 11.3, 11.8, 15.8; 10240 x 5120 19, 21, 28
+    against 24, 25, 31; rows of a power-of-two length were the slower ones when this was drawn, 6144 x 4096 is now 13.1,
+    14.3, 16.1 against 14.6, 15.1, 17.2) and the host 10 us instead of 26, which is what a step of few prompt
+    tokens waits for."""
     return rows <= 48 and 5120 <= n < TALL and not aliased_rows(k)
 
 
@@ -251,16 +253,17 @@ def plan_gated(rows: int, n_half: int, k: int, row_stride: int) -> Product:
     """``silu(x gate^T) * (x up^T)`` over a fused matrix of ``2 * n_half`` rows; "library" means
     its product followed by the activation kernel (up to 64 rows its float32 result).
 
-    Against the skinny kernel at 8 rows: 2x9728 x 2560 20 against 25 us, 2x25600 x 5120 90
-    against 105, 2x17408 x 5120 63 against 76, 2x6144 x 2048 13.8 against 15.2; but 2x12288 x
-    4096 44 against 39 (aliased rows; with the rows :func:`gated_row_padding` apart in memory
-    34.7 against 37.4) and 2x3072 x 1024 7.4 against 6.1 (a small matrix).
-    Against the library and the activation kernel from 17 to 64 rows: 2x9728 x 2560 21 to 27
-    against 30 to 34, 2x12288 x 4096 45 to 48 against 48 to 53, 2x17408 x 5120 67 to 86 against
-    78 to 93, 2x25600 x 5120 91 to 105 against 94 to 107, 2x3072 x 1024 9.3 to 12.8 against
-    13.8 to 14.3 (2x6144 x 2048 at 64 rows alone loses, 20.9 against 19.8).  A workgroup of the
-    rows kernel sees its gate rows and, ``n_half`` rows further, its up rows through one
-    descriptor, which spans at most 2 GB."""
+    Against the skinny kernel at 8 rows: 2x9728 x 2560 19.4 against 24.7 us, 2x25600 x 5120 91
+    against 103, 2x17408 x 5120 63 against 73, 2x6144 x 2048 10.6 against 14.4; but 2x12288 x
+    4096 42 against 39 (aliased rows; with the rows :func:`gated_row_padding` apart in memory
+    35.4 against 38.7).  Small matrices stay with the skinny kernel since an earlier form of the other (2x3072 x
+    1024 6.7, where the rows kernel now takes 6.0).
+    Against the library and the activation kernel from 17 to 64 rows: 2x9728 x 2560 19 to 23
+    against 25 to 30, 2x12288 x 4096 43 to 45 against 48 to 50 (apart 36 to 38 against 40 to 44), 2x17408 x
+    5120 66 to 76 against 82 to 89, 2x25600 x 5120 92 to 94 against 94 to 106, 2x6144 x 2048 11.4 to 15.0
+    against 17.2 to 18.6, 2x3072 x 1024 6.4 to 8.9 against 14.0 to 14.5.  Matrices whose up rows lie 2 GB and
+    more behind their gate rows are not the rows kernel's: one view once spanned both (each half now has its own), and
+    nothing of that size has been measured."""
     if rows > STREAM_ROWS:  # 2x9728 x 2560 at 65 to 128 rows: 41 to 48 us against the library's 36 to 38
         return Product("library")
     few = rows <= FEW_ROWS
