@@ -239,18 +239,26 @@ __global__ __launch_bounds__(512) void attention_sink_kernel(
       float sc[8];
       const int near = qpos[qt] - (kb + AS_BLOCK - 1);  // the smallest distance of the block for this query
       const bool all_far = bias == nullptr || near >= bucket_len - 1;
+      // (one question a block, of the whole wave, whose far queries find far_bias in the table's last entry.  A question a
+      // key was the compiler's to lay in or out of the walk: 2,048 tokens of 32 heads of 128 with a bias 218 us in and
+      // 228 out of it, without one 216 and 211; so 210 and 196.)
+      float by_distance[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) by_distance[e] = far_bias;
+      if (__builtin_amdgcn_ballot_w64(!all_far) != 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int dist = qpos[qt] - (kb + (e >> 2) * 16 + 4 * grp + (e & 3));
+          const int idx = dist < 0 ? 0 : dist;
+          by_distance[e] = tbl[idx < bucket_len - 1 ? idx : bucket_len - 1];
+        }
+      }
       float top = m_run[qt];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int key = kb + (e >> 2) * 16 + 4 * grp + (e & 3);
         const int dist = qpos[qt] - key;
-        float bias = far_bias;
-        if (!all_far) {
-          int idx = dist < 0 ? 0 : dist;
-          idx = idx < bucket_len - 1 ? idx : bucket_len - 1;
-          bias = tbl[idx];
-        }
-        const float v = capped_score(s[qt][e >> 2][e & 3], scale, softcap) + bias;
+        const float v = capped_score(s[qt][e >> 2][e & 3], scale, softcap) + by_distance[e];
         sc[e] = (dist >= 0 && key >= qfirst[qt]) ? v : -INFINITY;
         top = fmaxf(top, sc[e]);
       }
