@@ -17,7 +17,8 @@
 //
 // Scores come from the 16x16x32 bf16 matrix instruction with 16 keys as rows and the group's query heads, as often
 // as they fit, as columns; every copy then takes the softmax of other tiles.  The weighted sum of values takes
-// the probabilities as three bfloat16 parts each (exact for finite values; others are seen in the result).  Softmax statistics are float throughout.
+// the probabilities as three bfloat16 parts each (exact for finite values; others are seen in the result).
+// Softmax statistics are float throughout.
 //
 // The kernel can also take over the step that precedes attention: given the raw q/k/v
 // projection instead of prepared queries, each workgroup first norms and rotates its
