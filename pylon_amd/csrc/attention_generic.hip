@@ -65,6 +65,20 @@ __device__ __forceinline__ float att_over(float v, OP op) {
   }
 }
 
+// What a score becomes before the softmax: scaled, capped, with the bias by distance.
+__device__ __forceinline__ float att_score(float dot, float scale, float softcap, const float* __restrict__ rel,
+                                           const int* __restrict__ bucket, int bucket_len, int n_heads, int h, int far) {
+  float s = dot * scale;
+  if (softcap > 0.f) s = softcap * tanhf(s / softcap);
+  if (rel != nullptr) {
+    if (bucket != nullptr)
+      s += rel[static_cast<size_t>(bucket[far < bucket_len ? far : bucket_len - 1]) * n_heads + h];
+    else
+      s -= rel[h] * logf(1.0f + rel[n_heads + h] * static_cast<float>(far));
+  }
+  return s;
+}
+
 template <typename T, int DIMS_PER_LANE>
 __global__ void paged_attention_kernel(T* __restrict__ out, const T* __restrict__ q,
                                        const T* __restrict__ k_cache, const T* __restrict__ v_cache,
@@ -118,15 +132,7 @@ __global__ void paged_attention_kernel(T* __restrict__ out, const T* __restrict_
 #pragma unroll 8
         for (int d = 0; d < head_dim; d += 8) dot = Vec8<T>::dot(qbuf + d, kr + d, dot);
       }
-      s = dot * scale;
-      if (softcap > 0.f) s = softcap * tanhf(s / softcap);
-      if (rel != nullptr) {
-        const int far = pos - j;
-        if (bucket != nullptr)
-          s += rel[static_cast<size_t>(bucket[far < bucket_len ? far : bucket_len - 1]) * n_heads + h];
-        else
-          s -= rel[h] * logf(1.0f + rel[n_heads + h] * static_cast<float>(far));
-      }
+      s = att_score(dot, scale, softcap, rel, bucket, bucket_len, n_heads, h, pos - j);
     }
     const float m_new = fmaxf(m, att_over<T, DIMS_PER_LANE>(s, [](float a, float b) { return fmaxf(a, b); }));
     const float p = valid ? expf(s - m_new) : 0.f;
@@ -185,6 +191,174 @@ __global__ void paged_attention_kernel(T* __restrict__ out, const T* __restrict_
   }
 }
 
+// The same in float32 for few (token, head) pairs: a workgroup each, where the kernel above has a wavefront that makes
+// trip after trip to memory (of 120 keys: 4 for the keys, 16 for their values).  Four wavefronts score a block of 64
+// keys each, a key a lane, all of a key's elements under way at once; one or two more (64 elements of the values each)
+// have the values of two blocks on their way meanwhile.  Every number is formed as above and in its order: a key's dot
+// product along its elements, a block's maximum and sum over the lanes, blocks one after the other on the running
+// maximum, an element's products key by key; so the bits are the same, and which kernel runs is a matter of time
+// alone.  What bounds it is one trip to memory for the table and one for keys and values a round of 256 keys, and the
+// chain of products.  32 heads of 128 over 8, us of the kernel above and of this: 3 tokens of about 100 keys 25.7, 8.0; 16
+// of 120 27, 16.5; 8 of 700 142, 41; 1 of 8,000 1,496, 385; 1 of 1 5.9, 4.8.
+template <int KD>  // elements of a key: 64 KD
+__device__ __forceinline__ void paged_attention_few_body(
+    float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ k_cache,
+    const float* __restrict__ v_cache, const int* __restrict__ block_table, int table_width,
+    const int* __restrict__ tok_row, const int* __restrict__ positions, int n_heads, int n_kv_heads, int page_size,
+    int window, float scale, int v_dim, long long q_stride, const float* __restrict__ rel,
+    const int* __restrict__ bucket, int bucket_len, int sink, float softcap, const float* __restrict__ sink_logit,
+    int v_row) {
+  constexpr int DIM = 64 * KD, BLOCKS = 4;  // blocks of 64 keys a round
+  __shared__ __attribute__((aligned(16))) float qbuf[DIM];
+  // of a round and the one before: what weighs a block's keys, their sum, the blocks' maxima
+  __shared__ float weight[2][BLOCKS][PYLON_WAVE], total[2][BLOCKS], top[2][BLOCKS];
+  const int lane = threadIdx.x & (PYLON_WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PYLON_WAVE);
+  const int t = blockIdx.x / n_heads, h = blockIdx.x - t * n_heads;
+  const int kvh = h / (n_heads / n_kv_heads);
+  const int pos = __builtin_amdgcn_readfirstlane(positions[t]);
+  const int* table = block_table + static_cast<size_t>(__builtin_amdgcn_readfirstlane(tok_row[t])) * table_width;
+  const int first = first_visible(pos, window);
+  for (int i = threadIdx.x; i < DIM; i += blockDim.x)
+    qbuf[i] = q[static_cast<size_t>(t) * q_stride + static_cast<size_t>(h) * DIM + i];
+  __syncthreads();
+  auto slot_of = [&](int j) { return table[j / page_size] * page_size + (j % page_size); };
+
+  // The running maximum behind each block of a round, and what the sums so far are multiplied with there.
+  float m = -INFINITY;
+  auto follow = [&](int parity, int blocks, float (&after)[BLOCKS], float (&corr)[BLOCKS]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < BLOCKS; ++b)
+      if (b < blocks) {
+        after[b] = fmaxf(m, top[parity][b]);
+        corr[b] = expf(m - after[b]);
+        m = after[b];
+      }
+  };
+  int parity = 0;
+  if (wave < BLOCKS) {
+    for (int base = first; base <= pos; base += BLOCKS * PYLON_WAVE, parity ^= 1) {
+      const int blocks = (pos - base) / PYLON_WAVE + 1 < BLOCKS ? (pos - base) / PYLON_WAVE + 1 : BLOCKS;
+      const int j = base + wave * PYLON_WAVE + lane;
+      const bool valid = j <= pos;
+      float s = -INFINITY;
+      if (wave < blocks) {
+        if (valid) {
+          const float* kr = k_cache + (static_cast<size_t>(slot_of(j)) * n_kv_heads + kvh) * DIM;
+          float4 key[DIM / 4];
+#pragma unroll
+          for (int d = 0; d < DIM / 4; ++d) key[d] = *reinterpret_cast<const float4*>(kr + 4 * d);
+          float dot = 0.f;
+#pragma unroll
+          for (int d = 0; d < DIM / 4; ++d) {
+            const float4 e = *reinterpret_cast<const float4*>(qbuf + 4 * d);
+            dot = fmaf(e.x, key[d].x, dot);
+            dot = fmaf(e.y, key[d].y, dot);
+            dot = fmaf(e.z, key[d].z, dot);
+            dot = fmaf(e.w, key[d].w, dot);
+          }
+          s = att_score(dot, scale, softcap, rel, bucket, bucket_len, n_heads, h, pos - j);
+        }
+        const float most = wave_max(s);
+        if (lane == 0) top[parity][wave] = most;
+      }
+      __syncthreads();
+      float after[BLOCKS], corr[BLOCKS];
+      follow(parity, blocks, after, corr);
+#pragma unroll
+      for (int b = 0; b < BLOCKS; ++b)
+        if (b == wave && b < blocks) {
+          const float p = valid ? expf(s - after[b]) : 0.f;
+          const float sum = wave_sum(p);
+          weight[parity][b][lane] = p;
+          if (lane == 0) total[parity][b] = sum;
+        }
+      __syncthreads();
+    }
+    return;
+  }
+
+  const int d = (wave - BLOCKS) * PYLON_WAVE + lane;  // this lane's element of the values
+  const char* const values = reinterpret_cast<const char*>(v_cache + static_cast<size_t>(kvh) * v_row);
+  const unsigned row_bytes = static_cast<unsigned>(n_kv_heads) * v_row * 4u;
+  float l = 0.f, acc = 0.f;
+  for (int base = first; base <= pos; base += BLOCKS * PYLON_WAVE, parity ^= 1) {
+    const int blocks = (pos - base) / PYLON_WAVE + 1 < BLOCKS ? (pos - base) / PYLON_WAVE + 1 : BLOCKS;
+    float even[PYLON_WAVE], odd[PYLON_WAVE];
+    auto bring = [&](float (&v)[PYLON_WAVE], int b) __attribute__((always_inline)) {
+      if (b >= blocks) return;
+      const int j = base + b * PYLON_WAVE + lane;
+      const int slot = slot_of(j < pos ? j : pos);  // beyond the last key: that one again, not used
+      // a view of each row: lanes beyond its elements bring zeros, without a branch
+#pragma unroll
+      for (int k = 0; k < PYLON_WAVE; ++k) {
+        const unsigned long long row = static_cast<unsigned long long>(static_cast<unsigned>(__builtin_amdgcn_readlane(slot, k))) * row_bytes;
+        v[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(values + row), 0, v_dim * 4, 0x00020000), d * 4, 0, 0));
+      }
+    };
+    bring(even, 0);
+    bring(odd, 1);
+    __syncthreads();
+    float after[BLOCKS], corr[BLOCKS];
+    follow(parity, blocks, after, corr);
+    __syncthreads();
+    auto add = [&](const float (&v)[PYLON_WAVE], int b) __attribute__((always_inline)) {
+      if (b >= blocks) return;
+      l = l * corr[b] + total[parity][b];
+      acc *= corr[b];
+      const int count = pos - (base + b * PYLON_WAVE) + 1 < PYLON_WAVE ? pos - (base + b * PYLON_WAVE) + 1 : PYLON_WAVE;
+      const float p = weight[parity][b][lane];
+      auto weight_of = [&](int k) __attribute__((always_inline)) {
+        return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), k));
+      };
+      if (count == PYLON_WAVE) {
+#pragma unroll
+        for (int k = 0; k < PYLON_WAVE; ++k) acc = fmaf(weight_of(k), v[k], acc);
+      } else {
+#pragma unroll
+        for (int k = 0; k < PYLON_WAVE; ++k)
+          if (k < count) acc = fmaf(weight_of(k), v[k], acc);
+      }
+    };
+    add(even, 0);
+    bring(even, 2);
+    add(odd, 1);
+    bring(odd, 3);
+    add(even, 2);
+    add(odd, 3);
+  }
+  if (sink_logit != nullptr) {
+    const float z = sink_logit[h];
+    const float m_fin = fmaxf(m, z);
+    const float corr = expf(m - m_fin);
+    l = l * corr + expf(z - m_fin);
+    acc *= corr;
+  } else if (sink) {
+    l += expf(-m);
+  }
+  if (d < v_dim) out[(static_cast<size_t>(t) * n_heads + h) * v_dim + d] = acc * (1.0f / l);
+}
+
+template <int KD>
+__global__ __launch_bounds__(6 * PYLON_WAVE) void paged_attention_few_kernel(
+    float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ k_cache,
+    const float* __restrict__ v_cache, const int* __restrict__ block_table, int table_width,
+    const int* __restrict__ tok_row, const int* __restrict__ positions, int n_heads, int n_kv_heads, int page_size,
+    int window, float scale, int v_dim, long long q_stride, const float* __restrict__ rel,
+    const int* __restrict__ bucket, int bucket_len, int sink, float softcap, const float* __restrict__ sink_logit,
+    int v_row) {
+  paged_attention_few_body<KD>(out, q, k_cache, v_cache, block_table, table_width, tok_row, positions, n_heads, n_kv_heads,
+                               page_size, window, scale, v_dim, q_stride, rel, bucket, bucket_len, sink, softcap, sink_logit, v_row);
+}
+
+// Whether the kernel of a workgroup a pair takes a float32 launch: up to two workgroups a compute unit (beyond, the
+// wavefronts of the other hide each other's waits: 48 tokens of 120 keys, 32 heads, 41 us against 35; 16 of them 17
+// against 27).
+static bool att_few(long long items, int head_dim, int v_dim, int v_transposed) {
+  return items <= 2 * pylon_compute_units() && (head_dim == 64 || head_dim == 128) && v_dim <= 128 && !v_transposed;
+}
+
 template <typename T>
 static int launch_paged_attention(T* out, const T* q, const T* k_cache, const T* v_cache,
                                   const int* block_table, int table_width, const int* tok_row,
@@ -194,6 +368,21 @@ static int launch_paged_attention(T* out, const T* q, const T* k_cache, const T*
                                   int sink, int v_transposed, float softcap, const float* sink_logit,
                                   int v_row, hipStream_t stream) {
   const long long items = static_cast<long long>(tokens) * n_heads;
+  if constexpr (sizeof(T) == 4) {
+    if (att_few(items, head_dim, v_dim, v_transposed)) {
+      const dim3 few_grid(static_cast<unsigned>(items)), few_block((4 + (v_dim + 63) / 64) * PYLON_WAVE);
+#define FEW(KD)                                                                                                  \
+  hipLaunchKernelGGL((paged_attention_few_kernel<KD>), few_grid, few_block, 0, stream, out, q, k_cache, v_cache, \
+                     block_table, table_width, tok_row, positions, n_heads, n_kv_heads, page_size, window, scale, \
+                     v_dim, q_stride, rel, bucket, bucket_len, sink, softcap, sink_logit, v_row)
+      if (head_dim == 64)
+        FEW(1);
+      else
+        FEW(2);
+#undef FEW
+      return 0;
+    }
+  }
   const long long blocks = (items + ATT_WAVES - 1) / ATT_WAVES;
   dim3 grid((unsigned)blocks), block(ATT_WAVES * PYLON_WAVE);
   const size_t lds = sizeof(float) * ATT_WAVES * head_dim;

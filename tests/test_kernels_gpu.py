@@ -669,6 +669,40 @@ def test_paged_attention(ops, dtype, geom):
         assert np.abs(f64(got)[i] - want).max() <= tol(dtype, max(1.0, np.abs(want).max())), (i, r, p)
 
 
+# float32 heads of 64 and 128: a launch of few (token, head) pairs has a kernel of its own, which gives the bits of the
+# general one (the same tokens in a launch of many pairs); keys of part of a block, of whole rounds of four blocks of 64,
+# one more, and none before a window or a chunk; values of less than 64 elements and of up to 128
+@pytest.mark.parametrize("geom", [(8, 2, 128, 128, 16, {}), (4, 4, 64, 40, 32, {"window": 50}), (6, 3, 128, 65, 64, {"chunk": 100}),
+                                  (2, 1, 64, 128, 16, {"softcap": 5.0, "sink": True})])
+def test_float32_attention_of_few_pairs_has_the_bits_of_many(ops, geom):
+    nh, nkv, hd, vd, page, more = geom
+    more = {"window": None, **more}
+    last = [0, 1, 63, 64, 65, 255, 256, 257, 300, 511, 700]  # positions, all in one request
+    pages = -(-(max(last) + 1) // page)
+    kc, vc = rnd((pages, page, nkv, hd), 61).to(DEV), rnd((pages, page, nkv, vd), 62).to(DEV)
+    table = torch.randperm(pages, generator=torch.Generator().manual_seed(63)).to(torch.int32).reshape(1, -1).to(DEV)
+    q = rnd((len(last), nh, hd), 64).to(DEV)
+    pos = torch.tensor(last, dtype=torch.int32, device=DEV)
+    times = -(-(2 * ops.compute_units() + 1) // (len(last) * nh))
+
+    def attend(copies):
+        rows = torch.zeros(len(last) * copies, dtype=torch.int32, device=DEV)
+        return ops.paged_attention(q.repeat(copies, 1, 1), kc, vc, table, rows, pos.repeat(copies), page_size=page,
+                                   scale=hd ** -0.5, **more)
+
+    few, many = attend(1), attend(times)
+    for i in range(times):
+        assert torch.equal(few, many[i * len(last): (i + 1) * len(last)])
+    if not more.get("softcap"):
+        flat = [f64(c)[table[0].cpu().numpy()].reshape(pages * page, nkv, -1) for c in (kc, vc)]
+        for i, p in enumerate(last):
+            first = p // more["chunk"] * more["chunk"] if "chunk" in more else 0
+            keys, values = (f[first: p + 1].transpose(1, 0, 2) for f in flat)
+            want = np.stack([plain_attention(f64(q)[i], keys, np.ascontiguousarray(values[..., j: j + 1]).repeat(hd, 2),
+                                             hd ** -0.5, more["window"])[:, 0] for j in (0, vd - 1)], 1)
+            assert np.abs(f64(few)[i][:, [0, vd - 1]] - want).max() <= tol(torch.float32, 1.0), (i, p)
+
+
 @pytest.mark.parametrize("geom", [(8, 2, 128, 64, None), (4, 4, 64, 16, None), (16, 1, 256, 32, 100),
                                   (6, 2, 128, 256, None), (1, 1, 64, 16, 7)])
 @pytest.mark.parametrize("n_splits,n_cuts", [(1, 1), (2, 1), (4, 1), (8, 1), (1, 2), (4, 3), (8, 8), (2, 64)])
