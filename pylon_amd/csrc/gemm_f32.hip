@@ -10,7 +10,7 @@
 // which gemm_tiled takes: logits of six layers are 2.6e-6 off 64 bits instead of 6.7e-6.)
 //
 // gemm_f32_rows_kernel, up to 32 rows: a step of a few tokens, bound by reading w once.  A
-// workgroup owns a tile of 16 columns; its eight waves take one of the eight ranges
+// workgroup owns a tile of up to 16 columns (gf_row_cols); its eight waves take one of the eight ranges
 // each, so that even a matrix of 2560 rows has 1,280 waves that stream it, and the order of the
 // sums falls out of the order in which the waves' results are added through LDS.  A wave's share
 // of w goes from memory straight into LDS in whole 256-byte row segments (four rows a load;
@@ -20,15 +20,16 @@
 // 384 MB of other traffic, 1, 2, 3 and 4 tiles: 2560 x 9728 40, 51, 69, 83; 6144 x 2560 28, 28, 30, 32; 19456 x 2560
 // 66, 70, 70, 81; 151936 x 2560 289, 298, 311, 312).
 //
-// gemm_f32_tiles_kernel, more rows: LDS tiles, a chunk ahead, a wave a quarter of the tile.  One
-// 16-byte read from LDS feeds four matrix instructions of 32 clocks, so the matrix cores (157 TFLOP/s
-// in float32) are what bounds it: 64 x 64 for many rows; 32 x 32 otherwise, so that a launch of few
-// rows still reaches every compute unit's matrix cores, by two teams of four waves with half of K each.
+// gemm_f32_tiles_kernel, more rows: LDS tiles, a chunk ahead, a wave a quarter of the tile's.  One
+// 16-byte read from LDS feeds four matrix instructions of 32 clocks and more, so the matrix cores (157 TFLOP/s
+// in float32) are what bounds it, where a launch reaches all of them: seven tiles, from 32 x 32 to 96 x 64, some by two
+// teams of four waves with half of K each, chosen by a model of the launch's rounds (gf_tiling).
 //
 // Measured, 4B layer sizes, weights from memory, gemm_tiled (one chain per element on the vector ALUs)
-// before: of a step of 3 rows q/k/v 14 us, gate/up 35 (5.7 TB/s), out and down 34 together, the head 247 (6.3)
-// where a launch took 615 on average; 270 rows 106 + 79 + 299 + 177 (80 to 90 TFLOP/s); 2048 rows 112 TFLOP/s.
+// before: of a step of 3 rows q/k/v 14 us, gate/up 37 (5.4 TB/s), out and down 11 and 22, the head 247 (6.3)
+// where a launch took 615 on average; 270 rows 61 + 135 + 93 + 266 (93 to 106 TFLOP/s; 600 rows 106 to 110).
 #include "gemm_f32.h"
+#include <type_traits>
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef int intx4 __attribute__((ext_vector_type(4)));
@@ -61,8 +62,8 @@ __device__ __forceinline__ void gf_barrier() {
 // kernel that names it, launch stub and all.
 template <int MT>
 __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, const float* x,
-                                                   const float* __restrict__ w, int M, int N, int K, long long ldx,
-                                                   long long ldw, long long ldo) {
+                                                   const float* __restrict__ w, int M, int N, int K, int ldx, int ldw,
+                                                   long long ldo, int cols) {
   // per wave two stages of the tile of w; then the ranges' sums, [range][row tile][64 lanes][4]
   __shared__ __attribute__((aligned(1024))) unsigned char lds[GF_RANGES * 2 * GF_TILE_BYTES + GF_RANGES * MT * 1024];
   float* sums = reinterpret_cast<float*>(lds + GF_RANGES * 2 * GF_TILE_BYTES);
@@ -70,8 +71,8 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
   const int lane = threadIdx.x & (PYLON_WAVE - 1);
   const int range = __builtin_amdgcn_readfirstlane(threadIdx.x / PYLON_WAVE);
   const int r = lane & 15, g = lane >> 4;
-  const int row0 = blockIdx.x * 16;  // first row of w of this workgroup
-  const int rows = (N - row0 < 16) ? N - row0 : 16;
+  const int row0 = blockIdx.x * cols;  // first row of w of this workgroup
+  const int rows = (N - row0 < cols) ? N - row0 : cols;
   const int chunks = (K + GF_CHUNK - 1) / GF_CHUNK;
   const int c_begin = gf_range_begin(range, chunks), c_end = gf_range_begin(range + 1, chunks);
 
@@ -83,45 +84,50 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
 
   // A load brings rows 4 q .. 4 q + 3 of the tile: lane l, for row R = 4 q + l / 16, the 16-byte piece
   // (l % 16) ^ R, which lies at place l % 16 of that row in LDS: operand reads (lane r takes piece
-  // 4 s + g of row r) then fall into different groups of banks.
+  // 4 s + g of row r) then fall into different groups of banks.  The lanes' offsets are those of chunk 0, the chunk's is
+  // scalar; only the chunk that K ends within asks for the lanes' places (the range check of a view does not count the
+  // scalar offset).
   const int lrow = lane >> 4, lpos = lane & 15;
   unsigned char* stage_base = lds + range * 2 * GF_TILE_BYTES;
-  auto issue = [&](int chunk, int stage) {
-    const int k0 = chunk * GF_CHUNK;
+  unsigned w_at[4], x_at[MT], piece_at[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int R = 4 * q + lrow;
-      const int k = k0 + (lpos ^ R) * 4;
-      const bool ok = chunk < c_end && R < rows && k < K;
-      const unsigned at = static_cast<unsigned>(R) * static_cast<unsigned>(ldw) * 4u + static_cast<unsigned>(k) * 4u;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          wres, (GF_LDS(void)*)(stage_base + stage * GF_TILE_BYTES + q * 1024), 16, ok ? at : GF_OOB, 0, 0, 0);
-    }
-  };
-  unsigned piece_at[4];
+  for (int q = 0; q < 4; ++q) {
+    const int R = 4 * q + lrow;
+    w_at[q] = R < rows ? static_cast<unsigned>(R) * static_cast<unsigned>(ldw) * 4u + (lpos ^ R) * 16 : GF_OOB;
+  }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int m = 16 * t + r;
+    x_at[t] = m < M ? static_cast<unsigned>(m) * static_cast<unsigned>(ldx) * 4u + g * 16 : GF_OOB;
+  }
 #pragma unroll
   for (int s = 0; s < 4; ++s) piece_at[s] = (r >> 2) * 1024 + (r & 3) * 256 + (((4 * s + g) ^ r) * 16);
 
+  auto bring = [&](floatx4 (&xv)[MT][4], int chunk, int stage) __attribute__((always_inline)) {
+    const int at = chunk * (GF_CHUNK * 4);
+    auto send = [&](auto w_off, auto x_off, int offset) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          xv[t][s] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xres, x_off(t, s), offset, 0));
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (GF_LDS(void)*)(stage_base + stage * GF_TILE_BYTES + q * 1024), 16,
+                                                 w_off(q), offset, 0, 0);
+    };
+    if ((chunk + 1) * GF_CHUNK <= K) {
+      send([&](int q) { return w_at[q]; }, [&](int t, int s) { return x_at[t] + 64 * s; }, at);
+    } else {
+      const int left = K - chunk * GF_CHUNK;
+      send([&](int q) { return ((lpos ^ (4 * q + lrow)) * 4 < left) ? w_at[q] + at : GF_OOB; },
+           [&](int t, int s) { return 16 * s + 4 * g < left ? x_at[t] + 64 * s + at : GF_OOB; }, 0);
+    }
+  };
   floatx4 acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  auto load_x = [&](floatx4 (&xv)[MT][4], int chunk) {
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int k = chunk * GF_CHUNK + 16 * s + 4 * g;
-        const int m = 16 * t + r;
-        const bool ok = chunk < c_end && m < M && k < K;
-        const unsigned at = static_cast<unsigned>(m) * static_cast<unsigned>(ldx) * 4u + static_cast<unsigned>(k) * 4u;
-        xv[t][s] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xres, ok ? at : GF_OOB, 0, 0));
-      }
-  };
-  auto turn_of = [&](int chunk, floatx4 (&xv)[MT][4], floatx4 (&x_next)[MT][4], int stage) {
-    load_x(x_next, chunk + 1);
-    issue(chunk + 1, stage ^ 1);
-    gf_wait_loads<4 * MT + 4>();  // all but the loads just sent
+  auto multiply = [&](const floatx4 (&xv)[MT][4], int stage) __attribute__((always_inline)) {
     const GF_LDS(unsigned char)* base = (const GF_LDS(unsigned char)*)(stage_base + stage * GF_TILE_BYTES);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -132,15 +138,23 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
         for (int t = 0; t < MT; ++t)
           acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i], xv[t][s][i], acc[t], 0, 0, 0);
     }
-    // this wave's reads of the stage are over before the next turn's loads overwrite it
+    // this wave's reads of the stage are over before a later turn's loads overwrite it
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };
   floatx4 x_even[MT][4], x_odd[MT][4];
-  load_x(x_even, c_begin);
-  issue(c_begin, 0);
+  auto turn = [&](int chunk, const floatx4 (&xv)[MT][4], floatx4 (&x_next)[MT][4], int stage) __attribute__((always_inline)) {
+    if (chunk + 1 < c_end) {
+      bring(x_next, chunk + 1, stage ^ 1);
+      gf_wait_loads<4 * MT + 4>();  // all but the loads just sent
+    } else {
+      gf_wait_loads<0>();
+    }
+    multiply(xv, stage);
+  };
+  bring(x_even, c_begin, 0);
   for (int chunk = c_begin; chunk < c_end; chunk += 2) {
-    turn_of(chunk, x_even, x_odd, 0);
-    if (chunk + 1 < c_end) turn_of(chunk + 1, x_odd, x_even, 1);
+    turn(chunk, x_even, x_odd, 0);
+    if (chunk + 1 < c_end) turn(chunk + 1, x_odd, x_even, 1);
   }
 #pragma unroll
   for (int t = 0; t < MT; ++t)
@@ -148,7 +162,7 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
   gf_barrier();
 
   // Wave t now adds row tile t: element (row 16 t + r, column row0 + 4 g + i).
-  const bool wide = (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+  const bool wide = ((ldo | row0) & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
   if (range < MT) {
     const int t = range;
     floatx4 half[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -160,31 +174,34 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
     const int m = 16 * t + r, n = row0 + 4 * g;
     if (m >= M) return;
     float* p = out + static_cast<size_t>(m) * ldo + n;
-    if (wide && n + 3 < N) {
+    const int left = row0 + rows - n;  // columns from here on
+    if (wide && left >= 4) {
       *reinterpret_cast<floatx4*>(p) = v;
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (n + i < N) p[i] = v[i];
+        if (i < left) p[i] = v[i];
     }
   }
 }
 
+// What the first loads need are the first 14 words of the arguments, which come with the launch.
 template <int MT>
 __global__ __launch_bounds__(GF_RANGES* PYLON_WAVE) void gemm_f32_rows_kernel(
-    float* __restrict__ out, const float* x, const float* __restrict__ w, int M, int N, int K,
-    long long ldx, long long ldw, long long ldo) {
-  gemm_f32_rows_body<MT>(out, x, w, M, N, K, ldx, ldw, ldo);
+    const float* x, const float* __restrict__ w, int M, int N, int K, int cols, int ldx, int ldw,
+    float* __restrict__ out, long long ldo) {
+  gemm_f32_rows_body<MT>(out, x, w, M, N, K, ldx, ldw, ldo, cols);
 }
 
-// T: tiles of 16 rows and of 16 columns per wave; a workgroup's tile is 32 T by 32 T.  TEAMS: 1, or
+// TM, TN: tiles of 16 rows and of 16 columns per wave; WM, WN: waves of a team along them, four together.  TEAMS: 1, or
 // 2 teams of four waves that take half of K each.
-template <int T, int TEAMS>
+template <int TM, int TN, int WM, int WN, int TEAMS>
 __device__ __forceinline__ void gemm_f32_tiles_body(float* __restrict__ out, const float* __restrict__ x,
                                                     const float* __restrict__ w, int M, int N, int K, long long ldx,
                                                     long long ldw, long long ldo, int m_tiles, int n_tiles) {
-  constexpr int SIDE = 32 * T;
-  constexpr int STAGE_BYTES = 4 * T * GF_TILE_BYTES;  // 2 T tiles of x, then 2 T of w
+  static_assert(WM * WN == 4, "a team is four waves");
+  constexpr int X_TILES = TM * WM, W_TILES = TN * WN;
+  constexpr int STAGE_BYTES = (X_TILES + W_TILES) * GF_TILE_BYTES;  // the tiles of x, then those of w
   __shared__ __attribute__((aligned(1024))) unsigned char lds[TEAMS * 2 * STAGE_BYTES];
 
   // Workgroups that share columns of w run on one die (every eighth workgroup), one after the other,
@@ -192,14 +209,14 @@ __device__ __forceinline__ void gemm_f32_tiles_body(float* __restrict__ out, con
   const int die = blockIdx.x & 7, nth = blockIdx.x >> 3;
   const int mt = nth % m_tiles, nt = (nth / m_tiles) * 8 + die;
   if (nt >= n_tiles) return;
-  const int m0 = mt * SIDE, n0 = nt * SIDE;
-  const int m_rows = (M - m0 < SIDE) ? M - m0 : SIDE, n_rows = (N - n0 < SIDE) ? N - n0 : SIDE;
+  const int m0 = mt * 16 * X_TILES, n0 = nt * 16 * W_TILES;
+  const int m_rows = (M - m0 < 16 * X_TILES) ? M - m0 : 16 * X_TILES, n_rows = (N - n0 < 16 * W_TILES) ? N - n0 : 16 * W_TILES;
 
   const int lane = threadIdx.x & (PYLON_WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PYLON_WAVE) & 3;
   const int team = __builtin_amdgcn_readfirstlane(threadIdx.x / PYLON_WAVE) >> 2;
   const int r = lane & 15, g = lane >> 4;
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % WM, wn = wave / WM;
   const int chunks = (K + GF_CHUNK - 1) / GF_CHUNK;
   const int middle = gf_range_begin(GF_RANGES / 2, chunks);
   const int c_begin = (TEAMS == 2 && team == 1) ? middle : 0, c_end = (TEAMS == 2 && team == 0) ? middle : chunks;
@@ -218,35 +235,33 @@ __device__ __forceinline__ void gemm_f32_tiles_body(float* __restrict__ out, con
   const int R = 4 * wave + lrow;
   const int lk = (lpos ^ R) * 4;
   unsigned char* team_lds = lds + team * 2 * STAGE_BYTES;
+  const unsigned x_step = static_cast<unsigned>(ldx) * 64u, w_step = static_cast<unsigned>(ldw) * 64u;  // a tile's rows
+  const unsigned x_first = static_cast<unsigned>(R) * static_cast<unsigned>(ldx) * 4u + lk * 4u;
+  const unsigned w_first = static_cast<unsigned>(R) * static_cast<unsigned>(ldw) * 4u + lk * 4u;
   auto issue = [&](int chunk, int stage) {
-    const int k = chunk * GF_CHUNK + lk;
+    // a chunk's first byte; the range check of a view does not count the scalar offset, which rows beyond it need not
+    const int at = chunk * (GF_CHUNK * 4);
     unsigned char* base = team_lds + stage * STAGE_BYTES + wave * 1024;
-    const bool live = chunk < c_end && k < K;
+    const bool live = chunk < c_end && chunk * GF_CHUNK + lk < K;
 #pragma unroll
-    for (int t = 0; t < 2 * T; ++t) {
-      const int row = 16 * t + R;
-      const unsigned at = static_cast<unsigned>(row) * static_cast<unsigned>(ldx) * 4u + static_cast<unsigned>(k) * 4u;
+    for (int t = 0; t < X_TILES; ++t)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (GF_LDS(void)*)(base + t * GF_TILE_BYTES), 16,
-                                               live && row < m_rows ? at : GF_OOB, 0, 0, 0);
-    }
+                                               live && 16 * t + R < m_rows ? x_first + t * x_step : GF_OOB, at, 0, 0);
 #pragma unroll
-    for (int t = 0; t < 2 * T; ++t) {
-      const int row = 16 * t + R;
-      const unsigned at = static_cast<unsigned>(row) * static_cast<unsigned>(ldw) * 4u + static_cast<unsigned>(k) * 4u;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (GF_LDS(void)*)(base + (2 * T + t) * GF_TILE_BYTES), 16,
-                                               live && row < n_rows ? at : GF_OOB, 0, 0, 0);
-    }
+    for (int t = 0; t < W_TILES; ++t)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (GF_LDS(void)*)(base + (X_TILES + t) * GF_TILE_BYTES), 16,
+                                               live && 16 * t + R < n_rows ? w_first + t * w_step : GF_OOB, at, 0, 0);
   };
   unsigned piece_at[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) piece_at[s] = (r >> 2) * 1024 + (r & 3) * 256 + (((4 * s + g) ^ r) * 16);
 
   // of the range under way, of the half under way, of the first half (one team): [column tile][row tile]
-  floatx4 acc[T][T], half[T][T], first[T][T];
+  floatx4 acc[TN][TM], half[TN][TM], first[TN][TM];
 #pragma unroll
-  for (int j = 0; j < T; ++j)
+  for (int j = 0; j < TN; ++j)
 #pragma unroll
-    for (int t = 0; t < T; ++t) acc[j][t] = half[j][t] = first[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < TM; ++t) acc[j][t] = half[j][t] = first[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   issue(c_begin, 0);
   int range = team * (GF_RANGES / 2);
@@ -256,39 +271,40 @@ __device__ __forceinline__ void gemm_f32_tiles_body(float* __restrict__ out, con
     gf_barrier();
     if (turn + 1 < turns) issue(c + 1, stage ^ 1);
     if (c >= c_end) continue;
-    const GF_LDS(unsigned char)* xb = (const GF_LDS(unsigned char)*)(team_lds + stage * STAGE_BYTES + wm * T * GF_TILE_BYTES);
+    const GF_LDS(unsigned char)* xb =
+        (const GF_LDS(unsigned char)*)(team_lds + stage * STAGE_BYTES + wm * TM * GF_TILE_BYTES);
     const GF_LDS(unsigned char)* wb =
-        (const GF_LDS(unsigned char)*)(team_lds + stage * STAGE_BYTES + (2 * T + wn * T) * GF_TILE_BYTES);
+        (const GF_LDS(unsigned char)*)(team_lds + stage * STAGE_BYTES + (X_TILES + wn * TN) * GF_TILE_BYTES);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      floatx4 xf[T], wf[T];
+      floatx4 xf[TM], wf[TN];
 #pragma unroll
-      for (int t = 0; t < T; ++t) xf[t] = *reinterpret_cast<const GF_LDS(floatx4)*>(xb + t * GF_TILE_BYTES + piece_at[s]);
+      for (int t = 0; t < TM; ++t) xf[t] = *reinterpret_cast<const GF_LDS(floatx4)*>(xb + t * GF_TILE_BYTES + piece_at[s]);
 #pragma unroll
-      for (int j = 0; j < T; ++j) wf[j] = *reinterpret_cast<const GF_LDS(floatx4)*>(wb + j * GF_TILE_BYTES + piece_at[s]);
+      for (int j = 0; j < TN; ++j) wf[j] = *reinterpret_cast<const GF_LDS(floatx4)*>(wb + j * GF_TILE_BYTES + piece_at[s]);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < T; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-          for (int t = 0; t < T; ++t)
+          for (int t = 0; t < TM; ++t)
             acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j][i], xf[t][i], acc[j][t], 0, 0, 0);
     }
     if (gf_range_begin(range + 1, chunks) == c + 1) {  // the range ends with this chunk
       ++range;
 #pragma unroll
-      for (int j = 0; j < T; ++j)
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
+        for (int t = 0; t < TM; ++t) {
           half[j][t] += acc[j][t];
           acc[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
     }
     if (TEAMS == 1 && c + 1 == middle) {
 #pragma unroll
-      for (int j = 0; j < T; ++j)
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
+        for (int t = 0; t < TM; ++t) {
           first[j][t] = half[j][t];
           half[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
@@ -296,33 +312,34 @@ __device__ __forceinline__ void gemm_f32_tiles_body(float* __restrict__ out, con
   }
   if constexpr (TEAMS == 2) {
     // the second team's half goes to the first through LDS, which nobody reads any more
+    static_assert(4 * TM * TN * PYLON_WAVE * 16 <= TEAMS * 2 * STAGE_BYTES, "room for a team's sums");
     gf_barrier();
-    floatx4* meet = reinterpret_cast<floatx4*>(lds) + wave * T * T * PYLON_WAVE + lane;
+    floatx4* meet = reinterpret_cast<floatx4*>(lds) + wave * TM * TN * PYLON_WAVE + lane;
     if (team == 1) {
 #pragma unroll
-      for (int j = 0; j < T; ++j)
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int t = 0; t < T; ++t) meet[(j * T + t) * PYLON_WAVE] = half[j][t];
+        for (int t = 0; t < TM; ++t) meet[(j * TM + t) * PYLON_WAVE] = half[j][t];
     }
     gf_barrier();
     if (team == 1) return;
 #pragma unroll
-    for (int j = 0; j < T; ++j)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int t = 0; t < T; ++t) {
+      for (int t = 0; t < TM; ++t) {
         first[j][t] = half[j][t];
-        half[j][t] = meet[(j * T + t) * PYLON_WAVE];
+        half[j][t] = meet[(j * TM + t) * PYLON_WAVE];
       }
   }
 
   const bool wide = (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
 #pragma unroll
-  for (int t = 0; t < T; ++t) {
-    const int m = m0 + (wm * T + t) * 16 + r;
+  for (int t = 0; t < TM; ++t) {
+    const int m = m0 + (wm * TM + t) * 16 + r;
     if (m >= M) continue;
 #pragma unroll
-    for (int j = 0; j < T; ++j) {
-      const int n = n0 + (wn * T + j) * 16 + 4 * g;
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + (wn * TN + j) * 16 + 4 * g;
       const floatx4 v = first[j][t] + half[j][t];
       float* p = out + static_cast<size_t>(m) * ldo + n;
       if (wide && n + 3 < N) {
@@ -336,41 +353,85 @@ __device__ __forceinline__ void gemm_f32_tiles_body(float* __restrict__ out, con
   }
 }
 
-template <int T, int TEAMS>
+template <int TM, int TN, int WM, int WN, int TEAMS>
 __global__ __launch_bounds__(TEAMS * 256) void gemm_f32_tiles_kernel(float* __restrict__ out, const float* __restrict__ x,
                                                                      const float* __restrict__ w, int M, int N, int K,
                                                                      long long ldx, long long ldw, long long ldo,
                                                                      int m_tiles, int n_tiles) {
-  gemm_f32_tiles_body<T, TEAMS>(out, x, w, M, N, K, ldx, ldw, ldo, m_tiles, n_tiles);
+  gemm_f32_tiles_body<TM, TN, WM, WN, TEAMS>(out, x, w, M, N, K, ldx, ldw, ldo, m_tiles, n_tiles);
 }
 
-template <int T, int TEAMS>
+template <int TM, int TN, int WM, int WN, int TEAMS>
 static void launch_tiles(float* out, const float* x, const float* w, int M, int N, int K, long long ldx, long long ldw,
                          long long ldo, hipStream_t stream) {
-  const int side = 32 * T, m_tiles = (M + side - 1) / side, n_tiles = (N + side - 1) / side;
+  const int m_side = 16 * TM * WM, n_side = 16 * TN * WN;
+  const int m_tiles = (M + m_side - 1) / m_side, n_tiles = (N + n_side - 1) / n_side;
   const dim3 grid(static_cast<unsigned>((n_tiles + 7) / 8 * 8) * m_tiles), block(TEAMS * 256);
-  hipLaunchKernelGGL((gemm_f32_tiles_kernel<T, TEAMS>), grid, block, 0, stream, out, x, w, M, N, K, ldx, ldw, ldo, m_tiles, n_tiles);
+  hipLaunchKernelGGL((gemm_f32_tiles_kernel<TM, TN, WM, WN, TEAMS>), grid, block, 0, stream, out, x, w, M, N, K, ldx, ldw,
+                     ldo, m_tiles, n_tiles);
 }
 
-// Tiles of 64 x 64 for many rows that fill the chip three times over, else of 32 x 32 (us, 64 against
-// 32: 2048 rows 2560 x 9728 993, 1014 and 19456 x 2560 1861, 2057; 600 rows 19456 x 2560 591, 628; but
-// 400 rows 451, 440, 270 rows 2560 x 9728 245, 177 and 64 rows 230, 73; tiles of 128 x 128: 1487, 2024,
-// 606, 596, 743 and 727).  A launch holds less than 2^32 threads: 0 where neither does.
-static int gf_side(int M, int N, int units) {
-  auto fits = [&](int side, int threads) {
-    const long long groups = static_cast<long long>((M + side - 1) / side) * (((N + side - 1) / side + 7) / 8 * 8);
-    return groups * threads < (1ll << 32);
+// Columns a workgroup of the streaming kernel takes: 16, or an equal share where as many whole rounds of the units as
+// 16 would need then each have less to stream: in launches of several rounds, and in one if K is deep (us of 3 and of
+// 24 rows, 16 against the share: 2560 x 9728 in 10 25.1, 22.3 and 40.1, 39.2; 5120 x 8192 in 10 50.8, 42.5 and 71.7, 64.4;
+// 6144 x 2560 in 12 14.6, 13.9 and 25.2, 23.9; 6144 x 4096 in 12 21.6, 20.3; but 2560 x 4096 11.0 either way and 3072 x
+// 2560 in 12 8.6, 8.8).
+static int gf_row_cols(int N, int K, int units) {
+  const long long rounds = ((N + 15) / 16 + units - 1) / units;
+  if (rounds == 1 && (K < 8192 || N < 8 * units)) return 16;
+  const int even = static_cast<int>((N + rounds * units - 1) / (rounds * units));
+  return even < 8 ? 8 : even > 16 ? 16 : even;
+}
+
+// The tiles of a launch of more than 32 rows.  A workgroup's time for a chunk of K where one, two or three of its kind
+// share a compute unit (us, measured over 33 to 900 rows of 2560 x 4096, 2560 x 9728, 6144 x 2560 and 19456 x 2560): from
+// these and the number of rounds a launch is estimated, within 8 % of what it takes; the least is chosen.  Small tiles
+// reach every unit in a launch of few rows, large ones read less from the second-level cache and from LDS for each
+// product.  Two sizes alone, 32 x 32 and (from 512 rows on) 64 x 64, took, 4B layer sizes at 270 rows, 69 + 156 + 96 + 287
+// us where these take 61 + 135 + 93 + 266, at 600 135 + 296 + 189 + 557 and 118 + 274 + 181 + 546, at 900 212 + 479 + 282 +
+// 831 and 173 + 397 + 266 + 786.
+enum { GF_32_TEAMS, GF_32_WIDE, GF_48, GF_48_TEAMS, GF_64_TEAMS, GF_96, GF_64, GF_TILINGS };
+struct GfTiling {
+  int m, n, threads, resident;
+  float chunk[3];  // with as many on a unit
+};
+static const GfTiling gf_tilings[GF_TILINGS] = {
+    {32, 32, 512, 2, {0.46f, 0.64f, 0.f}}, {32, 64, 256, 3, {0.84f, 1.29f, 1.80f}}, {48, 64, 256, 2, {1.09f, 1.65f, 0.f}},
+    {48, 64, 512, 1, {0.88f, 0.f, 0.f}},   {64, 64, 512, 1, {1.12f, 0.f, 0.f}},    {96, 64, 256, 2, {1.91f, 3.19f, 0.f}},
+    {64, 64, 256, 2, {1.39f, 2.25f, 0.f}}};
+
+static int gf_tiling(int M, int N, int units) {
+  auto groups = [&](const GfTiling& t) {
+    return static_cast<long long>((M + t.m - 1) / t.m) * (((N + t.n - 1) / t.n + 7) / 8 * 8);
   };
+  // a launch holds less than 2^32 threads
+  auto fits = [&](int tiling) { return groups(gf_tilings[tiling]) * gf_tilings[tiling].threads < (1ll << 32); };
+  int best = GF_TILINGS;
+  if (M <= (1 << 15) && N <= (1 << 20)) {  // (larger ones have not been measured)
+    float least = 0.f;
+    for (int i = 0; i < GF_TILINGS; ++i) {
+      const GfTiling& t = gf_tilings[i];
+      if (!fits(i)) continue;
+      const long long round = static_cast<long long>(t.resident) * units;
+      const long long count = static_cast<long long>((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
+      const long long rest = count % round;
+      float us = static_cast<float>(count / round) * t.chunk[t.resident - 1];
+      if (rest > 0) us += t.chunk[(rest + units - 1) / units - 1];
+      if (best == GF_TILINGS || us < least) best = i, least = us;
+    }
+    if (best != GF_TILINGS) return best;
+  }
   const bool many = M >= 512 && static_cast<long long>((M + 63) / 64) * ((N + 63) / 64) >= 3ll * units;
-  if (!many && fits(32, 512)) return 32;
-  return fits(64, 256) ? 64 : 0;
+  if (!many && fits(GF_32_TEAMS)) return GF_32_TEAMS;
+  return fits(GF_64) ? GF_64 : GF_TILINGS;
 }
 
-// The side of the tiles in which a product of these sizes is computed in float32 (units: compute units), 16 for the
-// streaming kernel; 0 where gemm_tiled takes it.  Touches no device.
+// What computes a product of these sizes in float32 (units: compute units): 16 the streaming kernel, 32 tiles of fewer
+// than 64 rows, 64 larger ones; 0 where gemm_tiled takes it.  Touches no device.
 extern "C" int pylon_gemm_f32_plan(int M, int N, int units, int* side) {
   PYLON_REQUIRE(M >= 1 && N >= 1 && units >= 1 && side != nullptr, "gemm_f32_plan: bad arguments");
-  *side = M <= GF_ROWS ? 16 : gf_side(M, N, units);
+  const int tiling = gf_tiling(M, N, units);
+  *side = M <= GF_ROWS ? 16 : tiling == GF_TILINGS ? 0 : gf_tilings[tiling].m < 64 ? 32 : 64;
   return 0;
 }
 
@@ -391,17 +452,25 @@ bool gemm_f32_launch(float* out, const float* x, const float* w, int M, int N, i
   const int units = pylon_compute_units();
   if (units <= 0) return false;
   if (M <= GF_ROWS) {
-    const dim3 grid((N + 15) / 16), block(GF_RANGES * PYLON_WAVE);
+    const int cols = gf_row_cols(N, K, units);
+    const dim3 grid((N + cols - 1) / cols), block(GF_RANGES * PYLON_WAVE);
     if (M <= 16)
-      hipLaunchKernelGGL((gemm_f32_rows_kernel<1>), grid, block, 0, stream, out, x, w, M, N, K, ldx, ldw, ldo);
+      hipLaunchKernelGGL((gemm_f32_rows_kernel<1>), grid, block, 0, stream, x, w, M, N, K, cols, (int)ldx, (int)ldw, out, ldo);
     else
-      hipLaunchKernelGGL((gemm_f32_rows_kernel<2>), grid, block, 0, stream, out, x, w, M, N, K, ldx, ldw, ldo);
+      hipLaunchKernelGGL((gemm_f32_rows_kernel<2>), grid, block, 0, stream, x, w, M, N, K, cols, (int)ldx, (int)ldw, out, ldo);
     return true;
   }
-  const int side = gf_side(M, N, units);
-  if (side == 64)
-    launch_tiles<2, 1>(out, x, w, M, N, K, ldx, ldw, ldo, stream);
-  else if (side == 32)
-    launch_tiles<1, 2>(out, x, w, M, N, K, ldx, ldw, ldo, stream);
-  return side != 0;
+#define GO(TM, TN, WM, WN, TEAMS) launch_tiles<TM, TN, WM, WN, TEAMS>(out, x, w, M, N, K, ldx, ldw, ldo, stream)
+  switch (gf_tiling(M, N, units)) {
+    case GF_32_TEAMS: GO(1, 1, 2, 2, 2); break;
+    case GF_32_WIDE: GO(2, 1, 1, 4, 1); break;
+    case GF_48: GO(3, 1, 1, 4, 1); break;
+    case GF_48_TEAMS: GO(3, 1, 1, 4, 2); break;
+    case GF_64: GO(2, 2, 2, 2, 1); break;
+    case GF_64_TEAMS: GO(2, 2, 2, 2, 2); break;
+    case GF_96: GO(3, 2, 2, 2, 1); break;
+    default: return false;
+  }
+#undef GO
+  return true;
 }

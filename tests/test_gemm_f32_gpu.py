@@ -54,6 +54,19 @@ def test_tiles_of_64_agree_with_the_streaming_kernel(ops):
         assert torch.equal(ops.gemm_tiled(x[first:last].contiguous(), w), got[first:last])
 
 
+# sizes at which each of the tiles is chosen, one row and one column past whole tiles among them: 32 x 32, 32 x 64, 48 x
+# 64, 48 x 64 by two teams, 64 x 64, 64 x 64 by two teams, 96 x 64; and the streaming kernel's narrower shares
+@pytest.mark.parametrize("rows, n, k", [(97, 2560, 576), (100, 19455, 520), (181, 19457, 516), (270, 2561, 640),
+                                        (32770, 70, 520), (360, 2497, 1100), (287, 19455, 576), (5, 5121, 520),
+                                        (17, 2561, 8192)])
+def test_every_tile_against_float64(ops, rows, n, k):
+    x, w = draw(rows, rows, k), draw(n + k, n, k)
+    got = ops.gemm_tiled(x, w)
+    assert within_bound(got, x, w)
+    for first, last in ((0, 1), (rows // 2, rows // 2 + 9), (rows - 1, rows)):  # the streaming kernel's bits
+        assert torch.equal(ops.gemm_tiled(x[first:last].contiguous(), w), got[first:last])
+
+
 def test_strided_rows_and_rows_that_are_not_aligned(ops):
     x, w = draw(3, 40, 600), draw(4, 50, 604)
     for cut in (600, 599):  # 16-byte pieces, and a K that has none (the general kernel)
