@@ -26,6 +26,7 @@ from ..config.specs import ModelSpec
 from ..kernels import ops, plan
 from ..parts import build_part
 from ..parts.base import KVRequirement, Part, requirement_list
+from . import layer_run
 from .batch import StepContext
 
 
@@ -59,6 +60,7 @@ class Model(Part):
             block = build_part("block", layer, dtype=dtype, device=device)
             self.blocks.append(block)
             self.add_child(f"layers.{index}", block)
+        self.alike = dtype == torch.bfloat16 and layer_run.alike(spec)  # layers that one call may launch
         self.pass_entry = None
         if spec.pass_entry is not None:
             self.pass_entry = self.add_child("pass_entry", build_part("pass", spec.pass_entry, dtype=dtype, device=device))
@@ -122,7 +124,10 @@ class Model(Part):
         # a schedule may add the embedded tokens to the stream again before some of its runs
         embedded = resid.clone() if any(self.embedding_again) or self.begins_pass else None
         delta = None
-        for run, ((layer, cache_id, stores), again) in enumerate(zip(self.schedule, self.embedding_again)):
+        launched = layer_run.run_layers(self, ctx, resid) if self.alike else None
+        if launched is not None:
+            resid, delta = launched
+        for run, ((layer, cache_id, stores), again) in enumerate(zip(self.schedule, self.embedding_again)) if launched is None else ():
             if again:
                 ops.residual_add(resid, embedded)  # the pending output of the run before follows in the norm
             if run in self.begins_pass:

@@ -1,0 +1,123 @@
+"""The layers of a step of few prompt tokens, launched by one call: the bits of the parts' own launches, which steps it
+takes, and that what it does not take is left to the parts."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def config(**more):
+    return {"architectures": ["Qwen3ForCausalLM"], "model_type": "qwen3", "hidden_act": "silu", "num_hidden_layers": 3,
+            "hidden_size": 1024, "num_attention_heads": 32, "num_key_value_heads": 8, "head_dim": 128,
+            "intermediate_size": 4096, "vocab_size": 1500, "rope_theta": 1e6, "rms_norm_eps": 1e-6,
+            "tie_word_embeddings": True, "max_position_embeddings": 4096, **more}
+
+
+def runner_of(cfg, **options):
+    from pylon_amd.config import PylonConfig
+    from pylon_amd.engine import Runner
+
+    options = {"dtype": "bfloat16", "max_batch_size": 4, "page_size": 64, "num_pages": 40, "cuda_graphs": False, **options}
+    return Runner.from_random(cfg, 7, PylonConfig(**options), std=0.02, norm_jitter=0.1)
+
+
+@pytest.fixture(scope="module")
+def runner():
+    return runner_of(config())
+
+
+@pytest.fixture
+def taken(monkeypatch):
+    """For every step, whether one call launched its layers."""
+    from pylon_amd.engine import layer_run
+
+    seen, real = [], layer_run.run_layers
+
+    def watch(*args):
+        got = real(*args)
+        seen.append(got is not None)
+        return got
+
+    monkeypatch.setattr(layer_run, "run_layers", watch)
+    return seen
+
+
+def serve(runner, portions):
+    """Logits of steps whose entries are (request, tokens), every token's wanted, then of one token for each request."""
+    from pylon_amd.engine import StepEntry
+
+    ids = torch.arange(4096).mul(7919).remainder(1499).tolist()
+    seqs, out = {}, []
+    for portion in [*portions, [(r, 1) for r in sorted({r for p in portions for r, _ in p})]]:
+        entries = []
+        for r, count in portion:
+            seq = seqs.setdefault(r, None) or runner.open(r)
+            seqs[r] = seq
+            entries.append(StepEntry(seq, [ids[(seq.length + i) * 3 + r] for i in range(count)], list(range(count))))
+        out.append(runner.step(entries).clone())
+    for seq in seqs.values():
+        runner.close(seq)
+    return out
+
+
+# up to 16 rows, 17 to 48 and beyond 64 (the tiled kernel: bfloat16 results between the layers; up to 128 float sums),
+# several requests, a second portion behind cached tokens, and the most tokens that one call takes
+@pytest.mark.parametrize("portions, one_call", [
+    ([[(0, 2)]], [True]), ([[(0, 16)]], [True]), ([[(0, 17)]], [True]), ([[(0, 48)]], [True]), ([[(0, 20), (1, 21)]], [True]),
+    ([[(0, 65)]], [True]), ([[(0, 128)]], [True]), ([[(0, 129)], [(0, 40)]], [True, True]), ([[(0, 300), (1, 212)]], [True]),
+    ([[(0, 49)]], [False]), ([[(0, 513)]], [False]), ([[(0, 1)]], [False]), ([[(0, 30)], [(0, 1), (1, 20)]], [True, False])])
+def test_the_bits_of_the_parts_launches(runner, taken, portions, one_call):
+    got = serve(runner, portions)
+    assert taken == one_call + [False]  # and the decode step behind
+    runner.model.alike, kept = False, runner.model.alike
+    try:
+        want = serve(runner, portions)
+    finally:
+        runner.model.alike = kept
+    assert kept and len(got) == len(want)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_what_is_followed_or_of_another_kind_is_left_to_the_parts(runner, taken):
+    from pylon_amd.parts.norm import RMSNorm
+
+    weight = runner.model.blocks[1].mixer.params["out"]
+    weight.requires_grad_(True)
+    try:
+        serve(runner, [[(0, 20)]])
+    finally:
+        weight.requires_grad_(False)
+
+    class Other(RMSNorm):
+        pass
+
+    norm = runner.model.blocks[2].feed_forward_norm
+    norm.__class__ = Other
+    try:
+        serve(runner, [[(0, 20)]])
+    finally:
+        norm.__class__ = RMSNorm
+    apart = torch.empty((1024, 4096 + 64), dtype=torch.bfloat16, device="cuda:0")[:, :4096]
+    old = runner.model.blocks[1].feed_forward.params["down"]
+    apart.copy_(old)
+    runner.model.blocks[1].feed_forward.params["down"] = apart
+    try:
+        serve(runner, [[(0, 20)]])
+    finally:
+        runner.model.blocks[1].feed_forward.params["down"] = old
+    assert not any(taken)
+
+
+def test_models_of_unlike_layers_and_of_32_bits_are_not_asked():
+    assert not runner_of(config(), dtype="float32").model.alike
+    assert runner_of(config(num_hidden_layers=1)).model.alike
+
+
+def test_the_fields_that_both_sides_count():
+    import ctypes
+
+    from pylon_amd.kernels import library
+
+    fields = (ctypes.c_int * 3)()
+    library.call("pylon_layer_run_fields", ctypes.addressof(fields))
+    assert tuple(fields) == (18, 30, 4)
