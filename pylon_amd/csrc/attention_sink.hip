@@ -8,8 +8,9 @@
 // values lie transposed inside every page, [page, kv head, vdim, slot in page], so that the
 // eight keys a lane feeds to a matrix instruction are neighbours in memory.
 //
-// A workgroup owns up to 32 consecutive tokens of one request and the (up to four) query heads of
-// one key/value head; each of its eight wavefronts one head and 16 of the tokens (one tile of query columns).  It walks the keys in blocks of 32 (which never cross a page: pages are
+// A workgroup owns up to 32 consecutive tokens of one request and the (up to four) query heads of one key/value head;
+// each of its eight wavefronts one head and 16 of the tokens (one tile of query columns).  It walks the keys in blocks of
+// 32 (which never cross a page: pages are
 // multiples of 32).  Scores are computed transposed, S^T = K Q^T (16x16x32 instructions: rows are
 // keys, columns are queries), so that everything that belongs to a query (its running maximum,
 // its sum, its output) lives in the lanes of that query's column, and the exponentials are
@@ -31,8 +32,11 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 #define AS_BLOCK 32   // keys per step of the walk
-#define AS_QT 1       // query tiles of 16 per wave
 #define AS_MAX_BIAS 4096
+// Waves a SIMD of the prompt kernel: two workgroups a compute unit where the outputs and queries leave the registers.
+#define AS_WAVES(KS, NV) ((KS) <= 6 && (NV) <= 8 ? 4 : 2)
+#define AS_LOG2E 1.4426950408889634f
+#define AS_LN2 0.6931471805599453f
 
 __device__ __forceinline__ uint32_t as_pack(float a, float b) {
   return floats_to_bf16_pair(a, b);
@@ -48,19 +52,46 @@ __device__ __forceinline__ float capped_score(float s, float scale, float cap) {
   return cap * (1.0f - 2.0f / (e + 1.0f));
 }
 
-template <int KS, int NV>
-__global__ __launch_bounds__(512) void attention_sink_kernel(
+// v times log2 e; a finite number stays finite (a bias may be the type's lowest).
+__device__ __forceinline__ float as_to_log2(float v) {
+  const float r = v * AS_LOG2E;
+  return __builtin_isinf(r) && !__builtin_isinf(v) ? copysignf(3.402823466e38f, v) : r;
+}
+
+// The largest over the four lanes of a query's column, on the vector unit (two trips through LDS with shuffles).
+__device__ __forceinline__ float as_column_max(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
+}
+
+// FULL: keys of exactly 32 KS elements and values of exactly 16 NV, the strides in LDS constants.
+//
+// What bounds it is the issue of a block's vector and matrix instructions (1.1 us a block of 32 keys and compute unit with
+// four waves a SIMD, twice what the matrix instructions alone take), and for the tile with the longest walk that walk's own
+// length (1.2 us a block with nothing beside it).  The registers are kept at 128 so that two workgroups share a compute
+// unit: with 145 the second one waited for the first to end.  The questions that are the same for a whole wave (does it
+// work, is there a cap, are the keys near, far, hidden) are asked once a block: asked inside the loops over the operands
+// they had put a branch and a wait for all loads before every matrix instruction.  The loads of the queries are waited
+// for before the walk.  Keys are written to LDS in the order that makes a lane's eight weights those of eight neighbours:
+// one 16-byte piece of values.  32 heads of 128 over 8, 2,048 tokens, bias over 2,049 distances: 152 -> 88 us; behind
+// 952 cached ones 279 -> 138; behind 452 in a window of 1,024 without a bias 144 -> 71; 40 tokens 10.5 -> 9.2.
+template <int KS, int NV, bool FULL>
+__global__ __launch_bounds__(512, AS_WAVES(KS, NV)) void attention_sink_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, long long q_stride, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int* __restrict__ block_table, int table_width,
-    const int* __restrict__ tiles, const int* __restrict__ positions, int n_heads, int n_kv_heads, int dim, int vdim, int page_size, float scale,
+    const int* __restrict__ tiles, const int* __restrict__ positions, int n_heads, int n_kv_heads, int dim_arg, int vdim_arg, int page_size, float scale,
     const float* __restrict__ bias, int bucket_len, int sink, int cuts, float* __restrict__ partial, int window,
     float softcap, const float* __restrict__ sink_logit) {
-  // eight waves: wave & 3 names the head of the group, wave >> 2 which 16 of the tile's 32 tokens, so
-  // that every SIMD holds two waves that fill each other's waits
+  // eight waves: wave & 3 names the head of the group, wave >> 2 which 16 of the tile's 32 tokens
+  const int dim = FULL ? 32 * KS : dim_arg, vdim = FULL ? 16 * NV : vdim_arg;
   constexpr int waves_per_group = 4;
   constexpr int KL = (KS + 3) / 4, VL = (NV + 7) / 8;  // 16-byte pieces of a block a thread fetches
+  constexpr bool KEYS_FIT = FULL && KS % 4 == 0, VALUES_FIT = FULL && NV % 8 == 0;  // every thread has its pieces
   extern __shared__ float bias_lds[];  // [heads of the workgroup][bucket_len], then the block's keys and values
-  const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3, qsel = threadIdx.x >> 8;
+  const int lane = threadIdx.x & 63;
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wave_id & 3, qsel = wave_id >> 2;
   const int col = lane & 15, grp = lane >> 4;
   const int group = n_heads / n_kv_heads;
   const int chunks = (group + waves_per_group - 1) / waves_per_group;
@@ -78,12 +109,12 @@ __global__ __launch_bounds__(512) void attention_sink_kernel(
   const int tok0 = tiles ? tiles[4 * tile] : tile, count = tiles ? tiles[4 * tile + 1] : 1;
   const int row = tiles ? tiles[4 * tile + 2] : tile, pos0 = tiles ? tiles[4 * tile + 3] : positions[tile];
   const int kv_last = pos0 + count - 1;
-  const int n_qt = (qsel == 0 || count > 16) ? 1 : 0;  // a tile of up to 16 tokens leaves the second half's waves idle
+  const bool works = !idle && (qsel == 0 || count > 16);  // other waves only help to fetch
   const int* table = block_table + static_cast<size_t>(row) * table_width;
 
   const int tstride = (bucket_len + 3) & ~3;  // keeps what follows the tables 16-byte aligned
   float* tbl = bias_lds + wave * tstride;
-  const int kstr = dim + 8, vstr = AS_BLOCK + 4;  // LDS rows, padded
+  const int kstr = dim + 8, vstr = AS_BLOCK + 8;  // LDS rows, padded against bank conflicts
   // two buffers of a block's keys and values, used in turns
   bf16_t* kv_lds = reinterpret_cast<bf16_t*>(bias_lds + waves_per_group * tstride);
   const int buf_elems = AS_BLOCK * kstr + ((vdim + 15) & ~15) * vstr;
@@ -91,40 +122,35 @@ __global__ __launch_bounds__(512) void attention_sink_kernel(
   const float* bias_row = bias ? bias + static_cast<size_t>(head) * bucket_len : nullptr;
   if (bias != nullptr) {
 #pragma unroll 8
-    for (int d = lane; d < bucket_len; d += 64) tbl[d] = bias_row[d];
+    for (int d = lane; d < bucket_len; d += 64) tbl[d] = as_to_log2(bias_row[d]);
   }
-  const float far_bias = bias != nullptr ? bias_row[bucket_len - 1] : 0.f;
+  // Scores, biases and maxima are kept times log2 e: a weight is one subtraction and one exponential to base 2.
+  const float far_bias = bias != nullptr ? as_to_log2(bias_row[bucket_len - 1]) : 0.f;
+  const float scale2 = (softcap > 0.f ? 1.f : scale) * AS_LOG2E;  // a capped score has its scale
 
   // Q^T operands: column = query, eight key elements per lane and step
-  bf16x8 qf[AS_QT][KS];
-  int qpos[AS_QT], qfirst[AS_QT];  // a query's position and the first key it sees (a window, a chunk)
-#pragma unroll
-  for (int qt = 0; qt < AS_QT; ++qt) {
-    const int qi = (qt + qsel) * 16 + col;
-    qpos[qt] = pos0 + qi;
-    qfirst[qt] = first_visible(qpos[qt], window);
+  bf16x8 qf[KS];
+  const int qi = qsel * 16 + col;
+  const int qpos = pos0 + qi, qfirst = first_visible(qpos, window);  // the query's position and the first key it sees
+  {
     const int t = tok0 + (qi < count ? qi : count - 1);
     const bf16_t* qr = q + static_cast<size_t>(t) * q_stride + static_cast<size_t>(head) * dim;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int d = ks * 32 + grp * 8;
       u32x4 raw = {0u, 0u, 0u, 0u};
-      if (d < dim) raw = *reinterpret_cast<const u32x4*>(qr + d);
-      qf[qt][ks] = __builtin_bit_cast(bf16x8, raw);
+      if (FULL || d < dim) raw = *reinterpret_cast<const u32x4*>(qr + d);
+      qf[ks] = __builtin_bit_cast(bf16x8, raw);
     }
   }
 
-  floatx4 o[AS_QT][NV];
-  float m_run[AS_QT], l_run[AS_QT];
+  floatx4 o[NV];
+  // the sink: a key without a value (one lane of a query's four carries its one) whose score is 0,
+  // or the head's learned number
+  float m_run = (sink && cut == 0) ? (sink_logit != nullptr ? as_to_log2(sink_logit[head]) : 0.f) : -INFINITY;
+  float l_run = (sink && cut == 0 && grp == 0) ? 1.f : 0.f;
 #pragma unroll
-  for (int qt = 0; qt < AS_QT; ++qt) {
-    // the sink: a key without a value (one lane of a query's four carries its one) whose score is 0,
-    // or the head's learned number
-    m_run[qt] = (sink && cut == 0) ? (sink_logit != nullptr ? sink_logit[head] : 0.f) : -INFINITY;
-    l_run[qt] = (sink && cut == 0 && grp == 0) ? 1.f : 0.f;
-#pragma unroll
-    for (int dt = 0; dt < NV; ++dt) o[qt][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int dt = 0; dt < NV; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   // the walk starts at the block of the first key that the tile's first query sees
   const int kb_first = first_visible(pos0, window) / AS_BLOCK * AS_BLOCK;
@@ -132,149 +158,134 @@ __global__ __launch_bounds__(512) void attention_sink_kernel(
   const int per_cut = (n_blocks + cuts - 1) / cuts;
   const int kb_begin = kb_first + cut * per_cut * AS_BLOCK;
   const int kb_end = kb_first + ((cut + 1) * per_cut < n_blocks ? (cut + 1) * per_cut : n_blocks) * AS_BLOCK;
+  const int wave_first = pos0 + qsel * 16, last_first = first_visible(wave_first + 15, window);
   // A block's keys and values travel global -> registers -> LDS; the registers of block b + 1
   // are filled while block b is computed.
   u32x4 kreg[KL], vreg[VL];
   const int kchunks = dim >> 3;  // 16-byte pieces of a key row
-  auto fetch = [&](int kb) {
-    const int page = table[kb / page_size];
-    const int in_page = kb % page_size;
+  // where this thread's pieces lie, in the caches behind a block's first key and in LDS
+  int k_from[KL], k_to[KL], v_to[VL];
+  long long v_from[VL];
+#pragma unroll
+  for (int n = 0; n < KL; ++n) {
+    const int c = threadIdx.x + n * threads, r = c / kchunks, e = (c - r * kchunks) * 8;
+    k_from[n] = r * n_kv_heads * dim + e, k_to[n] = ((r & 4) * 4 + (r >> 3) * 4 + (r & 3)) * kstr + e;
+  }
+#pragma unroll
+  for (int n = 0; n < VL; ++n) {
+    const int c = threadIdx.x + n * threads, r = c / (AS_BLOCK / 8), e = (c - r * (AS_BLOCK / 8)) * 8;
+    v_from[n] = static_cast<long long>(r) * page_size + e, v_to[n] = AS_BLOCK * kstr + r * vstr + e;
+  }
+  int page_at = kb_begin / page_size, in_page = kb_begin - page_at * page_size;  // of the block that is fetched next
+  int kb_next = kb_begin, page = kb_begin < kb_end ? table[page_at] : 0;
+  auto fetch = [&]() {
     const bf16_t* kbase = k_cache + ((static_cast<size_t>(page) * page_size + in_page) * n_kv_heads + kvh) * dim;
 #pragma unroll
     for (int n = 0; n < KL; ++n) {
       const int c = threadIdx.x + n * threads;
-      if (c < AS_BLOCK * kchunks) {
-        const int r = c / kchunks, e = (c - r * kchunks) * 8;
-        kreg[n] = *reinterpret_cast<const u32x4*>(kbase + static_cast<size_t>(r) * n_kv_heads * dim + e);
-      }
+      if (KEYS_FIT || c < AS_BLOCK * kchunks) kreg[n] = *reinterpret_cast<const u32x4*>(kbase + k_from[n]);
     }
     const bf16_t* vbase = v_cache + (static_cast<size_t>(page) * n_kv_heads + kvh) * vdim * page_size + in_page;
 #pragma unroll
     for (int n = 0; n < VL; ++n) {
       const int c = threadIdx.x + n * threads;
-      if (c < vdim * (AS_BLOCK / 8)) {
-        const int r = c / (AS_BLOCK / 8), e = (c - r * (AS_BLOCK / 8)) * 8;
-        vreg[n] = *reinterpret_cast<const u32x4*>(vbase + static_cast<size_t>(r) * page_size + e);
+      if (VALUES_FIT || c < vdim * (AS_BLOCK / 8)) vreg[n] = *reinterpret_cast<const u32x4*>(vbase + v_from[n]);
+    }
+    in_page += AS_BLOCK, kb_next += AS_BLOCK;
+    if (in_page == page_size && kb_next < kb_end) in_page = 0, page = table[++page_at];
+  };
+  auto stage = [&](int turn, int kb) {
+    bf16_t* const block = kv_lds + turn * buf_elems;
+    if (kb + AS_BLOCK - 1 > kv_last) {  // slots past the request's end hold anything; their weights are 0, and so are they
+#pragma unroll
+      for (int n = 0; n < VL; ++n) {
+        const int first = kb + (threadIdx.x + n * threads) % (AS_BLOCK / 8) * 8;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (first + e > kv_last) vreg[n][e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
       }
     }
-  };
-  auto stage = [&](int turn) {
-    bf16_t* k_lds = kv_lds + turn * buf_elems;
-    bf16_t* v_lds = k_lds + AS_BLOCK * kstr;
 #pragma unroll
     for (int n = 0; n < KL; ++n) {
       const int c = threadIdx.x + n * threads;
-      if (c < AS_BLOCK * kchunks) {
-        const int r = c / kchunks, e = (c - r * kchunks) * 8;
-        *reinterpret_cast<u32x4*>(k_lds + r * kstr + e) = kreg[n];
-      }
+      if (KEYS_FIT || c < AS_BLOCK * kchunks) *reinterpret_cast<u32x4*>(block + k_to[n]) = kreg[n];
     }
 #pragma unroll
     for (int n = 0; n < VL; ++n) {
       const int c = threadIdx.x + n * threads;
-      if (c < vdim * (AS_BLOCK / 8)) {
-        const int r = c / (AS_BLOCK / 8), e = (c - r * (AS_BLOCK / 8)) * 8;
-        *reinterpret_cast<u32x2*>(v_lds + r * vstr + e) = u32x2{vreg[n][0], vreg[n][1]};
-        *reinterpret_cast<u32x2*>(v_lds + r * vstr + e + 4) = u32x2{vreg[n][2], vreg[n][3]};
-      }
+      if (VALUES_FIT || c < vdim * (AS_BLOCK / 8)) *reinterpret_cast<u32x4*>(block + v_to[n]) = vreg[n];
     }
   };
   // Block b is computed from one buffer while block b + 1, fetched during block b - 1's math, is
   // written to the other and block b + 2 is sent for: one barrier a block.
+  if (kb_begin < kb_end) fetch();
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // of all loads: a wait for the queries inside the walk would be one for the next block
   if (kb_begin < kb_end) {
-    fetch(kb_begin);
-    stage(0);
-    if (kb_begin + AS_BLOCK < kb_end) fetch(kb_begin + AS_BLOCK);
+    stage(0, kb_begin);
+    if (kb_begin + AS_BLOCK < kb_end) fetch();
   }
   __syncthreads();
   int turn = 0;
   for (int kb = kb_begin; kb < kb_end; kb += AS_BLOCK, turn ^= 1) {
     const bf16_t* k_lds = kv_lds + turn * buf_elems;
     const bf16_t* v_lds = k_lds + AS_BLOCK * kstr;
-    // K operands: row = key, eight elements per lane and step
-    floatx4 s[AS_QT][2];
+    if (works) {
+      // K operands: row 16 t + 4 g + i of the block in LDS = key 8 g + 4 t + i, eight elements per lane and step: a lane's
+      // eight scores are of eight keys side by side, whose values it then reads as one piece
+      floatx4 s[2];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const bf16_t* kr = k_lds + (t * 16 + col) * kstr;
+      for (int t = 0; t < 2; ++t) {
+        const bf16_t* kr = k_lds + (t * 16 + col) * kstr;
+        s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int qt = 0; qt < AS_QT; ++qt) s[qt][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int d = ks * 32 + grp * 8;
-        u32x4 raw = {0u, 0u, 0u, 0u};
-        if (d < dim) raw = *reinterpret_cast<const u32x4*>(kr + d);
-        const bf16x8 kf = __builtin_bit_cast(bf16x8, raw);
-#pragma unroll
-        for (int qt = 0; qt < AS_QT; ++qt)
-          if (qt < n_qt) s[qt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[qt][ks], s[qt][t], 0, 0, 0);
-      }
-    }
-    // V^T operands: row = value element, keys kb + 4 grp + {0..3} and kb + 16 + 4 grp + {0..3}
-    bf16x8 vf[NV];
-    const bool ragged = kb + AS_BLOCK - 1 > kv_last;  // slots past the request's end hold anything
-#pragma unroll
-    for (int dt = 0; dt < NV; ++dt) {
-      const int d = dt * 16 + col;
-      u32x4 raw = {0u, 0u, 0u, 0u};
-      if (d < vdim) {
-        const bf16_t* vr = v_lds + d * vstr + 4 * grp;
-        const u32x2 first = *reinterpret_cast<const u32x2*>(vr);
-        const u32x2 second = *reinterpret_cast<const u32x2*>(vr + 16);
-        raw = u32x4{first[0], first[1], second[0], second[1]};
-        if (ragged) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int key = kb + (e >> 2) * 16 + 4 * grp + (e & 3);
-            if (key > kv_last) raw[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
-          }
+        for (int ks = 0; ks < KS; ++ks) {
+          const int d = ks * 32 + grp * 8;
+          u32x4 raw = {0u, 0u, 0u, 0u};
+          if (FULL || d < dim) raw = *reinterpret_cast<const u32x4*>(kr + d);
+          s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, raw), qf[ks], s[t], 0, 0, 0);
         }
       }
-      vf[dt] = __builtin_bit_cast(bf16x8, raw);
-    }
-
-#pragma unroll
-    for (int qt = 0; qt < AS_QT; ++qt) {
-      if (qt >= n_qt) continue;
-      // scores of this lane: keys kb + 16 t + 4 grp + i for query qpos[qt]
+      // Scores of this lane: keys kb + 8 grp + e for query qpos.  Three ways, one question a block for the whole
+      // wave: every query sees every key and all are far (or there is no bias), or all near, or anything.
       float sc[8];
-      const int near = qpos[qt] - (kb + AS_BLOCK - 1);  // the smallest distance of the block for this query
-      const bool all_far = bias == nullptr || near >= bucket_len - 1;
-      // (one question a block, of the whole wave, whose far queries find far_bias in the table's last entry.  A question a
-      // key was the compiler's to lay in or out of the walk: 2,048 tokens of 32 heads of 128 with a bias 218 us in and
-      // 228 out of it, without one 216 and 211; so 210 and 196.)
-      float by_distance[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) by_distance[e] = far_bias;
-      if (__builtin_amdgcn_ballot_w64(!all_far) != 0) {
+      for (int e = 0; e < 8; ++e) sc[e] = s[e >> 2][e & 3];
+      if (softcap > 0.f) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sc[e] = capped_score(sc[e], scale, softcap);
+      }
+      const bool seen = kb + AS_BLOCK - 1 <= wave_first && kb >= last_first;
+      if (seen && (bias == nullptr || wave_first - (kb + AS_BLOCK - 1) >= bucket_len - 1)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sc[e] = fmaf(sc[e], scale2, far_bias);
+      } else if (seen && wave_first + 15 - kb < bucket_len) {
+        const float* const near = tbl + (qpos - kb - 8 * grp - 7);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sc[e] = fmaf(sc[e], scale2, near[7 - e]);
+      } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const int dist = qpos[qt] - (kb + (e >> 2) * 16 + 4 * grp + (e & 3));
-          const int idx = dist < 0 ? 0 : dist;
-          by_distance[e] = tbl[idx < bucket_len - 1 ? idx : bucket_len - 1];
+          const int key = kb + 8 * grp + e, dist = qpos - key;
+          const int idx = dist < 0 ? 0 : dist < bucket_len - 1 ? dist : bucket_len - 1;
+          const float v = fmaf(sc[e], scale2, bias == nullptr ? 0.f : tbl[idx]);
+          sc[e] = (dist >= 0 && key >= qfirst) ? v : -INFINITY;
         }
       }
-      float top = m_run[qt];
+      float top = m_run;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int key = kb + (e >> 2) * 16 + 4 * grp + (e & 3);
-        const int dist = qpos[qt] - key;
-        const float v = capped_score(s[qt][e >> 2][e & 3], scale, softcap) + by_distance[e];
-        sc[e] = (dist >= 0 && key >= qfirst[qt]) ? v : -INFINITY;
-        top = fmaxf(top, sc[e]);
-      }
-      top = fmaxf(top, __shfl_xor(top, 16, 64));
-      top = fmaxf(top, __shfl_xor(top, 32, 64));
+      for (int e = 0; e < 8; ++e) top = fmaxf(top, sc[e]);
+      top = as_column_max(top);
       // a query past the tile's end, or one whose every key so far is hidden, keeps -inf: no NaN from inf - inf
-      const float m_new = top;
-      const float corr = (m_new == -INFINITY) ? 1.f : __expf(m_run[qt] - m_new);
+      const float base = (top == -INFINITY) ? 0.f : top;
+      const float corr = (top == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run - top);
       float p[8], sum = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        p[e] = (sc[e] == -INFINITY) ? 0.f : __expf(sc[e] - m_new);
+        p[e] = __builtin_amdgcn_exp2f(sc[e] - base);
         sum += p[e];
       }
-      l_run[qt] = l_run[qt] * corr + sum;
-      m_run[qt] = m_new;
+      l_run = l_run * corr + sum;
+      m_run = top;
       u32x4 hi, lo;
 #pragma unroll
       for (int e = 0; e < 8; e += 2) {
@@ -285,58 +296,58 @@ __global__ __launch_bounds__(512) void attention_sink_kernel(
         lo[e >> 1] = __builtin_amdgcn_perm(__float_as_uint(rc), __float_as_uint(ra), 0x07060302u);
       }
       const bf16x8 p_hi = __builtin_bit_cast(bf16x8, hi), p_lo = __builtin_bit_cast(bf16x8, lo);
-      const bool rescale = __any(corr != 1.f);  // no query of the wave raised its maximum: nothing to scale
+      if (__any(corr != 1.f)) {  // else no query of the wave raised its maximum: nothing to scale
+#pragma unroll
+        for (int dt = 0; dt < NV; ++dt) o[dt][0] *= corr, o[dt][1] *= corr, o[dt][2] *= corr, o[dt][3] *= corr;
+      }
+      // V^T operands: row = value element, keys kb + 8 grp + {0..7}
 #pragma unroll
       for (int dt = 0; dt < NV; ++dt) {
-        floatx4 acc = o[qt][dt];
-        if (rescale) {
-          acc[0] *= corr; acc[1] *= corr; acc[2] *= corr; acc[3] *= corr;
-        }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], p_hi, acc, 0, 0, 0);
-        o[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], p_lo, acc, 0, 0, 0);
+        const int d = dt * 16 + col;
+        u32x4 raw = {0u, 0u, 0u, 0u};
+        if (FULL || d < vdim) raw = *reinterpret_cast<const u32x4*>(v_lds + d * vstr + 8 * grp);
+        const bf16x8 vf = __builtin_bit_cast(bf16x8, raw);
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p_hi, o[dt], 0, 0, 0);
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p_lo, o[dt], 0, 0, 0);
       }
     }
     if (kb + AS_BLOCK < kb_end) {
-      stage(turn ^ 1);  // nobody reads that buffer: the block before this one is done everywhere
-      if (kb + 2 * AS_BLOCK < kb_end) fetch(kb + 2 * AS_BLOCK);
+      stage(turn ^ 1, kb + AS_BLOCK);  // nobody reads that buffer: the block before this one is done everywhere
+      if (kb + 2 * AS_BLOCK < kb_end) fetch();
     }
     __syncthreads();
   }
 
-#pragma unroll
-  for (int qt = 0; qt < AS_QT; ++qt) {
-    float l = l_run[qt];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    const int qi = (qt + qsel) * 16 + col;
-    if (qi >= count || idle) continue;
-    if (cuts > 1) {
-      // [token, head, cut, 2 + vdim]: maximum, sum, unnormalised output
-      float* dst = partial + ((static_cast<size_t>(tok0 + qi) * n_heads + head) * cuts + cut) * (2 + vdim);
-      if (grp == 0) {
-        dst[0] = m_run[qt];
-        dst[1] = l;
-      }
-#pragma unroll
-      for (int dt = 0; dt < NV; ++dt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (dt * 16 + 4 * grp + i < vdim) dst[2 + dt * 16 + 4 * grp + i] = o[qt][dt][i];
-      continue;
+  float l = l_run;
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (qi >= count || idle) return;
+  if (cuts > 1) {
+    // [token, head, cut, 2 + vdim]: maximum, sum, unnormalised output
+    float* dst = partial + ((static_cast<size_t>(tok0 + qi) * n_heads + head) * cuts + cut) * (2 + vdim);
+    if (grp == 0) {
+      dst[0] = m_run * AS_LN2;
+      dst[1] = l;
     }
-    const float inv = 1.0f / l;
-    bf16_t* orow = out + (static_cast<size_t>(tok0 + qi) * n_heads + head) * vdim;
 #pragma unroll
-    for (int dt = 0; dt < NV; ++dt) {
-      const int d = dt * 16 + 4 * grp;
-      if (d + 3 < vdim) {
-        u32x2 packed = {as_pack(o[qt][dt][0] * inv, o[qt][dt][1] * inv), as_pack(o[qt][dt][2] * inv, o[qt][dt][3] * inv)};
-        *reinterpret_cast<u32x2*>(orow + d) = packed;
-      } else {
+    for (int dt = 0; dt < NV; ++dt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (d + i < vdim) orow[d + i].bits = float_to_bf16_bits(o[qt][dt][i] * inv);
-      }
+      for (int i = 0; i < 4; ++i)
+        if (dt * 16 + 4 * grp + i < vdim) dst[2 + dt * 16 + 4 * grp + i] = o[dt][i];
+    return;
+  }
+  const float inv = 1.0f / l;
+  bf16_t* orow = out + (static_cast<size_t>(tok0 + qi) * n_heads + head) * vdim;
+#pragma unroll
+  for (int dt = 0; dt < NV; ++dt) {
+    const int d = dt * 16 + 4 * grp;
+    if (d + 3 < vdim) {
+      u32x2 packed = {as_pack(o[dt][0] * inv, o[dt][1] * inv), as_pack(o[dt][2] * inv, o[dt][3] * inv)};
+      *reinterpret_cast<u32x2*>(orow + d) = packed;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (d + i < vdim) orow[d + i].bits = float_to_bf16_bits(o[dt][i] * inv);
     }
   }
 }
@@ -679,27 +690,31 @@ extern "C" int pylon_attention_sink(void* out, const void* q, long long q_stride
   const int table_len = bias != nullptr ? bucket_len : 1;
   const size_t lds = sizeof(float) * waves * ((table_len + 3) & ~3) +
                      2 * 2 * (static_cast<size_t>(AS_BLOCK) * (dim + 8) +
-                              static_cast<size_t>((vdim + 15) / 16 * 16) * (AS_BLOCK + 4));  // two buffers of bfloat16
+                              static_cast<size_t>((vdim + 15) / 16 * 16) * (AS_BLOCK + 8));  // two buffers of bfloat16
   PYLON_REQUIRE(lds <= 160 * 1024, "attention_sink: the bias table and a block do not fit LDS");
   const int ks = (dim + 31) / 32, nv = (vdim + 15) / 16;
-#define GO(KS, NV) \
+#define GO(KS, NV, FULL) \
   do { \
   if (lds > 48 * 1024) \
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_sink_kernel<KS, NV>), \
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_sink_kernel<KS, NV, FULL>), \
                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); \
-  hipLaunchKernelGGL((attention_sink_kernel<KS, NV>), grid, block, lds, stream, (bf16_t*)out, (const bf16_t*)q, \
+  hipLaunchKernelGGL((attention_sink_kernel<KS, NV, FULL>), grid, block, lds, stream, (bf16_t*)out, (const bf16_t*)q, \
                      q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, table_width, tiles, \
                      positions, n_heads, n_kv_heads, dim, vdim, page_size, scale, bias, table_len, sink, cuts, partial, window, \
                      softcap, sink_logit); \
   } while (0)
-#define PICK_NV(KS)                 \
-  do {                              \
-    if (nv <= 2) GO(KS, 2);         \
-    else if (nv <= 4) GO(KS, 4);    \
-    else if (nv <= 8) GO(KS, 8);    \
-    else GO(KS, 16);                \
+#define PICK_NV(KS)                        \
+  do {                                     \
+    if (nv <= 2) GO(KS, 2, false);         \
+    else if (nv <= 4) GO(KS, 4, false);    \
+    else if (nv <= 8) GO(KS, 8, false);    \
+    else GO(KS, 16, false);                \
   } while (0)
-  if (ks <= 1) PICK_NV(1);
+  // the sizes of the usual heads with their strides as constants (128 and 128, 2,048 tokens: 115 -> 106 registers)
+  if (dim == 64 && vdim == 64) GO(2, 4, true);
+  else if (dim == 128 && vdim == 128) GO(4, 8, true);
+  else if (dim == 192 && vdim == 128) GO(6, 8, true);
+  else if (ks <= 1) PICK_NV(1);
   else if (ks <= 2) PICK_NV(2);
   else if (ks <= 4) PICK_NV(4);
   else PICK_NV(8);

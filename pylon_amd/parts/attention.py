@@ -171,7 +171,8 @@ class Attention(Part):
         # the matrix-core kernels take values as large as keys, plain scores and no sink
         same_size = spec.value_dim == spec.head_dim and not self.special
         if on_cores:
-            tiles = None if ctx.decode_only else ctx.token_tiles(ops.SINK_TILE)
+            tiles = None if ctx.decode_only else ctx.token_tiles(ops.SINK_TILE, fold=ops.sink_fold(
+                spec.n_heads, spec.n_kv_heads, spec.head_dim, spec.value_dim, 0))
             cuts = ops.sink_cuts(tokens, spec.n_heads, spec.n_kv_heads, self._span(ctx)) if ctx.decode_only else 1
             context = ops.attention_sink(q, cache.k, v_cache, cache.block_table, tiles, ctx.positions,
                                          page_size=cache.page_size, scale=spec.scale, bias=None, sink=spec.sink,
@@ -348,10 +349,8 @@ class SinkAttention(Part):
         q = qkv.as_strided((tokens, spec.n_heads, spec.head_dim), (qkv.stride(0), spec.head_dim, 1))
         mask = dict(window=spec.window, chunk=spec.chunk)
         if self._matrix_cores(page_size) and qkv.stride(0) % 8 == 0:
-            # tiles heaviest first (turning every second run of the order round, as the plain prefill
-            # kernel's caller does, loses here: 227 -> 270 us a layer at 2,048 tokens with four waves a
-            # workgroup, 5.81 -> 5.92 ms for eight layers with eight; the heaviest tile should start first)
-            tiles = None if ctx.decode_only else ctx.token_tiles(ops.SINK_TILE)
+            tiles = None if ctx.decode_only else ctx.token_tiles(ops.SINK_TILE, fold=ops.sink_fold(
+                spec.n_heads, spec.n_kv_heads, spec.head_dim, spec.v_head_dim, self.bias_len))
             # a prompt portion's tiles keep their keys whole: cut in two or four, with the merge behind,
             # a 2,048-token prompt of eight layers took 6.18 and 6.58 ms against 5.82
             span = ctx.max_len if self.span is None else min(ctx.max_len, self.span)

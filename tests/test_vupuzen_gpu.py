@@ -529,3 +529,51 @@ def test_recurrent_state_of_every_layout(ops, form, dtype, dim, vdim):
     # float32 throughout: chains of at most `dim` terms, a few roundings each; the result rounded to its type once
     torch.testing.assert_close(state.double(), want_state, rtol=1e-5, atol=1e-5)
     torch.testing.assert_close(got.double(), want.flatten(1), rtol=1.01 * 2.0 ** -8 if dtype == torch.bfloat16 else 0, atol=float(dim * 2.0 ** -22 * max(1.0, want.abs().max())))
+
+
+# sizes with constant strides and without, a group that leaves waves idle; tables shorter than a block, than the keys, and
+# longer; blocks that are all near, all far, across a window's edge; a page a block; portions that end inside a tile
+@pytest.mark.parametrize("heads, groups, dim, vdim, page, buckets, window, softcap", [
+    (8, 2, 128, 128, 64, 700, None, None), (4, 1, 128, 128, 32, 40, 90, None), (2, 2, 192, 128, 96, 0, 33, None),
+    (6, 2, 64, 64, 32, 7, None, 20.0), (5, 1, 120, 72, 64, 200, None, None), (4, 4, 256, 36, 32, 0, None, 5.0)])
+@pytest.mark.parametrize("cuts, sink", [(1, True), (3, True), (1, False)])
+def test_prompt_portions_against_float64(ops, heads, groups, dim, vdim, page, buckets, window, softcap, cuts, sink):
+    portions = ((530, 200), (97, 97), (33, 1), (16, 16))  # length, tokens of it in the step
+    gen = torch.Generator(DEV).manual_seed(dim + page)
+    width = max(-(-n // page) for n, _ in portions)
+    k = torch.randn(4 * width, page, groups, dim, generator=gen, device=DEV).bfloat16()
+    v = torch.randn(4 * width, groups, vdim, page, generator=gen, device=DEV).bfloat16()
+    table = torch.randperm(4 * width, generator=gen, device=DEV).int().view(4, width)
+    count = sum(n for _, n in portions)
+    q = torch.randn(count, heads, dim, generator=gen, device=DEV).bfloat16()
+    bias = torch.randn(heads, buckets, generator=gen, device=DEV) if buckets else None
+    logit = torch.randn(heads, generator=gen, device=DEV) if sink and softcap else None
+    tiles, at = [], 0
+    for row, (n, new) in enumerate(portions):
+        tiles += [(at + a, min(32, new - a), row, n - new + a) for a in range(0, new, 32)]
+        at += new
+        if n % page:  # what lies behind a request's end is anything
+            k[table[row, n // page], n % page:] = float("nan")
+            v[table[row, n // page], :, :, n % page:] = float("nan")
+    got = ops.attention_sink(q, k, v, table, i32(np.array(tiles).reshape(-1)).view(-1, 4), None, page_size=page, scale=0.1,
+                             bias=bias, sink=sink, cuts=cuts, window=window, softcap=softcap, sink_logit=logit).double()
+    at = 0
+    for row, (n, new) in enumerate(portions):
+        keys = k[table[row].long()].reshape(-1, groups, dim)[:n].double()
+        values = v[table[row].long()].permute(0, 3, 1, 2).reshape(-1, groups, vdim)[:n].double()
+        far = torch.arange(n - new, n, device=DEV)[:, None] - torch.arange(n, device=DEV)[None]
+        hidden = (far < 0) | (far >= window) if window else far < 0
+        for h in range(heads):
+            g = h // (heads // groups)
+            s = q[at: at + new, h].double() @ keys[:, g].t().contiguous() * 0.1
+            s = softcap * torch.tanh(s / softcap) if softcap else s
+            s = s + bias[h].double()[far.clamp(0, buckets - 1)] if buckets else s
+            s = s.masked_fill(hidden, float("-inf"))
+            if sink:
+                s = torch.cat([s, torch.full((new, 1), float(logit[h]) if logit is not None else 0.0, device=DEV).double()], 1)
+            want = torch.softmax(s, 1)[:, :n] @ values[:, g].contiguous()
+            # a result rounded to bfloat16 (eight bits: 2^-8 of it at most), weights to 15 bits, scores below 64 in float32
+            # (the sum of 256 products, the cap's exponential and division: under 2^-13) that shift weights by as much
+            slack = 2.0 ** -8 * want.abs() + 2.0 ** -12 * values[:, g].abs().max()
+            assert (got[at: at + new, h] - want).abs().le(slack).all(), (row, h)
+        at += new
