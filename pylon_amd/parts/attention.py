@@ -173,7 +173,11 @@ class Attention(Part):
         if on_cores:
             tiles = None if ctx.decode_only else ctx.token_tiles(ops.SINK_TILE, fold=ops.sink_fold(
                 spec.n_heads, spec.n_kv_heads, spec.head_dim, spec.value_dim, 0))
-            cuts = ops.sink_cuts(tokens, spec.n_heads, spec.n_kv_heads, self._span(ctx)) if ctx.decode_only else 1
+            if tiles is None:
+                cuts = ops.sink_cuts(tokens, spec.n_heads, spec.n_kv_heads, self._span(ctx))
+            else:
+                cuts = ops.sink_portion_cuts(tiles.shape[0], spec.n_heads, spec.n_kv_heads, spec.head_dim, spec.value_dim,
+                                             0, self._span(ctx))
             context = ops.attention_sink(q, cache.k, v_cache, cache.block_table, tiles, ctx.positions,
                                          page_size=cache.page_size, scale=spec.scale, bias=None, sink=spec.sink,
                                          cuts=cuts, softcap=spec.softcap, sink_logit=self.params.get("sink"), **mask)
@@ -351,10 +355,12 @@ class SinkAttention(Part):
         if self._matrix_cores(page_size) and qkv.stride(0) % 8 == 0:
             tiles = None if ctx.decode_only else ctx.token_tiles(ops.SINK_TILE, fold=ops.sink_fold(
                 spec.n_heads, spec.n_kv_heads, spec.head_dim, spec.v_head_dim, self.bias_len))
-            # a prompt portion's tiles keep their keys whole: cut in two or four, with the merge behind,
-            # a 2,048-token prompt of eight layers took 6.18 and 6.58 ms against 5.82
             span = ctx.max_len if self.span is None else min(ctx.max_len, self.span)
-            cuts = ops.sink_cuts(tokens, spec.n_heads, spec.n_kv_heads, span) if ctx.decode_only else 1
+            if tiles is None:
+                cuts = ops.sink_cuts(tokens, spec.n_heads, spec.n_kv_heads, span)
+            else:
+                cuts = ops.sink_portion_cuts(tiles.shape[0], spec.n_heads, spec.n_kv_heads, spec.head_dim, spec.v_head_dim,
+                                             self.bias_len, span)
             context = ops.attention_sink(q, cache.k, v_cache, cache.block_table, tiles, ctx.positions,
                                          page_size=page_size, scale=spec.scale, bias=self.bias_by_distance(),
                                          sink=spec.sink, cuts=cuts, **mask)
