@@ -52,6 +52,11 @@ __device__ __forceinline__ float capped_score(float s, float scale, float cap) {
   return cap * (1.0f - 2.0f / (e + 1.0f));
 }
 
+template <bool V>
+struct as_flag {
+  static constexpr bool value = V;
+};
+
 // v times log2 e; a finite number stays finite (a bias may be the type's lowest).
 __device__ __forceinline__ float as_to_log2(float v) {
   const float r = v * AS_LOG2E;
@@ -366,19 +371,24 @@ __global__ __launch_bounds__(512, AS_WAVES(KS, NV)) void attention_sink_kernel(
 // filled for the next block as soon as this block is done with them.  The biases are gathered by distance
 // straight from the table: a workgroup needs a few hundred entries of it, and copying all of a group's
 // tables to LDS first (32 KB at 2,048 distances and four heads) took longer than the walk itself.
-// 32 heads of 128 over 8 and 2,048 distances, 4 requests of 1,524 keys in 4 cuts with the merge: 29.9 us
-// with the tables in LDS and a block fetched when its turn came, 18.1 so (14.1 in 16 cuts); 16 requests 47.0
-// and 30.3; 64 of 1,000 keys, uncut, 88.1 and 63.2; without a bias, 2 of 2,524 in 8 cuts 25.1 and 16.5.
-template <int KS, int NV>
-__global__ __launch_bounds__(256) void attention_sink_decode_kernel(
+// The last block is a step of its own and nothing in a step is asked per operand, so that a wait is one for what
+// it is about (the first matrix instruction had waited for every load, the values' too); a lane's eight keys are
+// neighbours, their values one piece of 16 bytes; two waves a SIMD are asked for, which keeps the sums out of the
+// accumulation registers (each block had moved them there and back).
+// 32 heads of 128 over 8 and 2,048 distances, with the merge: 4 requests of 1,524 keys in 16 cuts 12.8 -> 10.0 us,
+// 4 of 700 in 8 9.7 -> 7.7, 1 of 8,000 in 64 16.9 -> 13.6, 16 of 1,524 in 4 26.6 -> 20.2, 64 of 1,000, uncut, 48.5
+// -> 36.3, 4 of 40 6.4 -> 4.7; without a bias, 2 of 2,524 in a window of 1,024 and 8 cuts 11.7 -> 8.3.
+template <int KS, int NV, bool FULL>
+__global__ __launch_bounds__(256, 2) void attention_sink_decode_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, long long q_stride, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int* __restrict__ block_table, int table_width,
-    const int* __restrict__ positions, int n_heads, int n_kv_heads, int dim, int vdim, int page_size, float scale,
+    const int* __restrict__ positions, int n_heads, int n_kv_heads, int dim_arg, int vdim_arg, int page_size, float scale,
     const float* __restrict__ bias, int bucket_len, int sink, int cuts, float* __restrict__ partial, int window,
     float softcap, const float* __restrict__ sink_logit) {
   extern __shared__ float mrg[];  // [4 waves][group][2 + vdim]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
+  const int dim = FULL ? 32 * KS : dim_arg, vdim = FULL ? 16 * NV : vdim_arg;
   const int group = n_heads / n_kv_heads;
   int b = blockIdx.x;
   const int cut = b % cuts;
@@ -398,18 +408,20 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
   const int kb_end = kb_first + ((cut + 1) * per_cut < n_blocks ? (cut + 1) * per_cut : n_blocks) * AS_BLOCK;
 
   u32x4 kraw[2][KS];
-  u32x2 vraw[NV][2];
+  u32x4 vraw[NV];
   float add[8];
+  // row 4 g + i of tile t is key 8 g + 4 t + i of the block: a lane's eight scores are of eight neighbours
+  const int key_row = (col >> 2) * 8 + (col & 3);
   auto load_keys = [&](int kb, int page) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const size_t slot = static_cast<size_t>(page) * page_size + kb % page_size + t * 16 + col;
+      const size_t slot = static_cast<size_t>(page) * page_size + kb % page_size + key_row + 4 * t;
       const bf16_t* kr = k_cache + (slot * n_kv_heads + kvh) * dim;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         const int d = ks * 32 + grp * 8;
         kraw[t][ks] = u32x4{0u, 0u, 0u, 0u};
-        if (d < dim) kraw[t][ks] = *reinterpret_cast<const u32x4*>(kr + d);
+        if (FULL || d < dim) kraw[t][ks] = *reinterpret_cast<const u32x4*>(kr + d);
       }
     }
   };
@@ -421,54 +433,36 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      int idx = pos - (kb + (e >> 2) * 16 + 4 * grp + (e & 3));
+      int idx = pos - (kb + 8 * grp + e);
       idx = idx < 0 ? 0 : (idx < bucket_len - 1 ? idx : bucket_len - 1);
       add[e] = bias_row[idx];
     }
   };
   auto load_values = [&](int kb, int page) {
-    const bf16_t* block = v_cache + (static_cast<size_t>(page) * n_kv_heads + kvh) * vdim * page_size + kb % page_size + 4 * grp;
+    const bf16_t* block = v_cache + (static_cast<size_t>(page) * n_kv_heads + kvh) * vdim * page_size + kb % page_size + 8 * grp;
 #pragma unroll
     for (int dt = 0; dt < NV; ++dt) {
       const int d = dt * 16 + col;
-      vraw[dt][0] = vraw[dt][1] = u32x2{0u, 0u};
-      if (d < vdim) {
-        const bf16_t* vr = block + static_cast<size_t>(d) * page_size;
-        vraw[dt][0] = *reinterpret_cast<const u32x2*>(vr);
-        vraw[dt][1] = *reinterpret_cast<const u32x2*>(vr + 16);
-      }
+      vraw[dt] = u32x4{0u, 0u, 0u, 0u};
+      if (FULL || d < vdim) vraw[dt] = *reinterpret_cast<const u32x4*>(block + static_cast<size_t>(d) * page_size);
     }
   };
 
   int kb = kb_begin + wave * AS_BLOCK;
-  bf16x8 qf[KS];
-  {
-    const bf16_t* qr = q + static_cast<size_t>(tok) * q_stride + static_cast<size_t>(my_head) * dim;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int d = ks * 32 + grp * 8;
-      u32x4 raw = {0u, 0u, 0u, 0u};
-      if (d < dim) raw = *reinterpret_cast<const u32x4*>(qr + d);
-      qf[ks] = __builtin_bit_cast(bf16x8, raw);
-    }
-  }
-  if (kb < kb_end) {
-    const int page = table[kb / page_size];
-    load_keys(kb, page);
-    load_bias(kb);
-    load_values(kb, page);
-  }
   floatx4 o[NV];
 #pragma unroll
   for (int dt = 0; dt < NV; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const float scale2 = (softcap > 0.f ? 1.f : scale) * AS_LOG2E;  // scores and maxima are times log2 e; a capped score has its scale
   const bool first = sink && cut == 0 && wave == 0;  // the sink belongs to one partial result
-  float m_run = first ? (sink_logit != nullptr ? sink_logit[my_head] : 0.f) : -INFINITY;
+  float m_run = first ? (sink_logit != nullptr ? as_to_log2(sink_logit[my_head]) : 0.f) : -INFINITY;
   float l_run = (first && grp == 0) ? 1.f : 0.f;
+  bf16x8 qf[KS];
 
-  for (; kb < kb_end; kb += 4 * AS_BLOCK) {
-    const int next = kb + 4 * AS_BLOCK;
-    const bool more = next < kb_end;
-    const int next_page = more ? table[next / page_size] : 0;
+  // One block; with another behind it the registers are filled again as they come free (no branch in between, so that a
+  // wait for the keys is one for the keys).
+  auto step = [&](auto another) __attribute__((always_inline)) {
+    constexpr bool more = decltype(another)::value;
+    const int next = kb + 4 * AS_BLOCK, next_page = more ? table[next / page_size] : 0;
     floatx4 s[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -479,22 +473,28 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
     }
     if (more) load_keys(next, next_page);
     float sc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sc[e] = s[e >> 2][e & 3];
+    if (softcap > 0.f) {  // asked once: inside the loop it is a branch and a wait for all loads a score
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sc[e] = capped_score(sc[e], scale, softcap);
+    }
     float top = m_run;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const int key = kb + (e >> 2) * 16 + 4 * grp + (e & 3);
-      const float v = capped_score(s[e >> 2][e & 3], scale, softcap) + add[e];
+      const int key = kb + 8 * grp + e;
+      const float v = fmaf(sc[e], scale2, add[e] * AS_LOG2E);
       sc[e] = (key <= pos && key >= first_key) ? v : -INFINITY;
       top = fmaxf(top, sc[e]);
     }
     if (more) load_bias(next);
-    top = fmaxf(top, __shfl_xor(top, 16, 64));
-    top = fmaxf(top, __shfl_xor(top, 32, 64));
-    const float corr = (top == -INFINITY || m_run == -INFINITY) ? (m_run == -INFINITY ? 0.f : 1.f) : __expf(m_run - top);
+    top = as_column_max(top);
+    const float base = (top == -INFINITY) ? 0.f : top;  // no key so far: no NaN from inf - inf
+    const float corr = (top == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run - top);
     float p[8], sum = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      p[e] = (sc[e] == -INFINITY) ? 0.f : __expf(sc[e] - top);
+      p[e] = __builtin_amdgcn_exp2f(sc[e] - base);
       sum += p[e];
     }
     l_run = l_run * corr + sum;
@@ -508,24 +508,39 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
       lo[e >> 1] = __builtin_amdgcn_perm(__float_as_uint(rc), __float_as_uint(ra), 0x07060302u);
     }
     const bf16x8 p_hi = __builtin_bit_cast(bf16x8, hi), p_lo = __builtin_bit_cast(bf16x8, lo);
-    const bool ragged = kb + AS_BLOCK - 1 > pos;
+    if (!more && kb + AS_BLOCK - 1 > pos) {  // slots behind the token may hold anything; they lie in the last block
+#pragma unroll
+      for (int dt = 0; dt < NV; ++dt)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (kb + 8 * grp + e > pos) vraw[dt][e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
+    }
 #pragma unroll
     for (int dt = 0; dt < NV; ++dt) {
-      u32x4 raw = {vraw[dt][0][0], vraw[dt][0][1], vraw[dt][1][0], vraw[dt][1][1]};
-      if (ragged) {  // slots behind the token may hold anything
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int key = kb + (e >> 2) * 16 + 4 * grp + (e & 3);
-          if (key > pos) raw[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
-        }
-      }
-      const bf16x8 vf = __builtin_bit_cast(bf16x8, raw);
+      const bf16x8 vf = __builtin_bit_cast(bf16x8, vraw[dt]);
       floatx4 acc = o[dt];
       acc[0] *= corr; acc[1] *= corr; acc[2] *= corr; acc[3] *= corr;
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p_hi, acc, 0, 0, 0);
       o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p_lo, acc, 0, 0, 0);
     }
     if (more) load_values(next, next_page);
+    kb = next;
+  };
+  if (kb < kb_end) {  // all its loads in here: a path without them would end the loop's waits early
+    const bf16_t* qr = q + static_cast<size_t>(tok) * q_stride + static_cast<size_t>(my_head) * dim;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int d = ks * 32 + grp * 8;
+      u32x4 raw = {0u, 0u, 0u, 0u};
+      if (FULL || d < dim) raw = *reinterpret_cast<const u32x4*>(qr + d);
+      qf[ks] = __builtin_bit_cast(bf16x8, raw);
+    }
+    const int page = table[kb / page_size];
+    load_keys(kb, page);
+    load_bias(kb);
+    load_values(kb, page);
+    while (kb + 4 * AS_BLOCK < kb_end) step(as_flag<true>{});
+    step(as_flag<false>{});
   }
   float l = l_run;
   l += __shfl_xor(l, 16, 64);
@@ -554,7 +569,7 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float mw = src[w * stride];
-      const float f = (mw == -INFINITY) ? 0.f : __expf(mw - m);
+      const float f = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - m);
       total = fmaf(src[w * stride + 1], f, total);
       acc = fmaf(src[w * stride + 2 + d], f, acc);
     }
@@ -564,7 +579,7 @@ __global__ __launch_bounds__(256) void attention_sink_decode_kernel(
     } else {
       float* dst = partial + (item * cuts + cut) * (2 + vdim);
       if (d == 0) {
-        dst[0] = m;
+        dst[0] = m * AS_LN2;
         dst[1] = total;
       }
       dst[2 + d] = acc;
@@ -652,24 +667,26 @@ extern "C" int pylon_attention_sink(void* out, const void* q, long long q_stride
     PYLON_REQUIRE(wgs < (1ll << 31), "attention_sink: too many workgroups for one launch");
     const size_t lds_d = sizeof(float) * 4 * group * (2 + vdim);
     const int ks_d = (dim + 31) / 32, nv_d = (vdim + 15) / 16;
-#define GO_D(KS, NV)                                                                                                \
+#define GO_D(KS, NV, FULL)                                                                                                \
   do {                                                                                                              \
     if (lds_d > 48 * 1024)                                                                                          \
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_sink_decode_kernel<KS, NV>),                \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_sink_decode_kernel<KS, NV, FULL>),                \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_d));                \
-    hipLaunchKernelGGL((attention_sink_decode_kernel<KS, NV>), dim3(static_cast<unsigned>(wgs)), dim3(256), lds_d,    \
+    hipLaunchKernelGGL((attention_sink_decode_kernel<KS, NV, FULL>), dim3(static_cast<unsigned>(wgs)), dim3(256), lds_d,    \
                        stream, (bf16_t*)out, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache,           \
                        block_table, table_width, positions, n_heads, n_kv_heads, dim, vdim, page_size, scale, bias,  \
                        bias != nullptr ? bucket_len : 1, sink, cuts, partial, window, softcap, sink_logit);          \
   } while (0)
 #define PICK_D(KS)                  \
   do {                              \
-    if (nv_d <= 2) GO_D(KS, 2);     \
-    else if (nv_d <= 4) GO_D(KS, 4);\
-    else if (nv_d <= 8) GO_D(KS, 8);\
-    else GO_D(KS, 16);              \
+    if (nv_d <= 2) GO_D(KS, 2, false);     \
+    else if (nv_d <= 4) GO_D(KS, 4, false);\
+    else if (nv_d <= 8) GO_D(KS, 8, false);\
+    else GO_D(KS, 16, false);              \
   } while (0)
-    if (ks_d <= 1) PICK_D(1);
+    if (dim == 64 && vdim == 64) GO_D(2, 4, true);
+    else if (dim == 128 && vdim == 128) GO_D(4, 8, true);
+    else if (ks_d <= 1) PICK_D(1);
     else if (ks_d <= 2) PICK_D(2);
     else if (ks_d <= 4) PICK_D(4);
     else PICK_D(8);

@@ -586,3 +586,34 @@ def test_prompt_portions_against_float64(ops, heads, groups, dim, vdim, page, bu
     (1, 4, 1, 128, 0, 200000, 64), (32, 32, 8, 256, 0, 3000, 1), (16, 32, 8, 128, 4096, 3000, 2), (16, 64, 8, 128, 0, 640, 2)])
 def test_cuts_of_a_prompt_portion(ops, tiles, heads, groups, dim, buckets, span, want):
     assert ops.sink_portion_cuts(tiles, heads, groups, dim, 128, buckets, span, units=256) == want
+
+
+# the sizes whose strides are constants and one beside each; waves of no block, one and several, whole and ragged
+@pytest.mark.parametrize("heads, groups, dim, vdim", [(8, 2, 64, 64), (8, 2, 64, 60), (8, 1, 128, 128), (32, 2, 120, 128)])
+@pytest.mark.parametrize("cuts, softcap, buckets", [(1, None, 600), (2, 6.0, 9), (1, 6.0, 0), (7, None, 0)])
+def test_single_tokens_against_float64(ops, heads, groups, dim, vdim, cuts, softcap, buckets):
+    page, lengths = 32, (1, 32, 33, 128, 129, 160, 700)
+    gen = torch.Generator(DEV).manual_seed(dim + cuts)
+    width = -(-max(lengths) // page)
+    k = torch.randn(width, page, groups, dim, generator=gen, device=DEV).bfloat16()
+    v = torch.randn(width, groups, vdim, page, generator=gen, device=DEV).bfloat16()
+    q = torch.randn(len(lengths), heads, dim, generator=gen, device=DEV).bfloat16()
+    order = torch.randperm(width, generator=gen, device=DEV).int()
+    table = order.expand(len(lengths), -1).contiguous()
+    bias = torch.randn(heads, buckets, generator=gen, device=DEV) if buckets else None
+    logit = torch.randn(heads, generator=gen, device=DEV) if softcap else None
+    got = ops.attention_sink(q, k, v, table, None, i32([n - 1 for n in lengths]), page_size=page, scale=0.1, bias=bias, sink=True,
+                             cuts=cuts, softcap=softcap, sink_logit=logit).double()
+    keys = k[order.long()].reshape(-1, groups, dim).double()
+    values = v[order.long()].permute(0, 3, 1, 2).reshape(-1, groups, vdim).double()
+    for r, n in enumerate(lengths):
+        for h in range(heads):
+            g = h // (heads // groups)
+            s = keys[:n, g] @ q[r, h].double() * 0.1
+            s = softcap * torch.tanh(s / softcap) if softcap else s
+            s = s + bias[h].double()[torch.arange(n - 1, -1, -1, device=DEV).clamp(0, buckets - 1)] if buckets else s
+            s = torch.cat([s, torch.full((1,), float(logit[h]) if softcap else 0.0, device=DEV).double()])
+            want = torch.softmax(s, 0)[:n] @ values[:n, g].contiguous()
+            # as for the prompt portions above
+            slack = 2.0 ** -8 * want.abs() + 2.0 ** -12 * values[:n, g].abs().max()
+            assert (got[r, h] - want).abs().le(slack).all(), (n, h)
