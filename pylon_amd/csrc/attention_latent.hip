@@ -571,6 +571,11 @@ extern "C" int pylon_latent_decode(void* out, const void* q, const void* cache, 
                               partial_floats >= static_cast<long long>(tokens) * n_heads * cuts * (2 + rank)),
                 "latent_decode: %d cuts need a scratch buffer", cuts);
   if (tokens == 0) return 0;
+  // Heads beyond sixteen share a workgroup's keys where the launch fills the chip; where it leaves units idle their
+  // workgroups run beside it, with half the products, sums and merges in each one's chain.  32 heads, keys of 320 over a
+  // latent of 256, 900 keys in four cuts, shared and apart: 1 token 16.4 and 10.7 us, 6 16.5 and 11.0, 32 (256 workgroups)
+  // 18.5 and 13.2, 48 (shared) 20.1; 1 of 1,000 in eight cuts 13.9 and 9.4; keys of 192 over 128, 6 of 700 11.3 and 8.8.
+  const bool two_tiles = n_heads > 16 && static_cast<long long>(tokens) * ((n_heads + 15) / 16) * cuts > pylon_compute_units();
   int index = latent_shape(width, rank);
 #define AL_GO(KS, NT, QT)                                                                                            \
   do {                                                                                                               \
@@ -588,7 +593,7 @@ extern "C" int pylon_latent_decode(void* out, const void* q, const void* cache, 
 #define AL_PICK(KS, NT)                                       \
   if (index-- == 0) {                                         \
     if constexpr (NT <= 16 && KS >= 3) {                      \
-      if (n_heads > 16) AL_GO(KS, NT, 2);                     \
+      if (two_tiles) AL_GO(KS, NT, 2);                        \
       else AL_GO(KS, NT, 1);                                  \
     } else {                                                  \
       AL_GO(KS, NT, 1);                                       \

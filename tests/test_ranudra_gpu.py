@@ -774,3 +774,22 @@ def test_a_configuration_drawn_at_random_matches_the_plain_model(tmp, seed, dtyp
         if dtype == "float32":
             assert np.abs(got - whole[rid]).max() <= 2e-5 * np.abs(whole[rid]).max(), (seed, rid)
     assert runner.manager.free_pages == pages
+
+
+# heads beyond sixteen share a workgroup only in launches that fill the chip: a token's result is the same beside few and many
+@pytest.mark.parametrize("heads, width, rank", [(17, 192, 128), (32, 320, 256), (48, 320, 250)])
+@pytest.mark.parametrize("cuts", [1, 3])
+def test_latent_heads_shared_or_apart(ops, heads, width, rank, cuts):
+    page, length = 64, 300
+    many = ops._lib.compute_units() // cuts + 1
+    gen = torch.Generator(DEV).manual_seed(heads)
+    pages = -(-length // page)
+    cache = torch.randn(pages, page, 1, width, generator=gen, device=DEV).bfloat16()
+    table = torch.randperm(pages, generator=gen, device=DEV).int().expand(many, -1).contiguous()
+    q = torch.randn(3, heads, width, generator=gen, device=DEV).bfloat16().repeat(many // 3 + 1, 1, 1)[:many].contiguous()
+    pos = i32([length - 1, 33, 0] * (many // 3 + 1))[:many].contiguous()
+    run = lambda n: ops.latent_decode(q[:n], cache, table[:n], pos[:n], rank=rank, page_size=page, scale=0.1, cuts=cuts)
+    few, all_ = run(3), run(many)
+    assert torch.isfinite(few.float()).all()
+    for start in range(0, many - 2, 3):
+        assert torch.equal(all_[start: start + 3], few)
