@@ -126,6 +126,74 @@ latent_rotate_kernel(T* __restrict__ q_out, T* __restrict__ cache, const T* __re
   for (int i = tid; i < half; i += LP_THREADS) rotate(c + rank, dst + rank, i);
 }
 
+// The same for few tokens, whose time is the chain of trips to memory, sines and barriers of one workgroup a token: with
+// `store` the first workgroup of a token norms and stores its latent and turns the shared key part, the others take 256
+// pairs of the heads each; a pair's angle is computed by the thread that turns it, and every load of a workgroup goes out
+// before the first is used.  Bfloat16, 32 heads, 64 turned elements, a latent of 256: 1 token 3.9 -> 2.6 us, 6 4.1 -> 2.8,
+// 512 4.7 -> 3.9, 1,024 (5,120 workgroups, more angles than the other saves) 5.7 and 5.7, 2,048 8.3 and 9.3; 128 heads over
+// a latent of 512, 6 tokens 7.4 -> 2.8.
+#define LR_PIECES 4  // elements of a latent a thread holds
+template <typename T>
+__global__ void __launch_bounds__(LP_THREADS)
+latent_rotate_few_kernel(T* __restrict__ q_out, T* __restrict__ cache, const T* __restrict__ proj, long long ld, int q_off,
+                         int heads, int dim, int rot, int c_off, int rank, const float* __restrict__ c_weight, float eps,
+                         const float* __restrict__ inv_freq, float rot_scale, int interleaved,
+                         const int* __restrict__ positions, const int* __restrict__ slot_map, int store) {
+  __shared__ float scratch[16];
+  const int t = blockIdx.x, tid = threadIdx.x, half = rot / 2, width = rank + rot;
+  const T* row = proj + static_cast<size_t>(t) * ld;
+  const bool latent = store && blockIdx.y == 0;
+  const int e = latent ? tid : (blockIdx.y - (store ? 1 : 0)) * LP_THREADS + tid;
+  const int h = latent ? 0 : e / (half > 0 ? half : 1), i = latent ? tid : e - h * half;
+  const bool turns = latent ? tid < half : e < heads * half;
+  if (!latent && !turns) return;
+  const T* src = latent ? row + c_off + rank : row + q_off + static_cast<size_t>(h) * (dim + rot) + dim;
+  const int a = interleaved ? 2 * i : i, b = interleaved ? 2 * i + 1 : i + half;
+  T u_in, v_in;
+  float pos = 0.f, freq = 0.f;
+  if (turns) {
+    u_in = src[a];
+    v_in = src[b];
+    if (inv_freq != nullptr) pos = static_cast<float>(positions[t]), freq = inv_freq[i];
+  }
+  T c[LR_PIECES];
+  float weight[LR_PIECES];
+  int slot = 0;
+  if (latent) {
+    slot = slot_map[t];
+#pragma unroll
+    for (int n = 0; n < LR_PIECES; ++n) {  // a piece beyond the latent reads its last element and counts nothing
+      const int at = tid + n * LP_THREADS < rank ? tid + n * LP_THREADS : rank - 1;
+      c[n] = row[c_off + at];
+      weight[n] = c_weight[at];
+    }
+  }
+  T* dst = latent ? cache + static_cast<size_t>(slot) * width : q_out + (static_cast<size_t>(t) * heads + h) * width;
+  if (turns) {
+    const float u = to_float(u_in), v = to_float(v_in);
+    float x = u, y = v;
+    if (inv_freq != nullptr) {
+      float sn, cs;
+      sincosf(pos * freq, &sn, &cs);
+      cs *= rot_scale;
+      sn *= rot_scale;
+      x = u * cs - v * sn;
+      y = v * cs + u * sn;
+    }
+    dst[rank + a] = from_float<T>(x);
+    dst[rank + b] = from_float<T>(y);
+  }
+  if (!latent) return;
+  float sq = 0.f;
+#pragma unroll
+  for (int n = 0; n < LR_PIECES; ++n)
+    if (tid + n * LP_THREADS < rank) sq = fmaf(to_float(c[n]), to_float(c[n]), sq);
+  const float inv = 1.0f / sqrtf(block_sum(sq, scratch) / static_cast<float>(rank) + eps);
+#pragma unroll
+  for (int n = 0; n < LR_PIECES; ++n)
+    if (tid + n * LP_THREADS < rank) dst[tid + n * LP_THREADS] = from_float<T>(to_float(c[n]) * inv * weight[n]);
+}
+
 // proj: [tokens, ld] of dtype holding, from q_off, the heads of q as [dim | rot] each, and from c_off the
 // latent (rank elements) and behind it the shared rotated key part (rot elements).  q_out: [tokens, heads,
 // rank + rot], of which only the last rot elements of every head are written.  cache: [slots, rank + rot].
@@ -145,6 +213,19 @@ extern "C" int pylon_latent_rotate(void* q_out, void* cache, const void* proj, i
   PYLON_REQUIRE(!store || (cache != nullptr && slot_map != nullptr && c_weight != nullptr),
                 "latent_rotate: storing needs cache, slots and the norm's weight");
   if (tokens == 0) return 0;
+  const long long pairs = static_cast<long long>(heads) * (rot / 2), shares = (pairs + LP_THREADS - 1) / LP_THREADS + (store ? 1 : 0);
+  if (tokens * shares <= 10ll * pylon_compute_units() && rank <= LR_PIECES * LP_THREADS && rot <= 2 * LP_THREADS && shares >= 1 && shares <= 65535) {
+    const dim3 grid(tokens, static_cast<unsigned>(shares));
+    if (dtype == PYLON_F32)
+      hipLaunchKernelGGL((latent_rotate_few_kernel<float>), grid, dim3(LP_THREADS), 0, stream, (float*)q_out, (float*)cache,
+                         (const float*)proj, ld, q_off, heads, dim, rot, c_off, rank, c_weight, eps, inv_freq, rot_scale,
+                         interleaved, positions, slot_map, store);
+    else
+      hipLaunchKernelGGL((latent_rotate_few_kernel<bf16_t>), grid, dim3(LP_THREADS), 0, stream, (bf16_t*)q_out,
+                         (bf16_t*)cache, (const bf16_t*)proj, ld, q_off, heads, dim, rot, c_off, rank, c_weight, eps,
+                         inv_freq, rot_scale, interleaved, positions, slot_map, store);
+    PYLON_LAUNCHED("latent_rotate");
+  }
   const size_t lds = sizeof(float) * (rot > 0 ? rot : 2);
   if (dtype == PYLON_F32)
     hipLaunchKernelGGL((latent_rotate_kernel<float>), dim3(tokens), dim3(LP_THREADS), lds, stream, (float*)q_out,

@@ -793,3 +793,28 @@ def test_latent_heads_shared_or_apart(ops, heads, width, rank, cuts):
     assert torch.isfinite(few.float()).all()
     for start in range(0, many - 2, 3):
         assert torch.equal(all_[start: start + 3], few)
+
+
+# few tokens in several workgroups each, many in one each: a token's numbers are the same; sizes beyond a workgroup's pairs
+@pytest.mark.parametrize("heads, rot, rank, interleaved, turned", [
+    (32, 64, 256, False, True), (9, 128, 1000, True, True), (3, 2, 5, False, False), (2, 0, 40, False, False)])
+@pytest.mark.parametrize("stored", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_latent_rows_of_few_tokens_are_those_of_many(ops, heads, rot, rank, interleaved, turned, stored, dtype):
+    many, dim = 10 * ops._lib.compute_units() + 1, 8
+    gen = torch.Generator(DEV).manual_seed(rank)
+    c_off = heads * (dim + rot)
+    proj = torch.randn(7, c_off + rank + rot, generator=gen, device=DEV).to(dtype).repeat(many // 7 + 1, 1)[:many].contiguous()
+    weight = torch.rand(rank, generator=gen, device=DEV)
+    inv_freq = torch.rand(rot // 2, generator=gen, device=DEV) if turned else None
+    pos, got = i32([0, 1, 77, 4000, 123456, 5, 9] * (many // 7 + 1))[:many].contiguous(), []
+    for n in (7, many):
+        q = torch.zeros(n, heads, rank + rot, device=DEV, dtype=dtype)
+        cache = torch.zeros(n, 1, 1, rank + rot, device=DEV, dtype=dtype)
+        ops.latent_rotate(proj[:n], q, cache if stored else None, i32(range(n)) if stored else None, q_off=0, n_heads=heads,
+                          head_dim=dim, rot_dim=rot, c_off=c_off, kv_rank=rank, c_weight=weight, eps=1e-6, inv_freq=inv_freq,
+                          rot_scale=0.9, interleaved=interleaved, positions=pos[:n])
+        got.append((q, cache))
+    for few, all_ in zip(*got):
+        assert torch.equal(all_[:7], few) and torch.equal(all_[-7 - many % 7: many - many % 7], few)
+        assert few.any() == (stored if few.shape[1:] == (1, 1, rank + rot) else rot > 0)
