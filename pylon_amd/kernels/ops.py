@@ -5,6 +5,7 @@ it launches, and launches on torch's current stream.  None has a CPU path.
 """
 from __future__ import annotations
 
+import functools
 from typing import Optional, Tuple
 
 import torch
@@ -322,15 +323,22 @@ def sink_cuts(tokens: int, n_heads: int, n_kv_heads: int, max_len: int, units: O
     return cuts
 
 
-def sink_fold(n_heads: int, n_kv_heads: int, head_dim: int, v_dim: int, bias_len: int,
-              units: Optional[int] = None) -> int:
-    """Tiles whose workgroups fill the chip once where two of :func:`attention_sink`'s share a compute unit (registers
-    for keys of 192 and values of 128, and half the LDS), else 0: the unit in which the order of a step's tiles is folded
-    (2,048 tokens at 32 heads of 128 over 8: 88.1 -> 83.5 us, with a bias of 2,049 distances 92.3 -> 88.2)."""
+@functools.lru_cache(maxsize=256)
+def _sink_launch(n_heads: int, n_kv_heads: int, head_dim: int, v_dim: int, bias_len: int, units: int) -> Tuple[int, int, int]:
+    """(workgroups of :func:`attention_sink` a tile, workgroups the chip holds at once, tiles whose workgroups fill the chip
+    once where two share a compute unit, else 0): registers for keys of 192 and values of 128, and half the LDS.  Kept by
+    its sizes: a step asks once a layer."""
     lds = 16 * bias_len + 4 * (32 * (head_dim + 8) + -(-v_dim // 16) * 16 * 40)
+    per_tile = n_kv_heads * -(-(n_heads // n_kv_heads) // 4)
     if head_dim > 192 or v_dim > 128 or lds > 80 * 1024:
-        return 0
-    return max(1, (units or _lib.compute_units()) // (n_kv_heads * -(-(n_heads // n_kv_heads) // 4)))
+        return per_tile, units, 0
+    return per_tile, 2 * units, max(1, units // per_tile)
+
+
+def sink_fold(n_heads: int, n_kv_heads: int, head_dim: int, v_dim: int, bias_len: int) -> int:
+    """The unit in which the order of a step's tiles is folded for :func:`attention_sink`, 0 where no two workgroups share a
+    compute unit (2,048 tokens at 32 heads of 128 over 8: 88.1 -> 83.5 us, with a bias of 2,049 distances 92.3 -> 88.2)."""
+    return _sink_launch(n_heads, n_kv_heads, head_dim, v_dim, bias_len, _lib.compute_units())[2]
 
 
 def sink_portion_cuts(n_tiles: int, n_heads: int, n_kv_heads: int, head_dim: int, v_dim: int, bias_len: int, span: int,
@@ -338,14 +346,14 @@ def sink_portion_cuts(n_tiles: int, n_heads: int, n_kv_heads: int, head_dim: int
     """Workgroups that share the keys of a prompt portion's tile (``span``: the most keys a token sees): as many as the
     chip holds at once, each of 160 keys or more, for a tile's walk is a chain that nothing else shortens.  With the
     merge behind, at 32 heads of 128 over 8, uncut and as this deals them: 200 tokens behind 1,300 64.1 -> 32.8 us (8
-    cuts), 500 behind 2,500 119.8 -> 67.0 (4), 952 behind 2,048 119.6 -> 106.0 (2), 300 behind 7,700 295.6 -> 121.2 (4),
-    300 behind 300 31.7 -> 29.5 (2).  Past the chip's room (2,048 tokens, 2 cuts) 93.0 -> 120.5, with fewer keys a cut
-    (300 tokens alone, 2 cuts) 19.3 -> 23.2: one each."""
-    units = units or _lib.compute_units()
-    chunks = -(-(n_heads // n_kv_heads) // 4)
-    room = units * (2 if sink_fold(n_heads, n_kv_heads, head_dim, v_dim, bias_len, units) else 1)
+    cuts), 500 behind 2,500 119.8 -> 67.0 (4), 952 behind 2,048 119.6 -> 106.0 (2), 300 behind 7,700 295.6 -> 121.2 (4).
+    Past the chip's room (2,048 tokens, 2 cuts) 93.0 -> 120.5, with fewer keys a cut (300 tokens alone, 2 cuts) 19.3 -> 23.2.
+    Below 768 keys (300 behind 300, 2 cuts: 31.7 -> 29.5) the room for the parts costs the host what the walk saves."""
+    if span < 768:
+        return 1
+    per_tile, room, _ = _sink_launch(n_heads, n_kv_heads, head_dim, v_dim, bias_len, units or _lib.compute_units())
     cuts = 1
-    while cuts < 64 and n_tiles * n_kv_heads * chunks * cuts * 2 <= room and span >= cuts * 2 * 160:
+    while cuts < 64 and n_tiles * per_tile * cuts * 2 <= room and span >= cuts * 2 * 160:
         cuts *= 2
     return cuts
 

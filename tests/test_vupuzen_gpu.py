@@ -582,8 +582,8 @@ def test_prompt_portions_against_float64(ops, heads, groups, dim, vdim, page, bu
 # at the edges: more workgroups than the chip holds, too few keys for two cuts, one workgroup a compute unit
 @pytest.mark.parametrize("tiles, heads, groups, dim, buckets, span, want", [
     (64, 32, 8, 128, 2049, 2048, 1), (33, 32, 8, 128, 2049, 3000, 1), (32, 32, 8, 128, 2049, 3000, 2),
-    (7, 32, 8, 128, 2049, 1500, 8), (10, 32, 8, 128, 2049, 300, 1), (10, 32, 8, 128, 2049, 320, 2),
-    (1, 4, 1, 128, 0, 200000, 64), (32, 32, 8, 256, 0, 3000, 1), (16, 32, 8, 128, 4096, 3000, 2), (16, 64, 8, 128, 0, 640, 2)])
+    (7, 32, 8, 128, 2049, 1500, 8), (10, 32, 8, 128, 2049, 767, 1), (10, 32, 8, 128, 2049, 768, 4),
+    (1, 4, 1, 128, 0, 200000, 64), (32, 32, 8, 256, 0, 3000, 1), (16, 32, 8, 128, 4096, 3000, 2), (16, 64, 8, 128, 0, 800, 2)])
 def test_cuts_of_a_prompt_portion(ops, tiles, heads, groups, dim, buckets, span, want):
     assert ops.sink_portion_cuts(tiles, heads, groups, dim, 128, buckets, span, units=256) == want
 
