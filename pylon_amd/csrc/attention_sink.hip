@@ -74,7 +74,7 @@ __device__ __forceinline__ float as_column_max(float v) {
 // FULL: keys of exactly 32 KS elements and values of exactly 16 NV, the strides in LDS constants.
 //
 // What bounds it is the issue of a block's vector and matrix instructions (1.1 us a block of 32 keys and compute unit with
-// four waves a SIMD, twice what the matrix instructions alone take), and for the tile with the longest walk that walk's own
+// four waves a SIMD, of which the matrix instructions take 0.3), and for the tile with the longest walk that walk's own
 // length (1.2 us a block with nothing beside it).  The registers are kept at 128 so that two workgroups share a compute
 // unit: with 145 the second one waited for the first to end.  The questions that are the same for a whole wave (does it
 // work, is there a cap, are the keys near, far, hidden) are asked once a block: asked inside the loops over the operands
