@@ -36,7 +36,6 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 // Waves a SIMD of the prompt kernel: two workgroups a compute unit where the outputs and queries leave the registers.
 #define AS_WAVES(KS, NV) ((KS) <= 6 && (NV) <= 8 ? 4 : 2)
 #define AS_LOG2E 1.4426950408889634f
-#define AS_LN2 0.6931471805599453f
 
 __device__ __forceinline__ uint32_t as_pack(float a, float b) {
   return floats_to_bf16_pair(a, b);
@@ -57,11 +56,10 @@ struct as_flag {
   static constexpr bool value = V;
 };
 
-// v times log2 e; a finite number stays finite (a bias may be the type's lowest).
-__device__ __forceinline__ float as_to_log2(float v) {
-  const float r = v * AS_LOG2E;
-  return __builtin_isinf(r) && !__builtin_isinf(v) ? copysignf(3.402823466e38f, v) : r;
-}
+// e to the power of a difference.  (Scores stay as they are and only the differences are multiplied with log2 e: kept
+// times log2 e, they saved one multiplication each, but a finite one could become infinite, and beside biases of 60 and
+// of 400 the float sums were up to 2.0 and 2.6 times as far from 64 bits.)
+__device__ __forceinline__ float as_exp(float v) { return __builtin_amdgcn_exp2f(v * AS_LOG2E); }
 
 // The largest over the four lanes of a query's column, on the vector unit (two trips through LDS with shuffles).
 __device__ __forceinline__ float as_column_max(float v) {
@@ -127,11 +125,10 @@ __global__ __launch_bounds__(512, AS_WAVES(KS, NV)) void attention_sink_kernel(
   const float* bias_row = bias ? bias + static_cast<size_t>(head) * bucket_len : nullptr;
   if (bias != nullptr) {
 #pragma unroll 8
-    for (int d = lane; d < bucket_len; d += 64) tbl[d] = as_to_log2(bias_row[d]);
+    for (int d = lane; d < bucket_len; d += 64) tbl[d] = bias_row[d];
   }
-  // Scores, biases and maxima are kept times log2 e: a weight is one subtraction and one exponential to base 2.
-  const float far_bias = bias != nullptr ? as_to_log2(bias_row[bucket_len - 1]) : 0.f;
-  const float scale2 = (softcap > 0.f ? 1.f : scale) * AS_LOG2E;  // a capped score has its scale
+  const float far_bias = bias != nullptr ? bias_row[bucket_len - 1] : 0.f;
+  const float left = softcap > 0.f ? 1.f : scale;  // a capped score has its scale
 
   // Q^T operands: column = query, eight key elements per lane and step
   bf16x8 qf[KS];
@@ -152,7 +149,7 @@ __global__ __launch_bounds__(512, AS_WAVES(KS, NV)) void attention_sink_kernel(
   floatx4 o[NV];
   // the sink: a key without a value (one lane of a query's four carries its one) whose score is 0,
   // or the head's learned number
-  float m_run = (sink && cut == 0) ? (sink_logit != nullptr ? as_to_log2(sink_logit[head]) : 0.f) : -INFINITY;
+  float m_run = (sink && cut == 0) ? (sink_logit != nullptr ? sink_logit[head] : 0.f) : -INFINITY;
   float l_run = (sink && cut == 0 && grp == 0) ? 1.f : 0.f;
 #pragma unroll
   for (int dt = 0; dt < NV; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -262,17 +259,17 @@ __global__ __launch_bounds__(512, AS_WAVES(KS, NV)) void attention_sink_kernel(
       const bool seen = kb + AS_BLOCK - 1 <= wave_first && kb >= last_first;
       if (seen && (bias == nullptr || wave_first - (kb + AS_BLOCK - 1) >= bucket_len - 1)) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sc[e] = fmaf(sc[e], scale2, far_bias);
+        for (int e = 0; e < 8; ++e) sc[e] = fmaf(sc[e], left, far_bias);
       } else if (seen && wave_first + 15 - kb < bucket_len) {
         const float* const near = tbl + (qpos - kb - 8 * grp - 7);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sc[e] = fmaf(sc[e], scale2, near[7 - e]);
+        for (int e = 0; e < 8; ++e) sc[e] = fmaf(sc[e], left, near[7 - e]);
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int key = kb + 8 * grp + e, dist = qpos - key;
           const int idx = dist < 0 ? 0 : dist < bucket_len - 1 ? dist : bucket_len - 1;
-          const float v = fmaf(sc[e], scale2, bias == nullptr ? 0.f : tbl[idx]);
+          const float v = fmaf(sc[e], left, bias == nullptr ? 0.f : tbl[idx]);
           sc[e] = (dist >= 0 && key >= qfirst) ? v : -INFINITY;
         }
       }
@@ -282,11 +279,11 @@ __global__ __launch_bounds__(512, AS_WAVES(KS, NV)) void attention_sink_kernel(
       top = as_column_max(top);
       // a query past the tile's end, or one whose every key so far is hidden, keeps -inf: no NaN from inf - inf
       const float base = (top == -INFINITY) ? 0.f : top;
-      const float corr = (top == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run - top);
+      const float corr = (top == -INFINITY) ? 1.f : as_exp(m_run - top);
       float p[8], sum = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        p[e] = __builtin_amdgcn_exp2f(sc[e] - base);
+        p[e] = as_exp(sc[e] - base);
         sum += p[e];
       }
       l_run = l_run * corr + sum;
@@ -331,7 +328,7 @@ __global__ __launch_bounds__(512, AS_WAVES(KS, NV)) void attention_sink_kernel(
     // [token, head, cut, 2 + vdim]: maximum, sum, unnormalised output
     float* dst = partial + ((static_cast<size_t>(tok0 + qi) * n_heads + head) * cuts + cut) * (2 + vdim);
     if (grp == 0) {
-      dst[0] = m_run * AS_LN2;
+      dst[0] = m_run;
       dst[1] = l;
     }
 #pragma unroll
@@ -452,9 +449,9 @@ __global__ __launch_bounds__(256, 2) void attention_sink_decode_kernel(
   floatx4 o[NV];
 #pragma unroll
   for (int dt = 0; dt < NV; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const float scale2 = (softcap > 0.f ? 1.f : scale) * AS_LOG2E;  // scores and maxima are times log2 e; a capped score has its scale
+  const float left = softcap > 0.f ? 1.f : scale;  // a capped score has its scale
   const bool first = sink && cut == 0 && wave == 0;  // the sink belongs to one partial result
-  float m_run = first ? (sink_logit != nullptr ? as_to_log2(sink_logit[my_head]) : 0.f) : -INFINITY;
+  float m_run = first ? (sink_logit != nullptr ? sink_logit[my_head] : 0.f) : -INFINITY;
   float l_run = (first && grp == 0) ? 1.f : 0.f;
   bf16x8 qf[KS];
 
@@ -483,18 +480,18 @@ __global__ __launch_bounds__(256, 2) void attention_sink_decode_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int key = kb + 8 * grp + e;
-      const float v = fmaf(sc[e], scale2, add[e] * AS_LOG2E);
+      const float v = fmaf(sc[e], left, add[e]);
       sc[e] = (key <= pos && key >= first_key) ? v : -INFINITY;
       top = fmaxf(top, sc[e]);
     }
     if (more) load_bias(next);
     top = as_column_max(top);
     const float base = (top == -INFINITY) ? 0.f : top;  // no key so far: no NaN from inf - inf
-    const float corr = (top == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run - top);
+    const float corr = (top == -INFINITY) ? 1.f : as_exp(m_run - top);
     float p[8], sum = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      p[e] = __builtin_amdgcn_exp2f(sc[e] - base);
+      p[e] = as_exp(sc[e] - base);
       sum += p[e];
     }
     l_run = l_run * corr + sum;
@@ -569,7 +566,7 @@ __global__ __launch_bounds__(256, 2) void attention_sink_decode_kernel(
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float mw = src[w * stride];
-      const float f = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - m);
+      const float f = (mw == -INFINITY) ? 0.f : as_exp(mw - m);
       total = fmaf(src[w * stride + 1], f, total);
       acc = fmaf(src[w * stride + 2 + d], f, acc);
     }
@@ -579,7 +576,7 @@ __global__ __launch_bounds__(256, 2) void attention_sink_decode_kernel(
     } else {
       float* dst = partial + (item * cuts + cut) * (2 + vdim);
       if (d == 0) {
-        dst[0] = m * AS_LN2;
+        dst[0] = m;
         dst[1] = total;
       }
       dst[2 + d] = acc;

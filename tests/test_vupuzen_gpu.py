@@ -617,3 +617,35 @@ def test_single_tokens_against_float64(ops, heads, groups, dim, vdim, cuts, soft
             # as for the prompt portions above
             slack = 2.0 ** -8 * want.abs() + 2.0 ** -12 * values[:n, g].abs().max()
             assert (got[r, h] - want).abs().le(slack).all(), (n, h)
+
+
+# biases near the ends of the type: its lowest at every key (the plain mean of the values), at some, beside others that are
+# almost as low (which then have all the weight), and large ones; for prompt tiles and for single tokens, which see one table
+@pytest.mark.parametrize("low, high, sink", [(0, 200, False), (0, 200, True), (3, 90, False), (3, 90, True)])
+@pytest.mark.parametrize("value, others", [(-3.4028234663852886e38, 0.0), (3e38, 0.0), (-3.4028234663852886e38, -3e38)])
+@pytest.mark.parametrize("dim, cuts", [(128, 1), (128, 3), (96, 1)])
+def test_biases_at_the_ends_of_the_type(ops, low, high, sink, value, others, dim, cuts):
+    page, n, heads, vdim = 32, 150, 4, 64
+    gen = torch.Generator(DEV).manual_seed(dim)
+    pages = -(-n // page)
+    k = torch.randn(pages, page, 1, dim, generator=gen, device=DEV).bfloat16()
+    v = torch.randn(pages, 1, vdim, page, generator=gen, device=DEV).bfloat16()
+    q = torch.randn(n, heads, dim, generator=gen, device=DEV).bfloat16()
+    table = torch.arange(pages, device=DEV).int().view(1, -1)
+    bias = torch.randn(heads, 200, generator=gen, device=DEV) + others
+    bias[:, low:high] = value
+    tiles = i32(np.array([(a, min(32, n - a), 0, a) for a in range(0, n, 32)]).reshape(-1)).view(-1, 4)
+    opts = dict(page_size=page, scale=0.1, bias=bias, sink=sink, cuts=cuts)
+    prompt = ops.attention_sink(q, k, v, table, tiles, None, **opts).double()
+    single = ops.attention_sink(q, k, v, table.expand(n, -1).contiguous(), None, torch.arange(n, device=DEV).int(), **opts).double()
+    keys, values = k.reshape(-1, dim)[:n].double(), v.permute(0, 3, 1, 2).reshape(-1, vdim)[:n].double()
+    far = torch.arange(n, device=DEV)[:, None] - torch.arange(n, device=DEV)[None]
+    for h in range(heads):
+        s = q[:, h].double() @ keys.t().contiguous() * 0.1 + bias[h].double()[far.clamp(0, 199)]
+        s = s.masked_fill(far < 0, float("-inf"))
+        if sink:
+            s = torch.cat([s, torch.zeros(n, 1, device=DEV).double()], 1)
+        want = torch.softmax(s, 1)[:, :n] @ values
+        slack = 2.0 ** -8 * want.abs() + 2.0 ** -12 * values.abs().max()  # as for the prompt portions above
+        for got in (prompt, single):
+            assert (got[:, h] - want).abs().le(slack).all(), h
