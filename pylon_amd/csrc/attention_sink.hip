@@ -35,6 +35,9 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 #define AS_MAX_BIAS 4096
 // Waves a SIMD of the prompt kernel: two workgroups a compute unit where the outputs and queries leave the registers.
 #define AS_WAVES(KS, NV) ((KS) <= 6 && (NV) <= 8 ? 4 : 2)
+// And of the kernel of single tokens, whose largest instance (heads beyond 128 in both) needs more than half of the
+// registers: asked for two it had 67 of them in scratch memory (heads of 256, 128 requests of 500 keys: 129 -> 161 us).
+#define AS_SINGLE_WAVES(KS, NV) ((KS) > 4 && (NV) > 8 ? 1 : 2)
 #define AS_LOG2E 1.4426950408889634f
 
 __device__ __forceinline__ uint32_t as_pack(float a, float b) {
@@ -376,7 +379,7 @@ __global__ __launch_bounds__(512, AS_WAVES(KS, NV)) void attention_sink_kernel(
 // 4 of 700 in 8 9.7 -> 7.7, 1 of 8,000 in 64 16.9 -> 13.6, 16 of 1,524 in 4 26.6 -> 20.2, 64 of 1,000, uncut, 48.5
 // -> 36.3, 4 of 40 6.4 -> 4.7; without a bias, 2 of 2,524 in a window of 1,024 and 8 cuts 11.7 -> 8.3.
 template <int KS, int NV, bool FULL>
-__global__ __launch_bounds__(256, 2) void attention_sink_decode_kernel(
+__global__ __launch_bounds__(256, AS_SINGLE_WAVES(KS, NV)) void attention_sink_decode_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, long long q_stride, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int* __restrict__ block_table, int table_width,
     const int* __restrict__ positions, int n_heads, int n_kv_heads, int dim_arg, int vdim_arg, int page_size, float scale,
@@ -621,6 +624,58 @@ __global__ void attention_sink_merge_kernel(bf16_t* __restrict__ out, const floa
   if (mine) out[static_cast<size_t>(item) * vdim + d].bits = float_to_bf16_bits(acc * inv);
 }
 
+// The instances for heads of these sizes.
+typedef decltype(&attention_sink_kernel<1, 2, false>) SinkPrompt;
+typedef decltype(&attention_sink_decode_kernel<1, 2, false>) SinkSingle;
+#define AS_OF_VALUES(KERNEL, KS) \
+  (nv <= 2 ? &KERNEL<KS, 2, false> : nv <= 4 ? &KERNEL<KS, 4, false> : nv <= 8 ? &KERNEL<KS, 8, false> : &KERNEL<KS, 16, false>)
+#define AS_OF_SIZES(KERNEL)                                                                       \
+  (ks <= 1 ? AS_OF_VALUES(KERNEL, 1) : ks <= 2 ? AS_OF_VALUES(KERNEL, 2) : ks <= 4 ? AS_OF_VALUES(KERNEL, 4) \
+                                                                                   : AS_OF_VALUES(KERNEL, 8))
+
+static SinkPrompt prompt_kernel(int dim, int vdim) {
+  const int ks = (dim + 31) / 32, nv = (vdim + 15) / 16;
+  // the sizes of the usual heads with their strides as constants (128 and 128, 2,048 tokens: 115 -> 106 registers)
+  if (dim == 64 && vdim == 64) return &attention_sink_kernel<2, 4, true>;
+  if (dim == 128 && vdim == 128) return &attention_sink_kernel<4, 8, true>;
+  if (dim == 192 && vdim == 128) return &attention_sink_kernel<6, 8, true>;
+  return AS_OF_SIZES(attention_sink_kernel);
+}
+
+static SinkSingle single_kernel(int dim, int vdim) {
+  const int ks = (dim + 31) / 32, nv = (vdim + 15) / 16;
+  if (dim == 64 && vdim == 64) return &attention_sink_decode_kernel<2, 4, true>;
+  if (dim == 128 && vdim == 128) return &attention_sink_decode_kernel<4, 8, true>;
+  return AS_OF_SIZES(attention_sink_decode_kernel);
+}
+#undef AS_OF_SIZES
+#undef AS_OF_VALUES
+
+static size_t prompt_lds(int dim, int vdim, int table_len) {  // four heads' biases, two buffers of bfloat16
+  return sizeof(float) * 4 * ((table_len + 3) & ~3) +
+         2 * 2 * (static_cast<size_t>(AS_BLOCK) * (dim + 8) + static_cast<size_t>((vdim + 15) / 16 * 16) * (AS_BLOCK + 8));
+}
+
+// What a compute unit makes of the kernels for heads of these sizes: the workgroups of the prompt kernel that it holds at
+// once beside tables of `bucket_len` distances (0: no bias), and the scratch memory of a lane, of the prompt kernel and of
+// the one of single tokens (the registers that did not fit).
+extern "C" int pylon_attention_sink_resources(int dim, int vdim, int bucket_len, int* workgroups, int* prompt_scratch,
+                                              int* single_scratch) {
+  PYLON_REQUIRE(dim >= 8 && dim % 8 == 0 && dim <= 256 && vdim >= 4 && vdim % 4 == 0 && vdim <= 256 && bucket_len >= 0 &&
+                    bucket_len <= AS_MAX_BIAS && workgroups && prompt_scratch && single_scratch,
+                "attention_sink_resources: sizes that the kernels do not take");
+  const void* prompt = reinterpret_cast<const void*>(prompt_kernel(dim, vdim));
+  const size_t lds = prompt_lds(dim, vdim, bucket_len > 0 ? bucket_len : 1);
+  hipFuncAttributes of_prompt, of_single;
+  PYLON_REQUIRE(hipFuncGetAttributes(&of_prompt, prompt) == hipSuccess &&
+                    hipFuncGetAttributes(&of_single, reinterpret_cast<const void*>(single_kernel(dim, vdim))) == hipSuccess &&
+                    hipOccupancyMaxActiveBlocksPerMultiprocessor(workgroups, prompt, 512, lds) == hipSuccess,
+                "attention_sink_resources: the device does not say");
+  *prompt_scratch = static_cast<int>(of_prompt.localSizeBytes);
+  *single_scratch = static_cast<int>(of_single.localSizeBytes);
+  return 0;
+}
+
 // q: bf16 [tokens, n_heads, dim], rows q_stride elements apart; out: bf16 [tokens, n_heads, vdim].
 // k_cache: bf16 [pages * page_size, n_kv_heads, dim]; v_cache: bf16 [pages, n_kv_heads, vdim, page_size].
 // tiles: int [n_tiles, 4] = (first token, count <= 32, block-table row, first position) of runs of
@@ -663,32 +718,14 @@ extern "C" int pylon_attention_sink(void* out, const void* q, long long q_stride
     const long long wgs = static_cast<long long>(tokens) * n_kv_heads * cuts;
     PYLON_REQUIRE(wgs < (1ll << 31), "attention_sink: too many workgroups for one launch");
     const size_t lds_d = sizeof(float) * 4 * group * (2 + vdim);
-    const int ks_d = (dim + 31) / 32, nv_d = (vdim + 15) / 16;
-#define GO_D(KS, NV, FULL)                                                                                                \
-  do {                                                                                                              \
-    if (lds_d > 48 * 1024)                                                                                          \
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_sink_decode_kernel<KS, NV, FULL>),                \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_d));                \
-    hipLaunchKernelGGL((attention_sink_decode_kernel<KS, NV, FULL>), dim3(static_cast<unsigned>(wgs)), dim3(256), lds_d,    \
-                       stream, (bf16_t*)out, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache,           \
-                       block_table, table_width, positions, n_heads, n_kv_heads, dim, vdim, page_size, scale, bias,  \
-                       bias != nullptr ? bucket_len : 1, sink, cuts, partial, window, softcap, sink_logit);          \
-  } while (0)
-#define PICK_D(KS)                  \
-  do {                              \
-    if (nv_d <= 2) GO_D(KS, 2, false);     \
-    else if (nv_d <= 4) GO_D(KS, 4, false);\
-    else if (nv_d <= 8) GO_D(KS, 8, false);\
-    else GO_D(KS, 16, false);              \
-  } while (0)
-    if (dim == 64 && vdim == 64) GO_D(2, 4, true);
-    else if (dim == 128 && vdim == 128) GO_D(4, 8, true);
-    else if (ks_d <= 1) PICK_D(1);
-    else if (ks_d <= 2) PICK_D(2);
-    else if (ks_d <= 4) PICK_D(4);
-    else PICK_D(8);
-#undef PICK_D
-#undef GO_D
+    const SinkSingle kernel = single_kernel(dim, vdim);
+    if (lds_d > 48 * 1024)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                static_cast<int>(lds_d));
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(wgs)), dim3(256), lds_d, stream, (bf16_t*)out, (const bf16_t*)q,
+                       q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, table_width, positions,
+                       n_heads, n_kv_heads, dim, vdim, page_size, scale, bias, bias != nullptr ? bucket_len : 1, sink, cuts,
+                       partial, window, softcap, sink_logit);
     if (cuts > 1) {
       const int items = tokens * n_heads, units = items * ((vdim + 63) / 64);
       hipLaunchKernelGGL(attention_sink_merge_kernel, dim3((units + 3) / 4), dim3(256), 0, stream, (bf16_t*)out,
@@ -702,38 +739,15 @@ extern "C" int pylon_attention_sink(void* out, const void* q, long long q_stride
   PYLON_REQUIRE(blocks < (1ll << 31), "attention_sink: too many tiles for one launch");
   dim3 grid(static_cast<unsigned>(blocks)), block(2 * 64 * waves);
   const int table_len = bias != nullptr ? bucket_len : 1;
-  const size_t lds = sizeof(float) * waves * ((table_len + 3) & ~3) +
-                     2 * 2 * (static_cast<size_t>(AS_BLOCK) * (dim + 8) +
-                              static_cast<size_t>((vdim + 15) / 16 * 16) * (AS_BLOCK + 8));  // two buffers of bfloat16
+  const size_t lds = prompt_lds(dim, vdim, table_len);
   PYLON_REQUIRE(lds <= 160 * 1024, "attention_sink: the bias table and a block do not fit LDS");
-  const int ks = (dim + 31) / 32, nv = (vdim + 15) / 16;
-#define GO(KS, NV, FULL) \
-  do { \
-  if (lds > 48 * 1024) \
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_sink_kernel<KS, NV, FULL>), \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); \
-  hipLaunchKernelGGL((attention_sink_kernel<KS, NV, FULL>), grid, block, lds, stream, (bf16_t*)out, (const bf16_t*)q, \
-                     q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, table_width, tiles, \
-                     positions, n_heads, n_kv_heads, dim, vdim, page_size, scale, bias, table_len, sink, cuts, partial, window, \
-                     softcap, sink_logit); \
-  } while (0)
-#define PICK_NV(KS)                        \
-  do {                                     \
-    if (nv <= 2) GO(KS, 2, false);         \
-    else if (nv <= 4) GO(KS, 4, false);    \
-    else if (nv <= 8) GO(KS, 8, false);    \
-    else GO(KS, 16, false);                \
-  } while (0)
-  // the sizes of the usual heads with their strides as constants (128 and 128, 2,048 tokens: 115 -> 106 registers)
-  if (dim == 64 && vdim == 64) GO(2, 4, true);
-  else if (dim == 128 && vdim == 128) GO(4, 8, true);
-  else if (dim == 192 && vdim == 128) GO(6, 8, true);
-  else if (ks <= 1) PICK_NV(1);
-  else if (ks <= 2) PICK_NV(2);
-  else if (ks <= 4) PICK_NV(4);
-  else PICK_NV(8);
-#undef PICK_NV
-#undef GO
+  const SinkPrompt kernel = prompt_kernel(dim, vdim);
+  if (lds > 48 * 1024)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              static_cast<int>(lds));
+  hipLaunchKernelGGL(kernel, grid, block, lds, stream, (bf16_t*)out, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache,
+                     (const bf16_t*)v_cache, block_table, table_width, tiles, positions, n_heads, n_kv_heads, dim, vdim,
+                     page_size, scale, bias, table_len, sink, cuts, partial, window, softcap, sink_logit);
   if (cuts > 1) {
     const int items = tokens * n_heads, units = items * ((vdim + 63) / 64);
     hipLaunchKernelGGL(attention_sink_merge_kernel, dim3((units + 3) / 4), dim3(256), 0, stream, (bf16_t*)out, partial,

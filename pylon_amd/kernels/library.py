@@ -33,6 +33,7 @@ _SIGNATURES = {
     "pylon_qkv_prepare": [P, P, P, P, I, L, P, P, F, P, I, P, P, I, I, I, I, I, P],
     "pylon_paged_attention": [P, P, P, P, I, P, I, P, P, I, I, I, I, I, I, F, I, L, P, P, I, I, I, F, P, I, P],
     "pylon_attention_sink": [P, P, L, P, P, P, I, P, P, I, I, I, I, I, I, F, P, I, I, I, P, L, I, I, F, P, P],
+    "pylon_attention_sink_resources": [I, I, I, P, P, P],
     "pylon_add_normed_rmsnorm": [P, I, P, P, I, I, L, P, F, P, I, P, I, I, F, P, P, F, P],
     "pylon_norm_gate": [P, I, P, P, P, L, I, I, F, I, P],
     "pylon_pass_join": [P, I, P, P, I, I, L, F, P, I, I, P],

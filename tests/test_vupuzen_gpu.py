@@ -649,3 +649,26 @@ def test_biases_at_the_ends_of_the_type(ops, low, high, sink, value, others, dim
         slack = 2.0 ** -8 * want.abs() + 2.0 ** -12 * values.abs().max()  # as for the prompt portions above
         for got in (prompt, single):
             assert (got[:, h] - want).abs().le(slack).all(), h
+
+
+# the largest heads, whose instance needs more than half of a wavefront's registers
+@pytest.mark.parametrize("dim, vdim", [(256, 256), (136, 132)])
+@pytest.mark.parametrize("cuts, softcap, buckets", [(1, None, 600), (3, 6.0, 0)])
+def test_single_tokens_of_the_largest_heads(ops, dim, vdim, cuts, softcap, buckets):
+    test_single_tokens_against_float64(ops, 8, 2, dim, vdim, cuts, softcap, buckets)
+
+
+def sink_resources(ops, dim, vdim, bucket_len=0):
+    """(workgroups of a prompt that a compute unit holds at once, bytes of scratch memory a lane of a prompt and of single tokens)."""
+    import ctypes
+
+    got = (ctypes.c_int * 3)()
+    at = ctypes.addressof(got)
+    ops._lib.call("pylon_attention_sink_resources", dim, vdim, bucket_len, at, at + 4, at + 8)
+    return tuple(got)
+
+
+def test_no_size_of_head_spills_registers(ops):
+    for dim in (8, 32, 40, 64, 72, 128, 136, 192, 200, 256):
+        for vdim in (4, 32, 36, 64, 68, 128, 132, 256):
+            assert sink_resources(ops, dim, vdim)[1:] == (0, 0), (dim, vdim)
