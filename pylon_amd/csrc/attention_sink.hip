@@ -33,8 +33,9 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 #define AS_BLOCK 32   // keys per step of the walk
 #define AS_MAX_BIAS 4096
-// Waves a SIMD of the prompt kernel: two workgroups a compute unit where the outputs and queries leave the registers.
-#define AS_WAVES(KS, NV) ((KS) <= 6 && (NV) <= 8 ? 4 : 2)
+// Waves a SIMD of the prompt kernel: two workgroups a compute unit where the outputs and queries leave the registers, at
+// values of up to 128 (the host counts on two for keys of up to 192: ops._sink_launch).
+#define AS_WAVES(KS, NV) ((NV) <= 8 ? 4 : 2)
 // And of the kernel of single tokens, whose largest instance (heads beyond 128 in both) needs more than half of the
 // registers: asked for two it had 67 of them in scratch memory (heads of 256, 128 requests of 500 keys: 129 -> 161 us).
 #define AS_SINGLE_WAVES(KS, NV) ((KS) > 4 && (NV) > 8 ? 1 : 2)

@@ -326,8 +326,8 @@ def sink_cuts(tokens: int, n_heads: int, n_kv_heads: int, max_len: int, units: O
 @functools.lru_cache(maxsize=256)
 def _sink_launch(n_heads: int, n_kv_heads: int, head_dim: int, v_dim: int, bias_len: int, units: int) -> Tuple[int, int, int]:
     """(workgroups of :func:`attention_sink` a tile, workgroups the chip holds at once, tiles whose workgroups fill the chip
-    once where two share a compute unit, else 0): registers for keys of 192 and values of 128, and half the LDS.  Kept by
-    its sizes: a step asks once a layer."""
+    once where two share a compute unit, else 0): the kernel's instances for keys of up to 192 and values of up to 128 leave
+    the registers for two, tables of up to some 3,000 distances half the LDS.  Kept by its sizes: a step asks once a layer."""
     lds = 16 * bias_len + 4 * (32 * (head_dim + 8) + -(-v_dim // 16) * 16 * 40)
     per_tile = n_kv_heads * -(-(n_heads // n_kv_heads) // 4)
     if head_dim > 192 or v_dim > 128 or lds > 80 * 1024:

@@ -672,3 +672,13 @@ def test_no_size_of_head_spills_registers(ops):
     for dim in (8, 32, 40, 64, 72, 128, 136, 192, 200, 256):
         for vdim in (4, 32, 36, 64, 68, 128, 132, 256):
             assert sink_resources(ops, dim, vdim)[1:] == (0, 0), (dim, vdim)
+
+
+# keys that take the instance of one size and of the next, exactly 192 over 128 among them; tables around half of the LDS
+@pytest.mark.parametrize("dim", [8, 64, 128, 136, 160, 192, 200, 256])
+def test_two_prompt_workgroups_share_a_unit_where_the_host_counts_on_them(ops, dim):
+    for vdim in (4, 64, 68, 96, 128, 132):
+        for buckets in (0, 2049, 2700, 3000, 3600, 4096):
+            per_tile, room, fold = ops._sink_launch(32, 8, dim, vdim, buckets, 256)
+            assert (room == 512) == (fold > 0) and per_tile == 8
+            assert sink_resources(ops, dim, vdim, buckets)[0] >= room // 256, (dim, vdim, buckets)
