@@ -30,6 +30,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x4 u32x4_at8 __attribute__((aligned(8)));  // sixteen bytes of a cache of values, which begins at any eighth byte
 
 #define AS_BLOCK 32   // keys per step of the walk
 #define AS_MAX_BIAS 4096
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(512, AS_WAVES(KS, NV)) void attention_sink_kernel(
 #pragma unroll
     for (int n = 0; n < VL; ++n) {
       const int c = threadIdx.x + n * threads;
-      if (VALUES_FIT || c < vdim * (AS_BLOCK / 8)) vreg[n] = *reinterpret_cast<const u32x4*>(vbase + v_from[n]);
+      if (VALUES_FIT || c < vdim * (AS_BLOCK / 8)) vreg[n] = *reinterpret_cast<const u32x4_at8*>(vbase + v_from[n]);
     }
     in_page += AS_BLOCK, kb_next += AS_BLOCK;
     if (in_page == page_size && kb_next < kb_end) in_page = 0, page = table[++page_at];
@@ -445,7 +446,7 @@ __global__ __launch_bounds__(256, AS_SINGLE_WAVES(KS, NV)) void attention_sink_d
     for (int dt = 0; dt < NV; ++dt) {
       const int d = dt * 16 + col;
       vraw[dt] = u32x4{0u, 0u, 0u, 0u};
-      if (FULL || d < vdim) vraw[dt] = *reinterpret_cast<const u32x4*>(block + static_cast<size_t>(d) * page_size);
+      if (FULL || d < vdim) vraw[dt] = *reinterpret_cast<const u32x4_at8*>(block + static_cast<size_t>(d) * page_size);
     }
   };
 
@@ -701,7 +702,7 @@ extern "C" int pylon_attention_sink(void* out, const void* q, long long q_stride
                 "attention_sink: bad table width or q stride");
   PYLON_REQUIRE((reinterpret_cast<uintptr_t>(q) & 15) == 0 && (reinterpret_cast<uintptr_t>(k_cache) & 15) == 0 &&
                 (reinterpret_cast<uintptr_t>(v_cache) & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0,
-                "attention_sink: operands must be 16-byte aligned");
+                "attention_sink: q and keys must be 16-byte aligned, values and results 8-byte");
   PYLON_REQUIRE(tiles != nullptr || positions != nullptr, "attention_sink: tiles or positions are required");
   PYLON_REQUIRE(bias == nullptr || (bucket_len >= 1 && bucket_len <= AS_MAX_BIAS),
                 "attention_sink: a bias by distance is a table of 1 to %d entries a head", AS_MAX_BIAS);

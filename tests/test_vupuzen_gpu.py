@@ -682,3 +682,20 @@ def test_two_prompt_workgroups_share_a_unit_where_the_host_counts_on_them(ops, d
             per_tile, room, fold = ops._sink_launch(32, 8, dim, vdim, buckets, 256)
             assert (room == 512) == (fold > 0) and per_tile == 8
             assert sink_resources(ops, dim, vdim, buckets)[0] >= room // 256, (dim, vdim, buckets)
+
+
+@pytest.mark.parametrize("dim, vdim", [(128, 128), (96, 36)])
+def test_values_that_begin_at_an_eighth_byte(ops, dim, vdim):
+    page, n = 32, 100
+    gen = torch.Generator(DEV).manual_seed(vdim)
+    k = torch.randn(4, page, 1, dim, generator=gen, device=DEV).bfloat16()
+    v = torch.randn(4, 1, vdim, page, generator=gen, device=DEV).bfloat16()
+    apart = torch.empty(v.numel() + 4, dtype=v.dtype, device=DEV)[4:].view(v.shape).copy_(v)
+    assert apart.data_ptr() % 16 == 8
+    q = torch.randn(n, 4, dim, generator=gen, device=DEV).bfloat16()
+    table = torch.arange(4, device=DEV).int().view(1, -1)
+    tiles = i32(np.array([(a, min(32, n - a), 0, a) for a in range(0, n, 32)]).reshape(-1)).view(-1, 4)
+    for at in (dict(block_table=table, tiles=tiles, positions=None),
+               dict(block_table=table.expand(n, -1).contiguous(), tiles=None, positions=torch.arange(n, device=DEV).int())):
+        a, b = (ops.attention_sink(q, k, values, **at, page_size=page, scale=0.1, bias=None, sink=True) for values in (v, apart))
+        assert torch.equal(a, b)
