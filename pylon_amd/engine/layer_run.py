@@ -81,10 +81,28 @@ def _gated(x, weight) -> Optional[Tuple[int, int]]:
     return 1, 1
 
 
+# What the parts of a plain layer do when they are asked themselves, and what they were written to do.
+_STEPS = ((PreNormBlock, "forward"), (Attention, "forward"), (GatedFeedForward, "forward"), (RMSNorm, "add_forward"),
+          (RMSNorm, "weight"), (RotaryPosition, "rotary"), (NoPosition, "rotary"))
+_AS_WRITTEN = tuple(getattr(kind, name) for kind, name in _STEPS)
+
+
+def _as_written() -> bool:
+    """Whether no class of a plain layer's parts was given another method from outside."""
+    return all(getattr(kind, name) is method for (kind, name), method in zip(_STEPS, _AS_WRITTEN))
+
+
 def _plain(block) -> bool:
-    return (type(block) is PreNormBlock and type(block.mixer) is Attention and type(block.feed_forward) is GatedFeedForward
-            and type(block.mixer_norm) is RMSNorm and type(block.feed_forward_norm) is RMSNorm
-            and type(block.mixer.position) in (RotaryPosition, NoPosition) and block.mixer.plain and not block.mixer.special)
+    if type(block) is not PreNormBlock:
+        return False
+    mixer, ff, norm1, norm2 = block.mixer, block.feed_forward, block.mixer_norm, block.feed_forward_norm
+    if not (type(mixer) is Attention and type(ff) is GatedFeedForward and type(norm1) is RMSNorm and type(norm2) is RMSNorm
+            and type(mixer.position) in (RotaryPosition, NoPosition) and mixer.plain and not mixer.special):
+        return False
+    # a part of its own type whose step was replaced (a wrapper that watches it, say) has the step in its own attributes
+    return not ("forward" in block.__dict__ or "forward" in mixer.__dict__ or "forward" in ff.__dict__
+                or "add_forward" in norm1.__dict__ or "weight" in norm1.__dict__ or "add_forward" in norm2.__dict__
+                or "weight" in norm2.__dict__ or "rotary" in mixer.position.__dict__)
 
 
 def run_layers(model, ctx, resid: torch.Tensor) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
@@ -95,7 +113,7 @@ def run_layers(model, ctx, resid: torch.Tensor) -> Optional[Tuple[torch.Tensor, 
     if resid.dtype != torch.float32 or resid.dim() != 2 or not resid.is_contiguous():
         return None
     block = model.blocks[0]
-    if not all(map(_plain, model.blocks)):
+    if not (_as_written() and all(map(_plain, model.blocks))):
         return None
     spec, ff = block.mixer.spec, block.feed_forward.spec
     width, qkv_size = spec.hidden_size, (spec.n_heads + 2 * spec.n_kv_heads) * spec.head_dim

@@ -121,3 +121,21 @@ def test_the_fields_that_both_sides_count():
     fields = (ctypes.c_int * 3)()
     library.call("pylon_layer_run_fields", ctypes.addressof(fields))
     assert tuple(fields) == (18, 30, 4)
+
+
+@pytest.mark.parametrize("part, step", [("", "forward"), ("mixer", "forward"), ("feed_forward", "forward"),
+                                        ("mixer_norm", "add_forward"), ("feed_forward_norm", "weight"),
+                                        ("mixer.position", "rotary")])
+@pytest.mark.parametrize("of_its_type", [False, True])
+def test_a_replaced_step_of_a_part_is_taken(runner, taken, monkeypatch, part, step, of_its_type):
+    thing = runner.model.blocks[1]
+    for name in filter(None, part.split(".")):
+        thing = getattr(thing, name)
+    calls, real = [], getattr(thing, step)
+    if of_its_type:
+        method = getattr(type(thing), step)
+        monkeypatch.setattr(type(thing), step, lambda self, *args, **more: (calls.append(1), method(self, *args, **more))[1])
+    else:
+        monkeypatch.setattr(thing, step, lambda *args, **more: (calls.append(1), real(*args, **more))[1], raising=False)
+    serve(runner, [[(0, 20)]])
+    assert not any(taken) and len(calls) >= 2  # in the prompt's step and the one behind it
