@@ -149,6 +149,14 @@ def run_layers(model, ctx, resid: torch.Tensor) -> Optional[Tuple[torch.Tensor, 
         return (t.dtype == bf16 and t.shape == like.shape and t.stride() == like.stride() and t.stride(1) == 1
                 and t.get_device() == place and t.data_ptr() % 16 == 0 and not ops._watched(t, t))
 
+    def ints(t, numel) -> bool:
+        return t is not None and t.dtype == torch.int32 and t.get_device() == place and t.is_contiguous() and t.numel() == numel
+
+    views = [ctx.cache(index) for index in range(len(model.blocks))]
+    maps, tables = ({id(t): t for t in found}.values() for found in ([v.slot_map for v in views], [v.block_table for v in views]))
+    if not (resid.shape == (tokens, width) and ints(ctx.positions, tokens) and all(ints(m, tokens) for m in maps)
+            and all(t is not None and t.dim() == 2 and t.shape[0] >= ctx.rows and ints(t, t.numel()) for t in tables)):
+        return None  # what the parts refuse (the views of one group of pages hold the same map and table)
     shapes = dict(qkv=(qkv_size, width), out=(width, spec.q_size), gate_up=(2 * ff.intermediate_size, width),
                   down=(width, ff.intermediate_size))
     if any(tuple(p[name].shape) != shapes[name] for p, name in ((mine, "qkv"), (mine, "out"), (theirs, "gate_up"), (theirs, "down"))):

@@ -139,3 +139,29 @@ def test_a_replaced_step_of_a_part_is_taken(runner, taken, monkeypatch, part, st
         monkeypatch.setattr(thing, step, lambda *args, **more: (calls.append(1), real(*args, **more))[1], raising=False)
     serve(runner, [[(0, 20)]])
     assert not any(taken) and len(calls) >= 2  # in the prompt's step and the one behind it
+
+
+def test_maps_and_tables_that_the_parts_refuse_are_not_launched_on(runner, monkeypatch):
+    from dataclasses import replace
+
+    from pylon_amd.engine import layer_run
+
+    answers, real = [], layer_run.run_layers
+
+    def watch(model, ctx, resid):
+        def of_layer(i, **other):
+            return replace(ctx, views={**ctx.views, i: replace(ctx.views[i], **other)})
+
+        view = ctx.views[2]
+        if not ctx.decode_only:
+            for broken in (replace(ctx, positions=ctx.positions.long()), replace(ctx, positions=ctx.positions[:-1]),
+                           of_layer(2, slot_map=view.slot_map.long()), of_layer(2, slot_map=view.slot_map[:-1]),
+                           of_layer(2, slot_map=view.slot_map.repeat_interleave(2)[::2]), of_layer(2, slot_map=None),
+                           of_layer(2, block_table=view.block_table.long()), of_layer(2, block_table=view.block_table[:0]),
+                           of_layer(2, block_table=view.block_table.cpu())):
+                answers.append(real(model, broken, resid))
+        return real(model, ctx, resid)
+
+    monkeypatch.setattr(layer_run, "run_layers", watch)
+    serve(runner, [[(0, 20)]])
+    assert answers == [None] * 9
