@@ -4,8 +4,8 @@
 //
 // A step of few prompt tokens waits for the host: a launch through the parts costs it 12 us (a tensor's allocation,
 // its checks, the conversion of some fifteen arguments, the launch itself about 3), a hundred of them are longer than
-// the device takes.  Here the operands of all layers come as one array of addresses and the intermediate results as
-// one set that every layer uses again.  MEASURED
+// the device takes.  Here the operands of some layers come as one array of addresses and the intermediate results as
+// one set that every layer uses again.
 #include "common.h"
 
 extern "C" {
@@ -42,8 +42,9 @@ extern "C" int pylon_layer_run_fields(int* fields) {
 }
 
 // layers: [n_layers][LR_LAYER_FIELDS]; step: [LR_STEP_FIELDS]; reals: [LR_REALS].  The residual stream is that in front of
-// the first layer, with nothing still to be added; what the last layer leaves to be added is in LR_DOWN_SUM.
-extern "C" int pylon_layer_run(const long long* layers, int n_layers, const long long* step, const double* reals,
+// the first layer of these; `pending`: what the layer before them left to be added is in LR_DOWN_SUM (else there is
+// nothing), as is then what the last of these leaves.
+extern "C" int pylon_layer_run(const long long* layers, int n_layers, int pending, const long long* step, const double* reals,
                                hipStream_t stream) {
   PYLON_REQUIRE(layers && step && reals && n_layers >= 1, "layer_run: no layers");
   const int tokens = static_cast<int>(step[LR_TOKENS]), width = static_cast<int>(step[LR_WIDTH]);
@@ -72,7 +73,7 @@ extern "C" int pylon_layer_run(const long long* layers, int n_layers, const long
   };
   for (int i = 0; i < n_layers; ++i) {
     const long long* const l = layers + static_cast<size_t>(i) * LR_LAYER_FIELDS;
-    int rc = norm(i == 0 ? 0 : step[LR_DOWN_SUM], step[LR_DOWN_PARTS], l[LR_NORM1], real(LR_EPS1));
+    int rc = norm(i == 0 && !pending ? 0 : step[LR_DOWN_SUM], step[LR_DOWN_PARTS], l[LR_NORM1], real(LR_EPS1));
     if (!rc) rc = product(step[LR_PROJECTED], step[LR_NORMED], l[LR_QKV], l[LR_LD_QKV], qkv_size, width, step[LR_QKV_PARTS],
                           step[LR_QKV_TILES], false, false);
     if (!rc) rc = pylon_qkv_prepare(at(step[LR_Q]), at(l[LR_K_CACHE]), at(l[LR_V_CACHE]), at(step[LR_PROJECTED]), PYLON_BF16,

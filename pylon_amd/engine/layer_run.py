@@ -1,15 +1,16 @@
-"""The layers of a step of few prompt tokens, launched by one call.
+"""The layers of a step of few prompt tokens, launched a few at a time by one call.
 
 A step of up to a few hundred prompt tokens waits for the host, which spends 12 us on every launch that the parts make
 one by one.  Where all layers of a model are alike, plain (pre-normed attention with norms and rotation head by head,
 gated feed-forward) and every one of their products runs on the engine's own kernels, :func:`run_layers` gathers the
-addresses of what a layer reads and has them launched in a loop of native code (``csrc/layer_run.hip``): the same
-kernels with the same arguments in the same order, so the same bits.  Anything else, a part of another type, a product
-that is the library's, decoding requests in the step, a tensor that something follows, is left to the parts."""
+addresses of what a layer reads and has four layers at a time launched in a loop of native code
+(``csrc/layer_run.hip``): the same kernels with the same arguments in the same order, so the same bits.  The device works
+on them while the next four are gathered.  Anything else, a part of another type, a product that is the library's,
+decoding requests in the step, a tensor that something follows, is left to the parts, from the layer on where it shows."""
 from __future__ import annotations
 
-import ctypes
 from array import array
+from functools import lru_cache
 from typing import Optional, Tuple
 
 import torch
@@ -23,6 +24,7 @@ from ..parts.norm import RMSNorm
 from ..parts.position import NoPosition, RotaryPosition
 
 MOST_TOKENS = 512  # beyond, the device takes longer than the host either way
+TOGETHER = 4  # layers of one call: the device waits for the first of them only, the others are gathered while it works
 
 
 def alike(spec) -> bool:
@@ -39,46 +41,42 @@ def alike(spec) -> bool:
             and spec.resolved_schedule() == tuple((i, i, True) for i in range(len(spec.layers))))
 
 
-def _streams(weight: torch.Tensor) -> bool:
-    """What :func:`ops.gemm_rows` asks of a matrix (``x`` is made here: close rows, aligned)."""
-    return weight.shape[1] % 8 == 0 and weight.stride(0) % 8 == 0 and weight.data_ptr() % 16 == 0 and weight.stride(1) == 1
+def _projection(rows: int, n: int, k: int, stride: int, units: int) -> Optional[Tuple[int, int]]:
+    """(parts, col_tiles) of :func:`ops.linear` with a bfloat16 result, for a matrix of n rows of k elements ``stride``
+    apart; (0, 0) for :func:`ops.gemm_wide`; None where it takes neither."""
+    if rows > plan.STREAM_ROWS:
+        return (0, 0) if ops.wide_sizes_ok(rows, n, k, k, stride) and plan.wide_beats_library(rows, n, k, units=units) else None
+    if k % 8 or stride % 8 or n >= plan.TALL:
+        return None
+    choice = plan.plan_projection(rows, n, k, stride)
+    if choice.kernel == "rows":
+        return 1, choice.col_tiles
+    return (1, 1) if choice.kernel == "library" and plan.rows_match_library(rows, n, k) else None
 
 
-def _wide(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> Optional[Tuple[int, int]]:
-    return (0, 0) if ops._wide_ok(x, weight, gated=gated) else None
-
-
-def _projection(x, weight, units) -> Optional[Tuple[int, int]]:
-    """(parts, col_tiles) of :func:`ops.linear` with a bfloat16 result, (0, 0) for :func:`ops.gemm_wide`; None where it
-    takes neither."""
-    rows, (n, k) = x.shape[0], weight.shape
-    if rows <= plan.STREAM_ROWS:
-        if not _streams(weight) or n >= plan.TALL:
-            return None
-        choice = plan.plan_projection(rows, n, k, weight.stride(0))
-        if choice.kernel == "rows":
-            return 1, choice.col_tiles
-        return (1, 1) if choice.kernel == "library" and plan.rows_match_library(rows, n, k) else None
-    return _wide(x, weight) if plan.wide_beats_library(rows, n, k, units=units) else None
-
-
-def _residual(x, weight, units) -> Optional[Tuple[int, int]]:
+def _residual(rows: int, n: int, k: int, stride: int, units: int) -> Optional[Tuple[int, int]]:
     """The same of :func:`ops.linear_for_residual`."""
-    rows, (n, k) = x.shape[0], weight.shape
-    if rows <= plan.SPLIT_ROWS and _streams(weight):
+    if rows <= plan.SPLIT_ROWS and k % 8 == 0 and stride % 8 == 0:
         choice = plan.plan_residual(rows, n, k, units=units)
         return (choice.parts, choice.col_tiles) if choice.kernel == "rows" else None
-    return _projection(x, weight, units) if rows > plan.STREAM_ROWS else None
+    return _projection(rows, n, k, stride, units) if rows > plan.STREAM_ROWS else None
 
 
-def _gated(x, weight) -> Optional[Tuple[int, int]]:
+def _gated(rows: int, n: int, k: int, stride: int) -> Optional[Tuple[int, int]]:
     """The same of :func:`ops.linear_glu`."""
-    rows, n_half = x.shape[0], weight.shape[0] // 2
     if rows > plan.STREAM_ROWS:
-        return _wide(x, weight, gated=True) if plan.wide_gated_beats_library(rows, n_half) else None
-    if not _streams(weight) or plan.plan_gated(rows, n_half, weight.shape[1], weight.stride(0)).kernel != "rows":
+        return (0, 0) if ops.wide_sizes_ok(rows, n, k, k, stride, gated=True) and plan.wide_gated_beats_library(rows, n // 2) else None
+    if k % 8 or stride % 8 or plan.plan_gated(rows, n // 2, k, stride).kernel != "rows":
         return None
     return 1, 1
+
+
+@lru_cache(maxsize=1024)  # asked for every step of few prompt tokens
+def _products(rows: int, units: int, qkv, out, gate_up, down) -> Optional[tuple]:
+    """What the four products of a layer are, each matrix given as (rows, columns, row stride); None where one of them is
+    not the engine's own."""
+    found = (_projection(rows, *qkv, units), _residual(rows, *out, units), _gated(rows, *gate_up), _residual(rows, *down, units))
+    return None if None in found else tuple(number for product in found for number in product)
 
 
 # What the parts of a plain layer do when they are asked themselves, and what they were written to do.
@@ -107,96 +105,117 @@ def _plain(block) -> bool:
 
 def run_layers(model, ctx, resid: torch.Tensor) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
     """``(resid, delta)`` behind the last layer, as the blocks hand them on, or None: then nothing was launched."""
-    tokens = ctx.tokens
+    tokens, blocks = ctx.tokens, model.blocks
     if tokens > MOST_TOKENS or ctx.decode_only or ctx.fixed_shapes or ctx.leading_singles or not resid.is_cuda:
         return None
-    if resid.dtype != torch.float32 or resid.dim() != 2 or not resid.is_contiguous():
+    block = blocks[0]
+    if not (_as_written() and _plain(block)):
         return None
-    block = model.blocks[0]
-    if not (_as_written() and all(map(_plain, model.blocks))):
-        return None
+    # the choice of the products first: it is what a step is left to the parts for, and costs least
     spec, ff = block.mixer.spec, block.feed_forward.spec
-    width, qkv_size = spec.hidden_size, (spec.n_heads + 2 * spec.n_kv_heads) * spec.head_dim
+    width, ff_size, heads, kv_heads, dim = spec.hidden_size, ff.intermediate_size, spec.n_heads, spec.n_kv_heads, spec.head_dim
+    qkv_size = (heads + 2 * kv_heads) * dim
+    mine, theirs, units = block.mixer.params, block.feed_forward.params, ops.compute_units()
+    shapes = ((qkv_size, width), (width, spec.q_size), (2 * ff_size, width), (width, ff_size))
+    matrices = (mine["qkv"], mine["out"], theirs["gate_up"], theirs["down"])
+    if any(m.shape != shape or m.stride(1) != 1 or m.stride(0) < shape[1] for m, shape in zip(matrices, shapes)):
+        return None
+    products = _products(tokens, units, *((*m.shape, m.stride(0)) for m in matrices))
     first = ctx.cache(0)
-    rotary = block.mixer.position.rotary()
-    if first.k is None or first.k.dim() != 4 or ops._watched(resid, resid):
+    if products is None or first.k is None or not ops.prefill_sizes_ok(heads, kv_heads, dim, first.block_table.shape[1]):
         return None
-    device, bf16, f32 = resid.device, torch.bfloat16, torch.float32
-    place = resid.get_device()
-    if place != torch.cuda.current_device():
+    place, bf16, f32, grad = resid.get_device(), torch.bfloat16, torch.float32, torch.is_grad_enabled()
+    if (place != torch.cuda.current_device() or resid.dtype != f32 or resid.shape != (tokens, width) or not resid.is_contiguous()
+            or ops._watched(resid, resid) or ff.activation not in ops.GATE_ACTS):
         return None
-
-    def scratch(*shape, dtype=bf16):
-        return torch.empty(shape, dtype=dtype, device=device)
-
-    normed, projected = scratch(tokens, width), scratch(tokens, qkv_size)
-    q, context = scratch(tokens, spec.n_heads, spec.head_dim), scratch(tokens, spec.n_heads, spec.head_dim)
-    hidden = scratch(tokens, ff.intermediate_size)
-    if not ops.prefill_attention_ok(q, first.k, first.block_table) or ff.activation not in ops.GATE_ACTS:
-        return None
-    units = ops.compute_units()
-    mine, theirs = block.mixer.params, block.feed_forward.params
-    products = (_projection(normed, mine["qkv"], units), _residual(context.view(tokens, spec.q_size), mine["out"], units),
-                _gated(normed, theirs["gate_up"]), _residual(hidden, theirs["down"], units))
-    if None in products:
+    page, rotary = first.page_size, block.mixer.position.rotary()
+    slots, table = (first.k.shape[0], page, kv_heads, dim), first.block_table.shape
+    rot_dim = rotary[1] if rotary else 0
+    if slots[0] * page >= 2 ** 31 or len(table) != 2 or table[0] < ctx.rows:
         return None
 
-    def good(t, dtype, shape) -> bool:
-        return (t.dtype == dtype and t.shape == shape and t.get_device() == place and t.is_contiguous()
-                and not ops._watched(t, t))
+    def row(*shape):  # type, shape and strides of a tensor without gaps
+        strides = [1]
+        for size in shape[:0:-1]:
+            strides.insert(0, strides[0] * size)
+        return shape, tuple(strides)
 
-    def matrix(t, like) -> bool:
-        return (t.dtype == bf16 and t.shape == like.shape and t.stride() == like.stride() and t.stride(1) == 1
-                and t.get_device() == place and t.data_ptr() % 16 == 0 and not ops._watched(t, t))
+    wanted = [(bf16, shape, (m.stride(0), 1)) for m, shape in zip(matrices, shapes)]
+    as_qkv, as_out, as_gate_up, as_down = wanted
+    as_gain, as_head, as_turn, as_cache = (f32, *row(width)), (f32, *row(dim)), (f32, *row(rot_dim // 2)), (bf16, *row(*slots))
+    as_map, as_table = (torch.int32, *row(tokens)), (torch.int32, *row(*table))
+    refused = False
 
-    def ints(t, numel) -> bool:
-        return t is not None and t.dtype == torch.int32 and t.get_device() == place and t.is_contiguous() and t.numel() == numel
+    def at(t, like) -> int:
+        """The address of an operand, which is refused where the parts would do something else with it."""
+        nonlocal refused
+        if not (type(t) in ops._PLAIN_TENSORS and t.dtype == like[0] and t.shape == like[1] and t.stride() == like[2]
+                and t.get_device() == place and not (grad and t.requires_grad)):
+            refused = True
+            return 0
+        address = t.data_ptr()
+        if address & 15:
+            refused = True
+        return address
 
-    views = [ctx.cache(index) for index in range(len(model.blocks))]
-    maps, tables = ({id(t): t for t in found}.values() for found in ([v.slot_map for v in views], [v.block_table for v in views]))
-    if not (resid.shape == (tokens, width) and ints(ctx.positions, tokens) and all(ints(m, tokens) for m in maps)
-            and all(t is not None and t.dim() == 2 and t.shape[0] >= ctx.rows and ints(t, t.numel()) for t in tables)):
-        return None  # what the parts refuse (the views of one group of pages hold the same map and table)
-    shapes = dict(qkv=(qkv_size, width), out=(width, spec.q_size), gate_up=(2 * ff.intermediate_size, width),
-                  down=(width, ff.intermediate_size))
-    if any(tuple(p[name].shape) != shapes[name] for p, name in ((mine, "qkv"), (mine, "out"), (theirs, "gate_up"), (theirs, "down"))):
+    maps = (first.slot_map, first.block_table)  # the views of one group of pages hold the same two
+    slot_map, pages, positions = at(maps[0], as_map), at(maps[1], as_table), at(ctx.positions, as_map)
+    if refused:
         return None
-    fields = array("q")
-    for index, block in enumerate(model.blocks):
-        a, f, cache = block.mixer.params, block.feed_forward.params, ctx.cache(index)
-        gain1, gain2, q_norm, k_norm = block.mixer_norm.weight(), block.feed_forward_norm.weight(), a.get("q_norm"), a.get("k_norm")
-        turn = block.mixer.position.rotary()
-        if not (matrix(a["qkv"], mine["qkv"]) and matrix(a["out"], mine["out"]) and matrix(f["gate_up"], theirs["gate_up"])
-                and matrix(f["down"], theirs["down"]) and good(gain1, f32, (width,)) and good(gain2, f32, (width,))
-                and good(cache.k, bf16, first.k.shape) and good(cache.v, bf16, first.k.shape)
-                and cache.page_size == cache.k.shape[1] == first.page_size and cache.block_table.shape == first.block_table.shape
-                and (turn is None) == (rotary is None) and (turn is None or turn[1] == rotary[1] and good(turn[0], f32, (turn[1] // 2,)))):
+
+    def operands(index: int) -> Optional[tuple]:
+        """What layer ``index`` reads, in the order of csrc/layer_run.hip; None where it is none of the plain ones."""
+        block, cache = blocks[index], ctx.cache(index)
+        if not _plain(block) or cache.page_size != page:
             return None
-        if spec.qk_norm and not (good(q_norm, f32, (spec.head_dim,)) and good(k_norm, f32, (spec.head_dim,))):
+        a, f, turn = block.mixer.params, block.feed_forward.params, block.mixer.position.rotary()
+        if (turn is None) != (rotary is None) or turn is not None and turn[1] != rot_dim:
             return None
-        fields.extend((gain1.data_ptr(), a["qkv"].data_ptr(), a["qkv"].stride(0),
-                       q_norm.data_ptr() if spec.qk_norm else 0, k_norm.data_ptr() if spec.qk_norm else 0,
-                       0 if turn is None else turn[0].data_ptr(), cache.k.data_ptr(), cache.v.data_ptr(),
-                       cache.slot_map.data_ptr(), cache.block_table.data_ptr(), cache.block_table.shape[1],
-                       a["out"].data_ptr(), a["out"].stride(0), gain2.data_ptr(), f["gate_up"].data_ptr(),
-                       f["gate_up"].stride(0), f["down"].data_ptr(), f["down"].stride(0)))
-    if first.k.shape[0] * first.page_size >= 2 ** 31 or first.k.shape[2:] != (spec.n_kv_heads, spec.head_dim):
-        return None
-    group = spec.n_heads // spec.n_kv_heads
-    tile_rows = ops.prefill_rows(tokens, spec.n_heads, group)
-    tiles = ctx.token_tiles(tile_rows // group, skip_rows=0, fold=ops.prefill_fold(spec.n_kv_heads))
+        if cache.slot_map is maps[0] and cache.block_table is maps[1]:
+            here = slot_map, pages
+        else:
+            here = at(cache.slot_map, as_map), at(cache.block_table, as_table)
+        found = (at(block.mixer_norm.weight(), as_gain), at(a["qkv"], as_qkv), as_qkv[2][0],
+                 at(a["q_norm"], as_head) if spec.qk_norm else 0, at(a["k_norm"], as_head) if spec.qk_norm else 0,
+                 0 if turn is None else at(turn[0], as_turn), at(cache.k, as_cache), at(cache.v, as_cache), *here, table[1],
+                 at(a["out"], as_out), as_out[2][0], at(block.feed_forward_norm.weight(), as_gain),
+                 at(f["gate_up"], as_gate_up), as_gate_up[2][0], at(f["down"], as_down), as_down[2][0])
+        return None if refused else found
 
-    def sums(parts):
-        return scratch(parts, tokens, width, dtype=f32) if parts > 1 else scratch(tokens, width, dtype=f32 if parts else bf16)
-
-    out_sum, down_sum = sums(products[1][0]), sums(products[3][0])
-    step = array("q", (
-        tokens, width, spec.n_heads, spec.n_kv_heads, spec.head_dim, rotary[1] if rotary else 0, first.page_size,
-        ff.intermediate_size, ops.GATE_ACTS[ff.activation], ops.mask_code(spec.window, spec.chunk), ctx.positions.data_ptr(),
-        tiles.data_ptr(), tiles.shape[0], tile_rows, resid.data_ptr(), normed.data_ptr(), projected.data_ptr(), q.data_ptr(),
-        context.data_ptr(), out_sum.data_ptr(), hidden.data_ptr(), down_sum.data_ptr(),
-        *(number for product in products for number in product)))
-    reals = array("d", (block.mixer_norm.spec.eps, block.feed_forward_norm.spec.eps, spec.qk_norm_eps, spec.scale))
-    library.call("pylon_layer_run", fields.buffer_info()[0], len(model.blocks), step.buffer_info()[0], reals.buffer_info()[0],
-                 ops._stream())
-    return resid, down_sum
+    step = reals = delta = None
+    for start in range(0, len(blocks), TOGETHER):
+        fields, count = array("q"), 0
+        for index in range(start, min(start + TOGETHER, len(blocks))):
+            found = operands(index)
+            if found is None:
+                break
+            fields.extend(found)
+            count += 1
+        whole = start + count == min(start + TOGETHER, len(blocks))
+        if not whole and start == 0:
+            return None
+        if step is None:
+            device = resid.device
+            group = heads // kv_heads
+            tile_rows = ops.prefill_rows(tokens, heads, group)
+            tiles = ctx.token_tiles(tile_rows // group, skip_rows=0, fold=ops.prefill_fold(kv_heads))
+            # one set of intermediate results, which every layer uses again
+            narrow = [torch.empty((tokens, size), dtype=bf16, device=device)
+                      for size in (width, qkv_size, spec.q_size, spec.q_size, ff_size)]
+            sums = [torch.empty((parts, tokens, width) if parts > 1 else (tokens, width), dtype=f32 if parts else bf16, device=device)
+                    for parts in (products[2], products[6])]
+            normed, projected, q, context, hidden = (t.data_ptr() for t in narrow)
+            delta = sums[1]
+            step = array("q", (
+                tokens, width, heads, kv_heads, dim, rot_dim, page, ff_size, ops.GATE_ACTS[ff.activation],
+                ops.mask_code(spec.window, spec.chunk), positions, tiles.data_ptr(), tiles.shape[0], tile_rows, resid.data_ptr(),
+                normed, projected, q, context, sums[0].data_ptr(), hidden, delta.data_ptr(), *products))
+            reals = array("d", (block.mixer_norm.spec.eps, block.feed_forward_norm.spec.eps, spec.qk_norm_eps, spec.scale))
+        if count:
+            library.call("pylon_layer_run", fields.buffer_info()[0], count, int(start > 0), step.buffer_info()[0],
+                         reals.buffer_info()[0], ops._stream())
+        if not whole:  # from here on the parts
+            for index in range(start + count, len(blocks)):
+                resid, delta = blocks[index].forward(resid, delta, ctx, ctx.cache(index), True)
+            break
+    return resid, delta

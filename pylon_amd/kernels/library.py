@@ -59,7 +59,7 @@ _SIGNATURES = {
     "pylon_gemm_tiled": [P, I, P, I, P, I, I, I, I, L, L, L, P],
     "pylon_gemm_skinny": [P, I, P, P, I, I, I, L, L, L, I, L, I, P],
     "pylon_gemm_rows": [P, I, P, P, I, I, I, L, L, L, I, L, I, I, I, I, F, F, F, P],
-    "pylon_layer_run": [P, I, P, P, P],
+    "pylon_layer_run": [P, I, I, P, P, P],
     "pylon_layer_run_fields": [P],
     "pylon_gemm_rows_shape": [I, I, I, I, I, I, I, I, P],
     "pylon_gemm_wide": [P, P, P, I, I, I, L, L, L, I, F, F, F, I, P],

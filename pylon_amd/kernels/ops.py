@@ -1281,12 +1281,15 @@ def prefill_fold(n_kv_heads: int) -> int:
 PREFILL_MAX_PAGES = 4096  # block-table columns the prefill kernel keeps in LDS
 
 
+def prefill_sizes_ok(n_heads: int, n_kv_heads: int, head_dim: int, table_width: int = 0) -> bool:
+    return (head_dim in DECODE_HEAD_DIMS and n_heads % n_kv_heads == 0 and n_heads // n_kv_heads <= PREFILL_ROWS
+            and table_width <= PREFILL_MAX_PAGES)
+
+
 def prefill_attention_ok(q: torch.Tensor, k_cache: torch.Tensor, block_table: Optional[torch.Tensor] = None) -> bool:
     tokens, n_heads, head_dim = q.shape
-    n_kv_heads = k_cache.shape[2]
-    return (q.dtype == torch.bfloat16 and head_dim in DECODE_HEAD_DIMS and n_heads % n_kv_heads == 0
-            and n_heads // n_kv_heads <= PREFILL_ROWS
-            and (block_table is None or block_table.shape[1] <= PREFILL_MAX_PAGES))
+    return q.dtype == torch.bfloat16 and prefill_sizes_ok(n_heads, k_cache.shape[2], head_dim,
+                                                          0 if block_table is None else block_table.shape[1])
 
 
 def attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -1471,16 +1474,21 @@ WIDE_CHUNK = 64  # elements of K that the tiled kernel walks at a time
 _WIDE_EPILOGUES = {"none": 0, "silu": 1, "relu2": 2, "gelu_tanh": 3, "capped": 4}
 
 
+def wide_sizes_ok(rows: int, n: int, k: int, x_stride: int, w_stride: int, gated: bool = False) -> bool:
+    """Sizes that :func:`gemm_wide` takes and is meant for: more rows than the streaming kernels hold, K in whole
+    chunks, rows of multiples of 8 elements, results of a multiple of 4 columns, and rows of w that one view of 2 GB
+    spans."""
+    return (rows > STREAM_ROWS and k % WIDE_CHUNK == 0 and x_stride % 8 == 0 and w_stride % 8 == 0 and x_stride < 2 ** 22
+            and n % (8 if gated else 4) == 0 and n > 0 and ((n // 2 if gated else 0) + 256) * w_stride < 2 ** 30)
+
+
 def _wide_ok(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool:
-    """Operands that :func:`gemm_wide` takes and is meant for: bfloat16 on this device, more rows than the streaming
-    kernels hold, K in whole chunks, rows of multiples of 8 elements at 16-byte aligned addresses, results of
-    a multiple of 4 columns, and rows of w that one view of 2 GB spans."""
+    """Operands that :func:`gemm_wide` takes and is meant for: of such sizes (:func:`wide_sizes_ok`), bfloat16, on this
+    device, at 16-byte aligned addresses."""
     return (x.shape[0] > STREAM_ROWS and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_cuda
-            and x.dim() == 2 and weight.dim() == 2 and weight.shape[1] % WIDE_CHUNK == 0
-            and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 and x.stride(0) < 2 ** 22 and _here(x, weight)
-            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
-            and weight.shape[0] % (8 if gated else 4) == 0 and weight.shape[0] > 0 and _rows_apart(x) and _rows_apart(weight)
-            and ((weight.shape[0] // 2 if gated else 0) + 256) * weight.stride(0) < 2 ** 30)
+            and x.dim() == 2 and weight.dim() == 2
+            and wide_sizes_ok(x.shape[0], *weight.shape, x.stride(0), weight.stride(0), gated) and _here(x, weight)
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and _rows_apart(x) and _rows_apart(weight))
 
 
 def gemm_wide(x: torch.Tensor, weight: torch.Tensor, *, epilogue: str = "none", alpha: float = 1.0, offset: float = 0.0,

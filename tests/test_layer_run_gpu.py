@@ -165,3 +165,85 @@ def test_maps_and_tables_that_the_parts_refuse_are_not_launched_on(runner, monke
     monkeypatch.setattr(layer_run, "run_layers", watch)
     serve(runner, [[(0, 20)]])
     assert answers == [None] * 9
+
+
+def runner_of_layers(monkeypatch, cfg, change, **options):
+    """A runner whose layers are ``change(layer)`` of the plain ones."""
+    from dataclasses import replace
+
+    from pylon_amd.engine import runner as engine
+
+    def resolve(config, real=engine.resolve):
+        arch = real(config)
+
+        def spec(parsed):
+            plain = arch.model_spec(parsed)
+            return replace(plain, layers=tuple(map(change, plain.layers)))
+
+        return replace(arch, model_spec=spec)
+
+    monkeypatch.setattr(engine, "resolve", resolve)
+    return runner_of(cfg, **options)
+
+
+# other layers than those above: a window, the other gate, no rotation, other widths and heads, a deep product over gemm_wide
+@pytest.mark.parametrize("mixer, ff, sizes", [
+    (dict(window=24), {}, {}), ({}, dict(activation="gelu_tanh"), {}), (dict(position="none"), {}, {}),
+    (dict(window=100), dict(activation="gelu_tanh"), dict(hidden_size=2560, intermediate_size=1536)),
+    ({}, {}, dict(hidden_size=512, num_attention_heads=24, num_key_value_heads=3, head_dim=64, intermediate_size=5120))])
+def test_the_bits_of_other_layers(monkeypatch, taken, mixer, ff, sizes):
+    from dataclasses import replace
+
+    def change(layer):
+        more = dict(mixer)
+        if "position" in more:
+            more["position"] = replace(layer.mixer.position, kind="none")
+        return replace(layer, mixer=replace(layer.mixer, **more), feed_forward=replace(layer.feed_forward, **ff))
+
+    runner = runner_of_layers(monkeypatch, config(**sizes), change)
+    portions = [[(0, 12)], [(0, 70)], [(0, 30), (1, 40)], [(2, 200), (1, 111)]]
+    got = serve(runner, portions)
+    steps = list(taken)
+    runner.model.alike = False
+    assert any(steps) and all(torch.equal(a, b) for a, b in zip(got, serve(runner, portions), strict=True))
+
+
+def test_the_first_layers_are_launched_before_the_last_are_looked_at(monkeypatch):
+    from pylon_amd.engine import layer_run
+
+    runner = runner_of(config(num_hidden_layers=9))
+    events, plain, call = [], layer_run._plain, layer_run.library.call
+    monkeypatch.setattr(layer_run, "_plain", lambda block: (events.append("layer"), plain(block))[1])
+    monkeypatch.setattr(layer_run.library, "call", lambda name, *args: (
+        name == "pylon_layer_run" and events.append(args[1]), call(name, *args))[1])
+    serve(runner, [[(0, 20)]])
+    assert events == ["layer"] * 5 + [4] + ["layer"] * 4 + [4, "layer", 1]
+
+
+# a layer that only the parts run, where none was launched yet, inside a call's layers and as the first of a call's; sums in
+# float parts and a bfloat16 result on their way between the two
+@pytest.mark.parametrize("at", [3, 4, 6, 8])
+@pytest.mark.parametrize("tokens", [20, 140])
+def test_the_parts_go_on_where_a_layer_is_theirs(monkeypatch, taken, at, tokens):
+    runner = runner_of(config(num_hidden_layers=9))
+    want = serve(runner, [[(0, tokens)]])
+    block, calls = runner.model.blocks[at], []
+    monkeypatch.setattr(block, "forward", lambda *args, real=block.forward: (calls.append(1), real(*args))[1], raising=False)
+    got = serve(runner, [[(0, tokens)]])
+    assert taken == [True, False, at > 3, False] and len(calls) == 2
+    assert all(torch.equal(a, b) for a, b in zip(got, want, strict=True))
+
+
+def test_a_step_that_is_left_to_the_parts_allocates_nothing_for_the_question(runner, monkeypatch):
+    from pylon_amd.engine import layer_run
+
+    count, real, asked = (lambda: torch.cuda.memory_stats()["allocation.all.allocated"]), layer_run.run_layers, []
+
+    def watch(*args):
+        before = count()
+        asked.append((real(*args) is None, count() - before))
+        return None
+
+    monkeypatch.setattr(layer_run, "run_layers", watch)
+    serve(runner, [[(0, 49)], [(1, 600)]])
+    assert asked == [(True, 0)] * 3
