@@ -88,43 +88,36 @@ __global__ void short_conv_kernel(TO* __restrict__ out, const TI* __restrict__ h
 }
 
 // Steps of single tokens, which are nothing but their trips to memory: the weights, the state and the input are sent for
-// together, whatever the number of taps (TAPS, or 0 where only the launch knows it: a tap beyond the last reads the last
-// once more and counts nothing).  A load under a question about the taps had been waited for before the next question: 4
-// tokens of 2,560 and four taps 2.58 -> 2.28 us, 64 3.03 -> 2.49.
+// together, by an instance for every number of taps.  (A load under a question about the taps is waited for before the next
+// question; loads for the most taps there are, the last one's again and again, cost more than they save: 256 tokens of
+// 8,192 and two taps 9.0 us with questions, 12.9 with eight loads of each, 5.7 so.)  4 tokens of 2,560 and four taps
+// 2.58 -> 2.28 us, 64 3.03 -> 2.49.
 template <typename TI, typename TW, typename TO, int TAPS>
 __global__ void short_conv_single_kernel(TO* __restrict__ out, const TI* __restrict__ h, const TW* __restrict__ w,
                                          float* state, const int* __restrict__ row_start,
-                                         const int* __restrict__ row_slots, int width, int taps_arg, long long h_stride,
-                                         int mode) {
-  constexpr int MOST = TAPS ? TAPS : CONV_MAX_TAPS;
-  const int taps = TAPS ? TAPS : taps_arg, keep = taps - 1;
+                                         const int* __restrict__ row_slots, int width, long long h_stride, int mode) {
+  constexpr int KEEP = TAPS - 1;
   const int row = blockIdx.x, c = blockIdx.y * blockDim.x + threadIdx.x;
   const int begin = row_start[row], end = row_start[row + 1];
   int slot = row_slots[row];
   asm volatile("" : "+s"(slot));  // read with the others, not once it is known that they leave something to do
   if (c >= width || begin >= end) return;
-  TW wt[MOST];
-  float win[MOST];
-  float* st = state + (static_cast<size_t>(slot) * keep) * width + c;
+  TW wt[TAPS];
+  float win[TAPS];
+  float* st = state + (static_cast<size_t>(slot) * KEEP) * width + c;
   const TI x_in = h[static_cast<size_t>(begin) * h_stride + c];
 #pragma unroll
-  for (int j = 0; j < MOST; ++j) wt[j] = w[static_cast<size_t>(c) * taps + (j < taps ? j : taps - 1)];
-  if (keep > 0) {
+  for (int j = 0; j < TAPS; ++j) wt[j] = w[static_cast<size_t>(c) * TAPS + j];
 #pragma unroll
-    for (int j = 0; j < MOST - 1; ++j) win[j] = st[static_cast<size_t>(j < keep ? j : keep - 1) * width];
-  }
+  for (int j = 0; j < KEEP; ++j) win[j] = st[static_cast<size_t>(j) * width];
   const float x = to_float(x_in);
-#pragma unroll
-  for (int j = 0; j < MOST; ++j)
-    if (j == keep) win[j] = x;
+  win[KEEP] = x;
   float acc = 0.f;
 #pragma unroll
-  for (int j = 0; j < MOST; ++j)
-    if (j < taps) acc = fmaf(to_float(wt[j]), win[j], acc);
+  for (int j = 0; j < TAPS; ++j) acc = fmaf(to_float(wt[j]), win[j], acc);
   out[static_cast<size_t>(begin) * width + c] = from_float<TO>(mode == 1 ? acc / (1.0f + expf(-acc)) : x + acc);
 #pragma unroll
-  for (int j = 0; j < MOST - 1; ++j)
-    if (j < keep) st[static_cast<size_t>(j) * width] = win[j + 1];
+  for (int j = 0; j < KEEP; ++j) st[static_cast<size_t>(j) * width] = win[j + 1];
 }
 
 // h: [tokens, width] of in_dtype, rows h_stride elements apart; w: [width, taps] of w_dtype; out:
@@ -146,18 +139,23 @@ extern "C" int pylon_short_conv(void* out, int out_dtype, const void* h, int in_
   const int tiles_per_row = (max_count + CONV_TILE - 1) / CONV_TILE;
   PYLON_REQUIRE(static_cast<long long>(rows) * tiles_per_row < (1ll << 31), "short_conv: too many tiles");
   dim3 grid(static_cast<unsigned>(rows * tiles_per_row), (width + 255) / 256), block(256);
-#define SINGLE(TI, TW, TO, TAPS)                                                                                    \
-  hipLaunchKernelGGL((short_conv_single_kernel<TI, TW, TO, TAPS>), dim3(static_cast<unsigned>(rows), (width + 255) / 256), \
-                     block, 0, stream, (TO*)out, (const TI*)h, (const TW*)w, state, row_start, row_slots, width, taps, \
-                     h_stride, mode)
+#define SINGLE(TI, TW, TO, TAPS)                                                                                      \
+  case TAPS:                                                                                                          \
+    hipLaunchKernelGGL((short_conv_single_kernel<TI, TW, TO, TAPS>), dim3(static_cast<unsigned>(rows), (width + 255) / 256), \
+                       block, 0, stream, (TO*)out, (const TI*)h, (const TW*)w, state, row_start, row_slots, width,    \
+                       h_stride, mode);                                                                               \
+    break
 #define GO(TI, TW, TO)                                                                                            \
   do {                                                                                                            \
-    if (max_count == 1 && taps == 4) SINGLE(TI, TW, TO, 4);                                                       \
-    else if (max_count == 1) SINGLE(TI, TW, TO, 0);                                                               \
-    else                                                                                                          \
-      hipLaunchKernelGGL((short_conv_kernel<TI, TW, TO>), grid, block, 0, stream, (TO*)out, (const TI*)h, (const TW*)w, \
-                         state, row_start, row_slots, tiles_per_row, width, taps, h_stride, mode);                \
+    switch (max_count == 1 ? taps : 0) {                                                                          \
+      SINGLE(TI, TW, TO, 1); SINGLE(TI, TW, TO, 2); SINGLE(TI, TW, TO, 3); SINGLE(TI, TW, TO, 4);                 \
+      SINGLE(TI, TW, TO, 5); SINGLE(TI, TW, TO, 6); SINGLE(TI, TW, TO, 7); SINGLE(TI, TW, TO, 8);                 \
+      default:                                                                                                    \
+        hipLaunchKernelGGL((short_conv_kernel<TI, TW, TO>), grid, block, 0, stream, (TO*)out, (const TI*)h, (const TW*)w, \
+                           state, row_start, row_slots, tiles_per_row, width, taps, h_stride, mode);              \
+    }                                                                                                             \
   } while (0)
+  static_assert(CONV_MAX_TAPS == 8, "an instance for every number of taps");
   const int key = (in_dtype == PYLON_F32 ? 4 : 0) | (w_dtype == PYLON_F32 ? 2 : 0) | (out_dtype == PYLON_F32 ? 1 : 0);
   switch (key) {
     case 0: GO(bf16_t, bf16_t, bf16_t); break;

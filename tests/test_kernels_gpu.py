@@ -407,6 +407,11 @@ def test_a_convolution_of_single_tokens_is_that_of_a_tile(ops, taps, rows, width
         assert torch.equal(one, two)
 
 
+@pytest.mark.parametrize("taps", [3, 5, 6, 7])
+def test_single_tokens_at_every_other_number_of_taps(ops, taps):
+    test_a_convolution_of_single_tokens_is_that_of_a_tile(ops, taps, 5, 257)
+
+
 def test_rounding_to_bfloat16_is_torchs(ops):
     """Every high half of a float32 (zeros, subnormal numbers, infinities and NaN among them) with low halves around
     the ties: the nearest, ties to even, NaN stays NaN."""
