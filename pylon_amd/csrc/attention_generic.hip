@@ -289,12 +289,16 @@ __device__ __forceinline__ void paged_attention_few_body(
       if (b >= blocks) return;
       const int j = base + b * PYLON_WAVE + lane;
       const int slot = slot_of(j < pos ? j : pos);  // beyond the last key: that one again, not used
-      // a view of each row: lanes beyond its elements bring zeros, without a branch
+      // a view of each row: lanes beyond its elements bring zeros, without a branch; sixteen keys at a time, as many as there are
 #pragma unroll
-      for (int k = 0; k < PYLON_WAVE; ++k) {
-        const unsigned long long row = static_cast<unsigned long long>(static_cast<unsigned>(__builtin_amdgcn_readlane(slot, k))) * row_bytes;
-        v[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(values + row), 0, v_dim * 4, 0x00020000), d * 4, 0, 0));
+      for (int part = 0; part < PYLON_WAVE; part += 16) {
+        if (part > 0 && base + b * PYLON_WAVE + part > pos) break;
+#pragma unroll
+        for (int k = part; k < part + 16; ++k) {
+          const unsigned long long row = static_cast<unsigned long long>(static_cast<unsigned>(__builtin_amdgcn_readlane(slot, k))) * row_bytes;
+          v[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+              __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(values + row), 0, v_dim * 4, 0x00020000), d * 4, 0, 0));
+        }
       }
     };
     bring(even, 0);
@@ -354,7 +358,8 @@ __global__ __launch_bounds__(6 * PYLON_WAVE) void paged_attention_few_kernel(
 
 // Whether the kernel of a workgroup a pair takes a float32 launch: up to two workgroups a compute unit (beyond, the
 // wavefronts of the other hide each other's waits: 48 tokens of 120 keys, 32 heads, 41 us against 35; 16 of them 17
-// against 27).
+// against 27).  Where the second workgroup of a unit has five keys or fewer there is nothing to win: 9 to 16 tokens of one
+// key, heads of 128 and of 64, 6.2 and 5.5 us against 6.0 and 4.9; of ten keys 6.2 and 5.6 against 6.9 and 5.8.
 static bool att_few(long long items, int head_dim, int v_dim, int v_transposed) {
   return items <= 2 * pylon_compute_units() && (head_dim == 64 || head_dim == 128) && v_dim <= 128 && !v_transposed;
 }

@@ -708,6 +708,30 @@ def test_float32_attention_of_few_pairs_has_the_bits_of_many(ops, geom):
             assert np.abs(f64(few)[i][:, [0, vd - 1]] - want).max() <= tol(torch.float32, 1.0), (i, p)
 
 
+# values are brought sixteen keys at a time, as many as there are: around every sixteen, what lies behind the last key NaN
+@pytest.mark.parametrize("hd, vd", [(64, 64), (128, 100)])
+def test_float32_attention_of_few_pairs_brings_no_key_too_few(ops, hd, vd):
+    last = [p + q for p in (0, 15, 31, 47, 63, 79, 255, 271) for q in (0, 1)]
+    pages, page = 5, 64
+    kc, vc = rnd((pages, page, 2, hd), 71).to(DEV), rnd((pages, page, 2, vd), 72).to(DEV)
+    table = torch.tensor([[3, 0, 4, 1, 2]], dtype=torch.int32, device=DEV)
+    q = rnd((len(last), 4, hd), 73).to(DEV)
+    rows = torch.zeros(1, dtype=torch.int32, device=DEV)
+    for i, p in enumerate(last):
+        k, v = kc.clone(), vc.clone()
+        for c in (k, v):
+            flat = c[table[0].long()].reshape(pages * page, 2, -1)
+            flat[p + 1:] = float("nan")
+            c[table[0].long()] = flat.view(c.shape)
+        got = ops.paged_attention(q[i: i + 1], k, v, table, rows, torch.tensor([p], dtype=torch.int32, device=DEV), page_size=page,
+                                  scale=hd ** -0.5, window=None)
+        keys, values = (f64(c)[table[0].cpu().numpy()].reshape(pages * page, 2, -1)[: p + 1] for c in (kc, vc))
+        for h in range(4):
+            s = keys[:, h // 2] @ f64(q)[i, h] * hd ** -0.5
+            w = np.exp(s - s.max())
+            assert np.abs(f64(got)[0, h] - w @ values[:, h // 2] / w.sum()).max() <= tol(torch.float32, 1.0), (p, h)
+
+
 @pytest.mark.parametrize("geom", [(8, 2, 128, 64, None), (4, 4, 64, 16, None), (16, 1, 256, 32, 100),
                                   (6, 2, 128, 256, None), (1, 1, 64, 16, 7)])
 @pytest.mark.parametrize("n_splits,n_cuts", [(1, 1), (2, 1), (4, 1), (8, 1), (1, 2), (4, 3), (8, 8), (2, 64)])
