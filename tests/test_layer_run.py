@@ -1,10 +1,15 @@
-"""Which models have layers that one call may launch."""
+"""Which models have layers that one call may launch, and that their products are those the parts launch."""
+import warnings
 from dataclasses import replace
 
 import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 
 from pylon_amd.config.registry import resolve
+from pylon_amd.engine import layer_run
 from pylon_amd.engine.layer_run import alike
+from pylon_amd.kernels import ops
 
 CONFIG = {"architectures": ["Qwen3ForCausalLM"], "model_type": "qwen3", "hidden_act": "silu", "num_hidden_layers": 3,
           "hidden_size": 128, "num_attention_heads": 2, "num_key_value_heads": 1, "head_dim": 64, "intermediate_size": 256,
@@ -43,3 +48,47 @@ def test_others_are_not(change):
 def test_a_layer_that_borrows_a_cache_is_not():
     plain = spec()
     assert not alike(replace(plain, schedule=(*plain.schedule[:2], replace(plain.schedule[2], cache=1))))
+
+
+# (q/k/v, context, width, feed-forward): 4B, 8B and 32B sizes, narrow layers, a narrow and deep one, one whose rows are of no
+# multiple of 64; with the matrices' rows apart as well
+@pytest.mark.parametrize("qkv, context, width, ff", [
+    (6144, 4096, 2560, 9728), (6144, 4096, 4096, 12288), (10240, 8192, 5120, 25600), (3072, 1024, 1024, 3072),
+    (1920, 1536, 512, 5120), (5120, 2048, 2056, 4104)])
+@pytest.mark.parametrize("apart", [0, 64])
+def test_the_products_are_those_of_their_entry_points(monkeypatch, qkv, context, width, ff, apart):
+    """Where a step's layers are launched by one call, (ranges of K, column tiles) of every product, (0, 0) for the tiled
+    kernel, are what the entry point that the part calls launches."""
+    launched, bf16 = [], torch.bfloat16
+    monkeypatch.setattr(ops, "_raw_device", lambda: 0)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_watched", lambda x, weight: False)
+    monkeypatch.setattr(ops, "_dev", lambda t, name, dtype=None: 0)
+    monkeypatch.setattr(ops._lib, "compute_units", lambda: 256)
+    monkeypatch.setattr(ops._lib, "call", lambda name, *args: launched.append(
+        (args[10], args[12]) if name == "pylon_gemm_rows" else (0, 0) if name == "pylon_gemm_wide" else None))
+    monkeypatch.setattr(torch.nn.functional, "linear", lambda x, w: launched.append(None) or x.new_empty(x.shape[0], w.shape[0]))
+    monkeypatch.setattr(ops, "_library_float", lambda x, w, out=None: launched.append(None) or x.new_empty(
+        x.shape[0], w.shape[0], dtype=torch.float32))
+    taken = set()
+    with FakeTensorMode(), warnings.catch_warnings():
+        warnings.simplefilter("ignore")  # data pointers of tensors without data
+
+        def choice(entry, rows, n, k, **more):
+            x = torch.empty(rows, k, dtype=bf16, device="cuda:0")
+            launched.clear()
+            entry(x, torch.empty(n, k + apart, dtype=bf16, device="cuda:0")[:, :k], **more)
+            return launched[0]
+
+        for rows in (1, 2, 16, 17, 31, 32, 33, 48, 49, 64, 65, 100, 128, 129, 192, 193, 256, 300, 384, 385, 511, 512):
+            asked = (layer_run._projection(rows, qkv, width, width + apart, 256),
+                     layer_run._residual(rows, width, context, context + apart, 256),
+                     layer_run._gated(rows, 2 * ff, width, width + apart),
+                     layer_run._residual(rows, width, ff, ff + apart, 256))
+            made = (choice(ops.linear, rows, qkv, width), choice(ops.linear_for_residual, rows, width, context, out_dtype=bf16),
+                    choice(ops.linear_glu, rows, 2 * ff, width, out_dtype=bf16),
+                    choice(ops.linear_for_residual, rows, width, ff, out_dtype=bf16))
+            for name, mine, theirs in zip(("qkv", "out", "gate/up", "down"), asked, made):
+                assert mine == theirs, (rows, name)  # None: the library's, or the skinny kernel's
+                taken.add(None if mine is None else mine[0] > 0)
+    assert taken >= {True} and len(taken) > 1
