@@ -372,13 +372,17 @@ static void launch_tiles(float* out, const float* x, const float* w, int M, int 
 }
 
 // Columns a workgroup of the streaming kernel takes: 16, or an equal share where as many whole rounds of the units as
-// 16 would need then each have less to stream: in launches of several rounds, and in one if K is deep (us of 3 and of
-// 24 rows, 16 against the share: 2560 x 9728 in 10 25.1, 22.3 and 40.1, 39.2; 5120 x 8192 in 10 50.8, 42.5 and 71.7, 64.4;
-// 6144 x 2560 in 12 14.6, 13.9 and 25.2, 23.9; 6144 x 4096 in 12 21.6, 20.3; but 2560 x 4096 11.0 either way and 3072 x
-// 2560 in 12 8.6, 8.8).
+// 16 would need then each have less to stream: in launches of two rounds, in longer ones if K is not short, and in one if K is
+// deep (us, 16 against the share.  3 and 24 rows: 2560 x 9728 in 10 25.1, 22.3 and 40.1, 39.2; 5120 x 8192 in 10 50.8, 42.5 and
+// 71.7, 64.4; 6144 x 2560 in 12 14.6, 13.9 and 25.2, 23.9; 6144 x 4096 in 12 21.6, 20.3; but 2560 x 4096 11.0 either way and
+// 3072 x 2560 in 12 8.6, 8.8.  Three rounds, 3 and 17 rows: 8448 x 2560 in 11 19.4, 17.6 and 29.4, 28.9, 10240 x 2560 in 14 21.1,
+// 19.9 and 30.5, 30.8; but 8448 x 1536 13.0, 12.2 and 18.0, 22.3, 8448 x 768 8.0, 9.0 and 11.7, 13.8, 10240 x 1024 10.1, 9.9 and
+// 14.4, 16.9.)  Rows of exactly 8192 numbers, one or two of x and 2560 to 4096 columns, are 2 to 6 % slower than with every
+// load's place computed for itself (4096 x 8192 39.6 us, 37.4); no other length from 4096 to 16384 is.
 static int gf_row_cols(int N, int K, int units) {
   const long long rounds = ((N + 15) / 16 + units - 1) / units;
   if (rounds == 1 && (K < 8192 || N < 8 * units)) return 16;
+  if (rounds > 2 && K < 2048) return 16;
   const int even = static_cast<int>((N + rounds * units - 1) / (rounds * units));
   return even < 8 ? 8 : even > 16 ? 16 : even;
 }
@@ -432,6 +436,13 @@ extern "C" int pylon_gemm_f32_plan(int M, int N, int units, int* side) {
   PYLON_REQUIRE(M >= 1 && N >= 1 && units >= 1 && side != nullptr, "gemm_f32_plan: bad arguments");
   const int tiling = gf_tiling(M, N, units);
   *side = M <= GF_ROWS ? 16 : tiling == GF_TILINGS ? 0 : gf_tilings[tiling].m < 64 ? 32 : 64;
+  return 0;
+}
+
+// The columns that a workgroup of the streaming kernel takes of such a product.  Touches no device.
+extern "C" int pylon_gemm_f32_columns(int N, int K, int units, int* columns) {
+  PYLON_REQUIRE(N >= 1 && K >= 1 && units >= 1 && columns != nullptr, "gemm_f32_columns: bad arguments");
+  *columns = gf_row_cols(N, K, units);
   return 0;
 }
 

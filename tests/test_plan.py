@@ -240,6 +240,16 @@ def test_float32_products_that_one_launch_holds(m, n, side):
         assert -(-m // side) * (-(-n // side) + 7 & ~7) * {32: 512, 64: 256}[side] < 2 ** 32
 
 
+# even shares of whole rounds: of one round for deep rows, of two, of more for rows that are not short
+@pytest.mark.parametrize("n, k, columns", [
+    (2560, 9728, 10), (2560, 8188, 16), (2047, 8192, 16), (2048, 8192, 8), (4096, 9728, 16), (4097, 512, 9), (6144, 512, 12),
+    (8192, 512, 16), (8193, 2044, 16), (8193, 2048, 11), (10240, 768, 16), (10240, 2560, 14), (20000, 1024, 16), (16385, 2560, 13)])
+def test_columns_of_float32_products_of_few_rows(n, k, columns):
+    got = ctypes.c_int()
+    assert library.load().pylon_gemm_f32_columns(n, k, 256, ctypes.byref(got)) == 0
+    assert got.value == columns and -(-n // columns) <= max(-(-n // 16), 256 * -(-(-(-n // 16)) // 256))
+
+
 def test_every_tile_of_the_wide_product_is_the_best_for_some_size():
     lib, tile, us = library.load(), ctypes.c_int(), ctypes.c_float()
     count = 0
