@@ -23,7 +23,10 @@
 // (rows padded against bank conflicts).  Keys
 // may be cut over `cuts` workgroups, which then leave float partial results (maximum, sum,
 // unnormalised output) for a second small kernel to merge in order; the sink belongs to the
-// first cut.  The order of a query's sums depends on its position and the number of cuts only.
+// first cut.  The order of a query's sums: that of its keys, in blocks from the first key that its tile sees, cut at every
+// so many blocks of its tile's walk.  A single token is a tile of its own.  A prompt portion's tiles begin where the portion
+// does, and the host deals it more cuts the fewer tiles its step has and the longer the step's longest request is: the same
+// tokens alone and beside others are other roundings of the same sums, each as near to the exact ones.
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -83,8 +86,8 @@ __device__ __forceinline__ float as_column_max(float v) {
 // work, is there a cap, are the keys near, far, hidden) are asked once a block: asked inside the loops over the operands
 // they had put a branch and a wait for all loads before every matrix instruction.  The loads of the queries are waited
 // for before the walk.  Keys are written to LDS in the order that makes a lane's eight weights those of eight neighbours:
-// one 16-byte piece of values.  32 heads of 128 over 8, 2,048 tokens, bias over 2,049 distances: 152 -> 88 us; behind
-// 952 cached ones 279 -> 138; behind 452 in a window of 1,024 without a bias 144 -> 71; 40 tokens 10.5 -> 9.2.
+// one 16-byte piece of values.  32 heads of 128 over 8, 2,048 tokens, bias over 2,049 distances: 153 -> 90 us; behind
+// 952 cached ones 275 -> 134; behind 452 in a window of 1,024 without a bias 143 -> 71; 40 tokens 10.4 -> 9.0.
 template <int KS, int NV, bool FULL>
 __global__ __launch_bounds__(512, AS_WAVES(KS, NV)) void attention_sink_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, long long q_stride, const bf16_t* __restrict__ k_cache,

@@ -588,6 +588,41 @@ def test_cuts_of_a_prompt_portion(ops, tiles, heads, groups, dim, buckets, span,
     assert ops.sink_portion_cuts(tiles, heads, groups, dim, 128, buckets, span, units=256) == want
 
 
+# the same portion alone, in four cuts, beside short prompts, uncut, and beside one long request whose length deals it more
+@pytest.mark.parametrize("window, buckets", [(None, 600), (900, 0)])
+def test_a_prompt_portion_beside_others(ops, window, buckets):
+    heads, groups, dim, page, new, behind = 32, 8, 128, 64, 70, 1000
+    results, cuts = [], set()
+    for others in ((), ((0, 300),) * 7, ((3000, 40),)):
+        portions = ((behind, new), *others)
+        width = -(-max(a + b for a, b in portions) // page)
+        own = -(-(behind + new) // page)
+        gen = torch.Generator(DEV).manual_seed(1)
+        k = torch.randn(own, page, groups, dim, generator=gen, device=DEV).bfloat16()
+        v = torch.randn(own, groups, dim, page, generator=gen, device=DEV).bfloat16()
+        q = torch.randn(new, heads, dim, generator=gen, device=DEV).bfloat16()
+        bias = torch.randn(heads, buckets, generator=gen, device=DEV) if buckets else None
+        more = torch.randn(width, page, groups, dim, generator=gen, device=DEV).bfloat16()  # one set of pages for all the others
+        table = torch.zeros(len(portions), width, device=DEV, dtype=torch.int32)
+        table[0, :own] = torch.arange(own, device=DEV)
+        table[1:] = torch.arange(own, own + width, device=DEV)
+        tiles, at = [], 0
+        for row, (start, count) in enumerate(portions):
+            tiles += [(at + a, min(32, count - a), row, start + a) for a in range(0, count, 32)]
+            at += count
+        span = min(window or 2 ** 31, max(a + b for a, b in portions))
+        cuts.add(ops.sink_portion_cuts(len(tiles), heads, groups, dim, dim, buckets, span))
+        got = ops.attention_sink(torch.cat([q, q.new_zeros(at - new, heads, dim)]), torch.cat([k, more]),
+                                 torch.cat([v, more.permute(0, 2, 3, 1).contiguous()]), table,
+                                 i32(np.array(tiles).reshape(-1)).view(-1, 4), None, page_size=page, scale=0.1, bias=bias, sink=True,
+                                 window=window, cuts=ops.sink_portion_cuts(len(tiles), heads, groups, dim, dim, buckets, span))
+        results.append(got[:new].double())
+    assert len(cuts) >= 2 and 1 in cuts
+    most = 2.0 ** -12 * v.double().abs().max()  # each as near to the exact numbers as the portions above are
+    for other in results[1:]:
+        assert ((other - results[0]).abs() <= 2 * (2.0 ** -8 * torch.maximum(other.abs(), results[0].abs()) + most)).all()
+
+
 # the sizes whose strides are constants and one beside each; waves of no block, one and several, whole and ragged
 @pytest.mark.parametrize("heads, groups, dim, vdim", [(8, 2, 64, 64), (8, 2, 64, 60), (8, 1, 128, 128), (32, 2, 120, 128)])
 @pytest.mark.parametrize("cuts, softcap, buckets", [(1, None, 600), (2, 6.0, 9), (1, 6.0, 0), (7, None, 0)])
