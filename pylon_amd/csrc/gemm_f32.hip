@@ -27,7 +27,8 @@
 //
 // Measured, 4B layer sizes, weights from memory, gemm_tiled (one chain per element on the vector ALUs)
 // before: of a step of 3 rows q/k/v 14 us, gate/up 37 (5.4 TB/s), out and down 11 and 22, the head 247 (6.3)
-// where a launch took 615 on average; 270 rows 61 + 135 + 93 + 266 (93 to 106 TFLOP/s; 600 rows 106 to 110).
+// where a launch took 615 on average; out, down, q/k/v and gate/up of 270 rows 61, 135, 93 and 266 (91 to 101 TFLOP/s; 600 rows
+// 104 to 110).
 #include "gemm_f32.h"
 #include <type_traits>
 
@@ -391,9 +392,9 @@ static int gf_row_cols(int N, int K, int units) {
 // share a compute unit (us, measured over 33 to 900 rows of 2560 x 4096, 2560 x 9728, 6144 x 2560 and 19456 x 2560): from
 // these and the number of rounds a launch is estimated, within 8 % of what it takes; the least is chosen.  Small tiles
 // reach every unit in a launch of few rows, large ones read less from the second-level cache and from LDS for each
-// product.  Two sizes alone, 32 x 32 and (from 512 rows on) 64 x 64, took, 4B layer sizes at 270 rows, 69 + 156 + 96 + 287
-// us where these take 61 + 135 + 93 + 266, at 600 135 + 296 + 189 + 557 and 118 + 274 + 181 + 546, at 900 212 + 479 + 282 +
-// 831 and 173 + 397 + 266 + 786.
+// product.  Two sizes alone, 32 x 32 and (from 512 rows on) 64 x 64, took, out, down, q/k/v and gate/up of 4B sizes at 270
+// rows, 69, 156, 96 and 287 us where these take 61, 135, 93 and 266, at 600 135, 296, 189, 557 and 118, 274, 181, 546, at 900 212,
+// 479, 282, 831 and 173, 397, 266, 786.
 enum { GF_32_TEAMS, GF_32_WIDE, GF_48, GF_48_TEAMS, GF_64_TEAMS, GF_96, GF_64, GF_TILINGS };
 struct GfTiling {
   int m, n, threads, resident;

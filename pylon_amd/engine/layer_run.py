@@ -2,7 +2,8 @@
 
 A step of up to a few hundred prompt tokens waits for the host, which spends 12 us on every launch that the parts make
 one by one.  Where all layers of a model are alike, plain (pre-normed attention with norms and rotation head by head,
-gated feed-forward) and every one of their products runs on the engine's own kernels, :func:`run_layers` gathers the
+gated feed-forward) and every one of their products runs on the engine's own kernels (at 4B sizes 2 to 48 and 65 to 384
+tokens, 8B 2 to 16 and 65 to 256, 32B 2 to 48, 65 to 192 and 385 to 512), :func:`run_layers` gathers the
 addresses of what a layer reads and has four layers at a time launched in a loop of native code
 (``csrc/layer_run.hip``): the same kernels with the same arguments in the same order, so the same bits.  The device works
 on them while the next four are gathered.  Anything else, a part of another type, a product that is the library's,
@@ -23,7 +24,10 @@ from ..parts.feed_forward import GatedFeedForward
 from ..parts.norm import RMSNorm
 from ..parts.position import NoPosition, RotaryPosition
 
-MOST_TOKENS = 512  # beyond, the device takes longer than the host either way
+# Beyond, the device takes longer than the host either way: lone steps of 28 layers at a width of 1,024, by the parts and by
+# one call, 100 tokens 2,702 and 1,373 us, 300 2,762 and 2,179, 512 2,785 and 2,485, 700 2,809 and 2,677, 1,000 2,909 and 2,952; of
+# 36 at 4B sizes 21 tokens 3,346 and 2,418, from 100 on (3,927 and 3,951) no difference.
+MOST_TOKENS = 512
 TOGETHER = 4  # layers of one call: the device waits for the first of them only, the others are gathered while it works
 
 

@@ -311,9 +311,10 @@ def sink_cuts(tokens: int, n_heads: int, n_kv_heads: int, max_len: int, units: O
     an upper bound) has more than 64 keys a cut.  The kernel deals them in whole blocks of 32, as many to each cut:
     at least three, but for the last cut that gets any, and up to a third of the cuts get none (131 blocks in 64
     cuts: three each to 44) and leave partial results that weigh nothing.  With the merge behind, at 32 heads of
-    128 over 8: 4 requests of 300 keys in 1, 2, 4, 8 cuts 14.0, 13.0, 10.4, 9.9 us; 4 of 1,524 in 4, 8, 16, 32
-    18.1, 14.4, 14.1, 19.4; 1 of 8,000 in 8, 16, 32 30.0, 20.1, 16.2; 16 of 1,524 in 2, 4, 8 32.3, 30.3, 33.6; 64
-    of 1,000 in 1, 2, 4 63.2, 67.8, 71.2."""
+    128 over 8: 4 requests of 300 keys in 1, 2, 4, 8 cuts 8.8, 8.7, 7.5, 7.3 us; 4 of 1,524 in 4, 8, 16, 32
+    12.5, 9.8, 10.4, 14.4; 1 of 8,000 in 8, 16, 32, 64 23.1, 15.1, 12.0, 14.0; 16 of 1,524 in 1, 2, 4, 8 29.4, 21.2, 20.8,
+    23.1; 64 of 1,000 in 1, 2, 4 42.3, 45.5, 47.0 (the lines were drawn on a kernel half as fast, where the second number of
+    cuts won by more and 64 cuts had not lost)."""
     units = units or _lib.compute_units()
     group = n_heads // n_kv_heads
     groups = tokens * n_kv_heads * (-(-group // 4))
@@ -337,7 +338,7 @@ def _sink_launch(n_heads: int, n_kv_heads: int, head_dim: int, v_dim: int, bias_
 
 def sink_fold(n_heads: int, n_kv_heads: int, head_dim: int, v_dim: int, bias_len: int) -> int:
     """The unit in which the order of a step's tiles is folded for :func:`attention_sink`, 0 where no two workgroups share a
-    compute unit (2,048 tokens at 32 heads of 128 over 8: 88.1 -> 83.5 us, with a bias of 2,049 distances 92.3 -> 88.2)."""
+    compute unit (2,048 tokens at 32 heads of 128 over 8: 89.5 -> 84.7 us, with a bias of 2,049 distances 94.9 -> 89.7)."""
     return _sink_launch(n_heads, n_kv_heads, head_dim, v_dim, bias_len, _lib.compute_units())[2]
 
 
@@ -345,10 +346,11 @@ def sink_portion_cuts(n_tiles: int, n_heads: int, n_kv_heads: int, head_dim: int
                       units: Optional[int] = None) -> int:
     """Workgroups that share the keys of a prompt portion's tile (``span``: the most keys a token sees): as many as the
     chip holds at once, each of 160 keys or more, for a tile's walk is a chain that nothing else shortens.  With the
-    merge behind, at 32 heads of 128 over 8, uncut and as this deals them: 200 tokens behind 1,300 64.1 -> 32.8 us (8
-    cuts), 500 behind 2,500 119.8 -> 67.0 (4), 952 behind 2,048 119.6 -> 106.0 (2), 300 behind 7,700 295.6 -> 121.2 (4).
-    Past the chip's room (2,048 tokens, 2 cuts) 93.0 -> 120.5, with fewer keys a cut (300 tokens alone, 2 cuts) 19.3 -> 23.2.
-    Below 768 keys (300 behind 300, 2 cuts: 31.7 -> 29.5) the room for the parts costs the host what the walk saves."""
+    merge behind, at 32 heads of 128 over 8, uncut and as this deals them: 200 tokens behind 1,300 63.8 -> 33.0 us (8
+    cuts), 500 behind 2,500 120.4 -> 70.2 (4), 952 behind 2,048 120.4 -> 106.1 (2), 300 behind 7,700 296.2 -> 132.1 (4).
+    Past the chip's room (2,048 tokens, 2 cuts) 94.9 -> 119.1, with fewer keys a cut (300 tokens alone, 2 cuts) 19.2 -> 23.1.
+    Below 768 keys (300 behind 300, 2 cuts: 31.4 -> 29.4) the room for the parts costs the host what the walk saves.
+    How a portion is cut therefore depends on the other requests of its step."""
     if span < 768:
         return 1
     per_tile, room, _ = _sink_launch(n_heads, n_kv_heads, head_dim, v_dim, bias_len, units or _lib.compute_units())
@@ -1912,7 +1914,11 @@ def latent_prefill(q: torch.Tensor, cache: torch.Tensor, block_table: torch.Tens
 
 def latent_cuts(tokens: int, n_heads: int, span: int, units: Optional[int] = None) -> int:
     """Workgroups that share the keys of one token and group of heads in a step of single tokens: more
-    while the launch leaves compute units idle and every cut keeps 128 keys, a block for each wave."""
+    while the launch leaves compute units idle and every cut keeps 128 keys, a block for each wave.  Heads beyond sixteen
+    are counted in groups of 32, as they share a workgroup where the launch fills the chip; where it does not, each sixteen
+    have workgroups of their own and this line is drawn short or long of the best.  With the merge behind, 32 heads, keys
+    of 320 over a latent of 256, 900 of them: 1 token in 4 (dealt), 8, 16 cuts 10.8, 9.4, 10.0 us; 6 11.0, 10.1, 11.3; 32 in 2,
+    4 (dealt), 8 15.0, 13.4, 18.5; 48 in 1, 2, 4 (dealt) 17.5, 16.7, 20.3."""
     units = units or _lib.compute_units()
     groups = tokens * (-(-n_heads // (32 if n_heads > 16 else 16)))
     cuts = 1
