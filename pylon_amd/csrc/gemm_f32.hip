@@ -376,11 +376,12 @@ static void launch_tiles(float* out, const float* x, const float* w, int M, int 
 // 16 would need then each have less to stream: in launches of two rounds, in longer ones if K is not short, and in one if K is
 // deep (us, 16 against the share.  3 and 24 rows: 2560 x 9728 in 10 25.1, 22.3 and 40.1, 39.2; 5120 x 8192 in 10 50.8, 42.5 and
 // 71.7, 64.4; 6144 x 2560 in 12 14.6, 13.9 and 25.2, 23.9; 6144 x 4096 in 12 21.6, 20.3; but 2560 x 4096 10.5, 10.3 and 18.0, 18.2 and
-// 3072 x 2560 in 12 8.6, 8.8.  In between, where there are none yet: 2560 x 5120 13.7, 12.8 and 23.9, 22.7; 3072 x 6144 in 12 16.3,
-// 15.6 and 27.5, 26.7; 3584 x 7168 in 14 20.4, 20.3 and 31.5, 31.1.  Three rounds, 3 and 17 rows: 8448 x 2560 in 11 19.4, 17.6 and 29.4, 28.9, 10240 x 2560 in 14 21.1,
-// 19.9 and 30.5, 30.8; but 8448 x 1536 13.0, 12.2 and 18.0, 22.3, 8448 x 768 8.0, 9.0 and 11.7, 13.8, 10240 x 1024 10.1, 9.9 and
-// 14.4, 16.9.)  Rows of exactly 8192 numbers, one or two of x and 2560 to 4096 columns, are 2 to 6 % slower than with every
-// load's place computed for itself (4096 x 8192 39.6 us, 37.4); no other length from 4096 to 16384 is.
+// 3072 x 2560 in 12 8.6, 8.8.  In between, where there are none yet: 2560 x 5120 13.7, 12.8 and 23.9, 22.7; 3072 x 6144 in 12
+// 16.3, 15.6 and 27.5, 26.7; 3584 x 7168 in 14 20.4, 20.3 and 31.5, 31.1.  Three rounds, 3 and 17 rows: 8448 x 2560 in 11 19.4,
+// 17.6 and 29.4, 28.9, 10240 x 2560 in 14 21.1, 19.9 and 30.5, 30.8; but 8448 x 1536 13.0, 12.2 and 18.0, 22.3, 8448 x 768 8.0,
+// 9.0 and 11.7, 13.8, 10240 x 1024 10.1, 9.9 and 14.4, 16.9).  Rows of exactly 8192 numbers, one or two of x and 2560 to 4096
+// columns, are 2 to 6 % slower than with every load's place computed for itself (4096 x 8192 39.6 us, 37.4); no other
+// length from 4096 to 16384 is.
 static int gf_row_cols(int N, int K, int units) {
   const long long rounds = ((N + 15) / 16 + units - 1) / units;
   if (rounds == 1 && (K < 8192 || N < 8 * units)) return 16;
