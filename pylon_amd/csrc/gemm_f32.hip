@@ -61,7 +61,7 @@ __device__ __forceinline__ void gf_barrier() {
 
 // The body is a device function: the host pass does not know the descriptor type and would drop a
 // kernel that names it, launch stub and all.
-template <int MT>
+template <int MT, bool W_FIRST>
 __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, const float* x,
                                                    const float* __restrict__ w, int M, int N, int K, int ldx, int ldw,
                                                    long long ldo, int cols) {
@@ -107,15 +107,19 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
   auto bring = [&](floatx4 (&xv)[MT][4], int chunk, int stage) __attribute__((always_inline)) {
     const int at = chunk * (GF_CHUNK * 4);
     auto send = [&](auto w_off, auto x_off, int offset) __attribute__((always_inline)) {
+      auto send_w = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (GF_LDS(void)*)(stage_base + stage * GF_TILE_BYTES + q * 1024), 16,
+                                                   w_off(q), offset, 0, 0);
+      };
+      if (W_FIRST) send_w();
 #pragma unroll
       for (int t = 0; t < MT; ++t)
 #pragma unroll
         for (int s = 0; s < 4; ++s)
           xv[t][s] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xres, x_off(t, s), offset, 0));
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (GF_LDS(void)*)(stage_base + stage * GF_TILE_BYTES + q * 1024), 16,
-                                                 w_off(q), offset, 0, 0);
+      if (!W_FIRST) send_w();
     };
     if ((chunk + 1) * GF_CHUNK <= K) {
       send([&](int q) { return w_at[q]; }, [&](int t, int s) { return x_at[t] + 64 * s; }, at);
@@ -186,12 +190,15 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
   }
 }
 
-// What the first loads need are the first 14 words of the arguments, which come with the launch.
-template <int MT>
+// What the first loads need are the first 14 words of the arguments, which come with the launch.  W_FIRST: a chunk of w is
+// sent for before that of x, for up to 16 deep rows.  It is what rows of 8,192 numbers want (us, x first and w first: 1 x 4096 x
+// 8192 39.7, 37.4, 3 x 2560 x 8192 23.7, 23.3; of 9,216 to 25,600 numbers no difference beyond 3 %); shorter ones want x first
+// (3 x 6144 x 2560 13.3, 13.7, 16 x 8192 x 512 5.1, 5.4).
+template <int MT, bool W_FIRST>
 __global__ __launch_bounds__(GF_RANGES* PYLON_WAVE) void gemm_f32_rows_kernel(
     const float* x, const float* __restrict__ w, int M, int N, int K, int cols, int ldx, int ldw,
     float* __restrict__ out, long long ldo) {
-  gemm_f32_rows_body<MT>(out, x, w, M, N, K, ldx, ldw, ldo, cols);
+  gemm_f32_rows_body<MT, W_FIRST>(out, x, w, M, N, K, ldx, ldw, ldo, cols);
 }
 
 // TM, TN: tiles of 16 rows and of 16 columns per wave; WM, WN: waves of a team along them, four together.  TEAMS: 1, or
@@ -379,9 +386,7 @@ static void launch_tiles(float* out, const float* x, const float* w, int M, int 
 // 3072 x 2560 in 12 8.6, 8.8.  In between, where there are none yet: 2560 x 5120 13.7, 12.8 and 23.9, 22.7; 3072 x 6144 in 12
 // 16.3, 15.6 and 27.5, 26.7; 3584 x 7168 in 14 20.4, 20.3 and 31.5, 31.1.  Three rounds, 3 and 17 rows: 8448 x 2560 in 11 19.4,
 // 17.6 and 29.4, 28.9, 10240 x 2560 in 14 21.1, 19.9 and 30.5, 30.8; but 8448 x 1536 13.0, 12.2 and 18.0, 22.3, 8448 x 768 8.0,
-// 9.0 and 11.7, 13.8, 10240 x 1024 10.1, 9.9 and 14.4, 16.9).  Rows of exactly 8192 numbers, one or two of x and 2560 to 4096
-// columns, are 2 to 6 % slower than with every load's place computed for itself (4096 x 8192 39.6 us, 37.4); no other
-// length from 4096 to 16384 is.
+// 9.0 and 11.7, 13.8, 10240 x 1024 10.1, 9.9 and 14.4, 16.9.)
 static int gf_row_cols(int N, int K, int units) {
   const long long rounds = ((N + 15) / 16 + units - 1) / units;
   if (rounds == 1 && (K < 8192 || N < 8 * units)) return 16;
@@ -468,10 +473,12 @@ bool gemm_f32_launch(float* out, const float* x, const float* w, int M, int N, i
   if (M <= GF_ROWS) {
     const int cols = gf_row_cols(N, K, units);
     const dim3 grid((N + cols - 1) / cols), block(GF_RANGES * PYLON_WAVE);
-    if (M <= 16)
-      hipLaunchKernelGGL((gemm_f32_rows_kernel<1>), grid, block, 0, stream, x, w, M, N, K, cols, (int)ldx, (int)ldw, out, ldo);
-    else
-      hipLaunchKernelGGL((gemm_f32_rows_kernel<2>), grid, block, 0, stream, x, w, M, N, K, cols, (int)ldx, (int)ldw, out, ldo);
+#define GO(MT, W_FIRST)                                                                                            \
+  hipLaunchKernelGGL((gemm_f32_rows_kernel<MT, W_FIRST>), grid, block, 0, stream, x, w, M, N, K, cols, (int)ldx, (int)ldw, out, ldo)
+    if (M > 16) GO(2, false);
+    else if (K >= 8192) GO(1, true);
+    else GO(1, false);
+#undef GO
     return true;
   }
 #define GO(TM, TN, WM, WN, TEAMS) launch_tiles<TM, TN, WM, WN, TEAMS>(out, x, w, M, N, K, ldx, ldw, ldo, stream)

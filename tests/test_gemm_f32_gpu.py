@@ -58,7 +58,7 @@ def test_tiles_of_64_agree_with_the_streaming_kernel(ops):
 # 64, 48 x 64 by two teams, 64 x 64, 64 x 64 by two teams, 96 x 64; and the streaming kernel's narrower shares
 @pytest.mark.parametrize("rows, n, k", [(97, 2560, 576), (100, 19455, 520), (181, 19457, 516), (270, 2561, 640),
                                         (32770, 70, 520), (360, 2497, 1100), (287, 19455, 576), (5, 5121, 520),
-                                        (17, 2561, 8192)])
+                                        (17, 2561, 8192), (16, 2561, 8188), (16, 2561, 8196), (1, 17, 8192)])
 def test_every_tile_against_float64(ops, rows, n, k):
     x, w = draw(rows, rows, k), draw(n + k, n, k)
     got = ops.gemm_tiled(x, w)
