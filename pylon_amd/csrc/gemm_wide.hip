@@ -15,16 +15,26 @@
 // behind a counted wait: the next chunk has landed, and nobody reads this one's place any more.
 //
 // Two ways to lay chunks out in LDS.  STAGES > 0: that many stages of x and w, as many as fit.
-// STAGES = 0 (square tiles): a ring of five places, each x or w of one chunk; two and a half chunks of a
-// 256 x 256 tile fill the 160 KB, where two stages keep too few bytes in flight for the latency of
-// memory (2048 rows, gate/up 2 x 12288 x 4096: 346 -> 307 us).
+// STAGES = 0: three places for x and two for w, two and a half chunks; those of a 256 x 256 tile fill the 160 KB,
+// where two stages keep too few bytes in flight for the latency of memory (2048 rows, gate/up 2 x 12288 x 4096:
+// 346 -> 307 us).
 //
-// Which tile: gw_choose, by a model of the launch's rounds over the compute units.  A layer of a prompt step,
-// library products and activation kernel before, gate/up here after (us, in whole steps): 4B sizes at 250,
-// 600, 1024, 1600, 2048 tokens 195, 262, 352, 482, 567 -> 176, 253, 347, 438, 519; 8B sizes 263, 401, 502, 828,
-// 794 -> 248, 390, 488, 810, 773; 32B sizes at 1024 and 2048 1218, 1829 -> 1138, 1775.  The products without an
-// activation: plan.wide_beats_library.  256 x 256 tiles multiply at 1.45 PFLOP/s (2048 x 2 x 12288 x 4096 in 285
-// us with its activation; with loads and LDS reads left out the loop reaches 1.7).
+// What bounds it.  A 256 x 256 tile is bound by the matrix cores (2048 x 2 x 12288 x 4096 in 279 us with its activation,
+// 1.48 PFLOP/s; with loads and LDS reads left out the loop reaches 1.7).  Smaller tiles are bound by the way from the
+// second-level cache into the unit: its first-level cache has some 115 lines of 128 bytes on their way at any time, whatever
+// is sent, 200 clocks a line that the second level holds, 1,100 to 1,600 one that it does not (2048 x 2560 x 9728 in 128 x 160
+// tiles: 105 us, its loads alone 102, its matrix instructions alone 63, its LDS reads alone 34, its loads from the second
+// level 57).  Pulling lines there ahead of their use, by scalar loads or by other waves' loads, does not help; what does is
+// a large tile (fewer lines a product), and that the tiles a die has at one time share rows (gw_deep: the same product
+// in 111 us with 16 x 2 tiles a die, 101 with 8 x 4).  Hence for a matrix with too few large tiles for the units
+// K cut into ranges (pylon_gemm_wide_parts): that product in two ranges of 256 x 160 tiles 82 us.
+//
+// Which tile: gw_choose, by a model of the launch's rounds over the compute units; a last round that would leave most
+// of them idle is a launch of its own (gw_split).  Gate/up with its activation here, one tile for all (before the
+// tiles of 160 and 192 columns and that) -> now, and the library's product alone, us: 2 x 9728 x 2560 at 520, 1000,
+// 2048 rows 67, 107, 168 -> 56, 90, 157 (61, 104, 189); 2 x 12288 x 4096 at 1000, 2048, 2096 165, 290, 364 -> 149, 279, 322
+// (165, 269, 334); 2 x 25600 x 5120 at 1000, 2048 446, 796 -> 387, 739 (475, 772).  The products without an activation:
+// plan.wide_beats_library, plan.portion_beats_library, and pylon_gemm_wide_parts_plan for those into the residual stream.
 //
 // A kernel's code has to stay small: two compute units share 64 KB of instruction cache.  Results stored with
 // an unrolled fallback for odd widths, software rounding and a peeled first chunk (55 to 87 KB of code instead
@@ -41,10 +51,12 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 #define GW_LDS(T) __attribute__((address_space(3))) T
 #define GW_CHUNK 64
 #define GW_ROW_BYTES 128
-#define GW_PLACES 5  // of the ring of square tiles
+#define GW_X_PLACES 3  // of tiles that keep two and a half chunks
+#define GW_W_PLACES 2
 
 // What happens to the sums: nothing; act(gate) * up of a fused gate/up matrix; max(v, 0)^2.
-enum GwEpilogue { GW_PLAIN = 0, GW_SILU = 1, GW_RELU2 = 2, GW_GELU = 3, GW_CAPPED = 4 };
+// The last one is a part's float sums, unrounded.
+enum GwEpilogue { GW_PLAIN = 0, GW_SILU = 1, GW_RELU2 = 2, GW_GELU = 3, GW_CAPPED = 4, GW_SUMS = 5 };
 
 // A gate of up to GW_EXACT_ROWS rows is expf and a true division, as in the kernels for fewer rows: up to there
 // the activation of a request's tokens has one precision whatever shares its step.  Beyond, where the other
@@ -77,8 +89,11 @@ __device__ __forceinline__ void gw_sync() {
 
 struct GwShape {
   int M, N, K;
+  int m_tiles, n_tiles, deep;  // deep: tile rows that are walked together
   long long ldx, ldw, ldo;
-  int m_tiles, n_tiles;
+  int up_rows;                 // from a gate row of w to its up row
+  int parts;                   // ranges K is cut into, each with float sums of its own, part_apart elements apart
+  long long part_apart;
   float alpha, offset, limit;  // of the capped gate
   int epilogue;
 };
@@ -109,30 +124,38 @@ __device__ __forceinline__ float gw_capped(float g, float u, const GwShape& p) {
 template <int MT, int NT, int STAGES, int GATE>
 __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
                                                const uint16_t* __restrict__ w, const GwShape p) {
-  constexpr bool RING = STAGES == 0, GATED = GATE != GW_NO_GATE, EXACT = GATE == GW_EXACT_GATE;
-  static_assert(!RING || MT == NT, "the ring's places hold x or w");
+  constexpr bool HALVES = STAGES == 0, GATED = GATE != GW_NO_GATE, EXACT = GATE == GW_EXACT_GATE;
   static_assert(!GATED || NT % 2 == 0, "a gate tile and its up tile belong to one wave");
   constexpr int TM = 32 * MT, TN = 32 * NT;
   constexpr int XL = TM / 32, WL = TN / 32, LOADS = XL + WL;  // loads a wave sends per chunk
-  constexpr int STAGE_BYTES = (TM + TN) * GW_ROW_BYTES, PLACE_BYTES = TM * GW_ROW_BYTES;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[RING ? GW_PLACES * PLACE_BYTES : STAGES * STAGE_BYTES];
+  constexpr int STAGE_BYTES = (TM + TN) * GW_ROW_BYTES, X_BYTES = TM * GW_ROW_BYTES, W_BYTES = TN * GW_ROW_BYTES;
+  __shared__ __attribute__((aligned(1024))) unsigned char
+      lds[HALVES ? GW_X_PLACES * X_BYTES + GW_W_PLACES * W_BYTES : STAGES * STAGE_BYTES];
 
-  // Every eighth workgroup runs on one die: a die gets consecutive tiles, rows of tiles fastest, so that
-  // its cache serves most of what its workgroups read.
-  const int tiles = p.m_tiles * p.n_tiles, per_die = (tiles + 7) >> 3;
-  const int id = (blockIdx.x & 7) * per_die + (blockIdx.x >> 3);
-  if (static_cast<int>(blockIdx.x >> 3) >= per_die || id >= tiles) return;
-  constexpr int DEEP = TM >= 256 ? 8 : 16;  // tile rows walked together
-  const int deep_tiles = DEEP * p.n_tiles, stripe = id / deep_tiles, within = id - stripe * deep_tiles;
-  const int deep = p.m_tiles - stripe * DEEP < DEEP ? p.m_tiles - stripe * DEEP : DEEP;
-  const int m0 = (stripe * DEEP + within % deep) * TM, n0 = within / deep * (GATED ? TN / 2 : TN);
+  // Every eighth workgroup runs on one die: a die gets consecutive tiles of one part, `deep` rows of tiles walked
+  // together (gw_deep), so that its cache serves most of what its workgroups read.
+  const int tiles = p.m_tiles * p.n_tiles, all = tiles * p.parts, per_die = (all + 7) >> 3;
+  int id = (blockIdx.x & 7) * per_die + (blockIdx.x >> 3);
+  if (static_cast<int>(blockIdx.x >> 3) >= per_die || id >= all) return;
+  int part = 0;
+  if (p.parts > 1) {
+    part = id / tiles;
+    id -= part * tiles;
+  }
+  const int deep_tiles = p.deep * p.n_tiles, stripe = id / deep_tiles, within = id - stripe * deep_tiles;
+  const int deep = p.m_tiles - stripe * p.deep < p.deep ? p.m_tiles - stripe * p.deep : p.deep;
+  const int m0 = (stripe * p.deep + within % deep) * TM, n0 = within / deep * (GATED ? TN / 2 : TN);
 
   const int lane = threadIdx.x & (PYLON_WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PYLON_WAVE);
   const int r = lane & 15, g = lane >> 4, wm = wave & 1, wn = wave >> 1;
-  const int chunks = p.K / GW_CHUNK;
-  const uint16_t* xt = x + static_cast<size_t>(m0) * p.ldx;
-  const uint16_t* wt = w + static_cast<size_t>(n0) * p.ldw;
+  int chunks = p.K / GW_CHUNK, first = 0;
+  if (p.parts > 1) {
+    first = chunks * part / p.parts;
+    chunks = chunks * (part + 1) / p.parts - first;
+  }
+  const uint16_t* xt = x + static_cast<size_t>(m0) * p.ldx + first * GW_CHUNK;
+  const uint16_t* wt = w + static_cast<size_t>(n0) * p.ldw + first * GW_CHUNK;
 
   // Load i of wave v brings rows 8 (v XL + i) .. + 7 of the tile.  Rows beyond M or N are read as the last
   // one (their results go nowhere).
@@ -148,7 +171,7 @@ __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const
     const int row = 8 * (wave * WL + i) + (lane >> 3);
     int at = GATED ? (row >> 5) * 16 + (row & 15) : row;
     at = n0 + at < p.N ? at : p.N - 1 - n0;
-    if (GATED && (row & 16)) at += p.N;
+    if (GATED && (row & 16)) at += p.up_rows;
     w_at[i] = static_cast<unsigned>(at) * static_cast<unsigned>(p.ldw) * 2u + ((lane & 7) ^ (row & 7)) * 16;
   }
   // Beyond K the descriptor spans nothing and the chunk's offset is zero: the load fetches nothing, whether or
@@ -211,35 +234,33 @@ __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const
     });
   };
 
-  if constexpr (RING) {
-    // x of chunk c lies at place 2 c, w at 2 c + 1 (modulo five).  In flight besides the chunk in use: the
-    // next one and x of the one after it.
-    auto whole = [&](bool is_x, int chunk, int place) __attribute__((always_inline)) {
+  if constexpr (HALVES) {
+    // x has three places, w two.  In flight besides the chunk in use: the next one and x of the one after it.
+    constexpr int W_AT = GW_X_PLACES * X_BYTES;
+    auto whole = [&](bool is_x, int chunk, int at) __attribute__((always_inline)) {
       const __amdgpu_buffer_rsrc_t rows = rows_of(is_x, chunk);
 #pragma unroll
-      for (int i = 0; i < XL; ++i) load(rows, is_x, chunk, place * PLACE_BYTES, i);
+      for (int i = 0; i < (is_x ? XL : WL); ++i) load(rows, is_x, chunk, at, i);
     };
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      whole(true, c, 2 * c);
-      whole(false, c, 2 * c + 1);
+      whole(true, c, c * X_BYTES);
+      whole(false, c, W_AT + c * W_BYTES);
     }
-    gw_sync<2 * XL>();
+    gw_sync<LOADS>();
 #pragma unroll
-    for (int q = 0; q < READS; ++q) read(0, 0, PLACE_BYTES, q);
-    int place = 0;  // of the chunk's x
-    auto at = [&](int d) __attribute__((always_inline)) {
-      const int v = place + d;
-      return (v >= GW_PLACES ? v - GW_PLACES : v) * PLACE_BYTES;
-    };
+    for (int q = 0; q < READS; ++q) read(0, 0, W_AT, q);
+    int x_now = 0, w_now = W_AT;  // of the chunk in use
     for (int c = 0; c < chunks; ++c) {
+      const int x_next = x_now == 2 * X_BYTES ? 0 : x_now + X_BYTES, x_then = x_next == 2 * X_BYTES ? 0 : x_next + X_BYTES;
+      const int w_next = 2 * W_AT + W_BYTES - w_now;
       const __amdgpu_buffer_rsrc_t xr = rows_of(true, c + 2), wr = rows_of(false, c + 2);
-      turn(Int<0>{}, at(0), at(1), Int<XL>{}, Int<PRODUCTS>{},
-           [&](auto I) __attribute__((always_inline)) { load(xr, true, c + 2, at(4), decltype(I)::value); });
+      turn(Int<0>{}, x_now, w_now, Int<XL>{}, Int<PRODUCTS>{},
+           [&](auto I) __attribute__((always_inline)) { load(xr, true, c + 2, x_then, decltype(I)::value); });
       gw_sync<XL>();  // all of the next chunk; x of the one after it is on its way
-      turn(Int<1>{}, at(2), at(3), Int<WL>{}, Int<PRODUCTS / 2>{},
-           [&](auto I) __attribute__((always_inline)) { load(wr, false, c + 2, at(0), decltype(I)::value); });
-      place = place + 2 >= GW_PLACES ? place + 2 - GW_PLACES : place + 2;
+      turn(Int<1>{}, x_next, w_next, Int<WL>{}, Int<PRODUCTS / 2>{},
+           [&](auto I) __attribute__((always_inline)) { load(wr, false, c + 2, w_now, decltype(I)::value); });
+      x_now = x_next, w_now = w_next;
     }
   } else {
     constexpr int HALF = (LOADS + 1) / 2;  // of a chunk's loads, sent per turn
@@ -280,6 +301,21 @@ __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const
   // Loads beyond K fetch nothing but do write (zeros) into LDS: the wave sees them through before it leaves.
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 
+  if constexpr (!GATED) {
+    if (p.epilogue == GW_SUMS) {
+      float* const base = reinterpret_cast<float*>(out) + part * p.part_apart +
+                          static_cast<size_t>(m0 + wm * MT * 16 + r) * p.ldo + n0 + wn * NT * 16 + 4 * g;
+      const int rows = p.M - (m0 + wm * MT * 16 + r), cols = p.N - (n0 + wn * NT * 16 + 4 * g);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        if (16 * t >= rows) break;
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          if (16 * j < cols) *reinterpret_cast<floatx4*>(base + static_cast<size_t>(16 * t) * p.ldo + 16 * j) = acc[j][t];
+      }
+      return;
+    }
+  }
   // acc[j][t][i] is out[16 t + r][16 j + 4 g + i] of the wave's quarter (a pair of column tiles with GATED).
   // N is a multiple of four: a lane's four values are all there or all beyond it.
   auto store = [&](auto value) __attribute__((always_inline)) {
@@ -319,7 +355,7 @@ __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const
 // Two workgroups to a compute unit where their LDS fits.
 template <int MT, int NT, int STAGES>
 constexpr int gw_per_unit() {
-  const int bytes = (STAGES == 0 ? GW_PLACES * 32 * MT : STAGES * 32 * (MT + NT)) * GW_ROW_BYTES;
+  const int bytes = 32 * (STAGES == 0 ? GW_X_PLACES * MT + GW_W_PLACES * NT : STAGES * (MT + NT)) * GW_ROW_BYTES;
   return 2 * bytes <= 160 * 1024 ? 2 : 1;
 }
 
@@ -329,7 +365,7 @@ __global__ __launch_bounds__(256, (gw_per_unit<MT, NT, STAGES>())) void gemm_wid
   gemm_wide_body<MT, NT, STAGES, GATE>(out, x, w, p);
 }
 
-// The tiles: rows, columns, workgroups per compute unit, and what a chunk of 64 of K costs a workgroup in
+// The tiles (the sums depend on none): rows, columns, workgroups per compute unit, and what a chunk of 64 of K costs a workgroup in
 // nanoseconds where the launch's last round leaves it alone on its unit (for one workgroup a unit: leaves
 // units idle) and in full rounds (measured over the layer sizes of 4B to 32B, each launch behind 256 MB of
 // other traffic, as in a step: launched back to back the small tiles look a third faster than they are).
@@ -338,38 +374,74 @@ struct GwTile {
 };
 static const GwTile kTiles[] = {
     {64, 64, 2, 230, 380},      // 2 x 2, five stages
-    {128, 128, 1, 580, 600},    // 4 x 4, four stages
-    {128, 128, 2, 700, 930},    // 4 x 4, the ring
-    {128, 192, 1, 690, 700},    // 4 x 6, three stages
+    {128, 128, 1, 560, 575},    // 4 x 4, four stages
+    {128, 128, 2, 700, 930},    // 4 x 4, two and a half chunks
+    {128, 192, 1, 660, 670},    // 4 x 6, three stages
     {128, 192, 2, 850, 1330},   // 4 x 6, two stages
     {96, 256, 1, 740, 750},     // 3 x 8, three stages
-    {256, 128, 1, 840, 840},    // 8 x 4, three stages
+    {256, 128, 1, 855, 855},    // 8 x 4, three stages
     {128, 256, 1, 860, 870},    // 4 x 8, three stages
-    {160, 256, 1, 920, 970},    // 5 x 8, three stages
-    {256, 256, 1, 1300, 1380},  // 8 x 8, the ring
+    {160, 256, 1, 940, 990},    // 5 x 8, three stages
+    {256, 256, 1, 1300, 1380},  // 8 x 8, two and a half chunks
+    {128, 160, 1, 650, 660},    // 4 x 5, four stages; none of the next two with a gate, whose halves share a wave
+    {256, 160, 1, 940, 950},    // 8 x 5, three stages
+    {256, 192, 1, 1055, 1075},  // 8 x 6, two and a half chunks
+    {192, 256, 1, 1080, 1100},  // 6 x 8, two and a half chunks
 };
 #define GW_ROUND_US 3.5  // of a round: the first chunks' way to LDS, and the results' way out
 static const int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 
-static double gw_time_us(const GwTile& t, int M, int N, int K, bool gated, int units) {
+// A float result of a part leaves late: its bytes, in us a MB.
+#define GW_STORE_US_MB 0.27
+
+static double gw_time_us(const GwTile& t, int M, int N, int K, bool gated, int units, int parts = 1) {
   const int cols = gated ? t.cols / 2 : t.cols;
-  const long long tiles = static_cast<long long>((M + t.rows - 1) / t.rows) * ((N + cols - 1) / cols);
+  const long long tiles = static_cast<long long>((M + t.rows - 1) / t.rows) * ((N + cols - 1) / cols) * parts;
   const long long slots = static_cast<long long>(units) * t.per_unit;
   const long long rounds = tiles / slots, left = tiles - rounds * slots;
-  const double chunks = 1e-3 * (K / GW_CHUNK);
+  const double chunks = 1e-3 * (K / GW_CHUNK) / parts;
   const double last = left == 0 ? 0.0 : chunks * (left <= units ? t.alone_ns : t.full_ns) + GW_ROUND_US;
-  return rounds * (chunks * t.full_ns + GW_ROUND_US) + last;
+  const double stored = parts == 1 ? 0.0 : GW_STORE_US_MB * 4e-6 * parts * M * N / (rounds + (left > 0));
+  return rounds * (chunks * t.full_ns + GW_ROUND_US) + last + stored;
 }
 
-static int gw_choose(int M, int N, int K, bool gated, int units) {
+static bool gw_takes(const GwTile& t, int M, bool gated) {
+  return !gated || (t.cols % 64 == 0 && (M > GW_EXACT_ROWS || t.rows <= GW_EXACT_ROWS));
+}
+
+static int gw_choose(int M, int N, int K, bool gated, int units, double* us = nullptr) {
   int best = 0;
   double least = 1e30;
   for (int i = 0; i < kTileCount; ++i) {
-    if (gated && M <= GW_EXACT_ROWS && kTiles[i].rows > GW_EXACT_ROWS) continue;  // these have no exact gate
-    const double us = gw_time_us(kTiles[i], M, N, K, gated, units);
-    if (us < least) least = us, best = i;
+    if (!gw_takes(kTiles[i], M, gated)) continue;
+    const double now = gw_time_us(kTiles[i], M, N, K, gated, units);
+    if (now < least) least = now, best = i;
   }
+  if (us) *us = least;
   return best;
+}
+
+// A last round that leaves most units idle: the whole rounds of one tile in a launch of their own and the columns that are
+// left in a launch of the tile that suits them, where both are quicker than one launch (`us`).  Columns of the first
+// launch, 0 for one launch.
+#define GW_SECOND_US 2.5
+static int gw_split(int M, int N, int K, bool gated, int units, double us, int* first, int* rest) {
+  int ahead = 0;
+  if (M <= 4 * GW_EXACT_ROWS) return 0;
+  for (int i = 0; i < kTileCount; ++i) {
+    const GwTile& t = kTiles[i];
+    if (!gw_takes(t, M, gated)) continue;
+    const int cols = gated ? t.cols / 2 : t.cols, m_tiles = (M + t.rows - 1) / t.rows;
+    const long long slots = static_cast<long long>(units) * t.per_unit;
+    const long long rounds = static_cast<long long>(m_tiles) * (N / cols) / slots;
+    const long long n = rounds * slots / m_tiles * cols;
+    if (rounds == 0 || n >= N) continue;
+    double left;
+    const int other = gw_choose(M, N - static_cast<int>(n), K, gated, units, &left);
+    const double now = gw_time_us(t, M, static_cast<int>(n), K, gated, units) + left + GW_SECOND_US;
+    if (now < us) us = now, ahead = static_cast<int>(n), *first = i, *rest = other;
+  }
+  return ahead;
 }
 
 // The tile that pylon_gemm_wide takes for a product of these sizes (units 0: the current device's), and in
@@ -378,17 +450,60 @@ extern "C" int pylon_gemm_wide_plan(int M, int N, int K, int gated, int units, i
   PYLON_REQUIRE(tile != nullptr && us != nullptr && M >= 1 && N >= 1 && K >= GW_CHUNK, "gemm_wide_plan: bad arguments");
   if (units <= 0) units = pylon_compute_units();
   PYLON_REQUIRE(units > 0, "gemm_wide_plan: no device to take the number of compute units from");
-  *tile = gw_choose(M, N, K, gated != 0, units);
-  *us = static_cast<float>(gw_time_us(kTiles[*tile], M, N, K, gated != 0, units));
+  double least;
+  *tile = gw_choose(M, N, K, gated != 0, units, &least);
+  *us = static_cast<float>(least);
   return 0;
+}
+
+// Ranges of K for a product into the residual stream, with the tile, or one range and tile -1 (pylon_gemm_wide): the
+// quickest with what the residual norm pays for reading float sums of every range instead of one bfloat16 result.
+#define GW_ADD_US_MB 0.2
+#define GW_MOST_PARTS 4
+#define GW_LEAST_CHUNKS 8  // of a range
+extern "C" int pylon_gemm_wide_parts_plan(int M, int N, int K, int units, int* parts, int* tile, float* us) {
+  PYLON_REQUIRE(parts && tile && us && M >= 1 && N >= 1 && K >= GW_CHUNK, "gemm_wide_parts_plan: bad arguments");
+  if (units <= 0) units = pylon_compute_units();
+  PYLON_REQUIRE(units > 0, "gemm_wide_parts_plan: no device to take the number of compute units from");
+  double least;
+  gw_choose(M, N, K, false, units, &least);
+  int first, rest;
+  if (const int ahead = gw_split(M, N, K, false, units, least, &first, &rest)) {
+    double left;
+    gw_choose(M, N - ahead, K, false, units, &left);
+    least = gw_time_us(kTiles[first], M, ahead, K, false, units) + left + GW_SECOND_US;
+  }
+  *parts = 1, *tile = -1;
+  for (int n = 2; n <= GW_MOST_PARTS && n * GW_LEAST_CHUNKS <= K / GW_CHUNK; ++n)
+    for (int i = 0; i < kTileCount; ++i) {
+      const double now = gw_time_us(kTiles[i], M, N, K, false, units, n) + GW_ADD_US_MB * 1e-6 * (4 * n - 2) * M * N;
+      if (now < least) least = now, *parts = n, *tile = i;
+    }
+  *us = static_cast<float>(least);
+  return 0;
+}
+
+// Rows of tiles that a die walks together, of stripes of one depth: those with which the tiles that its units hold at
+// one time need the fewest rows of x and w.
+static int gw_deep(int m_tiles, int n_tiles, int rows, int cols, int held) {
+  int best = 1;
+  long long least = -1;
+  for (int stripes = 1; stripes <= m_tiles; ++stripes) {
+    const int deep = (m_tiles + stripes - 1) / stripes, down = deep < held ? deep : held;
+    const long long across = held <= deep ? 16 : 16ll * held / deep;  // sixteenths of a tile
+    const long long need = 16ll * down * rows + (across < 16ll * n_tiles ? across : 16ll * n_tiles) * cols;
+    if (least < 0 || need < least) least = need, best = deep;
+  }
+  return best;
 }
 
 template <int MT, int NT, int STAGES>
 static void launch_wide(void* out, const void* x, const void* w, GwShape p, hipStream_t stream) {
-  const bool gated = p.epilogue != GW_PLAIN && p.epilogue != GW_RELU2;
+  const bool gated = p.epilogue != GW_PLAIN && p.epilogue != GW_RELU2 && p.epilogue != GW_SUMS;
   const int cols = gated ? 16 * NT : 32 * NT;
   p.m_tiles = (p.M + 32 * MT - 1) / (32 * MT), p.n_tiles = (p.N + cols - 1) / cols;
-  const dim3 grid((static_cast<unsigned>(p.m_tiles) * p.n_tiles + 7) / 8 * 8), block(256);
+  p.deep = gw_deep(p.m_tiles, p.n_tiles, 32 * MT, 32 * NT, 32 * gw_per_unit<MT, NT, STAGES>());
+  const dim3 grid((static_cast<unsigned>(p.m_tiles) * p.n_tiles * p.parts + 7) / 8 * 8), block(256);
 #define GO(GATE)                                                                                                     \
   hipLaunchKernelGGL((gemm_wide_kernel<MT, NT, STAGES, GATE>), grid, block, 0, stream, (uint16_t*)out, (const uint16_t*)x, \
                      (const uint16_t*)w, p)
@@ -396,14 +511,35 @@ static void launch_wide(void* out, const void* x, const void* w, GwShape p, hipS
     GO(GW_NO_GATE);
     return;
   }
-  if constexpr (32 * MT <= GW_EXACT_ROWS) {
-    if (p.M <= GW_EXACT_ROWS) {
-      GO(GW_EXACT_GATE);
-      return;
+  if constexpr (NT % 2 == 0) {
+    if constexpr (32 * MT <= GW_EXACT_ROWS) {
+      if (p.M <= GW_EXACT_ROWS) {
+        GO(GW_EXACT_GATE);
+        return;
+      }
     }
+    GO(GW_FAST_GATE);
   }
-  GO(GW_FAST_GATE);
 #undef GO
+}
+
+static void gw_launch(int tile, void* out, const void* x, const void* w, const GwShape& p, hipStream_t stream) {
+  switch (tile) {
+    case 0: launch_wide<2, 2, 5>(out, x, w, p, stream); break;
+    case 1: launch_wide<4, 4, 4>(out, x, w, p, stream); break;
+    case 2: launch_wide<4, 4, 0>(out, x, w, p, stream); break;
+    case 3: launch_wide<4, 6, 3>(out, x, w, p, stream); break;
+    case 4: launch_wide<4, 6, 2>(out, x, w, p, stream); break;
+    case 5: launch_wide<3, 8, 3>(out, x, w, p, stream); break;
+    case 6: launch_wide<8, 4, 3>(out, x, w, p, stream); break;
+    case 7: launch_wide<4, 8, 3>(out, x, w, p, stream); break;
+    case 8: launch_wide<5, 8, 3>(out, x, w, p, stream); break;
+    case 9: launch_wide<8, 8, 0>(out, x, w, p, stream); break;
+    case 10: launch_wide<4, 5, 4>(out, x, w, p, stream); break;
+    case 11: launch_wide<8, 5, 3>(out, x, w, p, stream); break;
+    case 12: launch_wide<8, 6, 0>(out, x, w, p, stream); break;
+    default: launch_wide<6, 8, 0>(out, x, w, p, stream); break;
+  }
 }
 
 // x: [M, ldx] bf16; w: [N, ldw] bf16, or with a gate [2 N, ldw], gate rows first; out: [M, ldo] bf16, rounded
@@ -425,27 +561,49 @@ extern "C" int pylon_gemm_wide(void* out, const void* x, const void* w, int M, i
   PYLON_REQUIRE(N % 4 == 0 && ldo % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0,
                 "gemm_wide: rows of the result are multiples of 4 elements at 8-byte aligned addresses");
   PYLON_REQUIRE(tile >= -1 && tile < kTileCount, "gemm_wide: there is no tile %d", tile);
-  PYLON_REQUIRE(tile < 0 || !gated || M > GW_EXACT_ROWS || kTiles[tile].rows <= GW_EXACT_ROWS,
-                "gemm_wide: a gate of up to %d rows takes a tile of up to as many rows", GW_EXACT_ROWS);
+  PYLON_REQUIRE(tile < 0 || gw_takes(kTiles[tile], M, gated),
+                "gemm_wide: a gate takes no tile of %d columns, and up to %d rows one of up to as many rows", kTiles[tile].cols,
+                GW_EXACT_ROWS);
   PYLON_REQUIRE(static_cast<long long>((M + 63) / 64) * ((N + 31) / 32) < (1ll << 30), "gemm_wide: too many tiles for one launch");
   if (M == 0) return 0;
+  int ahead = 0;  // columns of a launch of its own
   if (tile < 0) {
     const int units = pylon_compute_units();
     PYLON_REQUIRE(units > 0, "gemm_wide: the device's number of compute units is unknown");
-    tile = gw_choose(M, N, K, gated, units);
+    double us;
+    tile = gw_choose(M, N, K, gated, units, &us);
+    int first, rest;
+    ahead = gw_split(M, N, K, gated, units, us, &first, &rest);
+    if (ahead > 0) {
+      gw_launch(first, out, x, w, GwShape{M, ahead, K, 0, 0, 0, ldx, ldw, ldo, N, 1, 0, alpha, offset, limit, epilogue}, stream);
+      tile = rest;
+    }
   }
-  const GwShape p{M, N, K, ldx, ldw, ldo, 0, 0, alpha, offset, limit, epilogue};
-  switch (tile) {
-    case 0: launch_wide<2, 2, 5>(out, x, w, p, stream); break;
-    case 1: launch_wide<4, 4, 4>(out, x, w, p, stream); break;
-    case 2: launch_wide<4, 4, 0>(out, x, w, p, stream); break;
-    case 3: launch_wide<4, 6, 3>(out, x, w, p, stream); break;
-    case 4: launch_wide<4, 6, 2>(out, x, w, p, stream); break;
-    case 5: launch_wide<3, 8, 3>(out, x, w, p, stream); break;
-    case 6: launch_wide<8, 4, 3>(out, x, w, p, stream); break;
-    case 7: launch_wide<4, 8, 3>(out, x, w, p, stream); break;
-    case 8: launch_wide<5, 8, 3>(out, x, w, p, stream); break;
-    default: launch_wide<8, 8, 0>(out, x, w, p, stream); break;
-  }
+  gw_launch(tile, static_cast<uint16_t*>(out) + ahead, x, static_cast<const uint16_t*>(w) + ahead * ldw,
+            GwShape{M, N - ahead, K, 0, 0, 0, ldx, ldw, ldo, N, 1, 0, alpha, offset, limit, epilogue}, stream);
   PYLON_LAUNCHED("gemm_wide");
+}
+
+// Float sums of `parts` ranges of K, each of them unrounded, for a consumer to add in order: out [parts][M][N] float.
+// tile: as pylon_gemm_wide_parts_plan says; -1 with one part for the rule of pylon_gemm_wide.
+extern "C" int pylon_gemm_wide_parts(float* out, const void* x, const void* w, int M, int N, int K, long long ldx,
+                                     long long ldw, int parts, int tile, hipStream_t stream) {
+  PYLON_REQUIRE(M >= 0 && N > 0 && K > 0 && K % GW_CHUNK == 0 && N % 4 == 0, "gemm_wide_parts: bad sizes M=%d N=%d K=%d", M, N, K);
+  PYLON_REQUIRE(parts >= 1 && parts <= 8 && parts <= K / GW_CHUNK, "gemm_wide_parts: cannot cut %d into %d parts", K, parts);
+  PYLON_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0, "gemm_wide_parts: bad row strides");
+  PYLON_REQUIRE((reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
+                    (reinterpret_cast<uintptr_t>(out) & 15) == 0, "gemm_wide_parts: operands must be 16-byte aligned");
+  PYLON_REQUIRE(ldx * 512 < (1ll << 31) && 256 * ldw * 2 < (1ll << 31),
+                "gemm_wide_parts: the rows of a tile are beyond the 2 GB that one view of them may span");
+  PYLON_REQUIRE(tile >= (parts == 1 ? -1 : 0) && tile < kTileCount, "gemm_wide_parts: there is no tile %d", tile);
+  PYLON_REQUIRE(static_cast<long long>((M + 63) / 64) * ((N + 31) / 32) < (1ll << 27), "gemm_wide_parts: too many tiles for one launch");
+  if (M == 0) return 0;
+  if (tile < 0) {
+    const int units = pylon_compute_units();
+    PYLON_REQUIRE(units > 0, "gemm_wide_parts: the device's number of compute units is unknown");
+    tile = gw_choose(M, N, K, false, units);
+  }
+  gw_launch(tile, out, x, w,
+            GwShape{M, N, K, 0, 0, 0, ldx, ldw, N, N, parts, static_cast<long long>(M) * N, 0.f, 0.f, 0.f, GW_SUMS}, stream);
+  PYLON_LAUNCHED("gemm_wide_parts");
 }

@@ -15,6 +15,7 @@ int pylon_gemm_rows(void*, int, const void*, const void*, int, int, int, long lo
                     int, int, int, float, float, float, hipStream_t);
 int pylon_gemm_wide(void*, const void*, const void*, int, int, int, long long, long long, long long, int, float, float, float,
                     int, hipStream_t);
+int pylon_gemm_wide_parts(float*, const void*, const void*, int, int, int, long long, long long, int, int, hipStream_t);
 int pylon_qkv_prepare(void*, void*, void*, const void*, int, long long, const float*, const float*, float, const float*, int,
                       const int*, const int*, int, int, int, int, int, hipStream_t);
 int pylon_attention_prefill(void*, const void*, const void*, const void*, const int*, int, const int*, int, int, int, int, int,
@@ -26,7 +27,8 @@ enum {
   LR_NORM1, LR_QKV, LR_LD_QKV, LR_Q_NORM, LR_K_NORM, LR_INV_FREQ, LR_K_CACHE, LR_V_CACHE, LR_SLOT_MAP, LR_TABLE,
   LR_TABLE_WIDTH, LR_OUT, LR_LD_OUT, LR_NORM2, LR_GATE_UP, LR_LD_GATE_UP, LR_DOWN, LR_LD_DOWN, LR_LAYER_FIELDS
 };
-// Of the step.  A product is two numbers: 0 for gemm_wide, else the ranges that gemm_rows cuts K into, and its col_tiles.
+// Of the step.  A product is two numbers: 0 for gemm_wide, else the ranges that K is cut into and gemm_rows' col_tiles, or,
+// for gemm_wide_parts, -1 less its tile.
 enum {
   LR_TOKENS, LR_WIDTH, LR_HEADS, LR_KV_HEADS, LR_HEAD_DIM, LR_ROT_DIM, LR_PAGE, LR_FF, LR_GELU, LR_MASK, LR_POSITIONS,
   LR_TILES, LR_N_TILES, LR_TILE_ROWS, LR_RESID, LR_NORMED, LR_PROJECTED, LR_Q, LR_CONTEXT, LR_OUT_SUM, LR_HIDDEN,
@@ -62,6 +64,9 @@ extern "C" int pylon_layer_run(const long long* layers, int n_layers, int pendin
     if (parts == 0)
       return pylon_gemm_wide(at(out), at(x), at(w), tokens, n, k, k, ldw, n, gated ? (step[LR_GELU] ? 3 : 1) : 0, 0.f, 0.f, 0.f,
                              -1, stream);
+    if (col_tiles < 0)
+      return pylon_gemm_wide_parts(static_cast<float*>(at(out)), at(x), at(w), tokens, n, k, k, ldw, static_cast<int>(parts),
+                                   static_cast<int>(-1 - col_tiles), stream);
     return pylon_gemm_rows(at(out), sums ? PYLON_F32 : PYLON_BF16, at(x), at(w), tokens, n, k, k, ldw, n, static_cast<int>(parts),
                            static_cast<long long>(tokens) * n, static_cast<int>(col_tiles),
                            gated ? (step[LR_GELU] ? 3 : 1) : 0, 0, 0, 0.f, 0.f, 0.f, stream);

@@ -66,6 +66,14 @@ def _residual(rows: int, n: int, k: int, stride: int, units: int) -> Optional[Tu
     return _projection(rows, n, k, stride, units) if rows > plan.STREAM_ROWS else None
 
 
+def _into_residual(rows: int, n: int, k: int, stride: int, units: int) -> Optional[Tuple[int, int]]:
+    """The same of :func:`ops.linear_into_residual`; (parts, -1 - tile) for :func:`ops.gemm_wide_parts`."""
+    if rows > plan.SPLIT_ROWS and ops.wide_sizes_ok(rows, n, k, k, stride):
+        parts, tile = ops.wide_parts(rows, n, k, units)
+        return (parts, -1 - tile) if parts > 1 else (0, 0)
+    return _residual(rows, n, k, stride, units)
+
+
 def _gated(rows: int, n: int, k: int, stride: int) -> Optional[Tuple[int, int]]:
     """The same of :func:`ops.linear_glu`."""
     if rows > plan.STREAM_ROWS:
@@ -79,7 +87,8 @@ def _gated(rows: int, n: int, k: int, stride: int) -> Optional[Tuple[int, int]]:
 def _products(rows: int, units: int, qkv, out, gate_up, down) -> Optional[tuple]:
     """What the four products of a layer are, each matrix given as (rows, columns, row stride); None where one of them is
     not the engine's own."""
-    found = (_projection(rows, *qkv, units), _residual(rows, *out, units), _gated(rows, *gate_up), _residual(rows, *down, units))
+    found = (_projection(rows, *qkv, units), _into_residual(rows, *out, units), _gated(rows, *gate_up),
+             _into_residual(rows, *down, units))
     return None if None in found else tuple(number for product in found for number in product)
 
 

@@ -6,6 +6,7 @@ it launches, and launches on torch's current stream.  None has a CPU path.
 from __future__ import annotations
 
 import functools
+from ctypes import byref, c_float, c_int
 from typing import Optional, Tuple
 
 import torch
@@ -1522,6 +1523,36 @@ def gemm_wide(x: torch.Tensor, weight: torch.Tensor, *, epilogue: str = "none", 
     return out
 
 
+def gemm_wide_parts(x: torch.Tensor, weight: torch.Tensor, *, parts: int, tile: int = -1) -> torch.Tensor:
+    """Float32 sums of ``x @ weight.T`` for many rows of bfloat16 ``x``: partial results ``[parts, M, N]`` of as many
+    ranges of K for the consumer to add in order, or ``[M, N]`` of the whole product.  ``tile``: as
+    :func:`wide_parts` says."""
+    if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
+        raise KernelError(f"gemm_wide_parts: cannot multiply {tuple(x.shape)} by the transpose of {tuple(weight.shape)}")
+    if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+        raise KernelError("gemm_wide_parts takes bfloat16 operands")
+    if not (x.is_cuda and weight.is_cuda) or x.stride(1) != 1 or weight.stride(1) != 1:
+        raise KernelError("gemm_wide_parts: operands must be on the GPU with contiguous rows")
+    if not _here(x, weight):
+        raise KernelError("gemm_wide_parts: operands must be on the current device")
+    m, k = x.shape
+    n = weight.shape[0]
+    out = torch.empty((parts, m, n) if parts > 1 else (m, n), dtype=torch.float32, device=x.device)
+    _lib.call("pylon_gemm_wide_parts", out.data_ptr(), x.data_ptr(), weight.data_ptr(), m, n, k, x.stride(0),
+              weight.stride(0), int(parts), int(tile), _stream())
+    return out
+
+
+@functools.lru_cache(maxsize=4096)  # asked for every product of a step
+def wide_parts(rows: int, n: int, k: int, units: int) -> Tuple[int, int]:
+    """(ranges that K is cut into, tile) of a product into the residual stream of more than
+    :data:`SPLIT_ROWS` rows: the quickest by the kernel's model of a launch, with what the consumer pays for adding
+    the ranges' sums; (1, -1): one bfloat16 result of :func:`gemm_wide`."""
+    parts, tile, us = c_int(), c_int(), c_float()
+    _lib.call("pylon_gemm_wide_parts_plan", rows, n, k, units, byref(parts), byref(tile), byref(us))
+    return parts.value, tile.value
+
+
 def _library_float(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``x @ weight.T`` of bfloat16 operands as float32: the library's product with a float32
     result, that is its float32 sums before any rounding."""
@@ -1602,6 +1633,31 @@ def linear_for_residual(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: tor
         if choice.kernel == "skinny":
             return gemm_skinny(x, weight, out_dtype=torch.float32, parts=choice.parts)
         return _library_float(x, weight)
+    return linear(x, weight, out_dtype=out_dtype)
+
+
+def linear_into_residual(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype) -> torch.Tensor:
+    """:func:`linear_for_residual`, but a prompt portion's product (more than :data:`SPLIT_ROWS` rows) is the tiled
+    kernel's wherever that takes it, with K cut into ranges where the uncut launch has fewer tiles than the device has
+    units, or small ones (:func:`wide_parts`): then float32 partial sums ``[parts, M, N]``, which the consumer adds.
+    (2560 x 9728 at 192, 640, 1200 and 2048 rows, with the norm's reading of the parts: 25, 42, 61 and 88 us, where
+    the uncut kernel or the library took 42, 61, 87 and 105; 5120 x 25600 at 256, 640 and 1500: 93, 149 and 283
+    against 265, 240 and 341.)  With a float32 ``out_dtype`` the sums come unrounded also where K is not cut."""
+    if (x.dim() == 2 and x.shape[0] > SPLIT_ROWS and out_dtype in (torch.bfloat16, torch.float32) and not _watched(x, weight)
+            and _wide_ok(x, weight)):
+        parts, tile = wide_parts(x.shape[0], *weight.shape, _lib.compute_units())
+        if parts > 1 or out_dtype == torch.float32:
+            return gemm_wide_parts(x, weight, parts=parts, tile=tile)
+        return gemm_wide(x, weight)
+    return linear_for_residual(x, weight, out_dtype=out_dtype)
+
+
+def linear_of_portion(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype) -> torch.Tensor:
+    """:func:`linear`, but a long portion's product with a bfloat16 result goes to the tiled kernel also where
+    :func:`plan.portion_beats_library` says so."""
+    if (out_dtype == torch.bfloat16 and x.dim() == 2 and x.shape[0] > plan.PORTION_ROWS
+            and plan.portion_beats_library(x.shape[0], *weight.shape) and not _watched(x, weight) and _wide_ok(x, weight)):
+        return gemm_wide(x, weight)
     return linear(x, weight, out_dtype=out_dtype)
 
 

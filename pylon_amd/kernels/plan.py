@@ -239,6 +239,23 @@ def wide_beats_library(rows: int, n: int, k: int, units: int = UNITS) -> bool:
     return rows <= 1700 or n <= 4096
 
 
+PORTION_ROWS = 512  # a long portion has more rows
+
+
+def portion_beats_library(rows: int, n: int, k: int) -> bool:
+    """Whether a portion's projection (q/k/v and the like) of more than :data:`PORTION_ROWS` rows takes the tiled
+    kernel, with its tiles of 160 and 192 columns and its whole rounds in a launch of their own, whatever
+    :func:`wide_beats_library` says of the tiles before those: everywhere but where 256 x 256 tiles fill five sixths of
+    their rounds and K is short, which is where the library has its best main loop.  us, here against the library:
+    6144 x 2560 at 1000, 1400 and 2048 rows 37 and 40, 46 and 54, 52 and 56; 6144 x 4096 at 2048 77 and 80; 10240 x 5120 at
+    1000 and 2048 86 and 95, 166 and 181; but 7168 x 4096 at 1800 and 2048 (224 tiles) 1.15 and 1.12 of the library's time,
+    6144 x 4096 at 2056 (216) 90 and 81, 8192 x 4096 at 2048 (256) 1.08; 16384 x 4096 at 2048 (512) 1.14; of rows of
+    5120 all but two of 88 products are within 3 % or quicker here."""
+    tiles = -(-rows // 256) * -(-n // 256)
+    full = 6 * tiles >= 5 * 256 * -(-tiles // 256)
+    return rows > PORTION_ROWS and n < TALL and not (full and k < 5120)
+
+
 def wide_gated_beats_library(rows: int, n_half: int) -> bool:
     """The same for gate/up, whose activation the own kernel has in its epilogue: everywhere
     but for very wide matrices where a third tile of 160 rows is begun and the library's two of 192 hold them

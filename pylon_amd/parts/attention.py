@@ -138,9 +138,9 @@ class Attention(Part):
                 slot_map=cache.slot_map if stores else None,
                 page_size=cache.page_size, window=spec.window, scale=spec.scale, n_splits=splits, n_cuts=cuts,
             )
-            return ops.linear_for_residual(context.view(tokens, spec.q_size), self.params["out"],
+            return ops.linear_into_residual(context.view(tokens, spec.q_size), self.params["out"],
                                            out_dtype=self.dtype)
-        qkv = ops.linear(h, weight, out_dtype=self.dtype)
+        qkv = ops.linear_of_portion(h, weight, out_dtype=self.dtype)
         q = torch.empty((tokens, spec.n_heads, spec.head_dim), dtype=self.dtype, device=h.device)
         on_cores = self._sink_kernel(cache.page_size) if cache.k is not None else False
         v_cache = cache.v
@@ -223,7 +223,7 @@ class Attention(Part):
         if spec.output_gate is not None:
             ops.sigmoid_gate_(context, qkv[:, self.gate_off: self.gate_off + spec.gate_size],
                               per=spec.value_dim if spec.output_gate == "head" else 1)
-        return ops.linear_for_residual(context, self.params["out"], out_dtype=self.dtype)
+        return ops.linear_into_residual(context, self.params["out"], out_dtype=self.dtype)
 
 
 def distance_buckets(rows: int, far: float) -> list:
@@ -346,7 +346,7 @@ class SinkAttention(Part):
                                      q_size=self.q_size, k_size=self.k_size, v_size=self.v_size, out_dtype=self.dtype,
                                      store=stores, v_transposed=True)
         else:
-            qkv = ops.linear(h, weight, out_dtype=self.dtype)
+            qkv = ops.linear_of_portion(h, weight, out_dtype=self.dtype)
             if stores:
                 ops.kv_store(qkv, cache.k, v_cache, cache.slot_map, k_off=self.q_size,
                              v_off=self.q_size + self.k_size, v_transposed=True)
@@ -374,7 +374,7 @@ class SinkAttention(Part):
                 q, cache.k, v_cache, cache.block_table, ctx.tok_row, ctx.positions, page_size=page_size,
                 scale=spec.scale, log_bias=self.params["log_bias"].view(2, spec.n_heads), sink=spec.sink,
                 v_transposed=True, **mask)
-        return ops.linear_for_residual(context.view(tokens, spec.n_heads * spec.v_head_dim), self.params["out"],
+        return ops.linear_into_residual(context.view(tokens, spec.n_heads * spec.v_head_dim), self.params["out"],
                                        out_dtype=self.dtype)
 
 

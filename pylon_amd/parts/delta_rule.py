@@ -71,7 +71,7 @@ class GatedDeltaRule(Part):
             dim=spec.head_dim, vdim=spec.v_head_dim, gate_off=self.gate_off, beta_off=self.beta_off,
             decay_off=self.decay_off, eps=spec.norm_eps, unit_eps=spec.unit_eps, q_scale=spec.head_dim ** -0.5,
             out_dtype=self.dtype, max_count=ctx.max_count)
-        return ops.linear_for_residual(mixed, self.params["out"], out_dtype=self.dtype)
+        return ops.linear_into_residual(mixed, self.params["out"], out_dtype=self.dtype)
 
 
 register_part("mixer", "delta_rule", GatedDeltaRule, replace=True)

@@ -38,11 +38,11 @@ class GatedFeedForward(Part):
     def forward(self, h: torch.Tensor, ctx) -> torch.Tensor:
         if not self.spec.bias:
             hidden = ops.linear_glu(h, self.params["gate_up"], out_dtype=self.dtype, act=self.spec.activation)
-            return ops.linear_for_residual(hidden, self.params["down"], out_dtype=self.dtype)
+            return ops.linear_into_residual(hidden, self.params["down"], out_dtype=self.dtype)
         sums = ops.linear(h, self.params["gate_up"], out_dtype=torch.float32)
         hidden = ops.gated_act(sums, alpha=1.0, offset=0.0, limit=0.0, out_dtype=self.dtype,
                                bias=self.params["gate_up_bias"])
-        out = ops.linear_for_residual(hidden, self.params["down"], out_dtype=self.dtype)
+        out = ops.linear_into_residual(hidden, self.params["down"], out_dtype=self.dtype)
         if self.defer_output_bias:
             return out
         if out.dim() == 3:  # partial sums: the bias joins the first
@@ -69,7 +69,7 @@ class CappedGatedFeedForward(Part):
         spec = self.spec
         hidden = ops.linear_capped(h, self.params["gate_up"], alpha=spec.alpha, offset=spec.offset, limit=spec.limit,
                                    out_dtype=self.dtype)
-        return ops.linear_for_residual(hidden, self.params["down"], out_dtype=self.dtype)
+        return ops.linear_into_residual(hidden, self.params["down"], out_dtype=self.dtype)
 
 
 class PlainFeedForward(Part):
@@ -87,7 +87,7 @@ class PlainFeedForward(Part):
 
     def forward(self, h: torch.Tensor, ctx) -> torch.Tensor:
         hidden = ops.linear_relu2(h, self.params["up"], out_dtype=self.dtype)
-        return ops.linear_for_residual(hidden, self.params["down"], out_dtype=self.dtype)
+        return ops.linear_into_residual(hidden, self.params["down"], out_dtype=self.dtype)
 
 
 register_part("feed_forward", "plain_mlp", PlainFeedForward, replace=True)

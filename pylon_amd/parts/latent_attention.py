@@ -163,11 +163,11 @@ class LatentAttention(Part):
                 down, cache.k if stores else None, cache.slot_map if stores else None, q_rank=spec.q_rank,
                 kv_rank=rank, n_gate=self.n_gate, q_weight=self.params["q_norm"], c_weight=self.params["c_norm"],
                 eps=spec.norm_eps, out_dtype=self.dtype)
-            q = ops.linear(q_latent, self.params["uq"], out_dtype=self.dtype)
+            q = ops.linear_of_portion(q_latent, self.params["uq"], out_dtype=self.dtype)
             q = self._into_latent(q.view(tokens, heads, spec.head_dim))
         mixed = self._attend(q, ctx, cache)
         context = self._into_values(mixed, **gating)
-        return ops.linear_for_residual(context.view(tokens, heads * spec.v_head_dim), self.params["out"],
+        return ops.linear_into_residual(context.view(tokens, heads * spec.v_head_dim), self.params["out"],
                                        out_dtype=self.dtype)
 
     def _queries(self, h: torch.Tensor, ctx, cache, stores: bool):
@@ -175,7 +175,7 @@ class LatentAttention(Part):
         None)`` of queries that come straight from the input; the tokens' rows go into the cache."""
         spec = self.spec
         tokens, heads, rank = h.shape[0], spec.n_heads, spec.kv_rank
-        proj = ops.linear(h, self.params["down"], out_dtype=self.dtype)
+        proj = ops.linear_of_portion(h, self.params["down"], out_dtype=self.dtype)
         q = torch.empty((tokens, heads, self.width), dtype=self.dtype, device=h.device)
         rotary = self.position.rotary() if self.position is not None else None
         ops.latent_rotate(

@@ -44,7 +44,7 @@ class LightningAttention(Part):
         spec = self.spec
         if not stores:
             raise ValueError("a lightning attention layer cannot borrow another run's state")
-        proj = ops.linear(h, self.params["qkvg"], out_dtype=self.dtype)
+        proj = ops.linear_of_portion(h, self.params["qkvg"], out_dtype=self.dtype)
         # prompt portions of a bfloat16 model run 32 tokens at a time on the matrix cores; steps of
         # single tokens, float32 models and odd head sizes token by token
         chunked = (not ctx.decode_only and ctx.max_count >= CHUNKED_FROM and ops.retention_chunked_ok(
@@ -54,7 +54,7 @@ class LightningAttention(Part):
             heads=spec.n_heads, dim=spec.head_dim, vdim=spec.v_head_dim, rot_dims=0, eps=spec.norm_eps, k_scale=1.0,
             chunked=chunked, max_count=ctx.max_count, form="lightning")
         mixed = ops.norm_gate(mixed, self.params["norm"], proj[:, self.gate_off:], spec.norm_eps)
-        return ops.linear_for_residual(mixed, self.params["out"], out_dtype=self.dtype)
+        return ops.linear_into_residual(mixed, self.params["out"], out_dtype=self.dtype)
 
 
 register_part("mixer", "lightning_attention", LightningAttention, replace=True)

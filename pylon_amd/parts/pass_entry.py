@@ -30,7 +30,7 @@ class JoinEmbedding(Part):
         elif delta is not None and not isinstance(delta, torch.Tensor):
             delta = summed(delta)
         joined = ops.pass_join(resid, delta, embedded, self.dtype, factor=factor)
-        product = ops.linear_for_residual(joined, self.params["join"], out_dtype=torch.float32)
+        product = ops.linear_into_residual(joined, self.params["join"], out_dtype=torch.float32)
         return ops.pass_begin(resid, product, self.params["step"][t]), None
 
 

@@ -47,7 +47,7 @@ class Retention(Part):
         if not stores:
             raise ValueError("a retention layer cannot borrow another run's state")
         rotary = self.position.rotary()
-        proj = ops.linear(h, self.params["qkvg"], out_dtype=self.dtype)
+        proj = ops.linear_of_portion(h, self.params["qkvg"], out_dtype=self.dtype)
         rot_dims = rotary[1] if rotary else 0
         # prompt portions of a bfloat16 model run 32 tokens at a time on the matrix cores; steps of
         # single tokens, float32 models and odd head sizes token by token
@@ -58,7 +58,7 @@ class Retention(Part):
             ctx.row_slots, rows=ctx.rows, heads=spec.n_heads, dim=spec.head_dim, vdim=spec.v_head_dim,
             rot_dims=rot_dims, eps=spec.norm_eps, k_scale=spec.head_dim ** -0.5, chunked=chunked,
             max_count=ctx.max_count)
-        return ops.linear_for_residual(mixed, self.params["out"], out_dtype=self.dtype)
+        return ops.linear_into_residual(mixed, self.params["out"], out_dtype=self.dtype)
 
 
 register_part("mixer", "retention", Retention, replace=True)

@@ -1,0 +1,99 @@
+"""Products of prompt portions with K cut into ranges, and projections of long portions: the rules, and what the parts'
+entry points launch for them."""
+import warnings
+
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+
+from pylon_amd.engine import layer_run
+from pylon_amd.kernels import ops, plan
+
+
+@pytest.mark.parametrize("rows", [129, 300, 512, 513, 640, 1024, 1500, 2048, 2112])
+@pytest.mark.parametrize("n, k", [(2560, 4096), (2560, 9728), (5120, 25600), (4096, 4096), (1024, 512), (64, 64), (512, 1024)])
+def test_ranges_of_k_are_whole_and_long(rows, n, k):
+    parts, tile = ops.wide_parts(rows, n, k, 256)
+    assert 1 <= parts <= 4 and (parts > 1) == (tile >= 0)
+    assert parts == 1 or k // 64 >= 8 * parts
+
+
+def test_deep_matrices_are_cut_and_full_launches_are_not():
+    assert ops.wide_parts(2048, 2560, 9728, 256)[0] > 1 and ops.wide_parts(640, 5120, 25600, 256)[0] > 1
+    assert ops.wide_parts(2048, 2560, 4096, 256)[0] == 1 and ops.wide_parts(2048, 5120, 25600, 256)[0] == 1
+
+
+# either side of whole rounds of 256 x 256 tiles (216 of 256 are five sixths, 192 are not), of the depth and of the rows
+@pytest.mark.parametrize("rows, n, k, own", [
+    (2048, 6144, 4096, True), (2049, 6144, 4096, False), (2049, 6144, 5120, True), (2048, 8192, 4096, False),
+    (513, 6144, 2560, True), (512, 6144, 2560, False), (1000, plan.TALL, 5120, False)])
+def test_projections_of_long_portions(rows, n, k, own):
+    assert plan.portion_beats_library(rows, n, k) is own
+
+
+@pytest.fixture
+def launched(monkeypatch):
+    seen = []
+
+    def call(name, *args):
+        if name.endswith("_plan"):
+            return real(name, *args)
+        seen.append((name.removeprefix("pylon_"), args))
+
+    real = ops._lib.call
+    monkeypatch.setattr(ops, "_raw_device", lambda: 0)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_watched", lambda x, weight: False)
+    monkeypatch.setattr(ops._lib, "compute_units", lambda: 256)
+    monkeypatch.setattr(ops._lib, "call", call)
+    plain = torch.nn.functional.linear
+    monkeypatch.setattr(torch.nn.functional, "linear", lambda x, w: (seen.append(("library", ())), plain(x, w))[1])
+    with FakeTensorMode(), warnings.catch_warnings():
+        warnings.simplefilter("ignore")  # data pointers of tensors without data
+        yield seen
+
+
+def empty(rows, k, gap=0, dtype=torch.bfloat16):
+    return torch.empty(rows, k + gap, dtype=dtype, device="cuda:0")[:, :k]
+
+
+@pytest.mark.parametrize("gap", [0, 64])
+def test_a_portions_residual_product_is_the_tiled_kernels(launched, gap):
+    """Float parts, or one bfloat16 result; as many as the layers launched by one call expect.  Few rows, operands that
+    the kernel does not take and products that something follows go where they went."""
+    for rows in (129, 192, 300, 512, 700, 2048):
+        for n, k in ((2560, 4096), (2560, 9728), (4096, 4096), (1024, 1024), (1024, 3072)):
+            launched.clear()
+            got = ops.linear_into_residual(empty(rows, k), empty(n, k, gap), out_dtype=torch.bfloat16)
+            parts, tile = ops.wide_parts(rows, n, k, 256)
+            (name, args), = launched
+            if parts > 1:
+                assert name == "gemm_wide_parts" and args[-3:-1] == (parts, tile)
+                assert got.dtype == torch.float32 and got.shape == (parts, rows, n)
+            else:
+                assert name == "gemm_wide" and got.dtype == torch.bfloat16 and got.shape == (rows, n)
+            assert layer_run._into_residual(rows, n, k, k + gap, 256) == ((parts, -1 - tile) if parts > 1 else (0, 0))
+            whole = ops.linear_into_residual(empty(rows, k), empty(n, k, gap), out_dtype=torch.float32)
+            assert whole.dtype == torch.float32 and whole.shape[-2:] == (rows, n) and (whole.dim() == 3) == (parts > 1)
+    for rows, n, k in ((128, 2560, 4096), (300, 2560, 4104), (300, 2562, 4096)):
+        asked = []
+        for entry in (ops.linear_into_residual, ops.linear_for_residual):
+            launched.clear()
+            entry(empty(rows, k), empty(n, k, gap), out_dtype=torch.bfloat16)
+            asked.append([name for name, _ in launched])
+        assert asked[0] == asked[1] and "gemm_wide_parts" not in asked[0]
+        assert layer_run._into_residual(rows, n, k, k + gap, 256) == layer_run._residual(rows, n, k, k + gap, 256)
+
+
+def test_a_followed_product_stays_with_the_library(launched, monkeypatch):
+    monkeypatch.setattr(ops, "_watched", lambda x, weight: True)
+    ops.linear_into_residual(empty(2048, 9728), empty(2560, 9728), out_dtype=torch.bfloat16)
+    ops.linear_of_portion(empty(2048, 2560), empty(6144, 2560), out_dtype=torch.bfloat16)
+    assert [name for name, _ in launched] == ["library"] * 2
+
+
+def test_a_long_portions_projection(launched):
+    for rows, n, k, name in ((2048, 6144, 2560, "gemm_wide"), (2048, 8192, 4096, "library"), (2048, 6144, 2564, "library")):
+        launched.clear()
+        assert ops.linear_of_portion(empty(rows, k), empty(n, k), out_dtype=torch.bfloat16).shape == (rows, n)
+        assert [seen for seen, _ in launched] == [name]

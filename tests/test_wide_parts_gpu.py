@@ -1,0 +1,106 @@
+"""The tiled bfloat16 product's float sums of ranges of K, its tiles of 160 and 192 columns, and its launches in two."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+TILES = [(64, 64), (128, 128), (128, 128), (128, 192), (128, 192), (96, 256), (256, 128), (128, 256), (160, 256), (256, 256),
+         (128, 160), (256, 160), (256, 192), (192, 256)]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from pylon_amd.kernels import ops
+
+    return ops
+
+
+def draw(seed, rows, k, pad=0):
+    gen = torch.Generator(DEV).manual_seed(seed)
+    return torch.randn(rows, k + pad, generator=gen, device=DEV).to(torch.bfloat16)[:, :k]
+
+
+# one chunk a range and ranges of unequal length; K of one chunk, a few, more than all that are in flight
+@pytest.mark.parametrize("k, parts", [(64, 1), (128, 2), (320, 3), (704, 4), (704, 1), (1088, 8)])
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_sums_of_ranges(ops, tile, k, parts):
+    rows, cols = TILES[tile]
+    for m, n in ((rows, cols), (rows + 1, cols - 4), (2 * rows - 3, cols + 4), (5, 3 * cols + 12)):
+        x, w = draw(m, m, k, 8), draw(n + k, n, k, 64)
+        got = ops.gemm_wide_parts(x, w, parts=parts, tile=tile)
+        assert got.dtype == torch.float32
+        chunks = k // 64
+        for p, sums in enumerate(got if parts > 1 else got[None]):
+            at = slice(chunks * p // parts * 64, chunks * (p + 1) // parts * 64)
+            want = x[:, at].double() @ w[:, at].double().T
+            # float32 sums of up to 1,088 exact products: 2^-24 of the running sum each, far below 2^-16 of the largest
+            assert (sums.double() - want).abs().max() <= want.abs().max() * 2.0 ** -16, (m, n, p)
+        assert torch.equal(got, ops.gemm_wide_parts(x, w, parts=parts, tile=(tile + 3) % len(TILES))), (m, n)
+
+
+@pytest.mark.parametrize("tile", [10, 11, 12, 13])
+def test_tiles_of_160_and_192_columns(ops, tile):
+    rows, cols = TILES[tile]
+    for k in (64, 128, 704):
+        for m, n in ((rows, cols), (rows + 1, cols - 4), (2 * rows - 3, cols + 4), (5, 3 * cols + 12)):
+            x, w = draw(m, m, k, 8), draw(n + k, n, k, 64)
+            assert torch.equal(ops.gemm_wide(x, w, tile=tile), ops.gemm_wide(x, w, tile=1))
+            assert torch.equal(ops.gemm_wide(x, w, epilogue="relu2", tile=tile), ops.gemm_wide(x, w, epilogue="relu2", tile=1))
+    x, w = draw(1, 300, 192), draw(2, 2 * 260, 192, 64) * 0.2
+    if cols % 64 == 0:
+        assert torch.equal(ops.gemm_wide(x, w, epilogue="silu", tile=tile), ops.gemm_wide(x, w, epilogue="silu", tile=6))
+    else:
+        with pytest.raises(ops.KernelError):  # a gate tile and its up tile belong to one wave
+            ops.gemm_wide(x, w, epilogue="silu", tile=tile)
+
+
+# sizes whose rounds are a launch of their own, their last columns another; the last tile of either ragged
+@pytest.mark.parametrize("m, n, k, epilogue", [
+    (1000, 9728, 256, "silu"), (2048, 9732, 256, "capped"), (1000, 10244, 320, "none"), (2040, 5124, 320, "relu2")])
+def test_launches_in_two(ops, m, n, k, epilogue):
+    gated = epilogue in ("silu", "capped")
+    x, w = draw(1, m, k), draw(2, 2 * n if gated else n, k, 64) * 0.2
+    got = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    options = dict(epilogue=epilogue, alpha=1.702, offset=1.0, limit=7.0)
+    ops.gemm_wide(x, w, out=got, **options)
+    assert torch.equal(got, ops.gemm_wide(x, w, tile=6, **options))
+
+
+def test_operands_that_end_where_their_memory_ends(ops):
+    """Loads ahead of a range's last chunk stay inside the operands."""
+    torch.cuda.empty_cache()
+    x, w = draw(1, 5120, 1024).contiguous(), draw(2, 5120, 1024).contiguous()
+    for tile in range(len(TILES)):
+        got = ops.gemm_wide_parts(x, w, parts=3, tile=tile)
+        if tile == 0:
+            first = got
+        assert torch.equal(got, first)
+
+
+def test_what_the_residual_norm_makes_of_parts(ops):
+    """A deep product of a portion with its norm, against 64 bits: as close as with the product rounded first."""
+    x, w = draw(3, 700, 9728), draw(4, 2560, 9728) * 0.02
+    resid, gain = torch.randn(700, 2560, device=DEV), torch.rand(2560, device=DEV)
+    delta = ops.linear_into_residual(x, w, out_dtype=torch.bfloat16)
+    assert delta.dtype == torch.float32 and delta.dim() == 3
+    want = resid.double() + x.double() @ w.double().T
+    scaled = want / torch.sqrt((want * want).mean(-1, keepdim=True) + 1e-6) * gain.double()
+    out = ops.add_rmsnorm(resid, delta, gain, 1e-6, torch.bfloat16)
+    assert ((resid.double() - want).abs() <= want.abs() * 2.0 ** -22 + want.abs().max() * 2.0 ** -17).all()
+    assert ((out.double() - scaled).abs() <= scaled.abs() * 1.01 * 2.0 ** -8 + scaled.abs().max() * 2.0 ** -16).all()
+
+
+def test_arguments_that_are_refused(ops):
+    from pylon_amd.kernels import library
+
+    x, w = draw(1, 200, 256), draw(2, 64, 256)
+    for parts, tile in ((5, 0), (0, 0), (9, 0), (2, -1), (2, len(TILES)), (1, -2)):  # four chunks: at most four ranges
+        with pytest.raises(ops.KernelError):
+            ops.gemm_wide_parts(x, w, parts=parts, tile=tile)
+    with pytest.raises(ops.KernelError):
+        ops.gemm_wide_parts(x, w[:62], parts=2, tile=0)
+    with pytest.raises(ops.KernelError):
+        ops.gemm_wide_parts(x[:, :200], w[:, :200], parts=2, tile=0)
+    assert library.load().pylon_gemm_wide_parts_plan(0, 64, 64, 256, None, None, None) != 0
