@@ -117,6 +117,16 @@ __device__ __forceinline__ float gw_capped(float g, float u, const GwShape& p) {
   return gw_gate<EXACT>(g, p.alpha * g) * (u + p.offset);
 }
 
+typedef unsigned int gw_u32x4 __attribute__((ext_vector_type(4), aligned(8)));
+
+// Four columns of two tiles in lanes g = lane / 16, columns 4 g of either -> eight columns: of the first tile 0 and 8 in
+// the lanes of g = 0 and 2, of the second in those of 1 and 3.
+__device__ __forceinline__ gw_u32x4 gw_pair(uint2 lo, uint2 hi) {
+  const auto x = __builtin_amdgcn_permlane16_swap(lo.x, hi.x, false, false);
+  const auto y = __builtin_amdgcn_permlane16_swap(lo.y, hi.y, false, false);
+  return gw_u32x4{x[0], y[0], x[1], y[1]};
+}
+
 // MT, NT: tiles of 16 rows and of 16 columns per wave.  With a gate w is a fused matrix of 2 N rows, gate rows
 // first; a pair of a wave's column tiles is 16 gate rows and their 16 up rows, N rows further down.
 // (The body is a device function: the host pass does not know the descriptor type and would drop a kernel
@@ -316,22 +326,40 @@ __device__ __forceinline__ void gemm_wide_body(uint16_t* __restrict__ out, const
       return;
     }
   }
-  // acc[j][t][i] is out[16 t + r][16 j + 4 g + i] of the wave's quarter (a pair of column tiles with GATED).
-  // N is a multiple of four: a lane's four values are all there or all beyond it.
+  // acc[j][t][i] is out[16 t + r][16 j + 4 g + i] of the wave's quarter (a pair of column tiles with GATED).  Of two
+  // neighbouring tiles the lanes of g = 0 and 1, and of 2 and 3, swap halves: a lane then has eight columns of one of
+  // them, and a store 64 bytes of each of 16 rows instead of 32 (gw_pair; 2048 x 16384 x 4096 205 -> 196 us, 2048 x 6144 x
+  // 2560 53 -> 50, 2048 x 2 x 12288 x 4096 with its gate 290 -> 279; nothing stored at all 182, 45, 273).
+  // N is a multiple of four: of a lane's eight values all, the first four or none lie within.
   auto store = [&](auto value) __attribute__((always_inline)) {
-    uint16_t* const base = out + static_cast<size_t>(m0 + wm * MT * 16 + r) * p.ldo + n0 + wn * NT * (GATED ? 8 : 16) + 4 * g;
-    const int rows = p.M - (m0 + wm * MT * 16 + r), cols = p.N - (n0 + wn * NT * (GATED ? 8 : 16) + 4 * g);
+    constexpr int OT = GATED ? NT / 2 : NT, PAIRS = OT / 2;  // tiles of the result
+    const int row0 = m0 + wm * MT * 16 + r, col0 = n0 + wn * OT * 16;
+    uint16_t* const base = out + static_cast<size_t>(row0) * p.ldo + col0;
+    const int rows = p.M - row0, cols = p.N - col0, eight = (g & 1) * 16 + (g >> 1) * 8;
+    auto four = [&](int j, int t) __attribute__((always_inline)) {
+      bf16x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = static_cast<__bf16>(GATED ? value(acc[2 * j % NT][t][i], acc[(2 * j + 1) % NT][t][i]) : value(acc[j][t][i], 0.f));
+      return __builtin_bit_cast(uint2, v);
+    };
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       if (16 * t >= rows) break;
       uint16_t* const row = base + static_cast<size_t>(16 * t) * p.ldo;
 #pragma unroll
-      for (int j = 0; j < NT; j += GATED ? 2 : 1) {
-        const int at = j * (GATED ? 8 : 16);
-        bf16x4 v;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = static_cast<__bf16>(value(acc[j][t][i], acc[GATED ? j + 1 : j][t][i]));
-        if (at < cols) *reinterpret_cast<bf16x4*>(row + at) = v;
+      for (int j = 0; j < PAIRS; ++j) {
+        const uint2 lo = four(2 * j, t), hi = four(2 * j + 1, t);
+        const gw_u32x4 v = gw_pair(lo, hi);
+        const int at = 32 * j + eight;
+        if (at + 8 <= cols)
+          *reinterpret_cast<gw_u32x4*>(row + at) = v;
+        else if (at < cols)
+          *reinterpret_cast<uint2*>(row + at) = uint2{v[0], v[1]};
+      }
+      if constexpr (OT % 2 == 1) {
+        const int at = 16 * (OT - 1) + 4 * g;
+        if (at < cols) *reinterpret_cast<uint2*>(row + at) = four(OT - 1, t);
       }
     }
   };
