@@ -199,7 +199,7 @@ __device__ __forceinline__ void gemm_rows_body(
       for (int q = 0; q < 4; ++q)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             GLU && j == 1 ? ures : wres, (GR_LDS(void)*)(base + (MT + wave * CT + j) * GR_TILE_BYTES + q * 1024), 16,
-            w_at[GLU ? 0 : j][q], at, 0, 0);
+            w_at[GLU ? 0 : j][q], at, 0, PYLON_STREAMED);
   };
   auto compute = [&](int stage, int left) __attribute__((always_inline)) {  // left: elements from the chunk's first to K
     const GR_LDS(unsigned char)* base = (const GR_LDS(unsigned char)*)(lds + stage * Shape::STAGE_BYTES);
