@@ -26,7 +26,8 @@
 // teams of four waves with half of K each, chosen by a model of the launch's rounds (gf_tiling).
 //
 // Measured, 4B layer sizes, weights from memory, gemm_tiled (one chain per element on the vector ALUs)
-// before: of a step of 3 rows q/k/v 14 us, gate/up 37 (5.4 TB/s), out and down 11 and 22, the head 247 (6.3)
+// before: of a step of 3 rows q/k/v 13 us, gate/up 34 (5.9 TB/s), out and down 10 and 22, the head 230 (6.8; the lines
+// of w not marked as read once 14, 37, 11, 24, 255)
 // where a launch took 615 on average; out, down, q/k/v and gate/up of 270 rows 61, 135, 93 and 266 (91 to 101 TFLOP/s; 600 rows
 // 104 to 110).
 #include "gemm_f32.h"
@@ -111,7 +112,7 @@ __device__ __forceinline__ void gemm_f32_rows_body(float* __restrict__ out, cons
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (GF_LDS(void)*)(stage_base + stage * GF_TILE_BYTES + q * 1024), 16,
-                                                   w_off(q), offset, 0, 0);
+                                                   w_off(q), offset, 0, PYLON_STREAMED);
       };
       if (W_FIRST) send_w();
 #pragma unroll
