@@ -39,8 +39,11 @@
 // within the chunk is computed once, the chunk's is scalar), what is asked before the first
 // load comes with the launch, and nothing is sent beyond the range.  With a check a load and
 // loads beyond the range 6144 x 2560, 2560 x 4096, 2560 x 9728 and 2 x 9728 x 2560 took 8.3,
-// 6.3, 11.8 and 20.9 us at 8 rows, now 7.6, 5.6, 11.0 and 20.0; at 48 rows 10.5, 9.3, 14.3
-// and 25.2, now 9.3, 8.3, 12.9 and 23.4 (under a graph, matrices that no cache holds).
+// 6.3, 11.8 and 20.9 us at 8 rows, then 7.6, 5.6, 11.0 and 20.0; at 48 rows 10.5, 9.3, 14.3
+// and 25.2, then 9.3, 8.3, 12.9 and 23.4 (under a graph, matrices that no cache holds).
+//
+// The lines of w are marked as read once (PYLON_STREAMED): the same products then 6.8, 5.3, 10.1 and 18.1 us at 8 rows
+// and 8.6, 7.2, 11.5 and 21.4 at 48 (heads of 151,936 rows 12 % less at 8, 4 to 10 at 64).
 #include "common.h"
 
 #include <type_traits>

@@ -2,8 +2,8 @@
 
 A step of up to a few hundred prompt tokens waits for the host, which spends 12 us on every launch that the parts make
 one by one.  Where all layers of a model are alike, plain (pre-normed attention with norms and rotation head by head,
-gated feed-forward) and every one of their products runs on the engine's own kernels (at 4B sizes 2 to 48 and 65 to 384
-tokens, 8B 2 to 16 and 65 to 256, 32B 2 to 48, 65 to 192 and 385 to 512), :func:`run_layers` gathers the
+gated feed-forward) and every one of their products runs on the engine's own kernels (at 4B sizes 2 to 48 and 65 to 512
+tokens, 8B 2 to 16 and 65 to 512, 32B 2 to 48, 65 to 320 and 385 to 512), :func:`run_layers` gathers the
 addresses of what a layer reads and has four layers at a time launched in a loop of native code
 (``csrc/layer_run.hip``): the same kernels with the same arguments in the same order, so the same bits.  The device works
 on them while the next four are gathered.  Anything else, a part of another type, a product that is the library's,

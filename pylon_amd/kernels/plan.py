@@ -2,7 +2,9 @@
 
 Pure functions of the shape: they touch no tensor and run anywhere, so the choices can be
 tested without a GPU.  Every figure below was measured on one MI355X, under a graph, over 36
-different matrices in turn (so that none came from a cache).
+different matrices in turn (so that none came from a cache).  Those of the rows kernel are from before its loads
+of w were marked as read once: it takes 4 to 16 % less since (2560 x 9728 at 8 rows 11.2 -> 10.1 us, 2 x 9728 x 2560 20.5
+-> 18.1, 6144 x 4096 12.9 -> 11.0; two halves of the rows 2 to 5 %), which moves no line against it.
 
 Three kernels take part.  ``rows`` (``gemm_rows``): both operands go through LDS in whole
 256-byte row segments, the rows of x are shared by a workgroup, K may be cut over workgroups.
