@@ -411,7 +411,7 @@ static const GwTile kTiles[] = {
     {128, 256, 1, 860, 870},    // 4 x 8, three stages
     {160, 256, 1, 940, 990},    // 5 x 8, three stages
     {256, 256, 1, 1300, 1380},  // 8 x 8, two and a half chunks
-    {128, 160, 1, 650, 660},    // 4 x 5, four stages; none of the next two with a gate, whose halves share a wave
+    {128, 160, 1, 600, 615},    // 4 x 5, four stages; none of the next two with a gate, whose halves share a wave
     {256, 160, 1, 940, 950},    // 8 x 5, three stages
     {256, 192, 1, 1055, 1075},  // 8 x 6, two and a half chunks
     {192, 256, 1, 1080, 1100},  // 6 x 8, two and a half chunks
