@@ -111,6 +111,9 @@ __global__ __launch_bounds__(512) void rmsnorm_kernel(TO* __restrict__ out, TX* 
 // it counts.  All arguments come with the launch (14 words do), and nothing waits for a store.
 // Launches in a row, four parts, 8 rows of 2,560, 4,096 and 5,120: 3.8, 4.2 and 4.2 us -> 2.5, 2.7 and 3.2 (of an
 // empty kernel's 1.5); 48 rows 4.3, 4.9, 4.7 -> 2.8, 3.3, 3.5.
+// For many rows, too (prompt portions; a workgroup a row): one that took two rows, all loads first, was the quicker one beside an
+// earlier form of this and takes longer than this now, 512, 1000 and 2048 rows of a bfloat16 product 6.2, 7.6, 14.2
+// us at 2,560 and 7.6, 11.7, 20.8 at 4,096 against 4.2, 6.1, 13.0 and 5.5, 10.5, 19.7 (5.1 TB/s).
 // Float residual rows of a multiple of 4 elements, at most 4 NV a thread.  parts_apart: fours of elements from one
 // part to the next; sizes: dim, from bit 16 on the number of parts (0: no delta), from bit 24 on whether the sum is
 // stored.  LOOSE: for rows that begin anywhere (8 rows of 2,560, four parts, 8.2 us element by element, 3.0 so).
@@ -182,92 +185,10 @@ static void launch_rmsnorm_few(void* out, float* x, const TD* delta, int n_delta
 #undef GO
 }
 
-// The same arithmetic, in the same order, for steps of many rows (prompt portions): a
-// workgroup takes R rows and issues the loads of all of them before the first sum, so that one
-// row's stores travel beside the next row's loads instead of every workgroup of the launch
-// reading at one time and writing at another (2,048 rows of 2,560: 19.5 -> 15.8 us on data
-// that no cache holds; four rows per workgroup lose again, 19.2 us).  Float residual, one
-// delta, rows of a multiple of 4 elements that fit 16 per thread; as many threads as the
-// kernel for few rows has at this width, so that a row's sum is formed in the same order.
-template <typename TD, typename TO, int R, int THREADS>
-__global__ __launch_bounds__(THREADS) void add_rmsnorm_many_kernel(TO* __restrict__ out, float* resid,
-                                                               const TD* __restrict__ delta,
-                                                               const float* __restrict__ w, int rows, int dim,
-                                                               float eps, float factor) {
-  __shared__ float scratch[16];
-  constexpr int VEC = 4;
-  const int chunks = dim >> 2;
-  const float4* w4 = reinterpret_cast<const float4*>(w);
-  float4 held[R][VEC], wt[VEC];
-  const int r0 = blockIdx.x * R;
-#pragma unroll
-  for (int n = 0; n < VEC; ++n) {
-    const int c = threadIdx.x + n * THREADS;
-    wt[n] = (c < chunks) ? w4[c] : float4{0.f, 0.f, 0.f, 0.f};
-  }
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const bool live = r0 + i < rows;
-    const float* xr = resid + static_cast<size_t>(live ? r0 + i : r0) * dim;
-    const TD* dr = delta + static_cast<size_t>(live ? r0 + i : r0) * dim;
-#pragma unroll
-    for (int n = 0; n < VEC; ++n) {
-      const int c = threadIdx.x + n * THREADS;
-      if (c < chunks) {
-        const float4 x = reinterpret_cast<const float4*>(xr)[c];
-        const float4 d = load4(dr, c);
-        held[i][n] = float4{fmaf(factor, d.x, x.x), fmaf(factor, d.y, x.y), fmaf(factor, d.z, x.z), fmaf(factor, d.w, x.w)};
-      } else {
-        held[i][n] = float4{0.f, 0.f, 0.f, 0.f};
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    if (r0 + i >= rows) break;  // the same for the whole workgroup
-    float ss = 0.f;
-#pragma unroll
-    for (int n = 0; n < VEC; ++n)
-      ss += row_squares(held[i][n]);
-    const float total = block_sum(ss, scratch);
-    const float inv = 1.0f / sqrtf(total / static_cast<float>(dim) + eps);
-    float* xr = resid + static_cast<size_t>(r0 + i) * dim;
-    TO* yr = out + static_cast<size_t>(r0 + i) * dim;
-#pragma unroll
-    for (int n = 0; n < VEC; ++n) {
-      const int c = threadIdx.x + n * THREADS;
-      if (c < chunks) {
-        reinterpret_cast<float4*>(xr)[c] = held[i][n];
-        store4(yr, c, (held[i][n].x * inv) * wt[n].x, (held[i][n].y * inv) * wt[n].y,
-               (held[i][n].z * inv) * wt[n].z, (held[i][n].w * inv) * wt[n].w);
-      }
-    }
-  }
-}
-
-#define PYLON_NORM_MANY_ROWS 512  // from this many rows on, a workgroup takes two
-
 template <typename TX, typename TD>
 static void launch_rmsnorm_out(void* out, int out_dtype, TX* x, const TD* delta, int n_delta,
                                long long delta_stride, const float* w, const int* row_idx, int rows,
                                int dim, float eps, int write_resid, float factor, hipStream_t stream) {
-  if constexpr (sizeof(TX) == 4) {
-    if (rows >= PYLON_NORM_MANY_ROWS && delta != nullptr && n_delta == 1 && row_idx == nullptr && write_resid &&
-        (dim & 3) == 0 && dim <= 8192) {
-      constexpr int R = 2;
-      dim3 grid((rows + R - 1) / R);
-#define GO(TO, THREADS)                                                                                    \
-  hipLaunchKernelGGL((add_rmsnorm_many_kernel<TD, TO, R, THREADS>), grid, dim3(THREADS), 0, stream, (TO*)out, x, \
-                     delta, w, rows, dim, eps, factor)
-      if (dim > 4096) {
-        if (out_dtype == PYLON_F32) GO(float, 512); else GO(bf16_t, 512);
-      } else {
-        if (out_dtype == PYLON_F32) GO(float, 256); else GO(bf16_t, 256);
-      }
-#undef GO
-      return;
-    }
-  }
   if constexpr (sizeof(TX) == 4) {
     if ((dim & 3) == 0 && dim <= 8192 && (delta_stride & 3) == 0 && delta_stride < (1ll << 33)) {
 #define GO(TO, THREADS) \
