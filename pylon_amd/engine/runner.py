@@ -18,14 +18,15 @@ from __future__ import annotations
 import logging
 import math
 import time
+from operator import ge
 from pathlib import Path
-from typing import Callable, Dict, Hashable, List, Mapping, Optional, Sequence as Seq
+from typing import Callable, Dict, Hashable, Iterable, List, Mapping, Optional, Sequence as Seq, Tuple
 
 import torch
 
 from ..cache.manager import CacheManager, Sequence, group_requirements, plan_pool
 from ..config.registry import load_model_config, resolve
-from ..kernels import check_device
+from ..kernels import check_device, ops
 from ..weights.loader import load_weights, stored_param_dtypes
 from ..weights.random_init import fill_random_model
 from .batch import MetadataArena, StepEntry, build_step
@@ -338,15 +339,28 @@ def cache_needs(requirements: Seq[object], dtype: torch.dtype, max_requests: int
     return groups, state_bytes
 
 
+def rows_to_measure(products: Iterable[Tuple[int, int]], most: int, units: int) -> List[int]:
+    """Row counts of the steps of up to ``most`` rows one of which takes the most memory: ``most``, and a smaller one
+    where no larger one of these takes as much for the result of each of ``products`` (their columns and depths).
+    Everything else of a step grows with its rows; float sums of ranges of K do not (:func:`ops.residual_bytes`)."""
+    products, kept = tuple(products), []
+    for rows in range(most, 0, -1):
+        taken = [ops.residual_bytes(rows, n, k, units) for n, k in products]
+        if rows == most or not any(all(map(ge, more, taken)) for _, more in kept):
+            kept.append((rows, taken))
+    return [rows for rows, _ in kept]
+
+
 def measure_activation_bytes(model: Model, config) -> int:
     """The most memory a step takes beside weights and cache: the largest step the serving
     options allow (a prompt portion of ``prefill_chunk_size`` tokens beside one token for each
     of the other ``max_batch_size - 1`` requests, all rows sampling) is run once over a
     throw-away pool of just the pages it needs, and the allocator's peak is read
-    (/root/reference/src/pylon/decode/warmup.py:33-120, kv/budget.py:85-95).  To it is added
-    what the decode graphs keep for good: their shared ``[max_batch_size, vocab]`` float32
-    logits and as much again as the peak of a decode-only step of ``max_batch_size`` rows.
-    The run also warms the library's matrix products up for the shapes of a full step."""
+    (/root/reference/src/pylon/decode/warmup.py:33-120, kv/budget.py:85-95).  So are the few smaller steps that
+    may take more (:func:`rows_to_measure`; two layers of 8B sizes beside 63 requests: 2,111 rows 156 MB,
+    2,048 rows 252).  To it is added what the decode graphs keep for good: their shared ``[max_batch_size, vocab]``
+    float32 logits and as much again as the peak of a decode-only step of up to ``max_batch_size`` rows.
+    The runs also warm the library's matrix products up for the shapes of a full step."""
     device = model.device
     spec = model.spec
     page = config.page_size
@@ -355,27 +369,34 @@ def measure_activation_bytes(model: Model, config) -> int:
     others = config.max_batch_size - 1
     pages = -(-chunk // page) + others + 1
     runner = Runner(model, page_size=page, num_pages=pages, max_requests=config.max_batch_size)
-    seqs = [runner.open(("warm-up", i)) for i in range(config.max_batch_size)]
-    try:
-        torch.cuda.synchronize(device)
-        base = torch.cuda.memory_allocated(device)
-        torch.cuda.reset_peak_memory_stats(device)
-        decode_peak = 0
-        if others:
-            runner.step([StepEntry(seq, [0], [0]) for seq in seqs[:others]])
+    # the matrices whose products go into the residual stream are among those of as many rows as it is wide
+    products = {tuple(owner.params[name].shape) for _, owner, name in model.named_params()
+                if owner.params[name].dim() == 2 and owner.params[name].dtype == torch.bfloat16
+                and owner.params[name].shape[0] == spec.hidden_size} if model.dtype == torch.bfloat16 else set()
+    units = ops.compute_units()
+
+    def peak_of(singles: int, portion: int) -> int:
+        seqs = [runner.open(("warm-up", i)) for i in range(singles + (portion > 0))]
+        try:
+            entries = [StepEntry(seq, [0], [0]) for seq in seqs[:singles]]
+            if portion:
+                entries.append(StepEntry(seqs[-1], [0] * portion, [portion - 1]))
             torch.cuda.synchronize(device)
-            decode_peak = torch.cuda.max_memory_allocated(device) - base
             torch.cuda.reset_peak_memory_stats(device)
-            entries = [StepEntry(seq, [0], [0]) for seq in seqs[:others]]
-        else:
-            entries = []
-        entries.append(StepEntry(seqs[-1], [0] * chunk, [chunk - 1]))
-        runner.step(entries)
-        torch.cuda.synchronize(device)
-        step_peak = torch.cuda.max_memory_allocated(device) - base
-    finally:
-        for seq in seqs:
-            runner.close(seq)
+            runner.step(entries)
+            torch.cuda.synchronize(device)
+            return torch.cuda.max_memory_allocated(device) - base
+        finally:
+            for seq in seqs:
+                runner.close(seq)
+
+    torch.cuda.synchronize(device)
+    base = torch.cuda.memory_allocated(device)
+    decode_peak = max([peak_of(rows, 0) for rows in rows_to_measure(products, others, units)], default=0)
+    step_peak = 0
+    for rows in rows_to_measure(products, others + chunk, units):
+        singles = min(others, rows - 1)  # as many rows that sample as the step can have
+        step_peak = max(step_peak, peak_of(singles, rows - singles))
     graphs = 0
     if config.cuda_graphs:
         graphs = config.max_batch_size * spec.vocab_size * 4 + max(decode_peak, 0)

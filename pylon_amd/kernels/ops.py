@@ -1652,6 +1652,17 @@ def linear_into_residual(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: to
     return linear_for_residual(x, weight, out_dtype=out_dtype)
 
 
+def residual_bytes(rows: int, n: int, k: int, units: int) -> int:
+    """Bytes of the result of :func:`linear_into_residual` for bfloat16 operands that lie as a part's do, a bfloat16 result
+    asked for.  They do not grow with the rows: 4096 x 12288 at 2,048 rows 67 MB in two ranges, at 2,049 17 MB."""
+    if rows > SPLIT_ROWS and wide_sizes_ok(rows, n, k, k, k):
+        parts, _ = wide_parts(rows, n, k, units)
+        return (4 * parts if parts > 1 else 2) * rows * n
+    if rows <= SPLIT_ROWS:
+        return 4 * plan.plan_residual(rows, n, k, units=units).parts * rows * n
+    return 2 * rows * n
+
+
 def linear_of_portion(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype) -> torch.Tensor:
     """:func:`linear`, but a long portion's product with a bfloat16 result goes to the tiled kernel also where
     :func:`plan.portion_beats_library` says so."""

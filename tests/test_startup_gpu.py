@@ -251,3 +251,33 @@ def test_groups_of_runs_get_pages_of_their_own_at_start_up(gpu, tmp_path):
                 ref.append(got)
     finally:
         unregister_architecture("ToyWindowedForCausalLM")
+
+
+def test_a_step_of_any_size_stays_within_the_measured_memory(gpu):
+    """Layers whose products into the residual stream take more memory for 2,048 rows (float sums of two ranges of K)
+    than for the 2,111 of the largest step."""
+    from pylon_amd.config import PylonConfig
+    from pylon_amd.engine import Runner, StepEntry
+
+    config = dict(CONFIGS["D"], hidden_size=4096, num_attention_heads=32, num_key_value_heads=8, head_dim=128,
+                  intermediate_size=12288, num_hidden_layers=2, vocab_size=1000, max_position_embeddings=4096)
+    options = PylonConfig(dtype="bfloat16", max_batch_size=64, prefill_chunk_size=2048, page_size=256, cuda_graphs=False,
+                          max_gpu_utilization=0.5)
+    runner = Runner.from_random(config, 1, options, std=0.02)
+    measured = runner.pool_sizing["activation_bytes"]
+    peaks = {}
+    for rows in (2111, 2049, 2048, 1500, 768, 129, 64):
+        singles = min(63, rows - 1)
+        seqs = [runner.open(i) for i in range(singles + 1)]
+        entries = [StepEntry(seq, [0], [0]) for seq in seqs[:singles]]
+        entries.append(StepEntry(seqs[-1], [0] * (rows - singles), [rows - singles - 1]))
+        torch.cuda.synchronize()
+        base = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        runner.step(entries)
+        torch.cuda.synchronize()
+        peaks[rows] = torch.cuda.max_memory_allocated() - base
+        for seq in seqs:
+            runner.close(seq)
+    print({rows: f"{peak / 1e6:.0f} MB" for rows, peak in peaks.items()}, f"measured {measured / 1e6:.0f} MB")
+    assert peaks[2048] > peaks[2111] and max(peaks.values()) <= measured
