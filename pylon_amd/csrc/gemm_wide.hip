@@ -401,7 +401,7 @@ struct GwTile {
   int rows, cols, per_unit, alone_ns, full_ns;
 };
 static const GwTile kTiles[] = {
-    {64, 64, 2, 230, 380},      // 2 x 2, five stages
+    {64, 64, 2, 230, 450},      // 2 x 2, five stages
     {128, 128, 1, 560, 575},    // 4 x 4, four stages
     {128, 128, 2, 700, 930},    // 4 x 4, two and a half chunks
     {128, 192, 1, 660, 670},    // 4 x 6, three stages
@@ -485,8 +485,13 @@ extern "C" int pylon_gemm_wide_plan(int M, int N, int K, int gated, int units, i
 }
 
 // Ranges of K for a product into the residual stream, with the tile, or one range and tile -1 (pylon_gemm_wide): the
-// quickest with what the residual norm pays for reading float sums of every range instead of one bfloat16 result.
+// quickest with what the residual norm pays for reading float sums of every range instead of one bfloat16 result, by
+// their size and each (three, which it reads one after the other, cost what four do).  Product and norm over 432 sizes of 2,560
+// to 5,120 columns and 129 to 2,112 rows take 0.79 of the time of the uncut kernel or the library, whichever it was before
+// (one of them 1.04, the others no more than 1.01); with 380 ns for a full round of the smallest tile and nothing for each range
+// 4096 x 4096 at 131, 435 and 512 rows took 21, 39 and 40 us against 20, 34 and 37, where one, two and two ranges take 20, 29 and 32.
 #define GW_ADD_US_MB 0.2
+#define GW_ADD_US_EACH 0.5
 #define GW_MOST_PARTS 4
 #define GW_LEAST_CHUNKS 8  // of a range
 extern "C" int pylon_gemm_wide_parts_plan(int M, int N, int K, int units, int* parts, int* tile, float* us) {
@@ -504,7 +509,8 @@ extern "C" int pylon_gemm_wide_parts_plan(int M, int N, int K, int units, int* p
   *parts = 1, *tile = -1;
   for (int n = 2; n <= GW_MOST_PARTS && n * GW_LEAST_CHUNKS <= K / GW_CHUNK; ++n)
     for (int i = 0; i < kTileCount; ++i) {
-      const double now = gw_time_us(kTiles[i], M, N, K, false, units, n) + GW_ADD_US_MB * 1e-6 * (4 * n - 2) * M * N;
+      const double now = gw_time_us(kTiles[i], M, N, K, false, units, n) + GW_ADD_US_MB * 1e-6 * (4 * n - 2) * M * N +
+                         GW_ADD_US_EACH * (n == 3 ? 4 : n);
       if (now < least) least = now, *parts = n, *tile = i;
     }
   *us = static_cast<float>(least);

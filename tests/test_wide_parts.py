@@ -23,6 +23,15 @@ def test_deep_matrices_are_cut_and_full_launches_are_not():
     assert ops.wide_parts(2048, 2560, 4096, 256)[0] == 1 and ops.wide_parts(2048, 5120, 25600, 256)[0] == 1
 
 
+# us of product and norm uncut, in two, three and four ranges, and by the route before there were any: 768 rows 37.1, 30.2, 30.9,
+# 30.7 and 34.9; 435 rows 38.9, 28.7, 31.5, 31.4 and 33.6; 512 rows 39.7, 31.5, 33.8, 32.4 and 37.3; 131 rows 19.7, 22.4, 20.3, 21.2
+# and 20.1
+@pytest.mark.parametrize("rows, n, k, cut", [(768, 2560, 4096, True), (435, 4096, 4096, True), (512, 4096, 4096, True),
+                                             (131, 4096, 4096, False)])
+def test_full_rounds_of_small_tiles_are_cut_and_small_products_are_not(rows, n, k, cut):
+    assert (ops.wide_parts(rows, n, k, 256)[0] > 1) is cut
+
+
 # either side of whole rounds of 256 x 256 tiles (216 of 256 are five sixths, 192 are not), of the depth and of the rows
 @pytest.mark.parametrize("rows, n, k, own", [
     (2048, 6144, 4096, True), (2049, 6144, 4096, False), (2049, 6144, 5120, True), (2048, 8192, 4096, False),
