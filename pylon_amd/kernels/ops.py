@@ -1639,7 +1639,8 @@ def linear_for_residual(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: tor
 def linear_into_residual(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype) -> torch.Tensor:
     """:func:`linear_for_residual`, but a prompt portion's product (more than :data:`SPLIT_ROWS` rows) is the tiled
     kernel's wherever that takes it, with K cut into ranges where the uncut launch has fewer tiles than the device has
-    units, or small ones (:func:`wide_parts`): then float32 partial sums ``[parts, M, N]``, which the consumer adds.
+    units, or small ones (:func:`wide_parts`): then float32 partial sums ``[parts, M, N]``, which the consumer adds.  Uncut
+    and with a bfloat16 result it is the library's where :func:`plan.library_fills_rounds`.
     (2560 x 9728 at 192, 640, 1200 and 2048 rows, with the norm's reading of the parts: 25, 42, 61 and 88 us, where
     the uncut kernel or the library took 42, 61, 87 and 105; 5120 x 25600 at 256, 640 and 1500: 93, 149 and 283
     against 265, 240 and 341.)  With a float32 ``out_dtype`` the sums come unrounded also where K is not cut."""
@@ -1648,6 +1649,8 @@ def linear_into_residual(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: to
         parts, tile = wide_parts(x.shape[0], *weight.shape, _lib.compute_units())
         if parts > 1 or out_dtype == torch.float32:
             return gemm_wide_parts(x, weight, parts=parts, tile=tile)
+        if plan.library_fills_rounds(x.shape[0], *weight.shape, units=_lib.compute_units()):
+            return torch.nn.functional.linear(x, weight)
         return gemm_wide(x, weight)
     return linear_for_residual(x, weight, out_dtype=out_dtype)
 
@@ -1664,11 +1667,12 @@ def residual_bytes(rows: int, n: int, k: int, units: int) -> int:
 
 
 def linear_of_portion(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: torch.dtype) -> torch.Tensor:
-    """:func:`linear`, but a long portion's product with a bfloat16 result goes to the tiled kernel also where
-    :func:`plan.portion_beats_library` says so."""
-    if (out_dtype == torch.bfloat16 and x.dim() == 2 and x.shape[0] > plan.PORTION_ROWS
-            and plan.portion_beats_library(x.shape[0], *weight.shape) and not _watched(x, weight) and _wide_ok(x, weight)):
-        return gemm_wide(x, weight)
+    """:func:`linear`, but a long portion's product with a bfloat16 result goes to the tiled kernel or to the library as
+    :func:`plan.portion_beats_library` says."""
+    if (out_dtype == torch.bfloat16 and x.dim() == 2 and x.shape[0] > plan.PORTION_ROWS and weight.shape[0] < plan.TALL
+            and not _watched(x, weight) and _wide_ok(x, weight)):
+        own = plan.portion_beats_library(x.shape[0], *weight.shape, units=_lib.compute_units())
+        return gemm_wide(x, weight) if own else torch.nn.functional.linear(x, weight)
     return linear(x, weight, out_dtype=out_dtype)
 
 

@@ -244,18 +244,42 @@ def wide_beats_library(rows: int, n: int, k: int, units: int = UNITS) -> bool:
 PORTION_ROWS = 512  # a long portion has more rows
 
 
-def portion_beats_library(rows: int, n: int, k: int) -> bool:
-    """Whether a portion's projection (q/k/v and the like) of more than :data:`PORTION_ROWS` rows takes the tiled
-    kernel, with its tiles of 160 and 192 columns and its whole rounds in a launch of their own, whatever
-    :func:`wide_beats_library` says of the tiles before those: everywhere but where 256 x 256 tiles fill five sixths of
-    their rounds and K is short, which is where the library has its best main loop.  us, here against the library:
-    6144 x 2560 at 1000, 1400 and 2048 rows 37 and 40, 46 and 54, 52 and 56; 6144 x 4096 at 2048 77 and 80; 10240 x 5120 at
-    1000 and 2048 86 and 95, 166 and 181; but 7168 x 4096 at 1800 and 2048 (224 tiles) 1.15 and 1.12 of the library's time,
-    6144 x 4096 at 2056 (216) 90 and 81, 8192 x 4096 at 2048 (256) 1.08; 16384 x 4096 at 2048 (512) 1.14; of rows of
-    5120 all but two of 88 products are within 3 % or quicker here."""
+def library_fills_rounds(rows: int, n: int, k: int, units: int = UNITS) -> bool:
+    """Whether an uncut product without an activation is the library's because its 256 x 256 tiles are those that fill the
+    rounds: of one round more than three quarters, and tiles of 192 rows or of 192 columns do not fit it, of several
+    more than five sixths.  Where rows of w are of a multiple of 8 KB its main loop is then the quicker one, us here and there:
+    8192 x 4096 at 1538, 1700, 2048 rows 92 and 82, 99 and 89, 103 and 94; 12288 x 4096 at 1100, 1280, 2049 99 and 92, 100 and
+    93, 177 and 167; 16384 x 4096 at 1600, 2048 183 and 174, 208 and 187; 7168 x 4096 at 1792 91 and 81; 8192 x 8192 at 2033
+    196 and 175; where smaller tiles fit, the own kernel is: 7168 x 4096 at 1700 (192 x 256) 77 and 79, 10240 x 4096 at 1134
+    76 and 77, 12288 x 4096 at 2000 (three quarters of two rounds) 154 and 166.  Up to 1,024 rows it is the one or the other
+    with no line between (16384 x 8192 at 972 187 and 244, 16384 x 4096 at 900 103 and 103, 20480 x 4096 at 668 102 and 94), as
+    with rows of more than 16 KB (8192 x 28672 at 1792 638 and 815, at 1900 681 and 671)."""
+    if rows <= 1024 or not aliased_rows(k) or k > 8192:
+        return False
     tiles = -(-rows // 256) * -(-n // 256)
-    full = 6 * tiles >= 5 * 256 * -(-tiles // 256)
-    return rows > PORTION_ROWS and n < TALL and not (full and k < 5120)
+    rounds = -(-tiles // units)
+    if rounds > 1:
+        return 6 * tiles > 5 * units * rounds
+    return 4 * tiles > 3 * units and min(-(-rows // 192) * -(-n // 256), -(-rows // 256) * -(-n // 192)) > units
+
+
+def portion_beats_library(rows: int, n: int, k: int, units: int = UNITS) -> bool:
+    """Whether a portion's projection (q/k/v and the like) of more than :data:`PORTION_ROWS` rows takes the tiled
+    kernel, with its tiles of 160 and 192 columns and its whole rounds in a launch of their own; else the library has it.
+    Where rows of w are of a multiple of 8 KB: unless :func:`library_fills_rounds`.  Else everywhere but where 256 x 256 tiles
+    fill five sixths of their rounds and K is short: there what :func:`wide_beats_library` says.  us, here
+    against the library: 6144 x 2560 at 1024, 1400 and 2048 rows 36 and 39, 45 and 55, 52 and 56, but at 2049 (216 tiles)
+    61 and 59; 10560 x 2560 at 1400, 1536 (252) 65 and 71, 66 and 72; 14592 x 2560 at 900 and 2048 (228, 456) 64 and 66,
+    127 and 123; 10240 x 5120 at 1024 and 2048 87 and 95, 170 and 185.  Over 934 sizes of 4,352 to 24,576 columns, K of 2,048 to
+    8,192 and 513 to 4,096 rows it takes 0.6 % longer than the quicker of the two at each (1.2 with one line of five sixths
+    for K below 5,120, and up to 1,700 rows none)."""
+    if rows <= PORTION_ROWS or n >= TALL:
+        return False
+    if aliased_rows(k):
+        return not library_fills_rounds(rows, n, k, units)
+    tiles = -(-rows // 256) * -(-n // 256)
+    full = 6 * tiles >= 5 * units * -(-tiles // units)
+    return not (full and k < 5120) or wide_beats_library(rows, n, k, units)
 
 
 def wide_gated_beats_library(rows: int, n_half: int) -> bool:

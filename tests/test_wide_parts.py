@@ -94,6 +94,18 @@ def test_a_portions_residual_product_is_the_tiled_kernels(launched, gap):
         assert layer_run._into_residual(rows, n, k, k + gap, 256) == layer_run._residual(rows, n, k, k + gap, 256)
 
 
+def test_an_uncut_product_that_the_librarys_tiles_fill_is_the_librarys(launched):
+    for rows, n, k, name in ((2048, 8192, 8192, "library"), (2049, 8192, 8192, "gemm_wide"), (3000, 5120, 8192, "library"),
+                             (2048, 5120, 8192, "gemm_wide"), (1000, 8192, 8192, "gemm_wide"), (1792, 8192, 28672, "gemm_wide")):
+        assert ops.wide_parts(rows, n, k, 256)[0] == 1
+        launched.clear()
+        got = ops.linear_into_residual(empty(rows, k), empty(n, k), out_dtype=torch.bfloat16)
+        assert [seen for seen, _ in launched] == [name] and got.dtype == torch.bfloat16 and got.shape == (rows, n)
+        launched.clear()
+        ops.linear_into_residual(empty(rows, k), empty(n, k), out_dtype=torch.float32)  # whose sums are to stay unrounded
+        assert [seen for seen, _ in launched] == ["gemm_wide_parts"]
+
+
 def test_a_followed_product_stays_with_the_library(launched, monkeypatch):
     monkeypatch.setattr(ops, "_watched", lambda x, weight: True)
     ops.linear_into_residual(empty(2048, 9728), empty(2560, 9728), out_dtype=torch.bfloat16)
@@ -106,3 +118,18 @@ def test_a_long_portions_projection(launched):
         launched.clear()
         assert ops.linear_of_portion(empty(rows, k), empty(n, k), out_dtype=torch.bfloat16).shape == (rows, n)
         assert [seen for seen, _ in launched] == [name]
+
+
+# rows of a multiple of 8 KB: either side of 1,024 rows, of tiles of 192 rows or columns that fit one round, of three quarters
+# of one and five sixths of several, of 16 KB; of other rows what there was
+@pytest.mark.parametrize("rows, n, k, own", [
+    (1700, 8192, 4096, False), (1538, 8192, 4096, False), (1536, 8192, 4096, True), (1024, 16384, 4096, True),
+    (1728, 7168, 4096, True), (1729, 7168, 4096, False), (1152, 10240, 4096, True), (1153, 10240, 4096, False),
+    (1300, 9216, 8192, True), (1345, 9216, 8192, False), (2048, 12288, 4096, True), (2049, 12288, 4096, False),
+    (4096, 10240, 4096, True), (2048, 8192, 8192, False), (2048, 8192, 12288, True), (1536, 10560, 2560, True),
+    (2048, 14592, 2560, False), (2048, 10240, 5120, True)])
+def test_the_rule_for_projections_decides_both_ways(launched, rows, n, k, own):
+    ops.linear_of_portion(empty(rows, k), empty(n, k), out_dtype=torch.bfloat16)
+    assert [seen for seen, _ in launched] == ["gemm_wide" if own else "library"]
+    assert plan.portion_beats_library(rows, n, k) is own
+    assert plan.portion_beats_library(rows, n, k, units=100000) is True  # a device whose rounds nothing fills
