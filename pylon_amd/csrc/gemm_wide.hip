@@ -30,7 +30,7 @@
 // K cut into ranges (pylon_gemm_wide_parts): that product in two ranges of 256 x 160 tiles 82 us.
 //
 // Which tile: gw_choose, by a model of the launch's rounds over the compute units; a last round that would leave most
-// of them idle is a launch of its own (gw_split).  Gate/up with its activation here, one tile for all (before the
+// of them idle is a launch of its own (gw_launches).  Gate/up with its activation here, one tile for all (before the
 // tiles of 160 and 192 columns and that) -> now, and the library's product alone, us: 2 x 9728 x 2560 at 520, 1000,
 // 2048 rows 67, 107, 168 -> 56, 90, 157 (61, 104, 189); 2 x 12288 x 4096 at 1000, 2048, 2096 165, 290, 364 -> 149, 279, 322
 // (165, 269, 334); 2 x 25600 x 5120 at 1000, 2048 446, 796 -> 387, 739 (475, 772).  The products without an activation:
@@ -449,13 +449,20 @@ static int gw_choose(int M, int N, int K, bool gated, int units, double* us = nu
   return best;
 }
 
-// A last round that leaves most units idle: the whole rounds of one tile in a launch of their own and the columns that are
-// left in a launch of the tile that suits them, where both are quicker than one launch (`us`).  Columns of the first
-// launch, 0 for one launch.
+// How a product is launched: the first `ahead` columns in a launch of tile `first` (0: no such launch), the others in one of
+// tile `rest`; us: by the model.
+struct GwLaunches {
+  int ahead, first, rest;
+  double us;
+};
+
+// One launch, or, where a last round would leave most units idle, the whole rounds of one tile in a launch of their own
+// and the columns that are left in a launch of the tile that suits them, where both are quicker.
 #define GW_SECOND_US 2.5
-static int gw_split(int M, int N, int K, bool gated, int units, double us, int* first, int* rest) {
-  int ahead = 0;
-  if (M <= 4 * GW_EXACT_ROWS) return 0;
+static GwLaunches gw_launches(int M, int N, int K, bool gated, int units) {
+  GwLaunches best{0, -1, 0, 0.0};
+  best.rest = gw_choose(M, N, K, gated, units, &best.us);
+  if (M <= 4 * GW_EXACT_ROWS) return best;
   for (int i = 0; i < kTileCount; ++i) {
     const GwTile& t = kTiles[i];
     if (!gw_takes(t, M, gated)) continue;
@@ -464,16 +471,17 @@ static int gw_split(int M, int N, int K, bool gated, int units, double us, int* 
     const long long rounds = static_cast<long long>(m_tiles) * (N / cols) / slots;
     const long long n = rounds * slots / m_tiles * cols;
     if (rounds == 0 || n >= N) continue;
+    const double whole = gw_time_us(t, M, static_cast<int>(n), K, gated, units) + GW_SECOND_US;
+    if (whole >= best.us) continue;  // what is left takes some time too
     double left;
-    const int other = gw_choose(M, N - static_cast<int>(n), K, gated, units, &left);
-    const double now = gw_time_us(t, M, static_cast<int>(n), K, gated, units) + left + GW_SECOND_US;
-    if (now < us) us = now, ahead = static_cast<int>(n), *first = i, *rest = other;
+    const int rest = gw_choose(M, N - static_cast<int>(n), K, gated, units, &left);
+    if (whole + left < best.us) best = GwLaunches{static_cast<int>(n), i, rest, whole + left};
   }
-  return ahead;
+  return best;
 }
 
-// The tile that pylon_gemm_wide takes for a product of these sizes (units 0: the current device's), and in
-// *us the time that the model gives it.  Touches no device memory.
+// The tile that suits a product of these sizes best in one launch (units 0: the current device's), and in *us the time that
+// the model gives it; pylon_gemm_wide_launches says whether there are two.  Touches no device memory.
 extern "C" int pylon_gemm_wide_plan(int M, int N, int K, int gated, int units, int* tile, float* us) {
   PYLON_REQUIRE(tile != nullptr && us != nullptr && M >= 1 && N >= 1 && K >= GW_CHUNK, "gemm_wide_plan: bad arguments");
   if (units <= 0) units = pylon_compute_units();
@@ -481,6 +489,17 @@ extern "C" int pylon_gemm_wide_plan(int M, int N, int K, int gated, int units, i
   double least;
   *tile = gw_choose(M, N, K, gated != 0, units, &least);
   *us = static_cast<float>(least);
+  return 0;
+}
+
+// The launches of pylon_gemm_wide for a product of these sizes: columns of the first of two (0: there is one), its tile, the
+// tile of the other columns, and the time that the model gives them.  Touches no device memory.
+extern "C" int pylon_gemm_wide_launches(int M, int N, int K, int gated, int units, int* ahead, int* first, int* rest, float* us) {
+  PYLON_REQUIRE(ahead && first && rest && us && M >= 1 && N >= 1 && K >= GW_CHUNK, "gemm_wide_launches: bad arguments");
+  if (units <= 0) units = pylon_compute_units();
+  PYLON_REQUIRE(units > 0, "gemm_wide_launches: no device to take the number of compute units from");
+  const GwLaunches found = gw_launches(M, N, K, gated != 0, units);
+  *ahead = found.ahead, *first = found.first, *rest = found.rest, *us = static_cast<float>(found.us);
   return 0;
 }
 
@@ -498,14 +517,7 @@ extern "C" int pylon_gemm_wide_parts_plan(int M, int N, int K, int units, int* p
   PYLON_REQUIRE(parts && tile && us && M >= 1 && N >= 1 && K >= GW_CHUNK, "gemm_wide_parts_plan: bad arguments");
   if (units <= 0) units = pylon_compute_units();
   PYLON_REQUIRE(units > 0, "gemm_wide_parts_plan: no device to take the number of compute units from");
-  double least;
-  gw_choose(M, N, K, false, units, &least);
-  int first, rest;
-  if (const int ahead = gw_split(M, N, K, false, units, least, &first, &rest)) {
-    double left;
-    gw_choose(M, N - ahead, K, false, units, &left);
-    least = gw_time_us(kTiles[first], M, ahead, K, false, units) + left + GW_SECOND_US;
-  }
+  double least = gw_launches(M, N, K, false, units).us;
   *parts = 1, *tile = -1;
   for (int n = 2; n <= GW_MOST_PARTS && n * GW_LEAST_CHUNKS <= K / GW_CHUNK; ++n)
     for (int i = 0; i < kTileCount; ++i) {
@@ -600,18 +612,14 @@ extern "C" int pylon_gemm_wide(void* out, const void* x, const void* w, int M, i
                 GW_EXACT_ROWS);
   PYLON_REQUIRE(static_cast<long long>((M + 63) / 64) * ((N + 31) / 32) < (1ll << 30), "gemm_wide: too many tiles for one launch");
   if (M == 0) return 0;
-  int ahead = 0;  // columns of a launch of its own
+  int ahead = 0;
   if (tile < 0) {
     const int units = pylon_compute_units();
     PYLON_REQUIRE(units > 0, "gemm_wide: the device's number of compute units is unknown");
-    double us;
-    tile = gw_choose(M, N, K, gated, units, &us);
-    int first, rest;
-    ahead = gw_split(M, N, K, gated, units, us, &first, &rest);
-    if (ahead > 0) {
-      gw_launch(first, out, x, w, GwShape{M, ahead, K, 0, 0, 0, ldx, ldw, ldo, N, 1, 0, alpha, offset, limit, epilogue}, stream);
-      tile = rest;
-    }
+    const GwLaunches found = gw_launches(M, N, K, gated, units);
+    ahead = found.ahead, tile = found.rest;
+    if (ahead > 0)
+      gw_launch(found.first, out, x, w, GwShape{M, ahead, K, 0, 0, 0, ldx, ldw, ldo, N, 1, 0, alpha, offset, limit, epilogue}, stream);
   }
   gw_launch(tile, static_cast<uint16_t*>(out) + ahead, x, static_cast<const uint16_t*>(w) + ahead * ldw,
             GwShape{M, N - ahead, K, 0, 0, 0, ldx, ldw, ldo, N, 1, 0, alpha, offset, limit, epilogue}, stream);

@@ -64,6 +64,7 @@ _SIGNATURES = {
     "pylon_gemm_rows_shape": [I, I, I, I, I, I, I, I, P],
     "pylon_gemm_wide": [P, P, P, I, I, I, L, L, L, I, F, F, F, I, P],
     "pylon_gemm_wide_plan": [I, I, I, I, I, P, P],
+    "pylon_gemm_wide_launches": [I, I, I, I, I, P, P, P, P],
     "pylon_gemm_wide_parts": [P, P, P, I, I, I, L, L, I, I, P],
     "pylon_gemm_wide_parts_plan": [I, I, I, I, P, P, P],
     "pylon_gemm_f32_plan": [I, I, I, P],

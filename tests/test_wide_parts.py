@@ -1,5 +1,6 @@
 """Products of prompt portions with K cut into ranges, and projections of long portions: the rules, and what the parts'
 entry points launch for them."""
+import ctypes
 import warnings
 
 import pytest
@@ -7,7 +8,7 @@ import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 
 from pylon_amd.engine import layer_run
-from pylon_amd.kernels import ops, plan
+from pylon_amd.kernels import library, ops, plan
 
 
 @pytest.mark.parametrize("rows", [129, 300, 512, 513, 640, 1024, 1500, 2048, 2112])
@@ -30,6 +31,36 @@ def test_deep_matrices_are_cut_and_full_launches_are_not():
                                              (131, 4096, 4096, False)])
 def test_full_rounds_of_small_tiles_are_cut_and_small_products_are_not(rows, n, k, cut):
     assert (ops.wide_parts(rows, n, k, 256)[0] > 1) is cut
+
+
+def launches(rows, n, k, gated):
+    """(columns of the first of two launches or 0, its tile, the tile of the others)"""
+    (ahead, first, rest), us = (ctypes.c_int() for _ in range(3)), ctypes.c_float()
+    call = library.load().pylon_gemm_wide_launches
+    assert call(rows, n, k, int(gated), 256, *map(ctypes.byref, (ahead, first, rest, us))) == 0
+    return ahead.value, first.value, rest.value, us.value
+
+
+# gate/up of 4B, 8B and 32B sizes, the sizes whose results are compared on the device, and some that stay one launch
+@pytest.mark.parametrize("rows, n, k, gated, ahead", [
+    (2048, 9728, 2560, True, 8192), (2096, 12288, 4096, True, 10880), (1000, 25600, 5120, True, 24576),
+    (1000, 9732, 832, True, 6144), (2048, 9732, 384, True, 8192), (1000, 16516, 832, False, 16384),
+    (2040, 8368, 832, False, 8192), (512, 25600, 5120, True, 0), (2048, 12288, 4096, True, 0), (2040, 5124, 320, False, 0)])
+def test_whole_rounds_in_a_launch_of_their_own(rows, n, k, gated, ahead):
+    columns, first, rest, us = launches(rows, n, k, gated)
+    assert columns == ahead and (first < 0) == (ahead == 0)
+    tile, alone = ctypes.c_int(), ctypes.c_float()
+    assert library.load().pylon_gemm_wide_plan(rows, n, k, int(gated), 256, ctypes.byref(tile), ctypes.byref(alone)) == 0
+    assert us < alone.value if ahead else (us, rest) == (alone.value, tile.value)  # what one launch of one tile takes
+
+
+def test_launches_are_asked_for_products_that_there_are():
+    place = ctypes.byref(ctypes.c_int())
+    time = ctypes.byref(ctypes.c_float())
+    call = library.load().pylon_gemm_wide_launches
+    assert call(100, 64, 64, 0, 256, place, place, place, time) == 0
+    assert call(0, 64, 64, 0, 256, place, place, place, time) != 0 and call(100, 64, 32, 0, 256, place, place, place, time) != 0
+    assert call(100, 64, 64, 0, 256, None, place, place, time) != 0
 
 
 # either side of whole rounds of 256 x 256 tiles (216 of 256 are five sixths, 192 are not), of the depth and of the rows

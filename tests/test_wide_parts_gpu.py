@@ -1,4 +1,5 @@
 """The tiled bfloat16 product's float sums of ranges of K, its tiles of 160 and 192 columns, and its launches in two."""
+import ctypes
 
 import pytest
 import torch
@@ -56,11 +57,18 @@ def test_tiles_of_160_and_192_columns(ops, tile):
             ops.gemm_wide(x, w, epilogue="silu", tile=tile)
 
 
-# sizes whose rounds are a launch of their own, their last columns another; the last tile of either ragged
-@pytest.mark.parametrize("m, n, k, epilogue", [
-    (1000, 9728, 256, "silu"), (2048, 9732, 256, "capped"), (1000, 10244, 320, "none"), (2040, 5124, 320, "relu2")])
-def test_launches_in_two(ops, m, n, k, epilogue):
+# whole rounds in a launch of their own, the other columns, the last tile of them ragged, in another (whose up rows are as far
+# from its gate rows as the whole matrix's); rows of whole tiles and ragged ones
+@pytest.mark.parametrize("m, n, k, epilogue, ahead", [
+    (1000, 9732, 832, "silu", 6144), (2048, 9732, 384, "capped", 8192), (1000, 16516, 832, "none", 16384),
+    (2040, 8368, 832, "relu2", 8192)])
+def test_launches_in_two(ops, m, n, k, epilogue, ahead):
+    from pylon_amd.kernels import library
+
     gated = epilogue in ("silu", "capped")
+    (columns, first, rest), us = (ctypes.c_int() for _ in range(3)), ctypes.c_float()
+    assert library.load().pylon_gemm_wide_launches(m, n, k, int(gated), 0, *map(ctypes.byref, (columns, first, rest, us))) == 0
+    assert columns.value == ahead and (n - ahead) % TILES[rest.value][1] != 0
     x, w = draw(1, m, k), draw(2, 2 * n if gated else n, k, 64) * 0.2
     got = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
     options = dict(epilogue=epilogue, alpha=1.702, offset=1.0, limit=7.0)
