@@ -57,16 +57,23 @@ def test_a_layer_that_borrows_a_cache_is_not():
     (1920, 1536, 512, 5120), (5120, 2048, 2056, 4104)])
 @pytest.mark.parametrize("apart", [0, 64])
 def test_the_products_are_those_of_their_entry_points(monkeypatch, qkv, context, width, ff, apart):
-    """Where a step's layers are launched by one call, (ranges of K, column tiles) of every product, (0, 0) for the tiled
-    kernel, are what the entry point that the part calls launches."""
+    """Where a step's layers are launched by one call, (ranges of K, column tiles) of every product, (ranges, -1 less the
+    tile) for ranges of the tiled kernel, (0, 0) for it uncut, are what the entry point that the part calls launches."""
     launched, bf16 = [], torch.bfloat16
     monkeypatch.setattr(ops, "_raw_device", lambda: 0)
     monkeypatch.setattr(ops, "_stream", lambda: 0)
     monkeypatch.setattr(ops, "_watched", lambda x, weight: False)
     monkeypatch.setattr(ops, "_dev", lambda t, name, dtype=None: 0)
     monkeypatch.setattr(ops._lib, "compute_units", lambda: 256)
-    monkeypatch.setattr(ops._lib, "call", lambda name, *args: launched.append(
-        (args[10], args[12]) if name == "pylon_gemm_rows" else (0, 0) if name == "pylon_gemm_wide" else None))
+    plan_of = ops._lib.call
+
+    def call(name, *args):
+        if name == "pylon_gemm_wide_parts_plan":  # on the host
+            return plan_of(name, *args)
+        launched.append((args[10], args[12]) if name == "pylon_gemm_rows" else (0, 0) if name == "pylon_gemm_wide"
+                        else (args[8], -1 - args[9]) if name == "pylon_gemm_wide_parts" else None)
+
+    monkeypatch.setattr(ops._lib, "call", call)
     monkeypatch.setattr(torch.nn.functional, "linear", lambda x, w: launched.append(None) or x.new_empty(x.shape[0], w.shape[0]))
     monkeypatch.setattr(ops, "_library_float", lambda x, w, out=None: launched.append(None) or x.new_empty(
         x.shape[0], w.shape[0], dtype=torch.float32))
@@ -82,13 +89,14 @@ def test_the_products_are_those_of_their_entry_points(monkeypatch, qkv, context,
 
         for rows in (1, 2, 16, 17, 31, 32, 33, 48, 49, 64, 65, 100, 128, 129, 192, 193, 256, 300, 384, 385, 511, 512):
             asked = (layer_run._projection(rows, qkv, width, width + apart, 256),
-                     layer_run._residual(rows, width, context, context + apart, 256),
+                     layer_run._into_residual(rows, width, context, context + apart, 256),
                      layer_run._gated(rows, 2 * ff, width, width + apart),
-                     layer_run._residual(rows, width, ff, ff + apart, 256))
-            made = (choice(ops.linear, rows, qkv, width), choice(ops.linear_for_residual, rows, width, context, out_dtype=bf16),
+                     layer_run._into_residual(rows, width, ff, ff + apart, 256))
+            made = (choice(ops.linear_of_portion, rows, qkv, width, out_dtype=bf16),
+                    choice(ops.linear_into_residual, rows, width, context, out_dtype=bf16),
                     choice(ops.linear_glu, rows, 2 * ff, width, out_dtype=bf16),
-                    choice(ops.linear_for_residual, rows, width, ff, out_dtype=bf16))
+                    choice(ops.linear_into_residual, rows, width, ff, out_dtype=bf16))
             for name, mine, theirs in zip(("qkv", "out", "gate/up", "down"), asked, made):
                 assert mine == theirs, (rows, name)  # None: the library's, or the skinny kernel's
-                taken.add(None if mine is None else mine[0] > 0)
-    assert taken >= {True} and len(taken) > 1
+                taken.add(None if mine is None else (mine[0] > 0) + (mine[1] < 0))
+    assert taken >= {1, 2}  # ranges of the rows kernel and of the tiled one

@@ -1,6 +1,6 @@
 """Every matrix product a step of the published Qwen3 dense sizes runs, at its real size,
-through the dispatchers the parts call (``ops.linear``, ``ops.linear_for_residual``,
-``ops.linear_glu``), against a float64 product: which kernel the plan picks for the case,
+through the dispatchers the parts call (``ops.linear``, ``ops.linear_of_portion``,
+``ops.linear_into_residual``, ``ops.linear_glu``), against a float64 product: which kernel the plan picks for the case,
 how that kernel is laid over the chip, and the numbers.
 
 The vocabulary head is /root/reference/src/pylon/model/model.py:140-144, q/k/v and the out
@@ -15,21 +15,21 @@ units, unless that would make it re-read more rows of x than it streams rows of 
 product    1, 8, 16 rows             17, 48, 64 rows                        130 rows
 =========  ========================  =====================================  ===================
 4b qkv     rows CT1 2w 256x1 c24     rows CT1 up to 48 rows, then library   gemm_wide
-4b out     rows CT1 4w 64x4 c40      rows CT1 4w 64x4 c40 at 17 rows,       gemm_wide
+4b out     rows CT1 4w 64x4 c40      rows CT1 4w 64x4 c40 at 17 rows,       gemm_wide, 2 ranges
                                      40x4 c64 at 48 and 64
 4b gate/up rows GLU 4w 256x1 c38     rows GLU 4w 256x1 c38                  gemm_wide, silu
-4b down    rows CT1 4w 64x4 c40      rows CT2 4w 32x8 c80                   gemm_wide
+4b down    rows CT1 4w 64x4 c40      rows CT2 4w 32x8 c80                   gemm_wide, 2 ranges
 4b head    rows CT2 4w 1277x1 c119   rows CT2 4w 1187x1 c128                library, float32
 8b qkv     rows CT1 2w 256x1 c24     library                                gemm_wide
 8b out     rows CT1 4w 64x4 c64      rows CT1 4w 64x4 c64                   gemm_wide
 8b gate/up skinny GLU                rows GLU 4w 256x1 c48                  gemm_wide, silu
-8b down    rows CT1 4w 64x4 c64      rows CT2 4w 32x8 c128                  gemm_wide
+8b down    rows CT1 4w 64x4 c64      rows CT2 4w 32x8 c128                  gemm_wide, 4 ranges
 8b head    rows CT1 4w 2533x1 c60    rows CT1 4w 2374x1 c64 at 17 rows,     library, float32
                                      library float32 at 48 and 64
 32b qkv    rows CT1 4w 256x1 c40     rows CT1 up to 48 rows, then library   gemm_wide
-32b out    rows CT2 4w 64x4 c80      rows CT2 4w 64x4 c80                   gemm_wide
+32b out    rows CT2 4w 64x4 c80      rows CT2 4w 64x4 c80                   gemm_wide, 4 ranges
 32b g/u    rows GLU 4w 512x1 c50     rows GLU 4w 512x1 c50                  gemm_wide, silu
-32b down   rows CT2 4w 64x4 c80      rows CT2 4w 64x4 c80                   gemm_wide
+32b down   rows CT2 4w 64x4 c80      rows CT2 4w 64x4 c80                   gemm_wide, 4 ranges
 32b head   rows CT2 4w 1277x1 c119   rows CT2 4w 1187x1 c128                library, float32
 =========  ========================  =====================================  ===================
 
@@ -41,6 +41,9 @@ as above.
 65 and 128 rows: the rows of x go as two halves, each to workgroups of its own, with the choices
 of 64 rows, for out, down and the q/k/v that a consumer adds; gate/up, the head and a plain q/k/v
 go where they go at 130 rows.
+
+Portions: out and down in one to four ranges of K (``PARTS``), q/k/v of more than 512 rows by the rule
+of projections (``PORTIONS``).
 """
 import ctypes
 import zlib
@@ -84,6 +87,12 @@ EXPECT = {
 EXPECT_SUMMED = {"4b": ((R, 2, 1, (4, 128, 48)), (R, 4, 2, (4, 64, 96))),
                  "8b": ((R, 2, 1, (4, 128, 48)), (R, 4, 2, (4, 64, 96))),
                  "32b": (None, (R, 2, 2, (4, 128, 80)))}
+
+# ranges of K of a product into the residual stream, by rows
+PARTS = {("4b", "out"): {130: 2, 400: 4, 640: 3, 900: 2, 2111: 1}, ("4b", "down"): {130: 2, 400: 4, 640: 3, 900: 4, 2111: 2},
+         ("8b", "out"): {130: 1, 400: 2, 640: 2, 900: 1, 2111: 1}, ("8b", "down"): {130: 4, 400: 4, 640: 4, 900: 3, 2111: 1},
+         ("32b", "out"): {130: 4, 400: 4, 640: 3, 900: 2, 2111: 1}, ("32b", "down"): {130: 4, 400: 4, 640: 3, 900: 3, 2111: 1}}
+PORTIONS = (513, 2048, 2111)  # rows of a projection
 
 
 @pytest.fixture(scope="module")
@@ -135,7 +144,8 @@ def test_a_product_at_its_real_size(ops, model, product):
     n, k = shape_of(model, product)
     gen = torch.Generator(device=DEV).manual_seed(zlib.crc32(f"{model}/{product}".encode()))
     w = (torch.randn((n, k), generator=gen, device=DEV) * 0.02).to(torch.bfloat16)
-    x = torch.randn((max(ROWS), k), generator=gen, device=DEV).to(torch.bfloat16)
+    every = ROWS + tuple(PARTS.get((model, product), ())) + (PORTIONS if product == "qkv" else ())
+    x = torch.randn((max(every), k), generator=gen, device=DEV).to(torch.bfloat16)
     want = torch.mm(x.double(), w.double().t())
     if product == "gate_up":
         g, u = want[:, : n // 2], want[:, n // 2:]
@@ -145,21 +155,23 @@ def test_a_product_at_its_real_size(ops, model, product):
     few, many = EXPECT[(model, product)]
     units = library.compute_units()
     assert units == 256  # the expectations above are those of an MI355X
-    for rows in ROWS:
+    for rows in sorted(set(every)):
         if rows <= 64:
             expected = few if rows <= 16 else (many[rows] if isinstance(many, dict) else many)
             assert chosen(model, product, rows, units) == expected, (model, product, rows)
         xr = x[:rows].contiguous()
         if product in ("out", "down"):
-            got = ops.linear_for_residual(xr, w, out_dtype=torch.bfloat16)
+            got = ops.linear_into_residual(xr, w, out_dtype=torch.bfloat16)
             if rows <= 128:  # float32 sums, never rounded: whole, or K cut into parts
                 assert got.dtype == torch.float32
                 if rows > 64:  # two halves of the rows, the choices of 64 rows
                     many64 = many[64] if isinstance(many, dict) else many
                     assert chosen(model, product, rows, units)[:3] == many64[:3], (model, product, rows)
-                got = got.sum(0, dtype=torch.float64) if got.dim() == 3 else got
-            else:
-                assert got.dtype == torch.bfloat16
+            else:  # the same of ranges of K; uncut it is rounded once
+                parts = PARTS[model, product][rows]
+                assert got.shape[:-2] == ((parts,) if parts > 1 else ()), (model, product, rows)
+                assert got.dtype == (torch.float32 if parts > 1 else torch.bfloat16)
+            got = got.sum(0, dtype=torch.float64) if got.dim() == 3 else got
         elif product == "gate_up":
             got = ops.linear_glu(xr, w, out_dtype=torch.bfloat16)
             assert got.dtype == torch.bfloat16
@@ -184,6 +196,9 @@ def test_a_product_at_its_real_size(ops, model, product):
                 assert np.abs(total - want[:rows]).max() <= 2e-6 * np.abs(want[:rows]).max(), (model, rows)
             else:
                 assert torch.equal(later, got)
+            portion = ops.linear_of_portion(xr, w, out_dtype=torch.bfloat16)
+            assert rows > 512 or torch.equal(portion, got)
+            got = portion
         ref = want[:rows]
         assert got.shape == ref.shape, (model, product, rows, tuple(got.shape))
         scale = np.abs(ref).max()
