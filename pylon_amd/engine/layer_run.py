@@ -70,7 +70,9 @@ def _into_residual(rows: int, n: int, k: int, stride: int, units: int) -> Option
     """The same of :func:`ops.linear_into_residual`; (parts, -1 - tile) for :func:`ops.gemm_wide_parts`."""
     if rows > plan.SPLIT_ROWS and ops.wide_sizes_ok(rows, n, k, k, stride):
         parts, tile = ops.wide_parts(rows, n, k, units)
-        return (parts, -1 - tile) if parts > 1 else (0, 0)
+        if parts > 1:
+            return parts, -1 - tile
+        return None if plan.library_fills_rounds(rows, n, k, units=units) else (0, 0)
     return _residual(rows, n, k, stride, units)
 
 

@@ -9,7 +9,7 @@ from torch._subclasses.fake_tensor import FakeTensorMode
 from pylon_amd.config.registry import resolve
 from pylon_amd.engine import layer_run
 from pylon_amd.engine.layer_run import alike
-from pylon_amd.kernels import ops
+from pylon_amd.kernels import ops, plan
 
 CONFIG = {"architectures": ["Qwen3ForCausalLM"], "model_type": "qwen3", "hidden_act": "silu", "num_hidden_layers": 3,
           "hidden_size": 128, "num_attention_heads": 2, "num_key_value_heads": 1, "head_dim": 64, "intermediate_size": 256,
@@ -48,6 +48,12 @@ def test_others_are_not(change):
 def test_a_layer_that_borrows_a_cache_is_not():
     plain = spec()
     assert not alike(replace(plain, schedule=(*plain.schedule[:2], replace(plain.schedule[2], cache=1))))
+
+
+def test_portions_by_other_rules_are_left_to_the_parts():
+    assert layer_run.MOST_TOKENS <= plan.PORTION_ROWS  # beyond, projections have a rule of their own
+    assert layer_run._into_residual(2048, 8192, 8192, 8192, 256) is None  # the library's
+    assert layer_run._into_residual(2049, 8192, 8192, 8192, 256) == (0, 0)
 
 
 # (q/k/v, context, width, feed-forward): 4B, 8B and 32B sizes, narrow layers, a narrow and deep one, one whose rows are of no
