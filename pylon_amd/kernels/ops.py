@@ -1641,9 +1641,9 @@ def linear_into_residual(x: torch.Tensor, weight: torch.Tensor, *, out_dtype: to
     kernel's wherever that takes it, with K cut into ranges where the uncut launch has fewer tiles than the device has
     units, or small ones (:func:`wide_parts`): then float32 partial sums ``[parts, M, N]``, which the consumer adds.  Uncut
     and with a bfloat16 result it is the library's where :func:`plan.library_fills_rounds`.
-    (2560 x 9728 at 192, 640, 1200 and 2048 rows, with the norm's reading of the parts: 25, 42, 61 and 88 us, where
-    the uncut kernel or the library took 42, 61, 87 and 105; 5120 x 25600 at 256, 640 and 1500: 93, 149 and 283
-    against 265, 240 and 341.)  With a float32 ``out_dtype`` the sums come unrounded also where K is not cut."""
+    (Product and norm, us: 2560 x 9728 at 160, 640, 1280 and 2048 rows 26, 48, 69 and 98, where the uncut kernel or the
+    library took 42, 68, 100 and 114; 5120 x 25600 at 256, 640 and 1536 94, 156 and 302 against 273, 248 and 371.)
+    With a float32 ``out_dtype`` the sums come unrounded also where K is not cut."""
     if (x.dim() == 2 and x.shape[0] > SPLIT_ROWS and out_dtype in (torch.bfloat16, torch.float32) and not _watched(x, weight)
             and _wide_ok(x, weight)):
         parts, tile = wide_parts(x.shape[0], *weight.shape, _lib.compute_units())

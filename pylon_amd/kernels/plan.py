@@ -4,7 +4,8 @@ Pure functions of the shape: they touch no tensor and run anywhere, so the choic
 tested without a GPU.  Every figure below was measured on one MI355X, under a graph, over 36
 different matrices in turn (so that none came from a cache).  Those of the rows kernel are from before its loads
 of w were marked as read once: it takes 4 to 16 % less since (2560 x 9728 at 8 rows 11.2 -> 10.1 us, 2 x 9728 x 2560 20.5
--> 18.1, 6144 x 4096 12.9 -> 11.0; two halves of the rows 2 to 5 %), which moves no line against it.
+-> 18.1, 6144 x 4096 12.9 -> 11.0; two halves of the rows 2 to 5 %).  No line was drawn again for that; where one was known
+to lie too far on the other kernel's side already, the text beside it says so.
 
 Three kernels take part.  ``rows`` (``gemm_rows``): both operands go through LDS in whole
 256-byte row segments, the rows of x are shared by a workgroup, K may be cut over workgroups.
@@ -204,8 +205,11 @@ def rows_match_library(rows: int, n: int, k: int) -> bool:
 
 def wide_beats_library(rows: int, n: int, k: int, units: int = UNITS) -> bool:
     """Whether a product of more than 64 rows without an activation behind it goes to the engine's own
-    tiled kernel (``gemm_wide``) or to the library's.  The own kernel's tile is chosen so that the launch fills
-    whole rounds of the compute units; for many rows the library's 256 x 256 tile is the faster main loop where
+    tiled kernel (``gemm_wide``) or to the library's: a projection of up to :data:`PORTION_ROWS` rows, a longer portion's where
+    :func:`portion_beats_library` has no line of its own, and whatever else :func:`ops.linear` is given.  (Out and down of more
+    than 128 rows have :func:`ops.wide_parts` and come here no more; the lines of matrices at least as deep as wide were
+    read off them, uncut and in the tiles of then, and hold for other products of such sizes.)  The own kernel's tile is chosen so
+    that the launch fills whole rounds of the compute units; for many rows the library's 256 x 256 tile is the faster main loop where
     a matrix is wide enough for it.  A layer of a prompt step in us, library against own kernel (both with
     gate/up in the own kernel's epilogue):
 
@@ -217,7 +221,7 @@ def wide_beats_library(rows: int, n: int, k: int, units: int = UNITS) -> bool:
     530, 569; 8B at 160, 1024, 1800, 2048 270, 502, 746, 794 against 265, 502, 759, 809; 32B at 2048 1829 against
     1902.
     A matrix at least as deep as wide has few tiles, and between one 64 x 64 tile a unit and a few of them the
-    own kernel, which does not cut K, leaves units waiting: out and down of 4B at 384, 450, 512, 700 tokens 211,
+    own kernel, uncut, leaves units waiting: out and down of 4B at 384, 450, 512, 700 tokens 211,
     231, 234, 280 against 206, 245, 270, 297; of 8B at 260, 384, 512, 640, 700 287, 310, 345, 408, 432 against 310,
     352, 365, 429, 438; of 32B at 260, 384, 450, 700 563, 609, 767, 927 against 584, 655, 693, 845.
     Full portions of a narrow matrix: one round of 128 x 192 tiles that leaves units idle, where the library has a
