@@ -112,9 +112,8 @@ def test_rmsnorm_and_fused_residual(ops, dtype, dim):
 @pytest.mark.parametrize("dim", [80, 2560 + 16, 5120 + 8, 8192])
 @pytest.mark.parametrize("delta_dtype", DTYPES)
 def test_residual_norm_of_many_rows_has_the_bits_of_few(ops, dim, delta_dtype):
-    """From 512 rows on another kernel takes the fused residual norm (two rows a workgroup):
-    it forms every row's sums in the order of the kernel for few rows, so a request's values do
-    not depend on how many tokens share its step."""
+    """One kernel takes the fused residual norm of any number of rows, a row a workgroup: a request's values
+    do not depend on how many tokens share its step, and are what 64 bits give."""
     eps, rows = 1e-6, 515
     x = rnd((rows, dim), 60, torch.float32, 2.0)
     delta = rnd((rows, dim), 61, delta_dtype)
