@@ -157,13 +157,14 @@ extern thread_local char pylon_error_text[512];
     return 0;                                                                         \
   } while (0)
 
-// Compute units of the current device (0 if there is none); asked of the runtime once per device.
 // The cache policy of a buffer load whose line nobody reads again (the nt bit).  A unit has some 115 lines on their way from
 // memory at any time, so a stream's rate is what one line's way allows: so marked 6.06 -> 6.90 TB/s from memory (319 MB,
-// three in turn), 6.85 -> 7.54 from the memory-side cache (84 MB).  Lines that other workgroups read too are lost
-// to them (prompt products 15 to 25 % slower).
+// three in turn), 6.85 -> 7.54 from the memory-side cache (84 MB).  Products whose matrices all stay in that cache (256 MB) gain
+// or lose by it: 60 to 200 MB of 1,024-wide ones 4 to 10 % less time, of 2,560-wide ones 2 to 10 % more (65 to 128 rows, whose
+// halves read w twice, up to 15).  Lines that other workgroups read too are lost to them (prompt products 15 to 25 % slower).
 #define PYLON_STREAMED 2
 
+// Compute units of the current device (0 if there is none); asked of the runtime once per device.
 extern "C" int pylon_compute_units();
 
 static inline bool pylon_valid_dtype(int d) { return d == PYLON_F32 || d == PYLON_BF16; }
