@@ -112,9 +112,9 @@ __global__ __launch_bounds__(512) void rmsnorm_kernel(TO* __restrict__ out, TX* 
 // Launches in a row, four parts, 8 rows of 2,560, 4,096 and 5,120: 3.8, 4.2 and 4.2 us -> 2.5, 2.7 and 3.2 (of an
 // empty kernel's 1.5); 48 rows 4.3, 4.9, 4.7 -> 2.8, 3.3, 3.5.
 // For many rows, too (prompt portions; a workgroup a row): one that took two rows, all loads first, was the quicker one beside an
-// earlier form of this.  512, 1,024 and 2,048 rows of a bfloat16 product, that and this, us: of 2,560 6.0, 7.4, 10.8 and 4.1, 6.0,
-// 10.5; of 4,096 7.4, 9.6, 18.1 and 5.3, 9.0, 19.2; of 5,120 7.4, 10.7, 27.7 and 6.1, 10.8, 23.3; of 8,192 8.9, 19.0, 42.9 and 9.5,
-// 20.3, 37.0 (two processes' figures of one size differ by up to 10 %).
+// earlier form of this.  512, 1,024 and 2,048 rows of a bfloat16 product, that and this, us: of 2,560 6.0, 7.5, 10.6 and 3.9, 6.0,
+// 10.3; of 4,096 7.5, 9.6, 18.1 and 5.3, 8.3, 18.2; of 5,120 7.4, 10.9, 27.8 and 6.1, 10.5, 22.6; of 8,192 9.0, 19.1, 42.9 and 8.4,
+// 18.5, 34.2 (2,048 rows of 8,192: 5.1 TB/s).
 // Float residual rows of a multiple of 4 elements, at most 4 NV a thread.  parts_apart: fours of elements from one
 // part to the next; sizes: dim, from bit 16 on the number of parts (0: no delta), from bit 24 on whether the sum is
 // stored.  LOOSE: for rows that begin anywhere (8 rows of 2,560, four parts, 8.2 us element by element, 3.0 so).

@@ -100,7 +100,7 @@ __device__ __forceinline__ float row_block_sum(float v, float* scratch) {
 }
 
 // d[n] = the sum over `parts` rows, `fours` fours of elements apart, of elements 4 (threadIdx.x + n THREADS) .. + 3, in
-// order; of 1, 2, 4 and 8 rows all loads are sent before the first sum.
+// order; of 1, 2, 4 and 8 rows (bfloat16: 1 and 2) all loads are sent before the first sum.
 template <typename TD, int NV, int THREADS, bool LOOSE = false>
 __device__ __forceinline__ void row_sum_parts(float4 (&d)[NV], const TD* row, int dim, int parts, unsigned fours) {
   auto part = [&](int p, float4* e) __attribute__((always_inline)) {
@@ -115,7 +115,10 @@ __device__ __forceinline__ void row_sum_parts(float4 (&d)[NV], const TD* row, in
     }
   };
   float4 e1[NV];
-  constexpr bool ROOM = THREADS <= 512;  // registers for them
+  // Registers for them.  Partial sums are float: with room for eight bfloat16 rows a residual norm of 6,148 to 8,192 elements
+  // holds 169 registers, one workgroup a unit, without it 80 and three (600, 1,024 and 2,048 rows of 8,192, a bfloat16 product, 11.7,
+  // 20.3 and 36.6 us -> 10.2, 18.5 and 34.2).
+  constexpr bool ROOM = THREADS <= 512 && sizeof(TD) == 4;
   if (ROOM && parts == 4) {
     float4 e2[NV], e3[NV];
     part(0, d); part(1, e1); part(2, e2); part(3, e3);

@@ -130,6 +130,24 @@ def test_residual_norm_of_many_rows_has_the_bits_of_few(ops, dim, delta_dtype):
             assert torch.equal(few, many[lo:hi]) and torch.equal(few_resid, many_resid[lo:hi])
 
 
+# as many parts as are sent for at once in one type or the other, and more; rows of one thread's fours up to four
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("dim", [80, 2560, 6144, 8192])
+def test_partial_sums_have_the_same_bits_in_either_type(ops, dim, parts):
+    """Parts are added in order, whatever is loaded ahead: bfloat16 parts and the same numbers in float."""
+    rows = 5
+    x, w = rnd((rows, dim), 63, torch.float32, 2.0).to(DEV), (1 + 0.3 * rnd((dim,), 64)).to(DEV)
+    delta = rnd((parts, rows, dim), 65, torch.bfloat16).to(DEV)
+    found = []
+    for d in (delta, delta.float()):
+        resid = x.clone()
+        found.append((ops.add_rmsnorm(resid, d, w, 1e-6, torch.bfloat16), resid))
+    assert torch.equal(found[0][0], found[1][0]) and torch.equal(found[0][1], found[1][1])
+    summed = f64(x) + f64(delta).sum(0)
+    # float32 sums of up to ten numbers: 2^-24 of a running sum each
+    assert np.abs(f64(found[0][1]) - summed).max() <= 10 * 2.0 ** -24 * np.abs(f64(delta)).sum(0).max() + 2.0 ** -23 * np.abs(summed).max()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_silu_gate(ops, dtype):
     gu = rnd((5, 2 * 176), 5, dtype, 3.0)
