@@ -419,6 +419,12 @@ static const GwTile kTiles[] = {
 #define GW_ROUND_US 3.5  // of a round: the first chunks' way to LDS, and the results' way out
 static const int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 
+// What a full round costs the smallest tile, which asks most of the way to the second-level caches, where these hold
+// w (nanoseconds a chunk, and the most bytes): 1,024 to 4,096 x 1,024 to 3,072 210 to 320 at 300 to 2,000 rows, 4,096 x 2,048 270 to 430,
+// from 2,560 x 4,096 on 400 to 490.
+#define GW_NEAR_NS 380
+#define GW_NEAR_BYTES 18000000
+
 // A float result of a part leaves late: its bytes, in us a MB.
 #define GW_STORE_US_MB 0.27
 
@@ -428,9 +434,11 @@ static double gw_time_us(const GwTile& t, int M, int N, int K, bool gated, int u
   const long long slots = static_cast<long long>(units) * t.per_unit;
   const long long rounds = tiles / slots, left = tiles - rounds * slots;
   const double chunks = 1e-3 * (K / GW_CHUNK) / parts;
-  const double last = left == 0 ? 0.0 : chunks * (left <= units ? t.alone_ns : t.full_ns) + GW_ROUND_US;
+  const bool near = t.rows == 64 && (gated ? 4ll : 2ll) * N * K <= GW_NEAR_BYTES;
+  const int full_ns = near ? GW_NEAR_NS : t.full_ns;
+  const double last = left == 0 ? 0.0 : chunks * (left <= units ? t.alone_ns : full_ns) + GW_ROUND_US;
   const double stored = parts == 1 ? 0.0 : GW_STORE_US_MB * 4e-6 * parts * M * N / (rounds + (left > 0));
-  return rounds * (chunks * t.full_ns + GW_ROUND_US) + last + stored;
+  return rounds * (chunks * full_ns + GW_ROUND_US) + last + stored;
 }
 
 static bool gw_takes(const GwTile& t, int M, bool gated) {
@@ -457,12 +465,16 @@ struct GwLaunches {
 };
 
 // One launch, or, where a last round would leave most units idle, the whole rounds of one tile in a launch of their own
-// and the columns that are left in a launch of the tile that suits them, where both are quicker.
+// and the columns that are left in a launch of the tile that suits them, where both take 2 % less than one.  (Measured, 183 products
+// that the model would split: where it gives less than 2 %, two launches take 1.006 of the time of one, where it gives 2 to 10 %
+// 0.98, beyond 0.91.)
 #define GW_SECOND_US 2.5
+#define GW_SECOND_SHARE 0.98
 static GwLaunches gw_launches(int M, int N, int K, bool gated, int units) {
   GwLaunches best{0, -1, 0, 0.0};
   best.rest = gw_choose(M, N, K, gated, units, &best.us);
   if (M <= 4 * GW_EXACT_ROWS) return best;
+  double least = GW_SECOND_SHARE * best.us;
   for (int i = 0; i < kTileCount; ++i) {
     const GwTile& t = kTiles[i];
     if (!gw_takes(t, M, gated)) continue;
@@ -472,10 +484,10 @@ static GwLaunches gw_launches(int M, int N, int K, bool gated, int units) {
     const long long n = rounds * slots / m_tiles * cols;
     if (rounds == 0 || n >= N) continue;
     const double whole = gw_time_us(t, M, static_cast<int>(n), K, gated, units) + GW_SECOND_US;
-    if (whole >= best.us) continue;  // what is left takes some time too
+    if (whole >= least) continue;  // what is left takes some time too
     double left;
     const int rest = gw_choose(M, N - static_cast<int>(n), K, gated, units, &left);
-    if (whole + left < best.us) best = GwLaunches{static_cast<int>(n), i, rest, whole + left};
+    if (whole + left < least) least = whole + left, best = GwLaunches{static_cast<int>(n), i, rest, least};
   }
   return best;
 }
@@ -505,12 +517,11 @@ extern "C" int pylon_gemm_wide_launches(int M, int N, int K, int gated, int unit
 
 // Ranges of K for a product into the residual stream, with the tile, or one range and tile -1 (pylon_gemm_wide): the
 // quickest with what the residual norm pays for reading float sums of every range instead of one bfloat16 result, by
-// their size and each (three, which it reads one after the other, cost what four do).  Product and norm over 432 sizes of 2,560
-// to 5,120 columns and 129 to 2,112 rows take 0.79 of the time of the uncut kernel or the library, whichever it was before
-// (one of them 1.04, the others no more than 1.01); with 380 ns for a full round of the smallest tile and nothing for each range
-// 4096 x 4096 at 131, 435 and 512 rows took 21, 39 and 40 us against 20, 34 and 37, where one, two and two ranges take 20, 29 and 32.
+// their size.  Product and norm over 1,096 sizes of 1,024 to 5,120 columns, K of 1,024 to 25,600 and 129 to 2,111 rows take 0.81 of the
+// time of the uncut kernel or the library, whichever it was before (1.03 to 1.06 in ten of them); with 380 ns for
+// every full round of the smallest tile 4096 x 4096 at 435 and 512 rows and 2560 x 4096 at 768 took 39, 40 and 37 us against
+// 34, 37 and 35, where two ranges take 29, 32 and 30.
 #define GW_ADD_US_MB 0.2
-#define GW_ADD_US_EACH 0.5
 #define GW_MOST_PARTS 4
 #define GW_LEAST_CHUNKS 8  // of a range
 extern "C" int pylon_gemm_wide_parts_plan(int M, int N, int K, int units, int* parts, int* tile, float* us) {
@@ -521,8 +532,7 @@ extern "C" int pylon_gemm_wide_parts_plan(int M, int N, int K, int units, int* p
   *parts = 1, *tile = -1;
   for (int n = 2; n <= GW_MOST_PARTS && n * GW_LEAST_CHUNKS <= K / GW_CHUNK; ++n)
     for (int i = 0; i < kTileCount; ++i) {
-      const double now = gw_time_us(kTiles[i], M, N, K, false, units, n) + GW_ADD_US_MB * 1e-6 * (4 * n - 2) * M * N +
-                         GW_ADD_US_EACH * (n == 3 ? 4 : n);
+      const double now = gw_time_us(kTiles[i], M, N, K, false, units, n) + GW_ADD_US_MB * 1e-6 * (4 * n - 2) * M * N;
       if (now < least) least = now, *parts = n, *tile = i;
     }
   *us = static_cast<float>(least);

@@ -21,7 +21,7 @@ product    1, 8, 16 rows             17, 48, 64 rows                        130 
 4b down    rows CT1 4w 64x4 c40      rows CT2 4w 32x8 c80                   gemm_wide, 2 ranges
 4b head    rows CT2 4w 1277x1 c119   rows CT2 4w 1187x1 c128                library, float32
 8b qkv     rows CT1 2w 256x1 c24     library                                gemm_wide
-8b out     rows CT1 4w 64x4 c64      rows CT1 4w 64x4 c64                   gemm_wide
+8b out     rows CT1 4w 64x4 c64      rows CT1 4w 64x4 c64                   gemm_wide, 4 ranges
 8b gate/up skinny GLU                rows GLU 4w 256x1 c48                  gemm_wide, silu
 8b down    rows CT1 4w 64x4 c64      rows CT2 4w 32x8 c128                  gemm_wide, 4 ranges
 8b head    rows CT1 4w 2533x1 c60    rows CT1 4w 2374x1 c64 at 17 rows,     library, float32
@@ -90,7 +90,7 @@ EXPECT_SUMMED = {"4b": ((R, 2, 1, (4, 128, 48)), (R, 4, 2, (4, 64, 96))),
 
 # ranges of K of a product into the residual stream, by rows
 PARTS = {("4b", "out"): {130: 2, 400: 4, 640: 3, 900: 2, 2111: 1}, ("4b", "down"): {130: 2, 400: 4, 640: 3, 900: 4, 2111: 2},
-         ("8b", "out"): {130: 1, 400: 2, 640: 2, 900: 1, 2111: 1}, ("8b", "down"): {130: 4, 400: 4, 640: 4, 900: 3, 2111: 1},
+         ("8b", "out"): {130: 4, 400: 2, 640: 2, 900: 1, 2111: 1}, ("8b", "down"): {130: 4, 400: 4, 640: 4, 900: 3, 2111: 1},
          ("32b", "out"): {130: 4, 400: 4, 640: 3, 900: 2, 2111: 1}, ("32b", "down"): {130: 4, 400: 4, 640: 3, 900: 3, 2111: 1}}
 PORTIONS = (513, 2048, 2111)  # rows of a projection
 

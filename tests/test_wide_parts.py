@@ -25,11 +25,11 @@ def test_deep_matrices_are_cut_and_full_launches_are_not():
 
 
 # us of product and norm uncut, in two, three and four ranges, and by the route before there were any: 768 rows 37.1, 30.2, 30.9,
-# 30.7 and 34.9; 435 rows 38.9, 28.7, 31.5, 31.4 and 33.6; 512 rows 39.7, 31.5, 33.8, 32.4 and 37.3; 131 rows 19.7, 22.4, 20.3, 21.2
-# and 20.1
+# 30.7 and 34.9; 435 rows 38.9, 28.7, 31.5, 31.4 and 33.6; 512 rows 39.7, 31.5, 33.8, 32.4 and 37.3; and a matrix that the
+# second-level caches hold, 335 rows 17.1, 18.7, 20.1, 22.2 and 20.9
 @pytest.mark.parametrize("rows, n, k, cut", [(768, 2560, 4096, True), (435, 4096, 4096, True), (512, 4096, 4096, True),
-                                             (131, 4096, 4096, False)])
-def test_full_rounds_of_small_tiles_are_cut_and_small_products_are_not(rows, n, k, cut):
+                                             (335, 4096, 2048, False), (1024, 2560, 9728, True), (440, 2048, 6144, True)])
+def test_full_rounds_of_small_tiles_are_cut_where_memory_holds_the_matrix(rows, n, k, cut):
     assert (ops.wide_parts(rows, n, k, 256)[0] > 1) is cut
 
 
@@ -44,14 +44,14 @@ def launches(rows, n, k, gated):
 # gate/up of 4B, 8B and 32B sizes, the sizes whose results are compared on the device, and some that stay one launch
 @pytest.mark.parametrize("rows, n, k, gated, ahead", [
     (2048, 9728, 2560, True, 8192), (2096, 12288, 4096, True, 10880), (1000, 25600, 5120, True, 24576),
-    (1000, 9732, 832, True, 6144), (2048, 9732, 384, True, 8192), (1000, 16516, 832, False, 16384),
+    (1000, 9732, 1280, True, 6144), (2048, 9732, 576, True, 8192), (1000, 16516, 832, False, 16384),
     (2040, 8368, 832, False, 8192), (512, 25600, 5120, True, 0), (2048, 12288, 4096, True, 0), (2040, 5124, 320, False, 0)])
 def test_whole_rounds_in_a_launch_of_their_own(rows, n, k, gated, ahead):
     columns, first, rest, us = launches(rows, n, k, gated)
     assert columns == ahead and (first < 0) == (ahead == 0)
     tile, alone = ctypes.c_int(), ctypes.c_float()
     assert library.load().pylon_gemm_wide_plan(rows, n, k, int(gated), 256, ctypes.byref(tile), ctypes.byref(alone)) == 0
-    assert us < alone.value if ahead else (us, rest) == (alone.value, tile.value)  # what one launch of one tile takes
+    assert us < 0.98 * alone.value if ahead else (us, rest) == (alone.value, tile.value)  # what one launch of one tile takes
 
 
 def test_launches_are_asked_for_products_that_there_are():

@@ -60,7 +60,7 @@ def test_tiles_of_160_and_192_columns(ops, tile):
 # whole rounds in a launch of their own, the other columns, the last tile of them ragged, in another (whose up rows are as far
 # from its gate rows as the whole matrix's); rows of whole tiles and ragged ones
 @pytest.mark.parametrize("m, n, k, epilogue, ahead", [
-    (1000, 9732, 832, "silu", 6144), (2048, 9732, 384, "capped", 8192), (1000, 16516, 832, "none", 16384),
+    (1000, 9732, 1280, "silu", 6144), (2048, 9732, 576, "capped", 8192), (1000, 16516, 832, "none", 16384),
     (2040, 8368, 832, "relu2", 8192)])
 def test_launches_in_two(ops, m, n, k, epilogue, ahead):
     from pylon_amd.kernels import library
